@@ -1,0 +1,209 @@
+"""CPU model of the bulge chase's message protocol (chase.hip, chase_kernel):
+sweeps run concurrently and hand each other the window of every step through
+slots that are doubled by the sweep's parity and hold EMPTY until a message
+element arrives.  Stores complete late and in random order; the only ordering
+the model grants is the kernel's: a step's sends are issued after the previous
+step's empties have completed.  Every interleaving must give the oracle's
+sequential result, no element may land in a slot that is not empty or be left
+behind in one that is loaded again, and without the start word or the ordering
+of empties before sends the model must fail."""
+import random
+
+import numpy as np
+import pytest
+
+from oracle import evd_oracle as O
+
+EMPTY = object()
+
+
+def _refl(x):
+    nrm = np.sqrt(x @ x)
+    if nrm > 0:
+        u = x / nrm
+        u[0] += 1.0 if x[0] >= 0 else -1.0
+        u /= np.sqrt(abs(u[0]))
+        return u, (-nrm if x[0] >= 0 else nrm)
+    return np.zeros_like(x), x[0]
+
+
+class Stale(Exception):
+    pass
+
+
+def _lens(n, b, p):
+    ln = min(b, n - p)
+    return ln, max(0, min(b, n - p - ln))
+
+
+def _window(n, b, p):
+    """The elements of a step's window that are loaded: ('S' | 'N', i, k)."""
+    ln, ln2 = _lens(n, b, p)
+    w = [("S", i, k) for i in range(ln) for k in range(ln)]
+    w += [("N", i, k) for i in range(ln2) for k in range(ln) if not (i == b - 1 and k < b - 1)]
+    return w
+
+
+def chase(Bd, b, seed, start_word=True, ordered=True, window=7):
+    n = Bd.shape[0]
+    rng = random.Random(seed)
+    nsw = n - 2
+    mem = {}  # (parity, slot | 'X', element) -> value; absent = EMPTY
+    for j in range(-(-n // b)):
+        p = 1 + j * b
+        if p < n:
+            ln, _ = _lens(n, b, p)
+            for what, i, k in _window(n, b, p):
+                r, c = (p + max(i, k), p + min(i, k)) if what == "S" else (p + ln + i, p + k)
+                mem[1, j, what, i, k] = Bd[r, c]
+    for i in range(min(b, n - 1)):
+        mem[1, "X", i] = Bd[1 + i, 0]
+    D, E, U = np.zeros(n), np.zeros(n - 1), np.zeros((n + b, n))
+    D[0] = Bd[0, 0]
+    started = set()
+
+    def flush(x, upto=None):
+        """Complete stores of sweep x: all empties up to step `upto`, or a random one."""
+        q = x["stores"]
+        if upto is None:
+            pick = [rng.randrange(len(q))] if q else []
+        else:
+            pick = [i for i, e in enumerate(q) if e[0] == "empty" and e[1] <= upto]
+        for i in reversed(pick):
+            kind, _, key, v = q.pop(i)
+            if kind == "empty":
+                mem.pop(key, None)
+            else:
+                if key in mem:
+                    raise Stale(f"{key} written twice")
+                mem[key] = v
+
+    def program(s):
+        """The sweep as a generator: yields None to be rescheduled."""
+        x = st[s]
+        rd, wr = (s + 1) % 2, s % 2
+        p = s + 1
+        ln, ln2 = _lens(n, b, p)
+        store = lambda kind, j, key, v=None: x["stores"].append((kind, j, key, v))
+        while start_word and s > 0 and s - 1 not in started:
+            yield
+        keys = [(rd, "X", i) for i in range(ln)]
+        got = {}
+        while len(got) < len(keys):
+            for k in keys:
+                if k not in got and k in mem:
+                    got[k] = mem[k]
+            yield
+        for k in keys:
+            store("empty", -1, k)
+        u, beta = _refl(np.array([got[k] for k in keys]))
+        U[p:p + ln, s] = u
+        E[s] = beta
+        j, B1 = 0, None
+        while True:
+            keys = [(rd, j, *e) for e in _window(n, b, p)]
+            got = {}
+            while len(got) < len(keys):  # elements are seen one by one, in any order
+                for k in keys:
+                    if k not in got and k in mem and rng.random() < 0.7:
+                        got[k] = mem[k]
+                yield
+            S = np.array([[got[rd, j, "S", i, k] for k in range(ln)] for i in range(ln)])
+            N = np.array([[got.get((rd, j, "N", i, k), 0.0) for k in range(ln)] for i in range(ln2)]).reshape(ln2, ln)
+            if ordered:
+                flush(x, j - 1)  # loads of this window were issued after the last step's empties
+            for k in keys:
+                store("empty", j, k)
+            yield
+            y = S @ u
+            w = y - 0.5 * (u @ y) * u
+            S = S - np.outer(u, w) - np.outer(w, u)
+            N = N - np.outer(N @ u, u)
+            send = lambda key, v: store("send", j, key, v)
+            if j == 0:
+                started.add(s)
+                D[s + 1] = S[0, 0]
+                for i in range(1, ln):
+                    send((wr, "X", i - 1), S[i, 0])
+                if s == nsw - 1:
+                    E[n - 2], D[n - 1] = S[1, 0], S[1, 1]
+            else:
+                B1 = B1 - np.outer(u, u @ B1)
+                for k in range(1, b):
+                    send((wr, j - 1, "S", b - 1, k - 1), B1[0, k])
+                    send((wr, j - 1, "S", k - 1, b - 1), B1[0, k])
+                    for i in range(1, ln):
+                        send((wr, j - 1, "N", i - 1, k - 1), B1[i, k])
+                send((wr, j - 1, "S", b - 1, b - 1), S[0, 0])
+                for i in range(1, ln):
+                    send((wr, j - 1, "N", i - 1, b - 1), S[i, 0])
+            for i in range(1, ln):
+                for k in range(1, ln):
+                    send((wr, j, "S", i - 1, k - 1), S[i, k])
+            if ln2 == 0:
+                break
+            un, betan = _refl(N[:, 0].copy()) if ln2 > 1 else (np.zeros(1), N[0, 0])
+            send((wr, "X", b - 1) if j == 0 else (wr, j - 1, "N", b - 1, b - 1), betan)
+            yield
+            p += ln
+            U[p:p + ln2, s] = un
+            u, B1 = un, N
+            ln, ln2 = _lens(n, b, p)
+            j += 1
+        while x["stores"]:
+            yield
+
+    st, ticket, idle = {}, 0, 0
+    while ticket < nsw or st:
+        cand = list(st)
+        if ticket < nsw and len(st) < window:
+            cand.append(-1)
+        s = rng.choice(cand)
+        if s == -1:
+            st[ticket] = {"stores": []}
+            st[ticket]["run"] = program(ticket)
+            ticket += 1
+            continue
+        if rng.random() < 0.5:
+            flush(st[s])
+        else:
+            try:
+                next(st[s]["run"])
+            except StopIteration:
+                del st[s]
+        idle += 1
+        if idle > 2_000_000:
+            raise Stale("no progress")
+    left = [k for k in mem if k[0] == nsw % 2]  # what sweep nsw - 2 sent: all of it was loaded
+    if left:
+        raise Stale(f"{len(left)} elements left behind")
+    return D, E, U
+
+
+def _band(n, b):
+    A = O.gen_symmetric(n, 3, 0).astype(np.float64)
+    return np.tril(np.triu(A, -b), b)
+
+
+@pytest.mark.parametrize("n,b", [(3, 4), (4, 3), (9, 4), (22, 4), (23, 4), (24, 4), (25, 4), (26, 5), (17, 2), (19, 7)])
+def test_messages_match_sequential_chase(n, b):
+    B = _band(n, b)
+    ref = O.sb2st(B, b)
+    for seed in range(3):
+        res = chase(B, b, seed)
+        assert max(np.abs(a - r).max() for a, r in zip(res, ref)) < 1e-11
+
+
+@pytest.mark.parametrize("unsafe", [{"start_word": False}, {"ordered": False}])
+def test_model_catches_unsafe_protocols(unsafe):
+    n, b = 25, 4
+    B = _band(n, b)
+    ref = O.sb2st(B, b)
+    bad = 0
+    for seed in range(30):
+        try:
+            res = chase(B, b, seed, **unsafe)
+            bad += max(np.abs(a - r).max() for a, r in zip(res, ref)) > 1e-6
+        except Stale:
+            bad += 1
+    assert bad

@@ -1,0 +1,56 @@
+"""The bulge chase at the edges of its message layout: bandwidths that do not
+fill a block or a plane of 8 columns, orders around multiples of the bandwidth
+(a last block of one row, of none, sweeps of a single step), bands of width 1,
+leading dimensions above 2 b, rows past the matrix that hold anything."""
+import numpy as np
+import pytest
+
+from oracle import evd_oracle as O
+from tests.helpers import to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+
+def _band(n, b, ld, rng):
+    B = np.zeros((n, n))
+    for d in range(min(b, n - 1) + 1):
+        v = rng.standard_normal(n - d)
+        B += np.diag(v, -d) + (np.diag(v, d) if d else 0.0)
+    band = np.full((ld, n), np.nan)
+    for c in range(n):
+        k = min(2 * b, n - c)  # rows past the matrix stay NaN: they are not read
+        band[:k, c] = 0.0
+        band[:min(b + 1, k), c] = B[c:c + min(b + 1, k), c]
+    return B, band
+
+
+@pytest.mark.parametrize("b", [1, 2, 7, 8, 9, 31, 32, 33, 57, 64])
+def test_chase_edges_match_oracle(ctx, b):
+    import evd4sc2025_amd as E
+
+    rng = np.random.default_rng(b)
+    for n in sorted({3, 4, 5, b, b + 1, b + 2, b + 3, 2 * b, 2 * b + 1, 2 * b + 2, 3 * b + 1, 5 * b + 2, 150}):
+        if n < 3:
+            continue
+        print(f"chase n={n} b={b}", flush=True)
+        B, band = _band(n, b, 2 * b + (n % 3), rng)
+        if b == 1 and n > 4:
+            B[4, 3] = B[3, 4] = band[1, 3] = 0.0
+        D0, E0, U0 = O.sb2st(B, b)
+        D, Ee, U = (to_host(x) for x in E.sb2st(ctx, to_dev(band), n, b))
+        # FP64 arithmetic of the same algorithm: rounding grows with the order
+        np.testing.assert_allclose(D, D0, atol=1e-10)
+        np.testing.assert_allclose(Ee, E0, atol=1e-10)
+        np.testing.assert_allclose(U, U0, atol=1e-5)
+
+
+def test_band_that_holds_the_empty_pattern_does_not_stall(ctx):
+    """A signalling NaN with the bits of an empty message element is an
+    ordinary NaN to the chase."""
+    import evd4sc2025_amd as E
+
+    n, b = 100, 32
+    _, band = _band(n, b, 2 * b, np.random.default_rng(0))
+    band[3, 7] = np.uint64(0x7FF7A5C300000000).view(np.float64)
+    D, _, _ = E.sb2st(ctx, to_dev(band), n, b)
+    assert np.isnan(to_host(D)).any()
