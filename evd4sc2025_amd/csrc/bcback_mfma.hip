@@ -26,11 +26,12 @@
 // eigenvector matrix of the tridiagonal stage has unit columns), so that
 // |Zw| and |X| stay below the FP16 range.
 //
-// MI355X mapping.  One workgroup owns 64 columns of Q; its NW waves form a
+// MI355X mapping.  One workgroup owns 16 NT columns of Q (NT = 4, or 2 and 1
+// where 64-column workgroups would leave CUs idle); its NW waves form a
 // pipeline over NW consecutive sweep blocks (wave k works on block S_top - k
 // one step behind wave k-1) and hand each other the 32 rows they have
 // finished through an LDS double buffer, so Q is streamed from HBM once per
-// 32 NW sweeps.  A wave holds its 64 x 64 window as 4 x 4 accumulator tiles of
+// 32 NW sweeps.  A wave holds its 64 x 16 NT window as 4 x NT accumulator tiles of
 // v_mfma_f32_16x16x32_f16; the K index of the 32-deep operands is permuted so
 // that the two 16-row accumulator tiles a lane holds are exactly the 8 K
 // values its operand slot needs (kmap below): accumulators become operands
@@ -206,24 +207,27 @@ __device__ __attribute__((always_inline)) inline f4 mma(float a, float b, const 
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// Element (row r, column c) of a 32 x 64 half window in accumulator order
-// (tile 4 mt + nt, lane 16 g + c16, component i), as a float index.
+// Element (row r, column c) of a 32 x 16 NT half window in accumulator order
+// (tile NT mt + nt, lane 16 g + c16, component i), as a float index.
+template <int NT>
 __device__ __attribute__((always_inline)) inline int half_index(int r, int c) {
-  return (((r >> 4) * 4 + (c >> 4)) * 64 + ((r >> 2) & 3) * 16 + (c & 15)) * 4 + (r & 3);
+  return (((r >> 4) * NT + (c >> 4)) * 64 + ((r >> 2) & 3) * 16 + (c & 15)) * 4 + (r & 3);
 }
 
-// LDS slot: 32 rows x 64 columns in accumulator order
-__device__ __attribute__((always_inline)) inline void put_half(f4 *slot, const f4 (&h)[2][4], int lane) {
+// LDS slot: 32 rows x 16 NT columns in accumulator order
+template <int NT>
+__device__ __attribute__((always_inline)) inline void put_half(f4 *slot, const f4 (&h)[2][NT], int lane) {
 #pragma unroll
   for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) slot[(mt * 4 + nt) * 64 + lane] = h[mt][nt];
+    for (int nt = 0; nt < NT; nt++) slot[(mt * NT + nt) * 64 + lane] = h[mt][nt];
 }
-__device__ __attribute__((always_inline)) inline void get_half(f4 (&h)[2][4], const f4 *slot, int lane) {
+template <int NT>
+__device__ __attribute__((always_inline)) inline void get_half(f4 (&h)[2][NT], const f4 *slot, int lane) {
 #pragma unroll
   for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) h[mt][nt] = slot[(mt * 4 + nt) * 64 + lane];
+    for (int nt = 0; nt < NT; nt++) h[mt][nt] = slot[(mt * NT + nt) * 64 + lane];
 }
 
 // fragments of a block: V^T of K step ks (4 x h8: mt 0 hi, lo, mt 1 hi, lo), -V T (8 x h8)
@@ -238,18 +242,19 @@ __device__ __attribute__((always_inline)) inline void load_frags(FR (&fr)[N], co
 // given, the next block's v0, v1 and wt are loaded as soon as the current ones
 // are consumed, so their latency hides behind the rest of the step and the
 // next one's start.
-__device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][4], f4 (&bot)[2][4], h8 (&v0)[4],
+template <int NT>
+__device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][NT], f4 (&bot)[2][NT], h8 (&v0)[4],
                                                                   h8 (&v1)[4], h8 (&wt)[8],
                                                                   const h8 *__restrict__ nxt, int lane) {
-  f4 x[2][4];
+  f4 x[2][NT];
 #pragma unroll
   for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) x[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; nt++) x[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
   // X = V^T Zw: K = 64 window rows in two steps, one column tile at a time
   // (products lo*hi, hi*lo, hi*hi)
 #pragma unroll
-  for (int nt = 0; nt < 4; nt++) {
+  for (int nt = 0; nt < NT; nt++) {
     h8 zh, zl;
     split8(top[0][nt], top[1][nt], zh, zl);
 #pragma unroll
@@ -262,7 +267,7 @@ __device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][4
   __builtin_amdgcn_sched_barrier(0);
   if (nxt) load_frags(v0, nxt, lane);
 #pragma unroll
-  for (int nt = 0; nt < 4; nt++) {
+  for (int nt = 0; nt < NT; nt++) {
     h8 zh, zl;
     split8(bot[0][nt], bot[1][nt], zh, zl);
 #pragma unroll
@@ -276,7 +281,7 @@ __device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][4
   if (nxt) load_frags(v1, nxt + 4 * kFrag, lane);
   // Zw += (-V T) X, K = 32 sweeps
 #pragma unroll
-  for (int nt = 0; nt < 4; nt++) {
+  for (int nt = 0; nt < NT; nt++) {
     h8 xh, xl;
     split8(x[0][nt], x[1][nt], xh, xl);
 #pragma unroll
@@ -298,14 +303,15 @@ __device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][4
 
 // The FP32 form of apply_block: V^T and -V T as f4 fragments, K = 4 per
 // v_mfma_f32_16x16x4f32; accumulator tiles are the B operands as they are.
-__device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][4], f4 (&bot)[2][4], f4 (&v0)[4],
+template <int NT>
+__device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][NT], f4 (&bot)[2][NT], f4 (&v0)[4],
                                                                   f4 (&v1)[4], f4 (&wt)[8],
                                                                   const f4 *__restrict__ nxt, int lane) {
-  f4 x[2][4];
+  f4 x[2][NT];
 #pragma unroll
   for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-    for (int nt = 0; nt < 4; nt++) x[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; nt++) x[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
   // X = V^T Zw.  Sweep tile mt of the staircase only reaches window tiles
   // mt .. mt+2, and column t of V T only rows 0 .. t+31: the zero tiles
   // (window tile 0 x sweep tile 1, window tile 3 x sweep tile 0) are skipped.
@@ -316,7 +322,7 @@ __device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][4
 #pragma unroll
       for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++)
+        for (int nt = 0; nt < NT; nt++)
           if (!(rt == 0 && mt == 1)) x[mt][nt] = mma(v0[2 * rt + mt][i], top[rt][nt][i], x[mt][nt]);
   __builtin_amdgcn_sched_barrier(0);
   if (nxt) load_frags(v0, nxt, lane);
@@ -327,7 +333,7 @@ __device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][4
 #pragma unroll
       for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++)
+        for (int nt = 0; nt < NT; nt++)
           if (!(rt == 1 && mt == 0)) x[mt][nt] = mma(v1[2 * rt + mt][i], bot[rt][nt][i], x[mt][nt]);
   __builtin_amdgcn_sched_barrier(0);
   if (nxt) load_frags(v1, nxt + 4 * kFrag, lane);
@@ -339,7 +345,7 @@ __device__ __attribute__((always_inline)) inline void apply_block(f4 (&top)[2][4
 #pragma unroll
       for (int mt = 0; mt < 4; mt++)
 #pragma unroll
-        for (int nt = 0; nt < 4; nt++) {
+        for (int nt = 0; nt < NT; nt++) {
           if (mt == 3 && st == 0) continue;
           if (mt < 2)
             top[mt][nt] = mma(wt[2 * mt + st][i], x[st][nt][i], top[mt][nt]);
@@ -355,24 +361,26 @@ __device__ __attribute__((always_inline)) inline void lds_barrier() {
 }
 
 // HBM <-> LDS traffic of a half window, spread over the 8 waves: wave k moves
-// columns 8k .. 8k+7, one instruction = 2 columns x 32 consecutive rows.
-// The accesses are raw buffer operations over the workgroup's 64 columns that
+// columns 2 NT k .. 2 NT (k + 1) - 1, one instruction = 2 columns x 32
+// consecutive rows.
+// The accesses are raw buffer operations over the workgroup's columns that
 // are always issued: a row or column that must be skipped gets an offset past
 // the buffer, which the hardware drops (stores) or reads as 0 (loads).  With a
 // fixed number of memory operations per step the compiler can wait for the
 // block fragments without also waiting for this traffic.
 constexpr unsigned kBufWord3 = 0x00020000u;  // raw buffer descriptor, 32-bit data
 constexpr unsigned kOutside = 0x80000000u;   // offset beyond every buffer here
+template <int NT>
 struct HalfIO {
   __amdgpu_buffer_rsrc_t rs;
-  int r, c;         // row of the lane, first column of the lane (within the 64)
+  int r, c;         // row of the lane, first column of the lane (within the workgroup's)
   unsigned cbytes;  // byte offset of the lane's first column
   int ncl;          // columns of this workgroup
   float scale;      // window scale (loads multiply, stores divide)
   __device__ HalfIO(float *Zc, long ldz, int n, int ncols_wg, int lane, int k, float sc)
       : rs(__builtin_amdgcn_make_buffer_rsrc(Zc, 0, (int)(((long)(ncols_wg - 1) * ldz + n) * 4), kBufWord3)),
         r(lane & 31),
-        c(8 * k + (lane >> 5)),
+        c(2 * NT * k + (lane >> 5)),
         cbytes((unsigned)(c * ldz * 4)),
         ncl(ncols_wg),
         scale(sc) {}
@@ -380,47 +388,48 @@ struct HalfIO {
     const long gr = row0 + r;
     return (on && gr < n && c + 2 * q < ncl) ? cbytes + (unsigned)((2 * q * ldz + gr) * 4) : kOutside;
   }
-  __device__ __attribute__((always_inline)) inline void load(float (&v)[4], bool on, long row0, int n, long ldz) const {
+  __device__ __attribute__((always_inline)) inline void load(float (&v)[NT], bool on, long row0, int n, long ldz) const {
 #pragma unroll
-    for (int q = 0; q < 4; q++)
+    for (int q = 0; q < NT; q++)
       v[q] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off(on, row0, n, ldz, q), 0, 0)) * scale;
   }
-  __device__ __attribute__((always_inline)) inline void park(f4 *slot, const float (&v)[4]) const {
+  __device__ __attribute__((always_inline)) inline void park(f4 *slot, const float (&v)[NT]) const {
     float *s = reinterpret_cast<float *>(slot);
 #pragma unroll
-    for (int q = 0; q < 4; q++) s[half_index(r, c + 2 * q)] = v[q];
+    for (int q = 0; q < NT; q++) s[half_index<NT>(r, c + 2 * q)] = v[q];
   }
   __device__ __attribute__((always_inline)) inline void store(const f4 *slot, bool on, long row0, int n,
                                                               long ldz) const {
     const float *s = reinterpret_cast<const float *>(slot);
 #pragma unroll
-    for (int q = 0; q < 4; q++) {
-      const float v = s[half_index(r, c + 2 * q)] / scale;
+    for (int q = 0; q < NT; q++) {
+      const float v = s[half_index<NT>(r, c + 2 * q)] / scale;
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rs, off(on, row0, n, ldz, q), 0, 0);
     }
   }
 };
 
-template <int NW, bool F32>
+template <int NW, bool F32, int NT>
 __global__ __launch_bounds__(NW * 64) void bcw_kernel(int n, int ncols, float *__restrict__ Z, long ldz,
                                                       const h8 *__restrict__ F16, int nsweeps, long z_stride,
                                                       long f_stride) {
   typedef typename std::conditional<F32, f4, h8>::type Frag;
   Z += blockIdx.y * z_stride;  // problem blockIdx.y of a batch
   const Frag *F = reinterpret_cast<const Frag *>(F16 + blockIdx.y * f_stride);
-  static_assert(NW == 8, "each wave moves 8 of the 64 columns of a half window");
+  static_assert(NW == 8, "each wave moves 2 NT of the 16 NT columns of a half window");
+  constexpr int kHalf = 128 * NT;  // f4 per half window
   // hand-off slots (2 per wave), the rows wave 0 takes in at each step, and
-  // the top rows of each wave's first step (both double-buffered): 160 KiB
-  __shared__ f4 xch[NW * 2 * 512];
-  __shared__ f4 stage[2 * 512];
-  __shared__ f4 stage_top[2 * 512];
+  // the top rows of each wave's first step (both double-buffered): 40 NT KiB
+  __shared__ f4 xch[NW * 2 * kHalf];
+  __shared__ f4 stage[2 * kHalf];
+  __shared__ f4 stage_top[2 * kHalf];
   const int lane = threadIdx.x & 63;
   const int k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col0 = blockIdx.x * 64;
+  const int col0 = blockIdx.x * (16 * NT);
   const int nblk = (int)wy_sweep_blocks(nsweeps);
   const long Jn = (n + kB - 1) / kB;
-  const HalfIO io(Z + (long)col0 * ldz, ldz, n, min(64, ncols - col0), lane, k, F32 ? 1.f : kScale);
-  f4 zt[2][4], zb[2][4];
+  const HalfIO<NT> io(Z + (long)col0 * ldz, ldz, n, min(16 * NT, ncols - col0), lane, k, F32 ? 1.f : kScale);
+  f4 zt[2][NT], zb[2][NT];
   Frag v0[4], v1[4], wt[8];
 
   const int ngroups = (nblk + NW - 1) / NW;
@@ -438,7 +447,7 @@ __global__ __launch_bounds__(NW * 64) void bcw_kernel(int n, int ncols, float *_
     // (lb, lt) and parked in LDS one step later from (pb, pt); the loop is
     // unrolled by two so the two register sets alternate without copies
     // (a copy would wait for the load).
-    auto body = [&](int tau, float(&lb)[4], float(&lt)[4], const float(&pb)[4], const float(&pt)[4])
+    auto body = [&](int tau, float(&lb)[NT], float(&lt)[NT], const float(&pb)[NT], const float(&pt)[NT])
                     __attribute__((always_inline)) {
       const int e = tau - k;
       const bool act = tau >= 0 && tau < T && k < nact && e >= 0 && e < J;
@@ -454,7 +463,7 @@ __global__ __launch_bounds__(NW * 64) void bcw_kernel(int n, int ncols, float *_
       }
       // (1) rows the last wave handed on at step tau-1 -> Q
       const int el = tau - 1 - kl;
-      io.store(xch + (kl * 2 + (el & 1)) * 512, el >= 0 && el < J, (long)(gtop - kl + el) * kB, n, ldz);
+      io.store(xch + (kl * 2 + (el & 1)) * kHalf, el >= 0 && el < J, (long)(gtop - kl + el) * kB, n, ldz);
       // (2) rows needed at step tau+2: wave 0's new bottom half, and the top
       // half of wave tau+2's first step
       io.load(lb, tau + 2 < J, (long)(gtop + tau + 3) * kB, n, ldz);
@@ -462,23 +471,23 @@ __global__ __launch_bounds__(NW * 64) void bcw_kernel(int n, int ncols, float *_
       // (3) this wave's step
       if (act) {
         if (e == 0) {
-          get_half(zt, stage_top + (k & 1) * 512, lane);
+          get_half(zt, stage_top + (k & 1) * kHalf, lane);
         } else {
 #pragma unroll
           for (int mt = 0; mt < 2; mt++)
 #pragma unroll
-            for (int nt = 0; nt < 4; nt++) zt[mt][nt] = zb[mt][nt];
+            for (int nt = 0; nt < NT; nt++) zt[mt][nt] = zb[mt][nt];
         }
-        get_half(zb, k == 0 ? stage + (e & 1) * 512 : xch + ((k - 1) * 2 + (e & 1)) * 512, lane);
+        get_half(zb, k == 0 ? stage + (e & 1) * kHalf : xch + ((k - 1) * 2 + (e & 1)) * kHalf, lane);
         if (app) apply_block(zt, zb, v0, v1, wt, (e + 1 < nst && e + 1 < J) ? cur + kBlockFrags * kFrag : nullptr, lane);
-        put_half(xch + (k * 2 + (e & 1)) * 512, zt, lane);
+        put_half(xch + (k * 2 + (e & 1)) * kHalf, zt, lane);
       }
       // (4) park the rows loaded at step tau-1 (for step tau+1)
-      if (tau >= -1 && tau + 1 < J) io.park(stage + ((tau + 1) & 1) * 512, pb);
-      if (tau >= -1 && tau + 1 < nact) io.park(stage_top + ((tau + 1) & 1) * 512, pt);
+      if (tau >= -1 && tau + 1 < J) io.park(stage + ((tau + 1) & 1) * kHalf, pb);
+      if (tau >= -1 && tau + 1 < nact) io.park(stage_top + ((tau + 1) & 1) * kHalf, pt);
       lds_barrier();
     };
-    float la[4], ta[4], lb2[4], tb2[4];
+    float la[NT], ta[NT], lb2[NT], tb2[NT];
     for (int tau = -2; tau <= T; tau += 2) {
       body(tau, la, ta, lb2, tb2);
       if (tau + 1 <= T) body(tau + 1, lb2, tb2, la, ta);
@@ -594,27 +603,29 @@ __global__ __launch_bounds__(256) void bcw64_prep_kernel(int n, const float *__r
   }
 }
 
-// A workgroup of the b = 64 kernel owns kC64 columns: a half window is 64
-// rows x kC64 columns, kNT64 column tiles of 16.
-constexpr int kC64 = 64, kNT64 = kC64 / 16, kHalf64 = 4 * kNT64 * 64;  // f4 per half window
+// A workgroup of the b = 64 kernel owns NT column tiles of 16: a half window
+// is 64 rows x 16 NT columns, 256 NT f4.
 
 // Element (row r, column c) of a half window in accumulator order (tile
-// kNT64 rt + nt, lane 16 g + c16, component i), as a float index.
+// NT rt + nt, lane 16 g + c16, component i), as a float index.
+template <int NT>
 __device__ __attribute__((always_inline)) inline int half64_index(int r, int c) {
-  return (((r >> 4) * kNT64 + (c >> 4)) * 64 + ((r >> 2) & 3) * 16 + (c & 15)) * 4 + (r & 3);
+  return (((r >> 4) * NT + (c >> 4)) * 64 + ((r >> 2) & 3) * 16 + (c & 15)) * 4 + (r & 3);
 }
 
-__device__ __attribute__((always_inline)) inline void put_half64(f4 *slot, const f4 (&h)[4][kNT64], int lane) {
+template <int NT>
+__device__ __attribute__((always_inline)) inline void put_half64(f4 *slot, const f4 (&h)[4][NT], int lane) {
 #pragma unroll
   for (int rt = 0; rt < 4; rt++)
 #pragma unroll
-    for (int nt = 0; nt < kNT64; nt++) slot[(rt * kNT64 + nt) * 64 + lane] = h[rt][nt];
+    for (int nt = 0; nt < NT; nt++) slot[(rt * NT + nt) * 64 + lane] = h[rt][nt];
 }
-__device__ __attribute__((always_inline)) inline void get_half64(f4 (&h)[4][kNT64], const f4 *slot, int lane) {
+template <int NT>
+__device__ __attribute__((always_inline)) inline void get_half64(f4 (&h)[4][NT], const f4 *slot, int lane) {
 #pragma unroll
   for (int rt = 0; rt < 4; rt++)
 #pragma unroll
-    for (int nt = 0; nt < kNT64; nt++) h[rt][nt] = slot[(rt * kNT64 + nt) * 64 + lane];
+    for (int nt = 0; nt < NT; nt++) h[rt][nt] = slot[(rt * NT + nt) * 64 + lane];
 }
 
 // HBM traffic of the b = 64 kernel.  Half windows staged through LDS (wave
@@ -624,8 +635,9 @@ __device__ __attribute__((always_inline)) inline void get_half64(f4 (&h)[4][kNT6
 // offset past the buffer (dropped stores, zero loads), so every step issues
 // the same memory operations.  load_acc brings a wave's own first top half
 // straight into its accumulator tiles.
+template <int NT>
 struct HalfIO64 {
-  static constexpr int kQ = kC64 / 4;
+  static constexpr int kQ = 4 * NT;
   __amdgpu_buffer_rsrc_t rs;
   int r, c;         // row of the lane, first column of the wave (within the workgroup's)
   unsigned cbytes;  // byte offset of the wave's first column
@@ -649,26 +661,26 @@ struct HalfIO64 {
   __device__ __attribute__((always_inline)) inline void park(f4 *slot, const float (&v)[kQ]) const {
     float *s = reinterpret_cast<float *>(slot);
 #pragma unroll
-    for (int q = 0; q < kQ; q++) s[half64_index(r, c + q)] = v[q];
+    for (int q = 0; q < kQ; q++) s[half64_index<NT>(r, c + q)] = v[q];
   }
   __device__ __attribute__((always_inline)) inline void store(const f4 *slot, bool on, long row0, int n,
                                                               long ldz) const {
     const float *s = reinterpret_cast<const float *>(slot);
 #pragma unroll
     for (int q = 0; q < kQ; q++)
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s[half64_index(r, c + q)]), rs,
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, s[half64_index<NT>(r, c + q)]), rs,
                                             off(on, row0, n, ldz, q), 0, 0);
   }
   // rows row0 .. row0+63 of all the workgroup's columns in accumulator order:
   // tile (rt, nt), lane 16 g + c16, component i = row 16 rt + 4 g + i of
   // column 16 nt + c16
-  __device__ __attribute__((always_inline)) inline void load_acc(f4 (&h)[4][kNT64], long row0, int n, long ldz,
+  __device__ __attribute__((always_inline)) inline void load_acc(f4 (&h)[4][NT], long row0, int n, long ldz,
                                                                  int lane) const {
     const int c16 = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int rt = 0; rt < 4; rt++)
 #pragma unroll
-      for (int nt = 0; nt < kNT64; nt++)
+      for (int nt = 0; nt < NT; nt++)
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           const long gr = row0 + 16 * rt + 4 * g + i;
@@ -693,18 +705,19 @@ __device__ __attribute__((always_inline)) inline void load_tiles(f4 (&fr)[M], co
 // the start, behind the X products, those of row tiles 4..7 (10) once X has
 // consumed most of vt, and the next block's V^T tiles (nxt, may be null) once
 // the first Zw half has consumed the first -V T part.  Every product loop runs
-// the kNT64 = 4 column tiles as independent accumulators.
-__device__ __attribute__((always_inline)) inline void apply_block64(f4 (&top)[4][kNT64], f4 (&bot)[4][kNT64],
+// the NT column tiles as independent accumulators.
+template <int NT>
+__device__ __attribute__((always_inline)) inline void apply_block64(f4 (&top)[4][NT], f4 (&bot)[4][NT],
                                                                     f4 (&vt)[20], const f4 *__restrict__ blk,
                                                                     const f4 *__restrict__ nxt, int lane) {
   f4 wa[16], wb[10];
   load_tiles<16>(wa, blk, woff64(0), lane);
   __builtin_amdgcn_sched_barrier(0);
-  f4 x[4][kNT64];
+  f4 x[4][NT];
 #pragma unroll
   for (int mt = 0; mt < 4; mt++)
 #pragma unroll
-    for (int nt = 0; nt < kNT64; nt++) x[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
+    for (int nt = 0; nt < NT; nt++) x[mt][nt] = f4{0.f, 0.f, 0.f, 0.f};
   // X = V^T Zw, window row tile by row tile (every loop has a constant trip
   // count, so all indices fold after unrolling and the arrays stay in
   // registers)
@@ -715,7 +728,7 @@ __device__ __attribute__((always_inline)) inline void apply_block64(f4 (&top)[4]
 #pragma unroll
       for (int mt = 0; mt < 4; mt++)
 #pragma unroll
-        for (int nt = 0; nt < kNT64; nt++) {
+        for (int nt = 0; nt < NT; nt++) {
           if (mt < vlo64(rt) || mt > vhi64(rt)) continue;
           x[mt][nt] = mma(vt[voff64(rt) + mt - vlo64(rt)][i], (rt < 4 ? top[rt & 3][nt] : bot[rt & 3][nt])[i],
                           x[mt][nt]);
@@ -740,7 +753,7 @@ __device__ __attribute__((always_inline)) inline void apply_block64(f4 (&top)[4]
 #pragma unroll
       for (int i = 0; i < 4; i++)
 #pragma unroll
-        for (int nt = 0; nt < kNT64; nt++) {
+        for (int nt = 0; nt < NT; nt++) {
           if (st < wlo64(rt)) continue;
           const int q = woff64(rt) + st - wlo64(rt);
           const f4 &w = rt < 4 ? wa[(q - woff64(0)) & 15] : wb[(q - woff64(4)) % 10];
@@ -753,7 +766,7 @@ __device__ __attribute__((always_inline)) inline void apply_block64(f4 (&top)[4]
 }
 
 // The b = 64 pipeline: as bcw_kernel (waves over consecutive sweep blocks,
-// rows handed on through LDS), with kC64 = 64 columns per workgroup and 4
+// rows handed on through LDS), with 16 NT columns per workgroup and 4
 // waves, one per SIMD (a wave's window, X and a block's fragments take
 // about 420 of its 512 registers).  Every workgroup streams all WY blocks,
 // so the column width sets the fragment traffic: 64 columns read the 6.2 GB
@@ -761,22 +774,23 @@ __device__ __attribute__((always_inline)) inline void apply_block64(f4 (&top)[4]
 // the hand-off slots and wave 0's incoming rows (160 KiB); each wave loads
 // the top half of its first step of a group straight into its registers, two
 // steps ahead.  Q is streamed from HBM once per 256 sweeps.
+template <int NT>
 __global__ __launch_bounds__(256) void bcw64_kernel(int n, int ncols, float *__restrict__ Z, long ldz,
                                                     const f4 *__restrict__ F, int nsweeps, long z_stride,
                                                     long f_stride) {
   constexpr int NW = 4;
-  constexpr int kQ = HalfIO64::kQ;
+  constexpr int kQ = HalfIO64<NT>::kQ, kCols = 16 * NT, kHalf64 = 256 * NT;
   Z += blockIdx.y * z_stride;
   F += blockIdx.y * f_stride;
   __shared__ f4 xch[NW * 2 * kHalf64];
   __shared__ f4 stage[2 * kHalf64];
   const int lane = threadIdx.x & 63;
   const int k = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int col0 = blockIdx.x * kC64;
+  const int col0 = blockIdx.x * kCols;
   const int nblk = (int)wy64_sweep_blocks(nsweeps);
   const long Jn = (n + kB64 - 1) / kB64;
-  const HalfIO64 io(Z + (long)col0 * ldz, ldz, n, min(kC64, ncols - col0), lane, k);
-  f4 zt[4][kNT64], zb[4][kNT64];
+  const HalfIO64<NT> io(Z + (long)col0 * ldz, ldz, n, min(kCols, ncols - col0), lane, k);
+  f4 zt[4][NT], zb[4][NT];
   f4 vt[20];
 
   const int ngroups = (nblk + NW - 1) / NW;
@@ -808,7 +822,7 @@ __global__ __launch_bounds__(256) void bcw64_kernel(int n, int ncols, float *__r
 #pragma unroll
           for (int rt = 0; rt < 4; rt++)
 #pragma unroll
-            for (int nt = 0; nt < kNT64; nt++) zt[rt][nt] = zb[rt][nt];
+            for (int nt = 0; nt < NT; nt++) zt[rt][nt] = zb[rt][nt];
         }
         get_half64(zb, k == 0 ? stage + (e & 1) * kHalf64 : xch + ((k - 1) * 2 + (e & 1)) * kHalf64, lane);
         if (app)
@@ -827,6 +841,30 @@ __global__ __launch_bounds__(256) void bcw64_kernel(int n, int ncols, float *__r
 }
 
 }  // namespace
+
+// Column tiles of 16 per workgroup (1, 2 or 4).  A launch lasts as long as the
+// CU with the most workgroups; a workgroup of 64 columns takes longer than one
+// of 16 but not four times as long, since a step's fragments, hand-off and
+// barriers are the same.  Relative times of one round, measured at n = 8192 (64 / 32
+// / 16 columns): b = 32 FP32 31.4 / 18.6 / 11-12.5 ms, b = 64 35.6 / 22.4 / 12-15.6
+// ms, FP16 14.2 / 12.4 / 8-9.9 ms.  With 64 columns throughout, up to half of
+// the CUs (n = 8192), all but 64 (n = 4096) or all but 16 (1000 vectors) had
+// nothing to do: n = 4096 8.4 -> 3.2 ms, n = 8192 31.4 -> 18.7 ms, 1000 vectors at n =
+// 8192 33.3 -> 12.3 ms.  Every column's arithmetic is the same for all widths.
+static int wy_column_tiles(const evd_ctx *ctx, long ncols, int count, bool split16) {
+  int best = 4;
+  long least = -1;
+  for (int nt : {4, 2, 1}) {
+    const long groups = (ncols + 16 * nt - 1) / (16 * nt) * count;
+    const long round = nt == 4 ? 100 : nt == 2 ? (split16 ? 86 : 60) : (split16 ? 57 : 35);
+    const long cost = (groups + ctx->num_cus - 1) / ctx->num_cus * round;
+    if (least < 0 || cost < least) {
+      least = cost;
+      best = nt;
+    }
+  }
+  return best;
+}
 
 size_t bc_back_wy_bytes(long n) {
   if (n <= 2) return 0;
@@ -860,13 +898,23 @@ int bc_back_wy_batched(evd_ctx *ctx, int count, long n, long ncols, float *Q, lo
   EVD_LAUNCHED(ctx);
   if (ctx->timing) hipEventRecord(ctx->kev[0], ctx->stream);
   constexpr int NW = 8;
-  const dim3 grid((unsigned)((ncols + 63) / 64), (unsigned)count);
-  if (split16)
-    bcw_kernel<NW, false><<<grid, NW * 64, 0, ctx->stream>>>((int)n, (int)ncols, Q, ldq, F, nsweeps, q_stride,
-                                                              f_stride);
+  auto launch = [&](auto tiles) {
+    constexpr int NT = decltype(tiles)::value;
+    const dim3 grid((unsigned)((ncols + 16 * NT - 1) / (16 * NT)), (unsigned)count);
+    if (split16)
+      bcw_kernel<NW, false, NT><<<grid, NW * 64, 0, ctx->stream>>>((int)n, (int)ncols, Q, ldq, F, nsweeps, q_stride,
+                                                                    f_stride);
+    else
+      bcw_kernel<NW, true, NT><<<grid, NW * 64, 0, ctx->stream>>>((int)n, (int)ncols, Q, ldq, F, nsweeps, q_stride,
+                                                                   f_stride);
+  };
+  const int nt = wy_column_tiles(ctx, ncols, count, split16);
+  if (nt == 1)
+    launch(std::integral_constant<int, 1>{});
+  else if (nt == 2)
+    launch(std::integral_constant<int, 2>{});
   else
-    bcw_kernel<NW, true><<<grid, NW * 64, 0, ctx->stream>>>((int)n, (int)ncols, Q, ldq, F, nsweeps, q_stride,
-                                                             f_stride);
+    launch(std::integral_constant<int, 4>{});
   EVD_LAUNCHED(ctx);
   if (ctx->timing) hipEventRecord(ctx->kev[1], ctx->stream);
   return 0;
@@ -879,7 +927,7 @@ size_t bc_back_wy64_bytes(long n) {
 }
 
 // the columns of a workgroup must be addressable with 32-bit buffer offsets
-bool bc_back_wy64_fits(long n, long ldq) { return ((kC64 - 1) * ldq + n) * 4 < (1L << 31); }
+bool bc_back_wy64_fits(long n, long ldq) { return (63 * ldq + n) * 4 < (1L << 31); }
 
 // Q <- H_1 .. H_K Q for b = 64 as WY blocks on FP32 MFMA (every precision
 // form), a batch of `count` same-size problems per launch.
@@ -897,8 +945,18 @@ int bc_back_wy64_batched(evd_ctx *ctx, int count, long n, long ncols, float *Q, 
       (int)n, U, ldu, nsweeps, F, u_stride, f_stride);
   EVD_LAUNCHED(ctx);
   if (ctx->timing) hipEventRecord(ctx->kev[0], ctx->stream);
-  bcw64_kernel<<<dim3((unsigned)((ncols + kC64 - 1) / kC64), (unsigned)count), 256, 0, ctx->stream>>>(
-      (int)n, (int)ncols, Q, ldq, F, nsweeps, q_stride, f_stride);
+  auto launch = [&](auto tiles) {
+    constexpr int NT = decltype(tiles)::value;
+    bcw64_kernel<NT><<<dim3((unsigned)((ncols + 16 * NT - 1) / (16 * NT)), (unsigned)count), 256, 0, ctx->stream>>>(
+        (int)n, (int)ncols, Q, ldq, F, nsweeps, q_stride, f_stride);
+  };
+  const int nt = wy_column_tiles(ctx, ncols, count, false);
+  if (nt == 1)
+    launch(std::integral_constant<int, 1>{});
+  else if (nt == 2)
+    launch(std::integral_constant<int, 2>{});
+  else
+    launch(std::integral_constant<int, 4>{});
   EVD_LAUNCHED(ctx);
   if (ctx->timing) hipEventRecord(ctx->kev[1], ctx->stream);
   return 0;
