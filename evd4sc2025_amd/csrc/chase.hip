@@ -104,22 +104,6 @@ __device__ __attribute__((always_inline)) inline double group_sum(double v) {
   return v;
 }
 
-// 1 / sqrt(x) and sqrt(x) for x > 0: the hardware estimate refined by two
-// coupled Newton steps (Goldschmidt's iteration), the root corrected once more
-// by its residual.  One short chain instead of a square root and a division.
-__device__ __attribute__((always_inline)) inline void rsqrt_sqrt(double x, double &inv, double &root) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double g = x * y, h = 0.5 * y;
-  double r = __builtin_fma(-g, h, 0.5);
-  g = __builtin_fma(g, r, g);
-  h = __builtin_fma(h, r, h);
-  r = __builtin_fma(-g, h, 0.5);
-  g = __builtin_fma(g, r, g);
-  h = __builtin_fma(h, r, h);
-  root = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-  inv = 2.0 * h;
-}
-
 // a b + c d with both products rounded, so that exchanging (a, d) and (b, c)
 // gives the same bits: the two halves of a symmetric block stay equal
 __device__ __attribute__((always_inline)) inline double sym_pair(double a, double b, double c, double d) {

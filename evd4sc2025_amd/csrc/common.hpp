@@ -39,7 +39,7 @@ struct Tuning {
 // level table + device copy of the merge descriptors, split flags and tile
 // offsets), kept per context.
 struct DcPlan {
-  int nmerge = 0, H = 0;
+  int nmerge = 0, H = 0, nleaf = 0;
   std::vector<int> level_off;    // merges of height h: [level_off[h], level_off[h + 1])
   std::vector<int> level_maxN;   // largest merge order of each height
   std::vector<int> level_tiles;  // grouped-GEMM tile budget of each height
@@ -258,6 +258,22 @@ __device__ inline double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
+// 1 / sqrt(x) and sqrt(x) for x > 0: the hardware estimate refined by two
+// coupled Newton steps (Goldschmidt's iteration), the root corrected once more
+// by its residual.  One short chain instead of a square root and a division.
+__device__ __attribute__((always_inline)) inline void rsqrt_sqrt(double x, double &inv, double &root) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double g = x * y, h = 0.5 * y;
+  double r = __builtin_fma(-g, h, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  r = __builtin_fma(-g, h, 0.5);
+  g = __builtin_fma(g, r, g);
+  h = __builtin_fma(h, r, h);
+  root = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  inv = 2.0 * h;
+}
+
 __device__ inline float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

@@ -15,7 +15,8 @@
 //  * Q_new = Q' [U 0; 0 I] by grouped FP64 MFMA GEMMs over the top and bottom
 //    row blocks (column types 1/2/3 as in dlaed2/dlaed3).
 //
-// GPU layout: the binary split tree is built on the host; all merges of one
+// GPU layout: the binary split tree is built on the host down to leaves of at
+// most kDcLeaf rows, which one wave each solves by the QR algorithm; all merges of one
 // tree height run in the same launches (grid.y = merge), every merge working
 // in the index range [start, start+N) of n-long scratch arrays and in the
 // diagonal block of the n x n Q / scratch matrices.  The deflation scan is
@@ -35,6 +36,17 @@ struct MergeDesc {
   double rho;  // |e| at the split
   double sgn;  // sign(e)
 };
+// a leaf of the tree: rows start .. start + size - 1 of problem `problem`
+struct LeafDesc {
+  int start, size, problem;
+};
+// Rows of a leaf.  A small merge level costs 35 to 60 us of dependent launches
+// whatever its size; the QR algorithm's rotations form one chain of about
+// 0.85 m^2 for a leaf of m rows, 0.1 us each, so leaves of 16 rows replace four
+// levels by one launch of 25 us, and leaves of 32 would spend 80 us to save one
+// level more.  With the parallel scans, products and copies below, whole solves of
+// T: n = 256 0.61 -> 0.25 ms, n = 2500 2.6 -> 1.3 ms.
+constexpr int kDcLeaf = 16;
 struct MergeOut {
   int K, K1, K2, K3, ndefl, nrot;
   double rho2;  // 2|e|
@@ -115,6 +127,87 @@ __global__ void dc_denormalize_kernel(long n, double *__restrict__ D, const doub
     D[q * n + i] *= s;
 }
 
+// Eigen-decomposition of one leaf (a symmetric tridiagonal of at most kDcLeaf
+// rows) by the implicit symmetric QR algorithm with Wilkinson's shift (Golub &
+// Van Loan, Matrix Computations, section 8.3): one wave, every lane runs the same
+// scalar recurrence and lane r applies its rotations to row r of the
+// vectors.  D and the vectors leave sorted.  Bound by the chain of rotations
+// (a reciprocal root each); the column a rotation finishes leaves for LDS while
+// the other one stays in a register as the next rotation's first.
+__global__ __launch_bounds__(64) void dc_leaf_kernel(const LeafDesc *__restrict__ lf, const double *__restrict__ E,
+                                                     double *__restrict__ D, double *__restrict__ Z, long ldz,
+                                                     long zmul, unsigned *__restrict__ err) {
+  __shared__ double d[kDcLeaf], e[kDcLeaf + 1], q[kDcLeaf][kDcLeaf + 1];
+  __shared__ int rank[kDcLeaf];
+  const LeafDesc l = lf[blockIdx.x];
+  const int m = l.size, st = l.start, lane = threadIdx.x;
+  const double eps = DBL_EPSILON * 0.5;
+  // entries whose square could underflow are zero beside the problem's norm, 1
+  const double tiny = 1e-140;
+  if (lane < m) {
+    d[lane] = D[st + lane];
+    e[lane] = lane < m - 1 ? E[st + lane] : 0.0;
+    for (int c = 0; c < m; c++) q[c][lane] = (c == lane) ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  int hi = m - 1, it = 0;
+  while (hi > 0) {
+    const bool small = lane < hi && fabs(e[lane]) <= eps * (fabs(d[lane]) + fabs(d[lane + 1])) + tiny;
+    const unsigned long long cut = __ballot(small);
+    if ((cut >> (hi - 1)) & 1) {
+      hi--;
+      continue;
+    }
+    if (++it > 40 * kDcLeaf) {
+      if (lane == 0) atomicOr(err, (unsigned)EVD_E_NOCONVERGE);
+      break;
+    }
+    // the unreduced block lo .. hi
+    const int lo = cut ? 64 - __clzll((long long)cut) : 0;
+    const double eh = e[hi - 1], dh = d[hi], del = 0.5 * (d[hi - 1] - dh);
+    const double mu = dh - eh * (eh / (del + copysign(sqrt(del * del + eh * eh), del)));
+    double dk = d[lo], ek = e[lo], x = dk - mu, z = ek;
+    double qk = lane < m ? q[lo][lane] : 0.0;
+    for (int k = lo; k < hi; k++) {
+      const double dn = d[k + 1], en = e[k + 1], qn = lane < m ? q[k + 1][lane] : 0.0;
+      double c = 1.0, s = 0.0, r = 0.0;
+      const double rr = x * x + z * z;
+      if (rr > 0.0) {
+        double inv;
+        rsqrt_sqrt(rr, inv, r);
+        c = x * inv;
+        s = -z * inv;
+      }
+      if (k > lo) e[k - 1] = r;
+      const double cs = c * s, t = 2.0 * cs * ek, cc = c * c, ss = s * s;
+      d[k] = cc * dk - t + ss * dn;
+      x = cs * (dk - dn) + (cc - ss) * ek;
+      dk = ss * dk + t + cc * dn;
+      if (lane < m) q[k][lane] = c * qk - s * qn;
+      qk = s * qk + c * qn;
+      z = -s * en;
+      ek = c * en;
+    }
+    e[hi - 1] = x;
+    d[hi] = dk;
+    if (lane < m) q[hi][lane] = qk;
+    __syncthreads();
+  }
+  if (lane < m) {
+    int pos = 0;
+    const double v = d[lane];
+    for (int i = 0; i < m; i++) pos += (d[i] < v || (d[i] == v && i < lane)) ? 1 : 0;
+    rank[lane] = pos;
+    D[st + pos] = v;
+  }
+  __syncthreads();
+  double *Zb = Z + ((long)l.problem * zmul + st + (long)st * ldz);
+  for (int i = lane; i < m * m; i += 64) {
+    const int row = i % m, c = i / m;
+    Zb[row + (long)rank[c] * ldz] = q[c][row];
+  }
+}
+
 // |e| and sign(e) at every split, read on the device so no host round trip
 // sits between the tridiagonal stage's producer and the merges.
 __global__ void dc_rho_kernel(int nmerge, MergeDesc *__restrict__ md, const double *__restrict__ E) {
@@ -125,11 +218,11 @@ __global__ void dc_rho_kernel(int nmerge, MergeDesc *__restrict__ md, const doub
   }
 }
 
-__global__ void dc_sort_kernel(const MergeDesc *__restrict__ md, const double *__restrict__ D,
-                               const double *__restrict__ Z, long ldz, DCScratch sc) {
-  const MergeDesc m = md[blockIdx.y];
+// d and z of one merge in ascending order of d, elements first, first + step, ...
+__device__ inline void merge_sorted(const MergeDesc &m, const double *__restrict__ D, const double *__restrict__ Z,
+                                    long ldz, const DCScratch &sc, int first, int step) {
   const int N = m.n1 + m.n2, st = m.start;
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < N; t += gridDim.x * blockDim.x) {
+  for (int t = first; t < N; t += step) {
     double d = D[st + t], z;
     int pos;
     if (t < m.n1) {
@@ -160,6 +253,12 @@ __global__ void dc_sort_kernel(const MergeDesc *__restrict__ md, const double *_
     sc.cs[st + pos] = t;
   }
 }
+__global__ void dc_sort_kernel(const MergeDesc *__restrict__ md, const double *__restrict__ D,
+                               const double *__restrict__ Z, long ldz, DCScratch sc) {
+  merge_sorted(md[blockIdx.y], D, Z, ldz, sc, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
+}
+// merges up to this order are sorted by their deflation workgroup
+constexpr int kDcSortInline = 512;
 
 // One thread per merge: deflation scan in sorted order (dlaed2 logic).
 // Block-wide helpers for one 256-thread workgroup.
@@ -171,23 +270,24 @@ __device__ inline double block_max256(double v, double *red) {
   __syncthreads();
   return fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
 }
-// exclusive prefix of per-thread counts (thread order); returns the total
-__device__ inline int block_scan256(int v, int *sh, int &excl) {
-  __syncthreads();
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int acc = 0;
-    for (int t = 0; t < 256; t++) {
-      const int x = sh[t];
-      sh[t] = acc;
-      acc += x;
-    }
-    sh[256] = acc;
+// exclusive prefix of per-thread counts (thread order); returns the total.
+// Three counts of up to 2^21 may share the word.
+__device__ inline unsigned long long block_scan256(unsigned long long v, unsigned long long *sh,
+                                                   unsigned long long &excl) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  unsigned long long x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned long long y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
   }
   __syncthreads();
-  excl = sh[threadIdx.x];
-  return sh[256];
+  if (lane == 63) sh[wave] = x;
+  __syncthreads();
+  unsigned long long before = 0;
+  for (int w = 0; w < wave; w++) before += sh[w];
+  excl = before + x - v;
+  return sh[0] + sh[1] + sh[2] + sh[3];
 }
 
 // Deflation of one merge (LAPACK dlaed2), one 256-thread workgroup per merge.
@@ -198,15 +298,21 @@ __device__ inline int block_scan256(int v, int *sh, int &excl) {
 // current values, accepts every pair before the first rotation, applies that
 // rotation and continues after it.  The deflated list is the in-order
 // z-deflated run merged with the (few) rotated entries; type counts and the
-// type-stable positions come from block scans.
+// type-stable positions come from block scans (shuffles within a wave; a scan
+// by one thread had made this kernel 16-23 us long, four times per merge level).
 __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__restrict__ md, MergeOut *__restrict__ mo,
-                                                         DCScratch sc) {
+                                                         const double *__restrict__ D, const double *__restrict__ Z,
+                                                         long ldz, int sort, DCScratch sc) {
   __shared__ double red[4];
-  __shared__ int sh[257];
+  __shared__ unsigned long long sh[4];
   __shared__ int s_nc, s_K, s_nrot;
   const MergeDesc m = md[blockIdx.x];
   const int N = m.n1 + m.n2, st = m.start, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const double rho = 2.0 * m.rho;
+  if (sort) {
+    merge_sorted(m, D, Z, ldz, sc, tid, 256);
+    __syncthreads();
+  }
   double *ds = sc.ds + st, *zs = sc.zs + st;
   const int *cs = sc.cs + st;
   int *types = sc.types + st;
@@ -237,10 +343,9 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
   // z-deflated run (in order) and the candidate list, by compaction
   int nz_loc = 0;
   for (int i = i0; i < i1; i++) nz_loc += (all_defl || rho * fabs(zs[i]) <= tol) ? 1 : 0;
-  int zoff;
-  const int nzd = block_scan256(nz_loc, sh, zoff);
-  int coff = (i0 - zoff > 0) ? i0 - zoff : 0;  // candidates before my chunk = i0 - (z-deflated before it)
-  coff = i0 - zoff;
+  unsigned long long before;
+  const int nzd = (int)block_scan256((unsigned long long)nz_loc, sh, before);
+  int zoff = (int)before, coff = i0 - zoff;  // candidates before my chunk = i0 - (z-deflated before it)
   for (int i = i0; i < i1; i++) {
     if (all_defl || rho * fabs(zs[i]) <= tol) {
       df_d[zoff] = ds[i];
@@ -383,22 +488,22 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
     c3 += (ty == 3);
     zs2 += nd_z[kk] * nd_z[kk];
   }
-  int e1, e2, e3;
-  const int K1 = block_scan256(c1, sh, e1);
-  const int K2 = block_scan256(c2, sh, e2);
-  const int K3 = block_scan256(c3, sh, e3);
+  const unsigned long long counts =
+      block_scan256((unsigned long long)c1 | (unsigned long long)c2 << 21 | (unsigned long long)c3 << 42, sh, before);
+  const int mask21 = (1 << 21) - 1;
+  const int K1 = (int)(counts & mask21), K2 = (int)(counts >> 21 & mask21), K3 = (int)(counts >> 42);
+  int e1 = (int)(before & mask21), e2 = (int)(before >> 21 & mask21), e3 = (int)(before >> 42);
   for (int kk = k0; kk < k1; kk++) {
     const int ty = types[nd_col[kk]];
     qpos[kk] = (ty == 1) ? e1++ : (ty == 2) ? K1 + e2++ : K1 + K2 + e3++;
   }
-  // z sum in a fixed order (deterministic): per-thread chunks, then thread order
+  // z sum in a fixed order (deterministic): per-thread chunks, waves, workgroup
+  zs2 = wave_sum(zs2);
   __syncthreads();
-  __shared__ double zpart[256];
-  zpart[tid] = zs2;
+  if (lane == 0) red[wave] = zs2;
   __syncthreads();
   if (tid == 0) {
-    double zsum = 0.0;
-    for (int t = 0; t < 256; t++) zsum += zpart[t];
+    const double zsum = ((red[0] + red[1]) + red[2]) + red[3];
     MergeOut o;
     o.K = K;
     o.K1 = K1;
@@ -432,23 +537,32 @@ __global__ void dc_rotate_kernel(const MergeDesc *__restrict__ md, const MergeOu
 }
 
 // Gather the permuted copy Qc = [non-deflated by type | deflated]: blocks of
-// 256 rows x 64 destination columns (grid z over merges).
-__global__ void dc_gather_kernel(const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo,
-                                 const double *__restrict__ Z, long ldz, DCScratch sc, long ldq) {
+// 64 rows x 16 destination columns, four independent copies per thread (grid z
+// over merges; a thread that copied 64 columns one by one took 12-16 us).
+__global__ __launch_bounds__(256) void dc_gather_kernel(const MergeDesc *__restrict__ md,
+                                                        const MergeOut *__restrict__ mo, const double *__restrict__ Z,
+                                                        long ldz, DCScratch sc, long ldq) {
   const MergeDesc m = md[blockIdx.z];
-  const MergeOut o = mo[blockIdx.z];
   const int N = m.n1 + m.n2, st = m.start;
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  const int c0 = blockIdx.y * 64, c1 = min(N, c0 + 64);
+  const int r = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int c0 = blockIdx.y * 16 + (threadIdx.x >> 6);
   if (r >= N || c0 >= N) return;
+  const int K = mo[blockIdx.z].K;
   const double *Zb = Z + ((long)m.pad * sc.zmul + st + (long)st * ldz);
   double *Qc = sc.Qc + ((long)m.pad * sc.qmul + st + (long)st * ldq);
-  for (int k = c0; k < c1; k++) {
-    if (k < o.K)
-      Qc[r + (long)sc.qpos[st + k] * ldq] = Zb[r + (long)sc.nd_col[st + k] * ldz];
-    else
-      Qc[r + (long)k * ldq] = Zb[r + (long)sc.df_col[st + (k - o.K)] * ldz];
+  int src[4], dst[4];
+  double v[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int k = min(c0 + 4 * i, N - 1);
+    src[i] = k < K ? sc.nd_col[st + k] : sc.df_col[st + (k - K)];
+    dst[i] = k < K ? sc.qpos[st + k] : k;
   }
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = Zb[r + (long)src[i] * ldz];
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    if (c0 + 4 * i < N) Qc[r + (long)dst[i] * ldq] = v[i];
 }
 
 // f(tau) pieces relative to pole `org`: psi over poles <= lower, phi over the rest.
@@ -595,121 +709,74 @@ __global__ void dc_secular_kernel(const MergeDesc *__restrict__ md, const MergeO
   }
 }
 
-// zhat_j^2 = prod_i (lambda_i - d_j) / (rho prod_{k != j} (d_k - d_j))
-__global__ void dc_loewner_kernel(const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo, DCScratch sc) {
+// zhat_j^2 = prod_i (lambda_i - d_j) / (rho prod_{k != j} (d_k - d_j)): one wave
+// per j, lane l takes the ratios k = l, l + 64, ... (each within the spread of
+// the poles, as is any product of them) and the lanes' products are multiplied in
+// a fixed order.  One thread per j had taken 73 us at n = 2500, a serial chain of
+// K divisions on K / 256 workgroups.
+__global__ __launch_bounds__(256) void dc_loewner_kernel(const MergeDesc *__restrict__ md,
+                                                         const MergeOut *__restrict__ mo, DCScratch sc) {
   const MergeDesc m = md[blockIdx.y];
   const MergeOut o = mo[blockIdx.y];
-  const int st = m.start, K = o.K;
+  const int st = m.start, K = o.K, lane = threadIdx.x & 63;
   const double *d = sc.nd_d + st, *z = sc.nd_z + st;
   const int *orig = sc.orig + st;
   const double *tau = sc.tau + st;
-  for (int j = blockIdx.x * blockDim.x + threadIdx.x; j < K; j += gridDim.x * blockDim.x) {
+  for (int j = blockIdx.x * 4 + (threadIdx.x >> 6); j < K; j += gridDim.x * 4) {
     const double dj = d[j];
-    double prod = ((d[orig[j]] - dj) + tau[j]) / o.rho2;  // (lambda_j - d_j)/rho
-    for (int k = 0; k < K; k++) {
-      if (k == j) continue;
+    double prod = 1.0;
+    for (int k = lane; k < K; k += 64) {
       const double lk = (d[orig[k]] - dj) + tau[k];  // lambda_k - d_j
-      prod *= lk / (d[k] - dj);
+      prod *= (k == j) ? lk / o.rho2 : lk / (d[k] - dj);
     }
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1) prod *= __shfl_xor(prod, s, 64);
     const double zh = sqrt(fabs(prod));
-    sc.zhat[st + j] = (z[j] >= 0.0) ? zh : -zh;
+    if (lane == 0) sc.zhat[st + j] = (z[j] >= 0.0) ? zh : -zh;
   }
 }
 
-// One workgroup per eigenvector column i of one merge: Uc[qpos[j], i].
-__global__ __launch_bounds__(256) void dc_vectors_kernel(const MergeDesc *__restrict__ md,
-                                                         const MergeOut *__restrict__ mo, DCScratch sc, long ldu) {
-  const MergeDesc m = md[blockIdx.y];
-  const MergeOut o = mo[blockIdx.y];
-  const int st = m.start, K = o.K;
-  const int i = blockIdx.x;
-  if (i >= K) return;
-  const double *d = sc.nd_d + st;
-  const double dorg = d[sc.orig[st + i]];
-  const double ti = sc.tau[st + i];
-  double *Uc = sc.Uc + ((long)m.pad * sc.qmul + st + (long)st * ldu);
-  __shared__ double red[4];
-  double ss = 0.0;
-  for (int j = threadIdx.x; j < K; j += 256) {
-    const double v = sc.zhat[st + j] / ((d[j] - dorg) - ti);
-    ss += v * v;
-  }
-  ss = wave_sum(ss);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
-  __syncthreads();
-  const double inv = 1.0 / sqrt(red[0] + red[1] + red[2] + red[3]);
-  for (int j = threadIdx.x; j < K; j += 256) {
-    const double v = sc.zhat[st + j] / ((d[j] - dorg) - ti);
-    Uc[sc.qpos[st + j] + (long)i * ldu] = v * inv;
-  }
-}
-
-// Final ascending order of [lambda (K) ; deflated (ndefl)], new D and column maps.
-__global__ void dc_order_kernel(const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo, DCScratch sc,
-                                double *__restrict__ D) {
-  const MergeDesc m = md[blockIdx.y];
-  const MergeOut o = mo[blockIdx.y];
-  const int st = m.start, K = o.K, nd = o.ndefl;
+// Ascending position of element t of [lambda (K) ; deflated (nd)]: the new D
+// and the column maps.
+__device__ inline void merged_position(int t, int st, int K, int nd, const DCScratch &sc, double *__restrict__ D) {
   const double *lam = sc.lam + st, *df = sc.df_d + st;
-  for (int t = blockIdx.x * blockDim.x + threadIdx.x; t < K + nd; t += gridDim.x * blockDim.x) {
-    if (t < K) {
-      const double v = lam[t];
-      int lo = 0, hi = nd;
-      while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (df[mid] < v)
-          lo = mid + 1;
-        else
-          hi = mid;
-      }
-      const int pos = t + lo;
-      D[st + pos] = v;
-      sc.colmap[st + t] = st + pos;
-    } else {
-      const int u = t - K;
-      const double v = df[u];
-      int lo = 0, hi = K;
-      while (lo < hi) {
-        int mid = (lo + hi) >> 1;
-        if (lam[mid] <= v)
-          lo = mid + 1;
-        else
-          hi = mid;
-      }
-      const int pos = u + lo;
-      D[st + pos] = v;
-      sc.dmap[st + u] = st + pos;
+  if (t < K) {
+    const double v = lam[t];
+    int lo = 0, hi = nd;
+    while (lo < hi) {
+      int mid = (lo + hi) >> 1;
+      if (df[mid] < v)
+        lo = mid + 1;
+      else
+        hi = mid;
     }
+    const int pos = t + lo;
+    D[st + pos] = v;
+    sc.colmap[st + t] = st + pos;
+  } else {
+    const int u = t - K;
+    const double v = df[u];
+    int lo = 0, hi = K;
+    while (lo < hi) {
+      int mid = (lo + hi) >> 1;
+      if (lam[mid] <= v)
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    const int pos = u + lo;
+    D[st + pos] = v;
+    sc.dmap[st + u] = st + pos;
   }
 }
 
-__global__ void dc_copy_deflated_kernel(const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo,
-                                        DCScratch sc, long ldq, double *__restrict__ Z, long ldz) {
-  const MergeDesc m = md[blockIdx.y];
-  const MergeOut o = mo[blockIdx.y];
-  const int st = m.start, N = m.n1 + m.n2;
-  const long total = (long)N * o.ndefl;
-  const double *Qc = sc.Qc + ((long)m.pad * sc.qmul + st + (long)st * ldq);
-  const long zsh = (long)m.pad * sc.zmul;
-  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
-    const int r = (int)(e % N);
-    const int u = (int)(e / N);
-    Z[zsh + (st + r) + (long)sc.dmap[st + u] * ldz] = Qc[r + (long)(o.K + u) * ldq];
-  }
-}
-
-// Grouped-GEMM problems of one tree level, built on the device from the
-// deflation results: merge i gives problem 2i (top rows: Qc[:, 0:K1+K2]) and
-// 2i+1 (bottom rows: Qc[:, K1:K]).  Tile offsets are fixed per level from the
-// bound K <= N; tiles past a problem's actual K columns exit at once, and a
-// merge with K = 0 gets m = 0.
-__global__ void dc_problems_kernel(int nm, const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo,
-                                   const int *__restrict__ tile_begin, DCScratch sc, long ldq, double *Z, long ldz,
-                                   DGemmProblem *__restrict__ probs) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nm) return;
-  const MergeDesc m = md[i];
-  const MergeOut o = mo[i];
+// Grouped-GEMM problems of one merge, from its deflation results: problem 2i
+// is the top rows (Qc[:, 0:K1+K2]), 2i+1 the bottom rows (Qc[:, K1:K]).  Tile
+// offsets are fixed per level from the bound K <= N; tiles past a problem's
+// actual K columns exit at once, and a merge with K = 0 gets m = 0.
+__device__ inline void merge_problems(int i, const MergeDesc &m, const MergeOut &o, const int *__restrict__ tile_begin,
+                                      const DCScratch &sc, long ldq, double *Z, long ldz,
+                                      DGemmProblem *__restrict__ probs) {
   const int st = m.start;
   const long zsh = (long)m.pad * sc.zmul, qsh = (long)m.pad * sc.qmul;
   DGemmProblem top;
@@ -740,6 +807,55 @@ __global__ void dc_problems_kernel(int nm, const MergeDesc *__restrict__ md, con
   probs[2 * i + 1] = bot;
 }
 
+// One workgroup per index i < N of one merge: eigenvector column i (Uc[qpos[j],
+// i], i < K), the position of element i in the merged order, and once per merge
+// its two product problems.
+__global__ __launch_bounds__(256) void dc_vectors_kernel(const MergeDesc *__restrict__ md,
+                                                         const MergeOut *__restrict__ mo, DCScratch sc, long ldu,
+                                                         double *__restrict__ D, const int *__restrict__ tile_begin,
+                                                         double *Z, long ldz, DGemmProblem *__restrict__ probs) {
+  const MergeDesc m = md[blockIdx.y];
+  const MergeOut o = mo[blockIdx.y];
+  const int st = m.start, K = o.K;
+  const int i = blockIdx.x;
+  if (threadIdx.x == 0 && i < K + o.ndefl) merged_position(i, st, K, o.ndefl, sc, D);
+  if (threadIdx.x == 64 && i == 0) merge_problems(blockIdx.y, m, o, tile_begin, sc, ldu, Z, ldz, probs);
+  if (i >= K) return;
+  const double *d = sc.nd_d + st;
+  const double dorg = d[sc.orig[st + i]];
+  const double ti = sc.tau[st + i];
+  double *Uc = sc.Uc + ((long)m.pad * sc.qmul + st + (long)st * ldu);
+  __shared__ double red[4];
+  double ss = 0.0;
+  for (int j = threadIdx.x; j < K; j += 256) {
+    const double v = sc.zhat[st + j] / ((d[j] - dorg) - ti);
+    ss += v * v;
+  }
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  const double inv = 1.0 / sqrt(red[0] + red[1] + red[2] + red[3]);
+  for (int j = threadIdx.x; j < K; j += 256) {
+    const double v = sc.zhat[st + j] / ((d[j] - dorg) - ti);
+    Uc[sc.qpos[st + j] + (long)i * ldu] = v * inv;
+  }
+}
+
+__global__ void dc_copy_deflated_kernel(const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo,
+                                        DCScratch sc, long ldq, double *__restrict__ Z, long ldz) {
+  const MergeDesc m = md[blockIdx.y];
+  const MergeOut o = mo[blockIdx.y];
+  const int st = m.start, N = m.n1 + m.n2;
+  const long total = (long)N * o.ndefl;
+  const double *Qc = sc.Qc + ((long)m.pad * sc.qmul + st + (long)st * ldq);
+  const long zsh = (long)m.pad * sc.zmul;
+  for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < total; e += (long)gridDim.x * blockDim.x) {
+    const int r = (int)(e % N);
+    const int u = (int)(e / N);
+    Z[zsh + (st + r) + (long)sc.dmap[st + u] * ldz] = Qc[r + (long)(o.K + u) * ldq];
+  }
+}
+
 struct TreeNode {
   int start, size, left, right, height;
 };
@@ -747,7 +863,7 @@ struct TreeNode {
 static int build_tree(std::vector<TreeNode> &nodes, int start, int size) {
   int id = (int)nodes.size();
   nodes.push_back({start, size, -1, -1, 0});
-  if (size > 1) {
+  if (size > kDcLeaf) {
     int n1 = size / 2;
     int l = build_tree(nodes, start, n1);
     int r = build_tree(nodes, start + n1, size - n1);
@@ -779,7 +895,7 @@ static size_t dc_per_problem(long n) {
 size_t stedc_workspace(long n) { return dc_per_problem(n) + align256(dc_lib_temp_words(n) * sizeof(double)) + (1 << 16); }
 
 // Merge plan of order n, built once per context: the tree (halving splits
-// down to single rows), merges grouped by height, the split flags and the
+// down to leaves), merges grouped by height, the split flags and the
 // per-level tile offsets of the grouped GEMMs, copied to device memory that
 // lives as long as the context.  Only the split values (rho, sign) change per
 // solve; dc_rho_kernel writes them into the device descriptors.
@@ -800,9 +916,13 @@ int dc_plan(evd_ctx *ctx, long n, int count, const DcPlan **out) {
   const int H = plan.H;
   std::vector<std::vector<int>> by_height(H + 1);
   for (int i = 0; i < (int)nodes.size(); i++)
-    if (nodes[i].size > 1) by_height[nodes[i].height].push_back(i);
+    by_height[nodes[i].height].push_back(i);
   std::vector<MergeDesc> all;
   std::vector<int> tiles;
+  std::vector<LeafDesc> leaves;
+  for (int q = 0; q < count; q++)
+    for (int id : by_height[0]) leaves.push_back({(int)(q * n) + nodes[id].start, nodes[id].size, q});
+  plan.nleaf = (int)leaves.size();
   plan.level_off.assign(H + 2, 0);
   plan.level_maxN.assign(H + 1, 0);
   plan.level_tiles.assign(H + 1, 0);
@@ -838,10 +958,11 @@ int dc_plan(evd_ctx *ctx, long n, int count, const DcPlan **out) {
   const size_t b_md = align256(sizeof(MergeDesc) * all.size()), b_split = align256(sizeof(int) * nt),
                b_tiles = align256(sizeof(int) * tiles.size());
   std::vector<char> &host = plan.host;
-  host.assign(b_md + b_split + b_tiles, 0);
-  memcpy(host.data(), all.data(), sizeof(MergeDesc) * all.size());
+  host.assign(b_md + b_split + b_tiles + sizeof(LeafDesc) * leaves.size(), 0);
+  if (!all.empty()) memcpy(host.data(), all.data(), sizeof(MergeDesc) * all.size());
   memcpy(host.data() + b_md, split.data(), sizeof(int) * nt);
-  memcpy(host.data() + b_md + b_split, tiles.data(), sizeof(int) * tiles.size());
+  if (!tiles.empty()) memcpy(host.data() + b_md + b_split, tiles.data(), sizeof(int) * tiles.size());
+  memcpy(host.data() + b_md + b_split + b_tiles, leaves.data(), sizeof(LeafDesc) * leaves.size());
   // device copy: carved from the context's plan pool (one allocation for all
   // plans), else an allocation of its own; the upload is stream-ordered and
   // its source stays alive with the plan
@@ -958,26 +1079,33 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
   const int *dsplit = reinterpret_cast<const int *>(pdev + align256(sizeof(MergeDesc) * nmerge));
   const int *dtiles = reinterpret_cast<const int *>(pdev + align256(sizeof(MergeDesc) * nmerge) +
                                                     align256(sizeof(int) * nt));
-  MergeOut *dmo = static_cast<MergeOut *>(arena_alloc(ctx, sizeof(MergeOut) * nmerge));
+  const LeafDesc *dleaf = reinterpret_cast<const LeafDesc *>(reinterpret_cast<const char *>(dtiles) +
+                                                             align256(sizeof(int) * 2 * nmerge));
+  MergeOut *dmo = static_cast<MergeOut *>(arena_alloc(ctx, sizeof(MergeOut) * std::max(1, nmerge)));
   // temporary of the library products (large merges, eager solves)
   double *libT = nullptr;
   if (ctx->blas && !ctx->tune.own_gemm && !ctx->capturing && dc_lib_temp_words(n) > 0) {
     libT = arena_alloc_n<double>(ctx, dc_lib_temp_words(n));
     if (!libT) return EVD_E_NOMEM;
   }
-  DGemmProblem *dprob = static_cast<DGemmProblem *>(arena_alloc(ctx, sizeof(DGemmProblem) * 2 * nmerge));
+  DGemmProblem *dprob = static_cast<DGemmProblem *>(arena_alloc(ctx, sizeof(DGemmProblem) * 2 * std::max(1, nmerge)));
   double *nrm = arena_alloc_n<double>(ctx, (size_t)count);
   if (!dmo || !dprob || !nrm) return EVD_E_NOMEM;
   unsigned *err = ctx->ctrl + kCtrlError;
 
-  // split values and signs, tearing of every split, then Q = I
+  // split values and signs, tearing of every split, then the leaves
   dc_normalize_kernel<<<(unsigned)count, 256, 0, ctx->stream>>>(n, D, E, nrm);
   EVD_LAUNCHED(ctx);
-  dc_rho_kernel<<<(unsigned)std::min((nmerge + 255) / 256, 1024), 256, 0, ctx->stream>>>(nmerge, dmd, E);
+  if (nmerge > 0) {
+    dc_rho_kernel<<<(unsigned)std::min((nmerge + 255) / 256, 1024), 256, 0, ctx->stream>>>(nmerge, dmd, E);
+    EVD_LAUNCHED(ctx);
+    dc_tear_kernel<<<(unsigned)std::min<long>((nt + 255) / 256, 1024), 256, 0, ctx->stream>>>(nt, dsplit, E, D);
+    EVD_LAUNCHED(ctx);
+    // outside the leaves' diagonal blocks Z starts as zeros
+    for (int q = 0; q < count; q++) EVD_TRY(fill_f64(ctx, Z + q * zs, n, n, ldz, 0.0));
+  }
+  dc_leaf_kernel<<<(unsigned)plan->nleaf, 64, 0, ctx->stream>>>(dleaf, E, D, Z, ldz, sc.zmul, err);
   EVD_LAUNCHED(ctx);
-  dc_tear_kernel<<<(unsigned)std::min<long>((nt + 255) / 256, 1024), 256, 0, ctx->stream>>>(nt, dsplit, E, D);
-  EVD_LAUNCHED(ctx);
-  for (int q = 0; q < count; q++) EVD_TRY(set_identity_f64(ctx, Z + q * zs, n, ldz));
 
   // Merges level by level (by height).  Launch shapes come from the largest
   // merge of the level; every kernel bounds its work by the deflation
@@ -989,27 +1117,24 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
     MergeOut *lmo = dmo + off;
     const int maxN = plan->level_maxN[h];
     const unsigned gx = (unsigned)std::min(64, (maxN + 255) / 256);
-    dc_sort_kernel<<<dim3(gx, nm), 256, 0, ctx->stream>>>(lmd, D, Z, ldz, sc);
-    EVD_LAUNCHED(ctx);
-    dc_deflate_kernel<<<nm, 256, 0, ctx->stream>>>(lmd, lmo, sc);
+    const bool sort_inline = maxN <= kDcSortInline;
+    if (!sort_inline) {
+      dc_sort_kernel<<<dim3(gx, nm), 256, 0, ctx->stream>>>(lmd, D, Z, ldz, sc);
+      EVD_LAUNCHED(ctx);
+    }
+    dc_deflate_kernel<<<nm, 256, 0, ctx->stream>>>(lmd, lmo, D, Z, ldz, sort_inline ? 1 : 0, sc);
     EVD_LAUNCHED(ctx);
     dc_rotate_kernel<<<dim3(gx, nm), 256, 0, ctx->stream>>>(lmd, lmo, Z, ldz, sc);
     EVD_LAUNCHED(ctx);
-    dc_gather_kernel<<<dim3((unsigned)((maxN + 255) / 256), (unsigned)((maxN + 63) / 64), nm), 256, 0, ctx->stream>>>(
+    dc_gather_kernel<<<dim3((unsigned)((maxN + 63) / 64), (unsigned)((maxN + 15) / 16), nm), 256, 0, ctx->stream>>>(
         lmd, lmo, Z, ldz, sc, ldq);
     EVD_LAUNCHED(ctx);
-    const unsigned gk = (unsigned)std::min(256, (maxN + 255) / 256);
     const unsigned gw = (unsigned)std::min(16384, (maxN + 3) / 4);  // 4 roots (waves) per workgroup
     dc_secular_kernel<<<dim3(gw, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc, err);
     EVD_LAUNCHED(ctx);
-    dc_loewner_kernel<<<dim3(gk, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc);
+    dc_loewner_kernel<<<dim3(gw, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc);
     EVD_LAUNCHED(ctx);
-    dc_vectors_kernel<<<dim3(maxN, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc, ldq);
-    EVD_LAUNCHED(ctx);
-    dc_order_kernel<<<dim3(gx, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc, D);
-    EVD_LAUNCHED(ctx);
-    dc_problems_kernel<<<(unsigned)((nm + 255) / 256), 256, 0, ctx->stream>>>(nm, lmd, lmo, dtiles + 2 * off, sc, ldq,
-                                                                             Z, ldz, dprob);
+    dc_vectors_kernel<<<dim3(maxN, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc, ldq, D, dtiles + 2 * off, Z, ldz, dprob);
     EVD_LAUNCHED(ctx);
     if (libT && maxN >= kDcLibMinN && !ctx->capturing)
       EVD_TRY(dc_level_library(ctx, dprob, 2 * nm, libT, dc_lib_temp_words(n)));
