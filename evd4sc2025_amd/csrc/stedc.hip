@@ -75,6 +75,15 @@ struct DCScratch {
   long zmul = 0, qmul = 0;
 };
 
+// Eigenvalues only: a merge needs just the last row of its first child's
+// vectors and the first row of its second's, so the vectors are never formed.
+// first / last hold those two rows of every node's vectors (by column, in the
+// place of D); rot_first / rot_last a merge's rows after its deflation
+// rotations.  Null when vectors are wanted.
+struct DCRows {
+  double *first = nullptr, *last = nullptr, *rot_first = nullptr, *rot_last = nullptr;
+};
+
 // Tearing of every split at once, one thread per diagonal entry (an entry
 // between two splits is adjusted by both): split[k] != 0 marks a split between
 // rows k-1 and k.
@@ -136,7 +145,7 @@ __global__ void dc_denormalize_kernel(long n, double *__restrict__ D, const doub
 // the other one stays in a register as the next rotation's first.
 __global__ __launch_bounds__(64) void dc_leaf_kernel(const LeafDesc *__restrict__ lf, const double *__restrict__ E,
                                                      double *__restrict__ D, double *__restrict__ Z, long ldz,
-                                                     long zmul, unsigned *__restrict__ err) {
+                                                     long zmul, DCRows rows, unsigned *__restrict__ err) {
   __shared__ double d[kDcLeaf], e[kDcLeaf + 1], q[kDcLeaf][kDcLeaf + 1];
   __shared__ int rank[kDcLeaf];
   const LeafDesc l = lf[blockIdx.x];
@@ -201,6 +210,13 @@ __global__ __launch_bounds__(64) void dc_leaf_kernel(const LeafDesc *__restrict_
     D[st + pos] = v;
   }
   __syncthreads();
+  if (rows.first) {
+    if (lane < m) {
+      rows.first[st + rank[lane]] = q[lane][0];
+      rows.last[st + rank[lane]] = q[lane][m - 1];
+    }
+    return;
+  }
   double *Zb = Z + ((long)l.problem * zmul + st + (long)st * ldz);
   for (int i = lane; i < m * m; i += 64) {
     const int row = i % m, c = i / m;
@@ -220,13 +236,13 @@ __global__ void dc_rho_kernel(int nmerge, MergeDesc *__restrict__ md, const doub
 
 // d and z of one merge in ascending order of d, elements first, first + step, ...
 __device__ inline void merge_sorted(const MergeDesc &m, const double *__restrict__ D, const double *__restrict__ Z,
-                                    long ldz, const DCScratch &sc, int first, int step) {
+                                    long ldz, const DCScratch &sc, const DCRows &rows, int first, int step) {
   const int N = m.n1 + m.n2, st = m.start;
   for (int t = first; t < N; t += step) {
     double d = D[st + t], z;
     int pos;
     if (t < m.n1) {
-      z = Z[(long)m.pad * sc.zmul + (st + m.n1 - 1) + (long)(st + t) * ldz];
+      z = rows.last ? rows.last[st + t] : Z[(long)m.pad * sc.zmul + (st + m.n1 - 1) + (long)(st + t) * ldz];
       int lo = 0, hi = m.n2;
       while (lo < hi) {
         int mid = (lo + hi) >> 1;
@@ -237,7 +253,7 @@ __device__ inline void merge_sorted(const MergeDesc &m, const double *__restrict
       }
       pos = t + lo;
     } else {
-      z = m.sgn * Z[(long)m.pad * sc.zmul + (st + m.n1) + (long)(st + t) * ldz];
+      z = m.sgn * (rows.first ? rows.first[st + t] : Z[(long)m.pad * sc.zmul + (st + m.n1) + (long)(st + t) * ldz]);
       int lo = 0, hi = m.n1;
       while (lo < hi) {
         int mid = (lo + hi) >> 1;
@@ -254,8 +270,8 @@ __device__ inline void merge_sorted(const MergeDesc &m, const double *__restrict
   }
 }
 __global__ void dc_sort_kernel(const MergeDesc *__restrict__ md, const double *__restrict__ D,
-                               const double *__restrict__ Z, long ldz, DCScratch sc) {
-  merge_sorted(md[blockIdx.y], D, Z, ldz, sc, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
+                               const double *__restrict__ Z, long ldz, DCScratch sc, DCRows rows) {
+  merge_sorted(md[blockIdx.y], D, Z, ldz, sc, rows, (int)(blockIdx.x * blockDim.x + threadIdx.x), (int)(gridDim.x * blockDim.x));
 }
 // merges up to this order are sorted by their deflation workgroup
 constexpr int kDcSortInline = 512;
@@ -302,7 +318,7 @@ __device__ inline unsigned long long block_scan256(unsigned long long v, unsigne
 // by one thread had made this kernel 16-23 us long, four times per merge level).
 __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__restrict__ md, MergeOut *__restrict__ mo,
                                                          const double *__restrict__ D, const double *__restrict__ Z,
-                                                         long ldz, int sort, DCScratch sc) {
+                                                         long ldz, int sort, DCScratch sc, DCRows rows) {
   __shared__ double red[4];
   __shared__ unsigned long long sh[4];
   __shared__ int s_nc, s_K, s_nrot;
@@ -310,7 +326,7 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
   const int N = m.n1 + m.n2, st = m.start, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const double rho = 2.0 * m.rho;
   if (sort) {
-    merge_sorted(m, D, Z, ldz, sc, tid, 256);
+    merge_sorted(m, D, Z, ldz, sc, rows, tid, 256);
     __syncthreads();
   }
   double *ds = sc.ds + st, *zs = sc.zs + st;
@@ -841,6 +857,117 @@ __global__ __launch_bounds__(256) void dc_vectors_kernel(const MergeDesc *__rest
   }
 }
 
+// Values only: the merge's two rows before the rotations (zero in the columns
+// of the other child) and the rotations on them.  Rotation t acts on columns
+// (p, n); its p is the n of rotation t - 1 or a column no rotation has touched,
+// so wave 0 takes 64 rotations' data at once and passes one pair of values on
+// from rotation to rotation.
+__global__ __launch_bounds__(256) void dc_rows_rotate_kernel(const MergeDesc *__restrict__ md,
+                                                             const MergeOut *__restrict__ mo, DCScratch sc,
+                                                             DCRows rows) {
+  const MergeDesc m = md[blockIdx.x];
+  const int N = m.n1 + m.n2, st = m.start, nrot = mo[blockIdx.x].nrot, tid = threadIdx.x;
+  double *rf = rows.rot_first + st, *rl = rows.rot_last + st;
+  for (int c = tid; c < N; c += 256) {
+    rf[c] = c < m.n1 ? rows.first[st + c] : 0.0;
+    rl[c] = c < m.n1 ? 0.0 : rows.last[st + c];
+  }
+  __syncthreads();
+  if (tid >= 64) return;
+  const int lane = tid;
+  double cf = 0.0, cl = 0.0;  // the rotated n column of the previous rotation
+  int cn = -1;
+  auto of_lane = [](double v, int i) {
+    const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+    const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, i);
+    const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), i);
+    return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+  };
+  for (int t0 = 0; t0 < nrot; t0 += 64) {
+    const int cnt = min(64, nrot - t0);
+    const bool on = lane < cnt;
+    const int p = on ? sc.rot_p[st + t0 + lane] : -1, n = on ? sc.rot_n[st + t0 + lane] : -1;
+    const double c = on ? sc.rot_c[st + t0 + lane] : 1.0, s = on ? sc.rot_s[st + t0 + lane] : 0.0;
+    const double pf = on ? rf[p] : 0.0, pl = on ? rl[p] : 0.0, nf = on ? rf[n] : 0.0, nl = on ? rl[n] : 0.0;
+    double of = 0.0, ol = 0.0, qf = 0.0, ql = 0.0;
+    for (int i = 0; i < cnt; i++) {
+      const bool chained = __builtin_amdgcn_readlane(p, i) == cn;
+      const double ci = of_lane(c, i), si = of_lane(s, i);
+      const double xf = chained ? cf : of_lane(pf, i), xl = chained ? cl : of_lane(pl, i);
+      const double yf = of_lane(nf, i), yl = of_lane(nl, i);
+      cf = ci * yf - si * xf;
+      cl = ci * yl - si * xl;
+      cn = __builtin_amdgcn_readlane(n, i);
+      if (lane == i) {
+        of = ci * xf + si * yf;
+        ol = ci * xl + si * yl;
+        qf = cf;
+        ql = cl;
+      }
+    }
+    // column n's value first: where the next rotation takes it on as its p,
+    // that rotation's store comes later (the next lane's below, or the next
+    // round's)
+    if (on) {
+      const int pnext = __shfl_down(p, 1, 64);
+      if (lane == cnt - 1 || pnext != n) {
+        rf[n] = qf;
+        rl[n] = ql;
+      }
+      rf[p] = of;
+      rl[p] = ol;
+    }
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+  }
+}
+
+// Values only: the merged node's two rows and the positions of its values, one
+// wave per index i < N.  Vector i has the entries zhat_j / (d_j - lambda_i) over
+// the non-deflated columns, so its first and last entries are two sums beside
+// its norm's; a deflated column keeps its entries.
+__global__ __launch_bounds__(256) void dc_rows_kernel(const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo,
+                                                      DCScratch sc, DCRows rows, int sums, double *__restrict__ D) {
+  const MergeDesc m = md[blockIdx.y];
+  const MergeOut o = mo[blockIdx.y];
+  const int st = m.start, K = o.K, lane = threadIdx.x & 63;
+  const int i = blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (i >= K + o.ndefl) return;
+  int pos = 0;
+  if (lane == 0) {
+    merged_position(i, st, K, o.ndefl, sc, D);
+    pos = i < K ? sc.colmap[st + i] : sc.dmap[st + i - K];
+  }
+  if (!sums) return;
+  const double *rf = rows.rot_first + st, *rl = rows.rot_last + st;
+  if (i >= K) {
+    if (lane == 0) {
+      const int c = sc.df_col[st + i - K];
+      rows.first[pos] = rf[c];
+      rows.last[pos] = rl[c];
+    }
+    return;
+  }
+  const double *d = sc.nd_d + st;
+  const double dorg = d[sc.orig[st + i]], ti = sc.tau[st + i];
+  double ss = 0.0, a = 0.0, b = 0.0;
+  for (int j = lane; j < K; j += 64) {
+    const double v = sc.zhat[st + j] / ((d[j] - dorg) - ti);
+    const int c = sc.nd_col[st + j];
+    ss += v * v;
+    a += v * rf[c];
+    b += v * rl[c];
+  }
+  ss = wave_sum(ss);
+  a = wave_sum(a);
+  b = wave_sum(b);
+  if (lane == 0) {
+    const double inv = 1.0 / sqrt(ss);
+    rows.first[pos] = a * inv;
+    rows.last[pos] = b * inv;
+  }
+}
+
 __global__ void dc_copy_deflated_kernel(const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo,
                                         DCScratch sc, long ldq, double *__restrict__ Z, long ldz) {
   const MergeDesc m = md[blockIdx.y];
@@ -890,6 +1017,14 @@ static size_t dc_per_problem(long n) {
   b += align256((size_t)n * sizeof(MergeOut));
   b += align256((size_t)2 * n * sizeof(DGemmProblem));
   return b;
+}
+
+// arena bytes of the values-only form (no matrices), count problems at a time
+size_t stedc_values_workspace(int count, long n) {
+  const int per = (int)std::max<long>(1, 65535 / ((n + 1) / 2));
+  return (dc_per_problem(n) - align256((size_t)n * n * sizeof(double)) * 2 + align256((size_t)n * sizeof(double)) * 4) *
+             (size_t)std::min(count, per) +
+         (1 << 16);
 }
 
 size_t stedc_workspace(long n) { return dc_per_problem(n) + align256(dc_lib_temp_words(n) * sizeof(double)) + (1 << 16); }
@@ -1042,11 +1177,13 @@ static int dc_level_library(evd_ctx *ctx, const DGemmProblem *dprob, int nprob, 
 
 // `count` same-size tridiagonals (D, E of problem q at q n, Z at q zs): every
 // merge level of all problems is one set of launches.  Each problem's merges
-// and their arithmetic are those of its single solve.
+// and their arithmetic are those of its single solve.  Z = nullptr: eigenvalues
+// only, by the two rows of each node's vectors that the merges read (O(n^2) work
+// instead of O(n^3): n = 3001 1.74 -> 0.70 ms, n = 16384 70 -> 5.4 ms).
 int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double *Z, long ldz, long zs) {
   if (n <= 0 || count <= 0) return 0;
   if (n == 1) {
-    for (int q = 0; q < count; q++) EVD_TRY(set_identity_f64(ctx, Z + q * zs, 1, ldz));
+    for (int q = 0; Z && q < count; q++) EVD_TRY(set_identity_f64(ctx, Z + q * zs, 1, ldz));
     return 0;
   }
   // the merges of one level are a launch dimension (at most 65535)
@@ -1054,20 +1191,29 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
   if (count > per) {
     for (int q0 = 0; q0 < count; q0 += per) {
       const int c = std::min(per, count - q0);
-      EVD_TRY(stedc_batched(ctx, c, n, D + q0 * n, E + q0 * n, Z + q0 * zs, ldz, zs));
+      EVD_TRY(stedc_batched(ctx, c, n, D + q0 * n, E + q0 * n, Z ? Z + q0 * zs : nullptr, ldz, zs));
     }
     return 0;
   }
   ArenaFrame frame(ctx);
   DCScratch sc;
   const long ldq = n, nt = n * count;
-  sc.Qc = arena_alloc_n<double>(ctx, (size_t)n * n * count);
-  sc.Uc = arena_alloc_n<double>(ctx, (size_t)n * n * count);
+  const bool vec = Z != nullptr;
+  DCRows rows;
+  if (vec) {
+    sc.Qc = arena_alloc_n<double>(ctx, (size_t)n * n * count);
+    sc.Uc = arena_alloc_n<double>(ctx, (size_t)n * n * count);
+    if (!sc.Qc || !sc.Uc) return EVD_E_NOMEM;
+  } else {
+    double **rbufs[] = {&rows.first, &rows.last, &rows.rot_first, &rows.rot_last};
+    for (auto p : rbufs) *p = arena_alloc_n<double>(ctx, (size_t)nt);
+    if (!rows.rot_last) return EVD_E_NOMEM;
+  }
   double **dbufs[] = {&sc.ds, &sc.zs, &sc.nd_d, &sc.nd_z, &sc.df_d, &sc.rot_c, &sc.rot_s, &sc.tau, &sc.lam, &sc.zhat};
   for (auto p : dbufs) *p = arena_alloc_n<double>(ctx, (size_t)nt);
   int **ibufs[] = {&sc.cs, &sc.nd_col, &sc.qpos, &sc.df_col, &sc.rot_p, &sc.rot_n, &sc.types, &sc.orig, &sc.colmap, &sc.dmap};
   for (auto p : ibufs) *p = arena_alloc_n<int>(ctx, (size_t)nt);
-  if (!sc.Qc || !sc.Uc || !sc.zhat || !sc.dmap) return EVD_E_NOMEM;
+  if (!sc.zhat || !sc.dmap) return EVD_E_NOMEM;
   sc.zmul = zs - n * (1 + ldz);
   sc.qmul = -n;
 
@@ -1084,7 +1230,7 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
   MergeOut *dmo = static_cast<MergeOut *>(arena_alloc(ctx, sizeof(MergeOut) * std::max(1, nmerge)));
   // temporary of the library products (large merges, eager solves)
   double *libT = nullptr;
-  if (ctx->blas && !ctx->tune.own_gemm && !ctx->capturing && dc_lib_temp_words(n) > 0) {
+  if (vec && ctx->blas && !ctx->tune.own_gemm && !ctx->capturing && dc_lib_temp_words(n) > 0) {
     libT = arena_alloc_n<double>(ctx, dc_lib_temp_words(n));
     if (!libT) return EVD_E_NOMEM;
   }
@@ -1102,9 +1248,9 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
     dc_tear_kernel<<<(unsigned)std::min<long>((nt + 255) / 256, 1024), 256, 0, ctx->stream>>>(nt, dsplit, E, D);
     EVD_LAUNCHED(ctx);
     // outside the leaves' diagonal blocks Z starts as zeros
-    for (int q = 0; q < count; q++) EVD_TRY(fill_f64(ctx, Z + q * zs, n, n, ldz, 0.0));
+    for (int q = 0; vec && q < count; q++) EVD_TRY(fill_f64(ctx, Z + q * zs, n, n, ldz, 0.0));
   }
-  dc_leaf_kernel<<<(unsigned)plan->nleaf, 64, 0, ctx->stream>>>(dleaf, E, D, Z, ldz, sc.zmul, err);
+  dc_leaf_kernel<<<(unsigned)plan->nleaf, 64, 0, ctx->stream>>>(dleaf, E, D, Z, ldz, sc.zmul, rows, err);
   EVD_LAUNCHED(ctx);
 
   // Merges level by level (by height).  Launch shapes come from the largest
@@ -1119,21 +1265,33 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
     const unsigned gx = (unsigned)std::min(64, (maxN + 255) / 256);
     const bool sort_inline = maxN <= kDcSortInline;
     if (!sort_inline) {
-      dc_sort_kernel<<<dim3(gx, nm), 256, 0, ctx->stream>>>(lmd, D, Z, ldz, sc);
+      dc_sort_kernel<<<dim3(gx, nm), 256, 0, ctx->stream>>>(lmd, D, Z, ldz, sc, rows);
       EVD_LAUNCHED(ctx);
     }
-    dc_deflate_kernel<<<nm, 256, 0, ctx->stream>>>(lmd, lmo, D, Z, ldz, sort_inline ? 1 : 0, sc);
+    dc_deflate_kernel<<<nm, 256, 0, ctx->stream>>>(lmd, lmo, D, Z, ldz, sort_inline ? 1 : 0, sc, rows);
     EVD_LAUNCHED(ctx);
-    dc_rotate_kernel<<<dim3(gx, nm), 256, 0, ctx->stream>>>(lmd, lmo, Z, ldz, sc);
-    EVD_LAUNCHED(ctx);
-    dc_gather_kernel<<<dim3((unsigned)((maxN + 63) / 64), (unsigned)((maxN + 15) / 16), nm), 256, 0, ctx->stream>>>(
-        lmd, lmo, Z, ldz, sc, ldq);
-    EVD_LAUNCHED(ctx);
+    if (vec) {
+      dc_rotate_kernel<<<dim3(gx, nm), 256, 0, ctx->stream>>>(lmd, lmo, Z, ldz, sc);
+      EVD_LAUNCHED(ctx);
+      dc_gather_kernel<<<dim3((unsigned)((maxN + 63) / 64), (unsigned)((maxN + 15) / 16), nm), 256, 0, ctx->stream>>>(
+          lmd, lmo, Z, ldz, sc, ldq);
+      EVD_LAUNCHED(ctx);
+    } else if (h < H) {
+      dc_rows_rotate_kernel<<<nm, 256, 0, ctx->stream>>>(lmd, lmo, sc, rows);
+      EVD_LAUNCHED(ctx);
+    }
     const unsigned gw = (unsigned)std::min(16384, (maxN + 3) / 4);  // 4 roots (waves) per workgroup
     dc_secular_kernel<<<dim3(gw, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc, err);
     EVD_LAUNCHED(ctx);
-    dc_loewner_kernel<<<dim3(gw, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc);
-    EVD_LAUNCHED(ctx);
+    if (vec || h < H) {  // the last merge's vectors are not needed for the values
+      dc_loewner_kernel<<<dim3(gw, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc);
+      EVD_LAUNCHED(ctx);
+    }
+    if (!vec) {
+      dc_rows_kernel<<<dim3((unsigned)((maxN + 3) / 4), nm), 256, 0, ctx->stream>>>(lmd, lmo, sc, rows, h < H ? 1 : 0, D);
+      EVD_LAUNCHED(ctx);
+      continue;
+    }
     dc_vectors_kernel<<<dim3(maxN, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc, ldq, D, dtiles + 2 * off, Z, ldz, dprob);
     EVD_LAUNCHED(ctx);
     if (libT && maxN >= kDcLibMinN && !ctx->capturing)

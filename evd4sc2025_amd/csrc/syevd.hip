@@ -5,10 +5,10 @@
 //
 // Differences from the reference driver, by design:
 //  * the tridiagonal stage runs on the GPU (FP64 divide and conquer) instead
-//    of host MKL, for eigenvalues-only requests too (their tridiagonal
-//    eigenvectors stay internal: the D&C's merges need them, and it runs
-//    every eigenvalue in parallel where a Sturm-count bisection is a serial
-//    chain of n steps per eigenvalue);
+//    of host MKL, for eigenvalues-only requests too (without the vectors,
+//    only the two rows of them that the merges read; it runs every eigenvalue
+//    in parallel where a Sturm-count bisection is a serial chain of n steps per
+//    eigenvalue);
 //  * eigenvectors are formed as Z = Q_SBR (Q_BC Z_T) by applying the
 //    reflectors to Z_T directly (4 n^3 flops) instead of forming Q and a
 //    final GEMM (6 n^3 in the reference);
@@ -28,6 +28,7 @@ int stedc(evd_ctx *ctx, long n, double *D, double *E, double *Z, long ldz);
 size_t stedc_workspace(long n);
 int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double *Z, long ldz, long zs);
 size_t stedc_batched_workspace(int count, long n);
+size_t stedc_values_workspace(int count, long n);
 size_t bc_back_pack_bytes(long n, long b);
 size_t bc_back_wy_bytes(long n);
 long sbr_back_blk(long knob, long b, long wcols);
@@ -188,11 +189,9 @@ size_t syevd_workspace(long n, long b, long nb, char jobz, int precision, long s
   s += align256((size_t)(n + b) * n * sizeof(float));         // U
   s += align256((size_t)n * sizeof(double)) * 2;              // D, E
   size_t later = std::max(sy2sb_workspace(n, b, nb), sb2st_batched_workspace(1, n, b));
-  // the tridiagonal stage is the D&C for both jobz (eigenvalues only: its
-  // vectors are internal)
-  s += align256((size_t)n * n * sizeof(double));  // Z_T
-  later = std::max(later, stedc_workspace(n));
+  later = std::max(later, stedc_values_workspace(1, n));
   if (jobz == 'V' || jobz == 'v') {
+    s += align256((size_t)n * n * sizeof(double));  // Z_T
     size_t dc = stedc_workspace(n);
     size_t back = align256((size_t)blk * n * sizeof(float)) + align256((size_t)(wc / 2) * blk * sizeof(float)) +
                   ((size_t)64 << 20);
@@ -220,10 +219,10 @@ int syevd(evd_ctx *ctx, char jobz, long n, long b, long nb, float *A, long lda, 
   float *U = arena_alloc_n<float>(ctx, (size_t)ldu * n);
   double *D = arena_alloc_n<double>(ctx, (size_t)n);
   double *E = arena_alloc_n<double>(ctx, (size_t)std::max<long>(n, 1));
-  double *Zt = arena_alloc_n<double>(ctx, (size_t)n * n);
+  double *Zt = vec ? arena_alloc_n<double>(ctx, (size_t)n * n) : nullptr;
   double *sigma = arena_alloc_n<double>(ctx, 1);
   unsigned *amax = arena_alloc_n<unsigned>(ctx, 1);
-  if (!W || !Y || !band || !U || !D || !E || !Zt || !sigma || !amax) return EVD_E_NOMEM;
+  if (!W || !Y || !band || !U || !D || !E || (vec && !Zt) || !sigma || !amax) return EVD_E_NOMEM;
 
   // full symmetric storage from the lower triangle, NaN/Inf screen, scaling
   EVD_TRY(prepare_inputs(ctx, 1, n, A, lda, 0, sigma, amax));
@@ -282,9 +281,10 @@ size_t syevd_batched_workspace(int count, long n, long b, long nb, char jobz, in
                align256((size_t)(n + b) * n * sizeof(float)) + align256((size_t)n * sizeof(double)) * 2;
   size_t s = per * count + 4 * 256;
   size_t later = std::max(sy2sb_batched_workspace(count, n, b, nb), sb2st_batched_workspace(count, n, b) + ((size_t)1 << 20));
-  s += align256((size_t)n * n * count * sizeof(double));  // tridiagonal eigenvectors (internal for jobz = N)
-  later = std::max(later, stedc_batched_workspace(count, n) + ((size_t)1 << 20));
+  later = std::max(later, stedc_values_workspace(count, n) + ((size_t)1 << 20));
   if (vec) {
+    s += align256((size_t)n * n * count * sizeof(double));  // tridiagonal eigenvectors
+    later = std::max(later, stedc_batched_workspace(count, n) + ((size_t)1 << 20));
     size_t back = syevd_workspace(n, b, nb, jobz, precision, sbr_knob);  // per-problem back transformation and D&C bound
     // batched SBR back transformation: merge products, block products, partials
     back = std::max(back, sy2sb_batched_workspace(count, n, b, nb) +
@@ -314,10 +314,10 @@ int syevd_batched(evd_ctx *ctx, char jobz, int count, long n, long b, long nb, f
   float *U = arena_alloc_n<float>(ctx, (size_t)u_stride * count);
   double *D = arena_alloc_n<double>(ctx, (size_t)n * count);
   double *E = arena_alloc_n<double>(ctx, (size_t)e_stride * count);
-  double *Zt = arena_alloc_n<double>(ctx, (size_t)n * n * count);
+  double *Zt = vec ? arena_alloc_n<double>(ctx, (size_t)n * n * count) : nullptr;
   double *sigma = arena_alloc_n<double>(ctx, (size_t)count);
   unsigned *amax = arena_alloc_n<unsigned>(ctx, (size_t)count);
-  if (!band || !U || !D || !E || !Zt || !sigma || !amax) return EVD_E_NOMEM;
+  if (!band || !U || !D || !E || (vec && !Zt) || !sigma || !amax) return EVD_E_NOMEM;
 
   EVD_TRY(prepare_inputs(ctx, count, n, A, lda, a_stride, sigma, amax));
 
