@@ -16,13 +16,6 @@ int panel_qr_f64(evd_ctx *ctx, long m, long nc, const double *A, long lda, doubl
 
 namespace {
 
-// upper triangle of C (n x n) <- its lower triangle
-__global__ void mirror_lower_f64_kernel(long n, double *__restrict__ C, long ldc) {
-  for (long c = blockIdx.y; c < n; c += gridDim.y)
-    for (long r = blockIdx.x * (long)blockDim.x + threadIdx.x; r < c; r += (long)gridDim.x * blockDim.x)
-      C[r + c * ldc] = C[c + r * ldc];
-}
-
 __global__ void add_identity_f64_kernel(long m, double *Q, long ldq) {
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < m; i += (long)gridDim.x * blockDim.x)
     Q[i + i * ldq] += 1.0;
@@ -41,23 +34,22 @@ dim3 grid2(long rows, long cols) {
 
 }  // namespace
 
-// C = alpha (A B^T + B A^T) + beta C, lower triangle computed as two FP64
-// MFMA products and mirrored to the upper (the semantics of
-// tc_ozimmu_syr2k, api/TCblas/tc_ozimmu_syr2k.cu:209-341).
+// C = alpha (A B^T + B A^T) + beta C, the lower triangle on the FP64 matrix
+// cores, mirrored to the upper (the semantics of tc_ozimmu_syr2k,
+// api/TCblas/tc_ozimmu_syr2k.cu:209-341).
 int syr2k_f64(evd_ctx *ctx, long n, long k, double alpha, const double *A, long lda, const double *B, long ldb,
               double beta, double *C, long ldc) {
   if (n <= 0) return 0;
-  EVD_TRY(dgemm(ctx, 'N', 'T', n, n, k, alpha, A, lda, B, ldb, beta, C, ldc));
-  EVD_TRY(dgemm(ctx, 'N', 'T', n, n, k, alpha, B, ldb, A, lda, 1.0, C, ldc));
-  mirror_lower_f64_kernel<<<grid2(n, n), 256, 0, ctx->stream>>>(n, C, ldc);
-  EVD_LAUNCHED(ctx);
-  return 0;
+  return dsyr2k_mirror(ctx, n, k, alpha, A, lda, B, ldb, beta, C, ldc);
 }
 
-// FP64 SBR: the ZY panel loop of sy2sb (sbr.hip) on FP64 storage.
-size_t sy2sb_f64_workspace(long n, long b, long nb) {
-  return align256((size_t)n * nb * sizeof(double)) + align256((size_t)nb * b * sizeof(double)) * 2 +
-         ((size_t)64 << 20);
+// FP64 SBR: the ZY panel loop of sy2sb (sbr.hip) on FP64 storage, with its
+// fused products: both corrections of Z_p and the b x b term as one product, the
+// lazy panel update as one, every product split over K.  Panels took 390 us at n = 1500
+// (17.8 ms in all) with a launch per product and no split.
+size_t sy2sb_f64_workspace(const evd_ctx *ctx, long n, long b, long nb) {
+  return align256((size_t)n * nb * sizeof(double)) + align256((size_t)nb * b * sizeof(double)) * 3 +
+         dgemm_pair_workspace(ctx, std::max(n, nb), 2 * b) + ((size_t)64 << 20);
 }
 
 int sy2sb_f64(evd_ctx *ctx, long n, long b, long nb, double *A, long lda, double *W, long ldw, double *Y, long ldy) {
@@ -69,7 +61,7 @@ int sy2sb_f64(evd_ctx *ctx, long n, long b, long nb, double *A, long lda, double
   ArenaFrame frame(ctx);
   const long ldz = n;
   double *Z = arena_alloc_n<double>(ctx, (size_t)n * nb);
-  double *t = arena_alloc_n<double>(ctx, (size_t)nb * b);
+  double *t = arena_alloc_n<double>(ctx, (size_t)2 * nb * b);  // [Z_q^T W_p; Y_q^T W_p]
   double *t3 = arena_alloc_n<double>(ctx, (size_t)b * b);
   if (!Z || !t || !t3) return EVD_E_NOMEM;
   const long P = nb / b;
@@ -83,26 +75,37 @@ int sy2sb_f64(evd_ctx *ctx, long n, long b, long nb, double *A, long lda, double
       double *Yp = Y + r0 + c * ldy;
       double *Zp = Z + r0 + p * b * ldz;
       EVD_TRY(panel_qr_f64(ctx, m, b, Ap, lda, Yp, ldy, Wp, ldw, nullptr, 0, Ap, lda, nullptr));
-      EVD_TRY(dgemm(ctx, 'N', 'N', m, b, m, 1.0, A + r0 + r0 * lda, lda, Wp, ldw, 0.0, Zp, ldz));
+      EVD_TRY(dgemm_pair(ctx, 'N', 'N', m, b, m, 0, 1.0, A + r0 + r0 * lda, lda, Wp, ldw, nullptr, 0, nullptr, 0, 0.0,
+                         Zp, ldz));
       if (p > 0) {
-        const long pb = p * b;
+        // as in sy2sb: [Z_q Z_p]^T W_p and [Y_q Y_p]^T W_p give t_z, t_y and
+        // X1 = Z_p^T W_p; t3^T / 2 = (X1 - t_y^T t_z - t_z^T t_y) / 2 takes X1's
+        // place, and Z_p -= Y_q t_z + Y_p t3 / 2 + Z_q t_y is one product
+        const long pb = p * b, pbx = pb + b;
         const double *Yq = Y + r0 + c0 * ldy;
         const double *Zq = Z + r0;
-        EVD_TRY(dgemm(ctx, 'T', 'N', pb, b, m, 1.0, Zq, ldz, Wp, ldw, 0.0, t, pb));
-        EVD_TRY(dgemm(ctx, 'N', 'N', m, b, pb, -1.0, Yq, ldy, t, pb, 1.0, Zp, ldz));
-        EVD_TRY(dgemm(ctx, 'T', 'N', pb, b, m, 1.0, Yq, ldy, Wp, ldw, 0.0, t, pb));
-        EVD_TRY(dgemm(ctx, 'N', 'N', m, b, pb, -1.0, Zq, ldz, t, pb, 1.0, Zp, ldz));
+        double *tz = t, *ty = t + pbx * b;
+        if (ldy == ldz) {
+          const long dYZ = (long)(reinterpret_cast<intptr_t>(Yq) - reinterpret_cast<intptr_t>(Zq)) / (long)sizeof(double);
+          EVD_TRY(dgemm_pair(ctx, 'T', 'N', pbx, b, m, 0, 1.0, Zq, ldz, Wp, ldw, nullptr, 0, nullptr, 0, 0.0, tz, pbx, 2,
+                             dYZ, pbx * b));
+        } else {
+          EVD_TRY(dgemm_pair(ctx, 'T', 'N', pbx, b, m, 0, 1.0, Zq, ldz, Wp, ldw, nullptr, 0, nullptr, 0, 0.0, tz, pbx));
+          EVD_TRY(dgemm_pair(ctx, 'T', 'N', pbx, b, m, 0, 1.0, Yq, ldy, Wp, ldw, nullptr, 0, nullptr, 0, 0.0, ty, pbx));
+        }
+        EVD_TRY(dgemm_pair(ctx, 'T', 'N', b, b, pb, pb, -0.5, ty, pbx, tz, pbx, tz, pbx, ty, pbx, 0.5, tz + pb, pbx));
+        EVD_TRY(dgemm_pair(ctx, 'N', 'N', m, b, pbx, pb, -1.0, Yq, ldy, tz, pbx, Zq, ldz, ty, pbx, 1.0, Zp, ldz));
+      } else {
+        EVD_TRY(dgemm_pair(ctx, 'T', 'N', b, b, m, 0, 1.0, Wp, ldw, Zp, ldz, nullptr, 0, nullptr, 0, 0.0, t3, b));
+        EVD_TRY(dgemm_pair(ctx, 'N', 'N', m, b, b, 0, -0.5, Yp, ldy, t3, b, nullptr, 0, nullptr, 0, 1.0, Zp, ldz));
       }
-      EVD_TRY(dgemm(ctx, 'T', 'N', b, b, m, 1.0, Wp, ldw, Zp, ldz, 0.0, t3, b));
-      EVD_TRY(dgemm(ctx, 'N', 'N', m, b, b, -0.5, Yp, ldy, t3, b, 1.0, Zp, ldz));
       const long kk = (p + 1) * b;
       const double *Ya = Y + r0 + c0 * ldy;
       const double *Za = Z + r0;
       const bool more = (p + 1 < P) && (n - (r0 + b) > 1);
       if (more) {
-        double *An = A + r0 + r0 * lda;
-        EVD_TRY(dgemm(ctx, 'N', 'T', m, b, kk, -1.0, Ya, ldy, Za, ldz, 1.0, An, lda));
-        EVD_TRY(dgemm(ctx, 'N', 'T', m, b, kk, -1.0, Za, ldz, Ya, ldy, 1.0, An, lda));
+        EVD_TRY(dgemm_pair(ctx, 'N', 'T', m, b, kk, kk, -1.0, Ya, ldy, Za, ldz, Za, ldz, Ya, ldy, 1.0, A + r0 + r0 * lda,
+                           lda));
         continue;
       }
       EVD_TRY(syr2k_f64(ctx, m, kk, -1.0, Ya, ldy, Za, ldz, 1.0, A + r0 + r0 * lda, lda));
@@ -302,7 +305,7 @@ extern "C" int evd_sy2sb_f64(evd_ctx *ctx, long n, long b, long nb, double *A, l
   EVD_ARG(ctx, lda >= std::max<long>(1, n), 6);
   EVD_ARG(ctx, ldw >= std::max<long>(1, n), 8);
   EVD_ARG(ctx, ldy >= std::max<long>(1, n), 10);
-  if (ctx->arena_top == 0) EVD_TRY(arena_ensure(ctx, sy2sb_f64_workspace(n, b, nb)));
+  if (ctx->arena_top == 0) EVD_TRY(arena_ensure(ctx, sy2sb_f64_workspace(ctx, n, b, nb)));
   return sy2sb_f64(ctx, n, b, nb, A, lda, W, ldw, Y, ldy);
 }
 

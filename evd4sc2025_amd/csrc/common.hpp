@@ -177,6 +177,12 @@ int sgemm_kcat(evd_ctx *ctx, char ta, char tb, long m, long n, long k1, long k2,
                long sC = 0);
 int dgemm(evd_ctx *ctx, char ta, char tb, long m, long n, long k, double alpha, const double *A, long lda,
           const double *B, long ldb, double beta, double *C, long ldc);
+int dgemm_pair(evd_ctx *ctx, char ta, char tb, long m, long n, long k1, long k2, double alpha, const double *A1,
+               long lda1, const double *B1, long ldb1, const double *A2, long lda2, const double *B2, long ldb2,
+               double beta, double *C, long ldc, long batch = 1, long sA = 0, long sC = 0);
+size_t dgemm_pair_workspace(const evd_ctx *ctx, long m, long n);
+int dsyr2k_mirror(evd_ctx *ctx, long n, long k, double alpha, const double *A, long lda, const double *B, long ldb,
+                  double beta, double *C, long ldc);
 int syr2k_lower_mirror(evd_ctx *ctx, long n, long k, float alpha, const float *A, long lda, const float *B, long ldb,
                        float beta, float *C, long ldc);
 int syr2k_lower_mirror_batched(evd_ctx *ctx, int count, long n, long k, float alpha, const float *A, long lda,

@@ -1170,6 +1170,150 @@ int dgemm(evd_ctx *ctx, char ta, char tb, long m, long n, long k, double alpha, 
   return 0;
 }
 
+// FP64 products of the band reduction: C = alpha (op(A1) op(B1) + op(A2) op(B2))
+// + beta C, the second pair optional, K split over workgroups.  The panels are 32 or 64
+// columns wide, so without a split their products ran on m / 64 workgroups (or one,
+// for the b x b and pb x b ones) for K up to n: 55 us a product at n = 1500.
+// SYM: A1 = B2, B1 = A2, the tiles on and below the diagonal, mirrored.
+template <bool TA, bool TB, int BN, bool SYM>
+__global__ __launch_bounds__(256) void dgemm_pair_kernel(int M, int N, int K1, int K2, double alpha,
+                                                         const double *__restrict__ A1, long lda1,
+                                                         const double *__restrict__ B1, long ldb1,
+                                                         const double *__restrict__ A2, long lda2,
+                                                         const double *__restrict__ B2, long ldb2, double beta,
+                                                         double *__restrict__ C, long ldc, int kchunk, int ksplit,
+                                                         double *__restrict__ P, long batches, long sA, long sC) {
+  constexpr int BM = 64, WM = BN == 32 ? 4 : 2, WN = 4 / WM, MI = BM / WM / 16, NI = BN / WN / 16;
+  using L = TileLoader<TA, TB, BM, BN, WM, WN, double>;
+  __shared__ __align__(16) double As[2 * kBK * L::LDSA];
+  __shared__ __align__(16) double Bs[2 * kBK * L::LDSB];
+  int ti = blockIdx.x, tj = blockIdx.y;
+  if (SYM) {
+    const long t = blockIdx.x;
+    ti = (int)((sqrt(8.0 * (double)t + 1.0) - 1.0) * 0.5);
+    while ((long)(ti + 1) * (ti + 2) / 2 <= t) ti++;
+    while ((long)ti * (ti + 1) / 2 > t) ti--;
+    tj = (int)(t - (long)ti * (ti + 1) / 2);
+  }
+  const long batch = blockIdx.z / ksplit;
+  const int kz = blockIdx.z % ksplit, kb = kz * kchunk, ke = min(K1 + K2, kb + kchunk);
+  const int m0 = ti * BM, n0 = tj * BN;
+  A1 += batch * sA;
+  C += batch * sC;
+  f64x4 acc[MI][NI];
+#pragma unroll
+  for (int mi = 0; mi < MI; mi++)
+#pragma unroll
+    for (int ni = 0; ni < NI; ni++) acc[mi][ni] = f64x4{0., 0., 0., 0.};
+  if (kb < K1)
+    tile_mainloop<TA, TB, BM, BN, WM, WN, double, f64x4>(A1, lda1, B1, ldb1, M, N, m0, n0, kb, min(ke, K1), As, Bs, acc);
+  if (ke > K1)
+    tile_mainloop<TA, TB, BM, BN, WM, WN, double, f64x4>(A2, lda2, B2, ldb2, M, N, m0, n0, max(kb, K1) - K1, ke - K1, As,
+                                                          Bs, acc);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int wm = wave % WM, wn = wave / WM;
+#pragma unroll
+  for (int mi = 0; mi < MI; mi++) {
+    const int row = m0 + wm * (BM / WM) + mi * 16 + (lane & 15);
+    if (row >= M) continue;
+#pragma unroll
+    for (int ni = 0; ni < NI; ni++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int col = n0 + wn * (BN / WN) + ni * 16 + acc_row(0.0, lane, r);
+        if (col >= N || (SYM && col > row)) continue;
+        if (ksplit > 1) {
+          P[((long)kz * batches + batch) * (long)M * N + row + (long)col * M] = acc[mi][ni][r];
+          continue;
+        }
+        const long o = row + (long)col * ldc;
+        const double v = (beta == 0.0) ? alpha * acc[mi][ni][r] : alpha * acc[mi][ni][r] + beta * C[o];
+        C[o] = v;
+        if (SYM && col != row) C[col + (long)row * ldc] = v;
+      }
+  }
+}
+
+__global__ void dsplitk_reduce_kernel(int M, int N, long batches, int ksplit, const double *__restrict__ P, double alpha,
+                                      double beta, double *__restrict__ C, long ldc, long sC) {
+  const long mn = (long)M * N, total = mn * batches;
+  for (long t = blockIdx.x * (long)blockDim.x + threadIdx.x; t < total; t += (long)gridDim.x * blockDim.x) {
+    const long b = t / mn, rc = t % mn;
+    const double *p = P + b * mn + rc;
+    double s = 0.0;
+    int kz = 0;
+    for (; kz + 8 <= ksplit; kz += 8) {
+      double v[8];
+#pragma unroll
+      for (int u = 0; u < 8; u++) v[u] = p[(long)(kz + u) * total];
+#pragma unroll
+      for (int u = 0; u < 8; u++) s += v[u];
+    }
+    for (; kz < ksplit; kz++) s += p[(long)kz * total];
+    const long o = b * sC + rc % M + (rc / M) * ldc;
+    C[o] = (beta == 0.0) ? alpha * s : alpha * s + beta * C[o];
+  }
+}
+
+template <bool TA, bool TB, int BN>
+static int launch_dgemm_pair(evd_ctx *ctx, long m, long n, long k1, long k2, double alpha, const double *A1, long lda1,
+                             const double *B1, long ldb1, const double *A2, long lda2, const double *B2, long ldb2,
+                             double beta, double *C, long ldc, long batch, long sA, long sC) {
+  // two workgroups per CU, chunks of at least 64 of K
+  const long tiles = ((m + 63) / 64) * ((n + BN - 1) / BN) * batch, k = k1 + k2;
+  long ksplit = std::max<long>(1, std::min<long>((2L * ctx->num_cus + tiles - 1) / tiles, std::min<long>(k / 64, 64)));
+  const long kchunk = ((k + ksplit - 1) / ksplit + kBK - 1) / kBK * kBK;
+  ksplit = std::max<long>(1, (k + kchunk - 1) / kchunk);
+  ArenaFrame frame(ctx);
+  double *P = nullptr;
+  if (ksplit > 1) {
+    P = arena_alloc_n<double>(ctx, (size_t)ksplit * batch * m * n);
+    if (!P) return EVD_E_NOMEM;
+  }
+  dgemm_pair_kernel<TA, TB, BN, false>
+      <<<dim3((unsigned)((m + 63) / 64), (unsigned)((n + BN - 1) / BN), (unsigned)(batch * ksplit)), 256, 0, ctx->stream>>>(
+          (int)m, (int)n, (int)k1, (int)k2, alpha, A1, lda1, B1, ldb1, A2, lda2, B2, ldb2, beta, C, ldc, (int)kchunk,
+          (int)ksplit, P, batch, sA, sC);
+  EVD_LAUNCHED(ctx);
+  if (ksplit > 1) {
+    dsplitk_reduce_kernel<<<(unsigned)std::min<long>((m * n * batch + 255) / 256, 4096), 256, 0, ctx->stream>>>(
+        (int)m, (int)n, batch, (int)ksplit, P, alpha, beta, C, ldc, sC);
+    EVD_LAUNCHED(ctx);
+  }
+  return 0;
+}
+
+// Partials a dgemm_pair call takes from the arena: at most two workgroups' tiles
+// per CU beyond one copy of the output, 64 x 64 each.
+size_t dgemm_pair_workspace(const evd_ctx *ctx, long m, long n) {
+  return ((size_t)m * n + (size_t)2 * ctx->num_cus * 64 * 64) * 2 * sizeof(double);
+}
+
+int dgemm_pair(evd_ctx *ctx, char ta, char tb, long m, long n, long k1, long k2, double alpha, const double *A1,
+               long lda1, const double *B1, long ldb1, const double *A2, long lda2, const double *B2, long ldb2,
+               double beta, double *C, long ldc, long batch, long sA, long sC) {
+  if (m <= 0 || n <= 0 || k1 + k2 <= 0) return 0;
+  const bool TA = ta == 'T', TB = tb == 'T', narrow = n <= 32;
+  if (TA && TB) return set_error(ctx, EVD_E_UNSUPPORTED, "dgemm_pair: transposes %c %c", ta, tb);
+  auto call = [&](auto fn) {
+    return fn(ctx, m, n, k1, k2, alpha, A1, lda1, B1, ldb1, A2, lda2, B2, ldb2, beta, C, ldc, batch, sA, sC);
+  };
+  if (TA) return narrow ? call(launch_dgemm_pair<true, false, 32>) : call(launch_dgemm_pair<true, false, 64>);
+  if (TB) return narrow ? call(launch_dgemm_pair<false, true, 32>) : call(launch_dgemm_pair<false, true, 64>);
+  return narrow ? call(launch_dgemm_pair<false, false, 32>) : call(launch_dgemm_pair<false, false, 64>);
+}
+
+// C = alpha (A B^T + B A^T) + beta C from the tiles on and below the diagonal
+int dsyr2k_mirror(evd_ctx *ctx, long n, long k, double alpha, const double *A, long lda, const double *B, long ldb,
+                  double beta, double *C, long ldc) {
+  const long nt = (n + 63) / 64;
+  dgemm_pair_kernel<false, true, 64, true><<<(unsigned)(nt * (nt + 1) / 2), 256, 0, ctx->stream>>>(
+      (int)n, (int)n, (int)k, (int)k, alpha, A, lda, B, ldb, B, ldb, A, lda, beta, C, ldc, (int)(2 * k), 1, nullptr, 1, 0,
+      0);
+  EVD_LAUNCHED(ctx);
+  return 0;
+}
+
 // Grouped FP64 GEMM: one workgroup per 64x64 output tile of one problem.
 __global__ __launch_bounds__(256) void dgemm_grouped_kernel(const DGemmProblem *__restrict__ probs, int nprob,
                                                             int total_tiles) {
