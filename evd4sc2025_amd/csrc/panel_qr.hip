@@ -392,6 +392,9 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
   }
 }
 
+// launches of the column-exchange kernel that may run on one card at once
+constexpr int kPanelLaunches = 16;
+
 template <int NB, int RPT, typename T>
 static int launch_panel(evd_ctx *ctx, long m, long nc, const T *A, long lda, T *Y, long ldy, T *W, long ldw, T *R,
                         long ldr, T *Aout, long ldo, double *tau_out, int count = 1, long s_in = 0, long s_y = 0,
@@ -415,9 +418,17 @@ static int launch_panel(evd_ctx *ctx, long m, long nc, const T *A, long lda, T *
   int mi = (int)m, ni = (int)nc;
   void *args[] = {&mi, &ni, (void *)&A, &lda, &Y, &ldy, &W, &ldw, &R, &ldr, &Aout, &ldo, &part, &tau_out,
                   &tags, &epoch_word, &err, &s_in, &s_y, &s_w, &s_out, (void *)&only_bad};
-  // one workgroup is trivially co-resident: a regular launch, which (unlike a
-  // cooperative one) may overlap with the work of other streams
-  if (G == 1)
+  // The groups of a launch wait for each other, so all of them have to become
+  // resident.  A cooperative launch sees to that, but goes through a queue of
+  // its own: 11 us before and 11 us after a kernel that, as the fallback of
+  // the Cholesky QR path, mostly has nothing to do.  A regular launch is as
+  // safe while all launches that can run at once fit together: every other
+  // kernel here ends by itself (the chase waits on running workgroups only), so
+  // groups that have to wait for room get it as long as these launches
+  // alone never fill the card.  HIP runs at most four kernels of a process at
+  // once (its hardware queues); 1/16 of the card leaves room for four
+  // processes that do: 32 groups, m <= 16384.  Larger panels stay cooperative.
+  if (G == 1 || (long)G * count <= maxres / kPanelLaunches)
     EVD_HIP(ctx, hipLaunchKernel((const void *)panel_qr_kernel<NB, RPT, T>, dim3(G, count), dim3(256), args, 0,
                                  ctx->stream));
   else

@@ -1,0 +1,66 @@
+"""Cholesky QR panels at the edges of their tiles: rows around the 64 of an
+output workgroup, the 256 of a Gram workgroup and the 2048 of a reduction
+group, fewer columns than the 32 of a tile, and rank-deficient panels whose
+fallback runs in one workgroup, in several on a regular launch, and above the
+limit of regular launches."""
+import numpy as np
+import pytest
+
+from oracle import evd_oracle as O
+from tests.helpers import to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+
+def _factor(ctx, P, dtype):
+    import torch
+
+    import evd4sc2025_amd as E
+
+    m, b = P.shape
+    dA = to_dev(P.astype(dtype))
+    tt = torch.float32 if dtype == np.float32 else torch.float64
+    dW, dR = E.colmajor(m, b, dtype=tt, fill=0.0), E.colmajor(b, b, dtype=tt, fill=0.0)
+    E.panelQR(ctx, dA, dW, dR)
+    torch.cuda.synchronize()
+    return [to_host(x).astype(np.float64) for x in (dA, dW, dR)]
+
+
+def _check(P, Y, W, R, eps):
+    m, b = P.shape
+    # the sums of the factorisation have m terms, those of its products b
+    tol = 4 * b * eps * np.sqrt(m) * max(1.0, np.abs(P).max())
+    Y = np.tril(Y, -1) + np.eye(m, b)
+    Rf = np.zeros((m, b))
+    Rf[:b] = np.triu(R)
+    assert np.abs(Rf - W @ (Y.T @ Rf) - P).max() < tol
+    Qt = np.eye(m, b) - W @ Y[:b].T
+    assert np.abs(Qt.T @ Qt - np.eye(b)).max() < tol
+    return Y, tol
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("m,b", [(2, 1), (34, 17), (64, 32), (65, 31), (129, 32), (256, 32), (257, 17), (2048, 32),
+                                 (2049, 32), (4097, 31)])
+def test_panel_edges(ctx, m, b, dtype):
+    print(f"panel m={m} b={b} {dtype.__name__}", flush=True)
+    P = np.random.default_rng(m + b).standard_normal((m, b)).astype(dtype)
+    Y, W, R = _factor(ctx, P, dtype)
+    P = P.astype(np.float64)
+    Y, tol = _check(P, Y, W, R, np.finfo(dtype).eps)
+    V, T, R0, _ = O.panel_qr(P)
+    # well conditioned: the reflectors themselves, sqrt(m) beyond the residual
+    # for the columns' norm
+    assert np.abs(Y - V).max() < tol * np.sqrt(m)
+    assert np.abs(W - V @ T).max() < tol * np.sqrt(m)
+
+
+@pytest.mark.parametrize("m", [300, 3000, 16384, 16900])
+def test_panel_fallback_launches(ctx, m):
+    print(f"panel fallback m={m}", flush=True)
+    P = np.random.default_rng(m).standard_normal((m, 32)).astype(np.float32)
+    P[:, 9] = P[:, 4]
+    P[:, 30] = 0.0
+    for _ in range(2):
+        Y, W, R = _factor(ctx, P, np.float32)
+        _check(P.astype(np.float64), Y, W, R, np.finfo(np.float32).eps)
