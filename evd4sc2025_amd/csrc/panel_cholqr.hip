@@ -41,7 +41,8 @@ namespace {
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kQ = 32;          // columns of a panel (padded)
-constexpr int kRows = 256;      // rows per workgroup of the row kernels
+constexpr int kRows = 256;      // rows per workgroup of the Gram passes
+constexpr int kOut = 64;        // rows per workgroup of the output kernel
 constexpr int kGroup = 8;       // partial Gram matrices summed per reduction step
 constexpr int kQQ = kQ * kQ;    // one 32 x 32 matrix
 constexpr int kLD = kQ + 1;     // LDS pitch of a 32 x 32 matrix or of a row
@@ -101,10 +102,10 @@ __device__ __forceinline__ void load_mat(const double *__restrict__ src, double 
   }
 }
 
-// dst = sum of the n 32 x 32 matrices src[0 .. n) (kQQ doubles apart), added
-// in index order; written by other workgroups of this launch, so read and
-// written with device-coherent accesses.  Call from all 256 threads.
-__device__ __forceinline__ void sum_slots(const double *src, int n, double *dst, int tid, double (&sum)[4]) {
+// sum of the n 32 x 32 matrices src[0 .. n) (kQQ doubles apart), added in index
+// order; written by other workgroups of this launch, so read with
+// device-coherent accesses.  Call from all 256 threads.
+__device__ __forceinline__ void sum_slots(const double *src, int n, double (&sum)[4], int tid) {
 #pragma unroll
   for (int r = 0; r < 4; r++) sum[r] = 0.0;
   for (int g0 = 0; g0 < n; g0 += 8) {
@@ -118,8 +119,6 @@ __device__ __forceinline__ void sum_slots(const double *src, int n, double *dst,
 #pragma unroll
       for (int r = 0; r < 4; r++) sum[r] += (g0 + u < n) ? v[u][r] : 0.0;
   }
-#pragma unroll
-  for (int r = 0; r < 4; r++) st_dev(&dst[tid + 256 * r], sum[r]);
 }
 
 // Counts this workgroup into *cnt (n members) after its coherent stores are
@@ -138,38 +137,39 @@ __device__ __forceinline__ bool last_arrival(unsigned *cnt, unsigned n) {
   return s_last != 0;
 }
 
-// Rows 64w .. 64w+63 of xs (LDS, pitch kLD) times the 32 x 32 matrix B (LDS,
-// pitch kLD) on wave w: acc[p][t][r] = C[64w + 16p + (lane & 15)][16t +
-// (lane >> 4) + 4r].  The MFMA takes B as its first operand, so the
-// accumulator lane index runs down the rows.
-__device__ __forceinline__ void wave_rows_times(const double *xs, const double *B, int w, int lane,
-                                                f64x4 (&acc)[4][2]) {
+// The 16 P rows at xs (LDS, pitch kLD) times the 32 x 32 matrix B (LDS, pitch
+// kLD) on one wave: acc[p][t][r] = C[16p + (lane & 15)][16t + (lane >> 4) +
+// 4r].  The MFMA takes B as its first operand, so the accumulator lane index
+// runs down the rows.
+template <int P>
+__device__ __forceinline__ void wave_rows_times(const double *xs, const double *B, int lane, f64x4 (&acc)[P][2]) {
 #pragma unroll
-  for (int p = 0; p < 4; p++)
+  for (int p = 0; p < P; p++)
 #pragma unroll
     for (int t = 0; t < 2; t++) acc[p][t] = f64x4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
   for (int ks = 0; ks < kQ / 4; ks++) {
     const int k = 4 * ks + (lane >> 4);
-    double a[4], b[2];
+    double a[P], b[2];
 #pragma unroll
-    for (int p = 0; p < 4; p++) a[p] = xs[(64 * w + 16 * p + (lane & 15)) * kLD + k];
+    for (int p = 0; p < P; p++) a[p] = xs[(16 * p + (lane & 15)) * kLD + k];
 #pragma unroll
     for (int t = 0; t < 2; t++) b[t] = B[k * kLD + 16 * t + (lane & 15)];
 #pragma unroll
-    for (int p = 0; p < 4; p++)
+    for (int p = 0; p < P; p++)
 #pragma unroll
       for (int t = 0; t < 2; t++) acc[p][t] = mfma64(b[t], a[p], acc[p][t]);
   }
 }
 
-__device__ __forceinline__ void wave_store_rows(double *xs, int w, int lane, const f64x4 (&acc)[4][2]) {
+template <int P>
+__device__ __forceinline__ void wave_store_rows(double *xs, int lane, const f64x4 (&acc)[P][2]) {
 #pragma unroll
-  for (int p = 0; p < 4; p++)
+  for (int p = 0; p < P; p++)
 #pragma unroll
     for (int t = 0; t < 2; t++)
 #pragma unroll
-      for (int r = 0; r < 4; r++) xs[(64 * w + 16 * p + (lane & 15)) * kLD + 16 * t + (lane >> 4) + 4 * r] = acc[p][t][r];
+      for (int r = 0; r < 4; r++) xs[(16 * p + (lane & 15)) * kLD + 16 * t + (lane >> 4) + 4 * r] = acc[p][t][r];
 }
 
 // Gram matrix of the panel's rows: rows of A (MODE 0) or of Q1 = A R1^-1
@@ -180,7 +180,7 @@ __device__ __forceinline__ void wave_store_rows(double *xs, int w, int lane, con
 // group of kGroup sums the group's partials into a level-2 slot, and the
 // last group to finish sums those into the final slot (always in index
 // order, so the sum does not depend on arrival order).  part per problem:
-// [ng partials][ngroups level-2 sums][final]; cnt: ngroups + 1 counters per
+// [ng partials][ngroups level-2 sums]; cnt: ngroups + 1 counters per
 // problem, zero between launches.  Returns true in the workgroup that formed
 // the final sum, whose thread t then holds its elements t + 256 r in gv[r].
 // A, fac, part and cnt point at this problem's data; xs has kRows * kLD
@@ -200,9 +200,9 @@ __device__ __forceinline__ bool gram_pass(int m, int nc, const T *__restrict__ A
   if (MODE == 1) {
     __syncthreads();  // ri
     f64x4 qa[4][2];
-    wave_rows_times(xs, ri, w, lane, qa);
+    wave_rows_times(xs + 64 * w * kLD, ri, lane, qa);
     lds_order();
-    wave_store_rows(xs, w, lane, qa);
+    wave_store_rows(xs + 64 * w * kLD, lane, qa);
   }
   lds_order();
   // acc[0] = G[0:16][0:16], acc[1] = G[0:16][16:32], acc[2] = G[16:32][16:32];
@@ -232,13 +232,22 @@ __device__ __forceinline__ bool gram_pass(int m, int nc, const T *__restrict__ A
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const int e = tid + 256 * r;
-    st_dev(&part[(long)g * kQQ + e], ((xs[e] + xs[kQQ + e]) + xs[2 * kQQ + e]) + xs[3 * kQQ + e]);
+    gv[r] = ((xs[e] + xs[kQQ + e]) + xs[2 * kQQ + e]) + xs[3 * kQQ + e];
   }
+  if (ng == 1) {
+    __syncthreads();  // xs is free
+    return true;
+  }
+#pragma unroll
+  for (int r = 0; r < 4; r++) st_dev(&part[(long)g * kQQ + tid + 256 * r], gv[r]);
   const int grp = g / kGroup, gsize = min(kGroup, ng - grp * kGroup);
   if (!last_arrival(cnt + grp, (unsigned)gsize)) return false;
-  sum_slots(part + (long)grp * kGroup * kQQ, gsize, part + (long)(ng + grp) * kQQ, tid, gv);
+  sum_slots(part + (long)grp * kGroup * kQQ, gsize, gv, tid);
+  if (ngroups == 1) return true;
+#pragma unroll
+  for (int r = 0; r < 4; r++) st_dev(&part[(long)(ng + grp) * kQQ + tid + 256 * r], gv[r]);
   if (!last_arrival(cnt + ngroups, (unsigned)ngroups)) return false;
-  sum_slots(part + (long)ng * kQQ, ngroups, part + (long)(ng + ngroups) * kQQ, tid, gv);
+  sum_slots(part + (long)ng * kQQ, ngroups, gv, tid);
   return true;
 }
 
@@ -304,22 +313,20 @@ __device__ __forceinline__ bool wave_cholesky(const double *G, double *R, int la
 // X = U^-1 for an upper triangular 32 x 32 U on one wave: lane c forms column
 // c by right-looking back substitution (x_k is final once the rows below k
 // are applied, and the updates of the rows above it are independent, so the
-// dependent chain is one multiply-add per step; the diagonal's reciprocals
-// are formed up front).  UNIT_LT: U is the transpose of the unit lower
+// dependent chain is one multiply-add per step; lane i divides for the
+// diagonal's reciprocal i).  UNIT_LT: U is the transpose of the unit lower
 // triangle stored in M (U[i][k] = M[k][i], unit diagonal); otherwise U is
 // M's upper triangle.
 template <bool UNIT_LT>
 __device__ __forceinline__ void wave_upper_inverse(const double *M, double *X, int lane) {
   const int c = lane & (kQ - 1);
-  double s[kQ], rd[kQ];
+  const double rd = UNIT_LT ? 1.0 : 1.0 / M[c * kLD + c];
+  double s[kQ];
 #pragma unroll
-  for (int i = 0; i < kQ; i++) {
-    s[i] = (i == c) ? 1.0 : 0.0;
-    rd[i] = UNIT_LT ? 1.0 : 1.0 / M[i * kLD + i];
-  }
+  for (int i = 0; i < kQ; i++) s[i] = (i == c) ? 1.0 : 0.0;
 #pragma unroll
   for (int k = kQ - 1; k >= 0; k--) {
-    const double xk = s[k] * rd[k];
+    const double xk = UNIT_LT ? s[k] : s[k] * lane_value(rd, k);
     s[k] = xk;
 #pragma unroll
     for (int i = 0; i < k; i++) s[i] -= (UNIT_LT ? M[k * kLD + i] : M[i * kLD + k]) * xk;
@@ -533,9 +540,12 @@ __global__ __launch_bounds__(256) void cq_pass_kernel(int m, int nc, const T *__
 }
 
 
-// Outputs, 256 rows per workgroup: V = A M (rows < 32: V1), W = V T on MFMA
-// through LDS (each wave on its own 64 rows), then Y = V, W, [R_H; 0] (Aout),
-// R and tau with one thread per row.
+// Outputs, kOut rows per workgroup: V = A M (rows < 32: V1), W = V T on MFMA
+// through LDS (each wave on its own 16 rows), then Y = V, W, [R_H; 0] (Aout),
+// R and tau.  A wave moves eight columns of the 64 rows.  The kernel is one
+// chain of loads, two products and stores; 64 rows a workgroup (256 before)
+// spread it over four times the CUs and shorten each part: m = 1000:
+// 14.7 -> 7.9 us; mean over the panels of n = 16384: 9.9 us.
 template <typename T>
 __global__ __launch_bounds__(256) void cq_out_kernel(int m, int nc, const T *__restrict__ A, long lda, long s_in,
                                                      const double *__restrict__ fac, T *__restrict__ Y, long ldy,
@@ -543,79 +553,75 @@ __global__ __launch_bounds__(256) void cq_out_kernel(int m, int nc, const T *__r
                                                      T *__restrict__ Aout, long ldo, long s_out, T *__restrict__ R,
                                                      long ldr, double *__restrict__ tau_out,
                                                      const int *__restrict__ state) {
-  const int g = blockIdx.x, q = blockIdx.y, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int g = blockIdx.x, q = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   // every global load of the kernel is issued before the first wait: the
-  // state word, this group's rows, M and T, and (group 0) V1 and R_H
+  // state word, this workgroup's rows, M and T, and (rows < 32) V1 and R_H
   const int st = state[q];
   A += q * s_in;
   Y += q * s_y;
   W += q * s_w;
   if (Aout) Aout += q * s_out;
   fac += (long)q * kFactorWords;
-  __shared__ double xs[kRows * kLD];
-  __shared__ double Ms[kQ * kLD], Ts[kQ * kLD], V1s[kQ * kLD], RHs[kQ * kLD];
-  const long r = (long)g * kRows + tid;
-  double a[kQ], fv[4][4];
-  load_row(A, lda, m, nc, r, a);
+  __shared__ double xs[kOut * kLD];
+  __shared__ double Ms[kQ * kLD], Ts[kQ * kLD];
+  const long r = (long)g * kOut + lane;
+  const bool rin = r < m, top = r < kQ;
+  T a[8];
+  double fv[2][4], v1[8], rh[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const int c = 8 * w + k;
+    a[k] = A[(rin ? r : 0) + (long)(c < nc ? c : 0) * lda];
+  }
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     fv[0][u] = fac[kF_M + tid + 256 * u];
     fv[1][u] = fac[kF_T + tid + 256 * u];
   }
-  if (g == 0) {
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-      fv[2][u] = fac[kF_V1 + tid + 256 * u];
-      fv[3][u] = fac[kF_RH + tid + 256 * u];
-    }
+  for (int k = 0; k < 8; k++) {
+    v1[k] = top ? fac[kF_V1 + r * kQ + 8 * w + k] : 0.0;
+    rh[k] = top ? fac[kF_RH + r * kQ + 8 * w + k] : 0.0;
   }
   if (st != kDone) return;
 #pragma unroll
-  for (int c = 0; c < kQ; c++) xs[tid * kLD + c] = a[c];
+  for (int k = 0; k < 8; k++) xs[lane * kLD + 8 * w + k] = (rin && 8 * w + k < nc) ? (double)a[k] : 0.0;
 #pragma unroll
   for (int u = 0; u < 4; u++) {
     const int e = tid + 256 * u, o = (e / kQ) * kLD + e % kQ;
     Ms[o] = fv[0][u];
     Ts[o] = fv[1][u];
-    if (g == 0) {
-      V1s[o] = fv[2][u];
-      RHs[o] = fv[3][u];
-    }
   }
   __syncthreads();
-  f64x4 acc[4][2];
-  wave_rows_times(xs, Ms, w, lane, acc);
+  f64x4 acc[1][2];
+  wave_rows_times(xs + 16 * w * kLD, Ms, lane, acc);
   lds_order();
-  wave_store_rows(xs, w, lane, acc);  // V (wave-local rows)
-  if (r < kQ) {
+  wave_store_rows(xs + 16 * w * kLD, lane, acc);  // V
+  __syncthreads();
 #pragma unroll
-    for (int c = 0; c < kQ; c++) xs[tid * kLD + c] = V1s[r * kLD + c];
+  for (int k = 0; k < 8; k++) {
+    const int c = 8 * w + k;
+    if (top) xs[lane * kLD + c] = v1[k];
+    const double v = top ? v1[k] : xs[lane * kLD + c];
+    if (rin && c < nc && Y) Y[r + (long)c * ldy] = (T)v;
   }
+  __syncthreads();
+  wave_rows_times(xs + 16 * w * kLD, Ts, lane, acc);  // W = V T
   lds_order();
-  wave_rows_times(xs, Ts, w, lane, acc);  // W = V T
-  if (r < m && Y) {
+  wave_store_rows(xs + 16 * w * kLD, lane, acc);
+  __syncthreads();
+  if (rin) {
 #pragma unroll
-    for (int c = 0; c < kQ; c++)
-      if (c < nc) Y[r + (long)c * ldy] = (T)xs[tid * kLD + c];
-  }
-  lds_order();
-  wave_store_rows(xs, w, lane, acc);
-  lds_order();
-  if (r < m) {
-#pragma unroll
-    for (int c = 0; c < kQ; c++) {
-      if (c >= nc) continue;
-      if (W) W[r + (long)c * ldw] = (T)xs[tid * kLD + c];
-      if (r < kQ) {
-        const double rv = (r <= c) ? RHs[r * kLD + c] : 0.0;
-        if (Aout) Aout[r + (long)c * ldo] = (T)rv;
-        if (R && r < nc) R[r + (long)c * ldr] = (T)rv;
-      } else if (Aout) {
-        Aout[r + (long)c * ldo] = (T)0;
-      }
+    for (int k = 0; k < 8; k++) {
+      const int c = 8 * w + k;
+      const T rv = (T)((r <= c) ? rh[k] : 0.0);
+      if (c < nc && W) W[r + (long)c * ldw] = (T)xs[lane * kLD + c];
+      if (c < nc && Aout) Aout[r + (long)c * ldo] = rv;
+      if (c < nc && R && r < nc) R[r + (long)c * ldr] = rv;
     }
   }
-  if (tau_out && r < nc) tau_out[r] = fac[kF_TAU + r];
+  if (tau_out && tid < kQ && r < nc) tau_out[r] = fac[kF_TAU + r];
 }
 
 }  // namespace
@@ -630,7 +636,7 @@ int panel_cholqr(evd_ctx *ctx, int count, long m, long nc, const T *A, long lda,
                  int *bad) {
   const int ng = (int)((m + kRows - 1) / kRows);  // row workgroups
   const int ngroups = (ng + kGroup - 1) / kGroup;
-  const long s_part = (long)(ng + ngroups + 1) * kQQ;
+  const long s_part = (long)(ng + ngroups) * kQQ;
   // problems per launch: the reduction counters of one launch must fit
   const int per = std::max(1, std::min(count, kCqCountWords / (ngroups + 1)));
   if (ngroups + 1 > kCqCountWords) return set_error(ctx, EVD_E_UNSUPPORTED, "panel of %ld rows", m);
@@ -648,14 +654,14 @@ int panel_cholqr(evd_ctx *ctx, int count, long m, long nc, const T *A, long lda,
     const T *Aq = A + q0 * s_in;
     T *Yq = Y + q0 * s_y, *Wq = W + q0 * s_w, *Oq = Aout ? Aout + q0 * s_out : nullptr;
     int *st = bad + q0;
-    const dim3 rows_grid((unsigned)ng, (unsigned)cq);
+    const dim3 rows_grid((unsigned)ng, (unsigned)cq), out_grid((unsigned)((m + kOut - 1) / kOut), (unsigned)cq);
     cq_pass_kernel<0, T><<<rows_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, part, s_part, cnt, st,
                                                              one_pass_max);
     EVD_LAUNCHED(ctx);
     cq_pass_kernel<1, T><<<rows_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, part, s_part, cnt, st,
                                                              one_pass_max);
     EVD_LAUNCHED(ctx);
-    cq_out_kernel<T><<<rows_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, Yq, ldy, s_y, Wq, ldw, s_w, Oq,
+    cq_out_kernel<T><<<out_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, Yq, ldy, s_y, Wq, ldw, s_w, Oq,
                                                         ldo, s_out, R, ldr, tau_out, st);
     EVD_LAUNCHED(ctx);
   }
