@@ -10,13 +10,14 @@
 //   N <- N H (block below S, which becomes the next B1 - the bulge).
 // u is stored in U[p .. p+len-1, s] ("noBandU" layout, FP32).
 //
-// MI355X design: sweeps are handed out by an atomic ticket in increasing
-// order, so a sweep's predecessor is always owned by a running workgroup and
-// no co-residency (cooperative launch) is needed.  A sweep does not update a
-// band in memory: it receives the window of each of its steps from its
-// predecessor as a message and sends the next sweep's windows on (chase_kernel
-// below).  Every access that crosses workgroups is device-coherent (sc1 loads
-// and stores, which bypass the non-coherent caches of a CU and of an XCD).
+// MI355X design: sweeps are handed out by atomic tickets, runs of consecutive
+// ones to one XCD, in an order that leaves every sweep's predecessor finished
+// or owned by a running workgroup, so no co-residency (cooperative launch) is
+// needed.  A sweep does not update a band in memory: it receives the window of
+// each of its steps from its predecessor as a message and sends the next
+// sweep's windows on (chase_kernel below).  A message within an XCD goes
+// through its L2 (plain stores, loads that pass the CU's cache by); one that
+// crosses XCDs is device-coherent on both sides (sc1).
 // Every wait is bounded by a watchdog so the grid always drains.
 #include <climits>
 #include <map>
@@ -42,9 +43,10 @@ constexpr unsigned kOutOfRange = 0x80000000u;
 __device__ __attribute__((always_inline)) inline double ld_band_at(__amdgpu_buffer_rsrc_t r, unsigned byte_off) {
   return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, byte_off, 0, kSc1));
 }
+template <int POLICY>
 __device__ __attribute__((always_inline)) inline void st_band_at(__amdgpu_buffer_rsrc_t r, unsigned byte_off, double v) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned, v),
-                                        r, byte_off, 0, kSc1);
+                                        r, byte_off, 0, POLICY);
 }
 
 __device__ __attribute__((always_inline)) inline void grp_barrier() {
@@ -177,11 +179,17 @@ __device__ __attribute__((always_inline)) inline double chase_reflector(double x
 // Measured against one workgroup per sweep on a band in HBM with progress
 // words (window loads, stores and a flag in every step's chain): b = 32,
 // n = 6000: 49.2 -> 25.6 ms, n = 16384: 137 -> 85 ms; b = 64, n = 8192:
-// 156 -> 92 ms.
+// 156 -> 92 ms (with every message between XCDs, see below).
 //
-// A batch of `count` same-size problems shares one launch: ticket t is sweep
-// t / count of problem t % count, so each problem's sweeps are still handed
-// out in increasing order.
+// Where the messages go decides the hand-off: from one XCD to another a store
+// reaches a poll after 820 ns, through the XCD's own L2 after 340 ns (a message
+// of 64 doubles sent to and fro).  So consecutive sweeps run on one XCD, each
+// of which has a box of slots of its own: a slot of a box is only ever
+// accessed through one L2.  All messages between
+// XCDs -> this: b = 32: n = 1000 3.88 -> 3.33 ms, n = 6000 25.6 -> 21.1 ms,
+// n = 16384 85.7 -> 59.6 ms; b = 64, n = 8192: 93.5 -> 86.5 ms.
+//
+// A batch of `count` same-size problems shares one launch, its units mixed.
 template <int BW>
 struct ChaseShape {
   static constexpr int EPT = BW / 8;    // window columns per thread
@@ -202,15 +210,22 @@ __host__ __device__ inline long mail_slot(long b) { return 2 * ((b + 7) / 8) * m
 __host__ __device__ inline long mail_slots(long n, long b) { return (n + b - 1) / b; }
 __host__ __device__ inline long mail_half(long n, long b) { return mail_slots(n, b) * mail_slot(b) + kXWords; }
 
-// Messages of parity 1 for sweep 0, from the band; everything else empty.
+// Messages of parity 1 for sweep 0, from the band, into the box between XCDs
+// (grid z = 0); everything else, the other boxes included, empty.
 __global__ __launch_bounds__(256) void mail_fill_kernel(int n, int b, const double *__restrict__ band_all, long ldb,
                                                         long band_stride, double *__restrict__ mail_all,
-                                                        double *__restrict__ D_all, long d_stride) {
+                                                        double *__restrict__ boxes, double *__restrict__ D_all,
+                                                        long d_stride) {
   const long q = blockIdx.y;
   const double *band = band_all + q * band_stride;
   const long half = mail_half(n, b), slot = mail_slot(b), plane = mail_plane(b), nslots = mail_slots(n, b);
-  double *mail = mail_all + q * 2 * half;
   const double empty = __builtin_bit_cast(double, (unsigned long long)kEmptyHi << 32);
+  if (blockIdx.z > 0) {
+    double *box = boxes + ((blockIdx.z - 1L) * gridDim.y + q) * 2 * half;
+    for (long e = blockIdx.x * 256L + threadIdx.x; e < 2 * half; e += gridDim.x * 256L) box[e] = empty;
+    return;
+  }
+  double *mail = mail_all + q * 2 * half;
   if (blockIdx.x == 0 && threadIdx.x == 0) D_all[q * d_stride] = band[0];
   for (long e = blockIdx.x * 256L + threadIdx.x; e < 2 * half; e += gridDim.x * 256L) {
     double v = empty;
@@ -241,17 +256,84 @@ __global__ __launch_bounds__(256) void mail_fill_kernel(int n, int b, const doub
   }
 }
 
-template <int BW>
+// Handing out sweeps.  A unit is a run of `len` consecutive sweeps of one
+// problem; units are numbered run by run over the problems (run u / count of
+// problem u % count) and an XCD takes the next one when all sweeps of its last
+// are handed out.  So the first sweep that is not finished is running or next
+// in its XCD's unit, whose workgroups have only finished ones behind them:
+// the chain always moves.  Units go to the first `members` XCDs that ask; the
+// workgroups of the others leave.
+// Words at `ticket`: the next unit, the members so far, and at
+// kXcdWords (x + 1) the 64-bit state of XCD x: member number << 61 | unit + 1
+// << 30 | sweeps handed out (0: no unit yet).
+constexpr int kXcds = 8, kXcdWords = 32;
+constexpr long kTicketWords = (long)kXcdWords * (kXcds + 1);
+constexpr unsigned kNoUnit = 0x7fffffffu;
+
+struct ChaseUnits {
+  int len, total, members;
+};
+
+// sweep (s of problem q) for this workgroup, whose XCD is member m; false: no
+// more.  One thread calls.
+__device__ inline bool next_sweep(unsigned *ticket, int x, const ChaseUnits &units, int count, int nsweeps,
+                                  unsigned *err, int &s, int &q, int &m) {
+  unsigned long long *state = reinterpret_cast<unsigned long long *>(ticket + kXcdWords * (x + 1));
+  auto field = [](unsigned long long v) -> unsigned { return (unsigned)(v >> 30) & kNoUnit; };
+  while (true) {
+    const unsigned long long v = __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned unit = field(v), idx = (unsigned)v & 0x3fffffffu;
+    m = (int)(v >> 61);
+    if (unit == kNoUnit) return false;
+    if (unit != 0 && idx < (unsigned)units.len) {
+      s = (int)((unit - 1) / count) * units.len + (int)idx;
+      q = (int)((unit - 1) % count);
+      if (s < nsweeps) return true;
+      continue;
+    }
+    if (idx == (unit == 0 ? 0u : (unsigned)units.len)) {  // fetch the XCD's next unit, and take its first sweep
+      if (unit == 0) m = (int)__hip_atomic_fetch_add(ticket + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      unsigned u = kNoUnit - 1;
+      if (m < units.members) {
+        const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (t < (unsigned)units.total) u = t;
+      }
+      const bool none = u == kNoUnit - 1;
+      __hip_atomic_store(state, (none ? 0ull : (unsigned long long)m << 61) | (unsigned long long)(u + 1) << 30 | 1ull,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (none) return false;
+      s = (int)(u / count) * units.len;
+      q = (int)(u % count);
+      return true;
+    }
+    // another workgroup fetches it
+    const unsigned long long t0 = clock100();
+    while (field(__hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == unit) {
+      __builtin_amdgcn_s_sleep(2);
+      if (clock100() - t0 > kWatchdogTicks) {
+        atomicOr(err, (unsigned)EVD_E_TIMEOUT);
+        return false;
+      }
+    }
+  }
+}
+
+// LOCAL: messages between sweeps of one unit go through box m of the XCD's
+// member number (boxes; one per member and problem) and stay in its L2; the
+// first sweep of a unit receives, and the last one sends, through mail_all.
+// Otherwise every message goes through mail_all.
+template <int BW, bool LOCAL>
 __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
-    int n, int b, double *__restrict__ mail_all, float *__restrict__ U_all, long ldu, long u_stride,
-    int *__restrict__ com_all, unsigned *__restrict__ ticket, unsigned *__restrict__ err, int count,
-    double *__restrict__ D_all, long d_stride, double *__restrict__ E_all, long e_stride) {
+    int n, int b, double *__restrict__ mail_all, double *__restrict__ boxes, ChaseUnits units,
+    float *__restrict__ U_all, long ldu, long u_stride, int *__restrict__ com_all, unsigned *__restrict__ ticket,
+    unsigned *__restrict__ err, int count, double *__restrict__ D_all, long d_stride, double *__restrict__ E_all,
+    long e_stride) {
   using Sh = ChaseShape<BW>;
   constexpr int EPT = Sh::EPT, NT = Sh::NT, NW = Sh::NW, LD = Sh::LD;
   __shared__ double sB[BW * LD];      // N^T of the last step: the next B1
   __shared__ double sU[NW][BW];       // each wave's copy of u
   __shared__ double sY[BW], sQ[BW], sN0[BW], sX[BW];
-  __shared__ int s_ticket, s_abort;
+  __shared__ int s_sweep, s_problem, s_member, s_abort;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int ri = tid >> 3, kc = tid & 7, xi = lane & (BW - 1);
@@ -264,18 +346,15 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
   // byte offset of S'(i, k) in a slot (N' at + nb0)
   auto at = [&](int i, int k) -> unsigned { return (unsigned)(k >> 3) * pb + (unsigned)(i * 8 + (k & 7)) * 8u; };
 
-  while (true) {
-    if (tid == 0) {
-      s_ticket = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      s_abort = 0;
-    }
-    grp_barrier();
-    const int tk = __builtin_amdgcn_readfirstlane(s_ticket);
-    grp_barrier();
-    if (tk >= nsweeps * count) return;
-    const int q = tk % count, s = tk / count;
-    double *mail = mail_all + (long)q * 2 * half;
-    double *rd = mail + ((s + 1) & 1) * half, *wr = mail + (s & 1) * half;  // slot 0 of this sweep's messages in, out
+  const int xcd = LOCAL ? (int)__builtin_amdgcn_s_getreg((3 << 11) | 20) & (kXcds - 1) : 0;  // HW_REG_XCC_ID
+
+  // one sweep, messages in and out with these store policies (0: within the
+  // XCD, kSc1: device-coherent); true: aborted
+  auto sweep = [&](auto in_policy, auto out_policy, const int s, const int q, double *mail_in, double *mail_out)
+                   __attribute__((always_inline)) -> bool {
+    constexpr int IN = decltype(in_policy)::value, OUT = decltype(out_policy)::value;
+    // slot 0 of this sweep's messages in, out
+    double *rd = mail_in + ((s + 1) & 1) * half, *wr = mail_out + (s & 1) * half;
     const __amdgpu_buffer_rsrc_t rxi =
         __builtin_amdgcn_make_buffer_rsrc(rd + half - kXWords, 0, kXWords * 8, kBufferWord3);
     const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(
@@ -340,7 +419,7 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
         const bool ready = (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32) != kEmptyHi;
         if (__all(ready) || expired(t0)) break;
       }
-      __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rxi, ox, 0, kSc1);
+      __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rxi, ox, 0, IN);
       if (lane < BW) sX[lane] = x;
     }
     grp_barrier();
@@ -392,8 +471,8 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(rd, 0, slot_bytes, kBufferWord3);
 #pragma unroll
         for (int r = 0; r < EPT; r++) {
-          __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rs, oS[r], 0, kSc1);
-          __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rs, oN[r], 0, kSc1);
+          __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rs, oS[r], 0, IN);
+          __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rs, oN[r], 0, IN);
         }
       }
       rd += slot;
@@ -453,23 +532,23 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
         sB[kk * LD + ri] = N[r];
         // ---- B1 <- H B1 (the first step has none and issues dropped stores)
         bt[r] -= uk[r] * t;
-        st_band_at(rv, first ? kOutOfRange : oB[r], bt[r]);
+        st_band_at<OUT>(rv, first ? kOutOfRange : oB[r], bt[r]);
       }
-      st_band_at(rv, first ? kOutOfRange : oM, bt[0]);
+      st_band_at<OUT>(rv, first ? kOutOfRange : oM, bt[0]);
 #pragma unroll
       for (int r = 0; r < EPT; r++) {
         const double wk = yk[r] - psi * uk[r];
         S[r] -= sym_pair(ui, wk, wi, uk[r]);
-        st_band_at(rw, oA[r], S[r]);
+        st_band_at<OUT>(rw, oA[r], S[r]);
       }
       // S(:, 0) and the next beta complete message j - 1 (X in the first step)
       {
         const unsigned ob = first ? (unsigned)(b - 1) * 8u : nb0 + at(b - 1, b - 1);
         const unsigned oc = tid == 1 ? (len2 > 0 ? ob : kOutOfRange) : (first ? oX : oC);
         const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
-            first ? mail + (s & 1) * half + (half - kXWords) : wr - slot, 0, first ? kXWords * 8 : slot_bytes,
+            first ? mail_out + (s & 1) * half + (half - kXWords) : wr - slot, 0, first ? kXWords * 8 : slot_bytes,
             kBufferWord3);
-        st_band_at(rc, oc, tid == 1 ? betan : S[0]);
+        st_band_at<OUT>(rc, oc, tid == 1 ? betan : S[0]);
       }
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)uu), ru,
                                             (wave == 0 && lane < len2) ? (unsigned)(pn + lane) * 4u : kOutOfRange, 0, 0);
@@ -504,7 +583,35 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
       if (end) break;
       end = step(std::false_type{}, Sa, Na, Sb, Nb);
     }
-    if (end == 2) return;
+    return end == 2;
+  };
+
+  const std::integral_constant<int, 0> local{};
+  const std::integral_constant<int, kSc1> coherent{};
+  while (true) {
+    if (tid == 0) {
+      int s, q, m;
+      s_sweep = next_sweep(ticket, xcd, units, count, nsweeps, err, s, q, m) ? s : -1;
+      s_problem = q;
+      s_member = m;
+      s_abort = 0;
+    }
+    grp_barrier();
+    const int s = __builtin_amdgcn_readfirstlane(s_sweep), q = __builtin_amdgcn_readfirstlane(s_problem);
+    const int m = __builtin_amdgcn_readfirstlane(s_member);
+    grp_barrier();
+    if (s < 0) return;
+    double *mail = mail_all + (long)q * 2 * half, *box = boxes + ((long)m * count + q) * 2 * half;
+    bool aborted;
+    if (!LOCAL)
+      aborted = sweep(coherent, coherent, s, q, mail, mail);
+    else if (s % units.len == 0)
+      aborted = sweep(coherent, local, s, q, mail, box);
+    else if ((s + 1) % units.len == 0)
+      aborted = sweep(local, coherent, s, q, box, mail);
+    else
+      aborted = sweep(local, local, s, q, box, box);
+    if (aborted) return;
   }
 }
 
@@ -928,29 +1035,56 @@ static int launch_chase_group(evd_ctx *ctx, int count, long n, long b, double *b
   return 0;
 }
 
+// Sweeps in flight of one problem (a sweep trails its predecessor by two to
+// three steps of b rows) and the XCDs that run the chase: 32 sweeps an XCD, one
+// per CU, keep a chain of up to 32 on one XCD; at b = 64, 16, whose slots (64
+// KiB, two steps apart, both parities) fit the 4 MiB of its L2.
+static long chase_inflight(long n, long b) { return (2 * n + 5 * b - 1) / (5 * b) + 4; }
+static int chase_members(int count, long n, long b) {
+  const long per = b <= 32 ? 32 : 16;
+  return (int)std::min<long>(kXcds, (chase_inflight(n, b) * count + per - 1) / per);
+}
+
 template <int BW>
 static int launch_chase(evd_ctx *ctx, int count, long n, long b, const double *band, long ldb, long band_stride,
-                        double *mail, float *U, long ldu, long u_stride, int *com, unsigned *ticket, double *D,
-                        long d_stride, double *E, long e_stride) {
-  // workgroups: sweep s+1 trails sweep s by between three and four b-row
-  // steps, so about n / (3b) sweeps of a problem are in flight; by default
-  // that many plus a few per problem (a workgroup takes its next sweep by
-  // ticket as soon as it finishes one), at most the resident count.
-  // Workgroups beyond that only poll and crowd out concurrent solves.
+                        double *mail, double *boxes, float *U, long ldu, long u_stride, int *com, unsigned *ticket,
+                        double *D, long d_stride, double *E, long e_stride) {
+  // workgroups: as many as sweeps are in flight (a workgroup takes its next
+  // sweep as soon as it finishes one), at most the resident count.  Those
+  // beyond that only poll and crowd out concurrent solves.  With boxes that many
+  // on each member XCD: workgroups are dealt to the XCDs in turn, so eight
+  // times as many are launched, of which those on other XCDs leave at once.
   int resident = 0;
-  EVD_TRY(max_coresident_blocks(ctx, (const void *)chase_kernel<BW>, ChaseShape<BW>::NT, 0, &resident));
-  const long inflight = ((n + 3 * b - 1) / (3 * b) + 4) * count;
-  long G = ctx->tune.chase_groups > 0 ? ctx->tune.chase_groups
-                                      : std::min<long>(inflight, (long)std::max(ctx->num_cus, resident));
-  G = std::min<long>(G, std::max<long>(1, (n - 2) * count));
+  const void *kernel = boxes ? (const void *)chase_kernel<BW, true> : (const void *)chase_kernel<BW, false>;
+  EVD_TRY(max_coresident_blocks(ctx, kernel, ChaseShape<BW>::NT, 0, &resident));
+  resident = std::max(ctx->num_cus, resident);
+  const long nsweeps = n - 2, inflight = chase_inflight(n, b);
+  const int members = boxes ? chase_members(count, n, b) : 1;
+  // units: everything on one XCD where that holds a problem's sweeps in
+  // flight; else as many sweeps as an XCD holds; batches mix the problems
+  long per = std::min<long>(inflight * count, resident), len = 1;
+  if (boxes) {
+    per = std::min<long>((per + members - 1) / members + 2, resident / kXcds);
+    len = count > 1 ? std::min(inflight, per) : members == 1 ? nsweeps : per;
+    len = std::max<long>(2, std::min(len, nsweeps));
+    per *= kXcds;
+  }
+  long G = ctx->tune.chase_groups > 0 ? ctx->tune.chase_groups : per;
+  G = std::min<long>(G, std::max<long>(1, nsweeps * count * (boxes ? kXcds : 1)));
+  const ChaseUnits units{(int)len, (int)(((nsweeps + len - 1) / len) * count), members};
   unsigned *err = ctx->ctrl + kCtrlError;
   const long words = 2 * mail_half(n, b);
-  mail_fill_kernel<<<dim3((unsigned)std::min<long>((words + 255) / 256, 4096), (unsigned)count), 256, 0, ctx->stream>>>(
-      (int)n, (int)b, band, ldb, band_stride, mail, D, d_stride);
+  mail_fill_kernel<<<dim3((unsigned)std::min<long>((words + 255) / 256, 4096), (unsigned)count,
+                          boxes ? members + 1u : 1u),
+                     256, 0, ctx->stream>>>((int)n, (int)b, band, ldb, band_stride, mail, boxes, D, d_stride);
   EVD_LAUNCHED(ctx);
   if (ctx->timing && !ctx->capturing) hipEventRecord(ctx->cev[0], ctx->stream);
-  chase_kernel<BW><<<(unsigned)G, ChaseShape<BW>::NT, 0, ctx->stream>>>((int)n, (int)b, mail, U, ldu, u_stride, com,
-                                                                         ticket, err, count, D, d_stride, E, e_stride);
+  if (boxes)
+    chase_kernel<BW, true><<<(unsigned)G, ChaseShape<BW>::NT, 0, ctx->stream>>>(
+        (int)n, (int)b, mail, boxes, units, U, ldu, u_stride, com, ticket, err, count, D, d_stride, E, e_stride);
+  else
+    chase_kernel<BW, false><<<(unsigned)G, ChaseShape<BW>::NT, 0, ctx->stream>>>(
+        (int)n, (int)b, mail, boxes, units, U, ldu, u_stride, com, ticket, err, count, D, d_stride, E, e_stride);
   EVD_LAUNCHED(ctx);
   if (ctx->timing && !ctx->capturing) hipEventRecord(ctx->cev[1], ctx->stream);
   return 0;
@@ -990,7 +1124,14 @@ __global__ void chase_signs_kernel(int n, const double *__restrict__ band, long 
 }
 
 size_t sb2st_batched_workspace(int count, long n, long b) {
-  return align256((size_t)count * 2 * mail_half(n, b) * sizeof(double) + ((size_t)count * n * kComStride + 1) * sizeof(int));
+  return align256((size_t)count * 2 * mail_half(n, b) * sizeof(double) +
+                  ((size_t)count * n * kComStride + kTicketWords) * sizeof(int));
+}
+
+// The XCDs' boxes are scratch on top of that, used where the arena has room
+// (a call never fails for want of them; the results are the same).
+static size_t chase_boxes_bytes(int count, long n, long b) {
+  return (size_t)chase_members(count, n, b) * count * 2 * mail_half(n, b) * sizeof(double);
 }
 
 // Bulge chasing of `count` same-size bands in one persistent launch (problem q
@@ -1006,7 +1147,7 @@ int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ld
     // messages, then progress words com[q * n * kComStride + s * kComStride]
     // and the ticket
     const long com_stride = n * kComStride;
-    const size_t words = (size_t)count * com_stride + 1;
+    const size_t words = (size_t)count * com_stride + kTicketWords;
     double *mail = ext_com ? reinterpret_cast<double *>(ext_com)
                            : arena_alloc_n<double>(ctx, sb2st_batched_workspace(count, n, b) / sizeof(double));
     if (!mail) return EVD_E_NOMEM;
@@ -1018,6 +1159,11 @@ int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ld
     // workgroup's waves share SIMDs and the grouped kernel's registers spill)
     const int depth = std::min({ctx->tune.chase_depth > 0 ? ctx->tune.chase_depth : 1, group_depth_max(b), 3});
     if (b > 64) return set_error(ctx, EVD_E_UNSUPPORTED, "bandwidth %ld > 64", b);
+    auto boxes = [&]() -> double * {
+      const size_t bytes = chase_boxes_bytes(count, n, b);
+      const size_t room = ctx->arena_bytes - std::min(ctx->arena_bytes, align256(ctx->arena_top));
+      return ext_com || bytes > room ? nullptr : static_cast<double *>(arena_alloc(ctx, bytes));
+    };
     if (b <= 32 && depth > 1) {
       if (depth == 3)
         EVD_TRY(launch_chase_group<3>(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, com, com_stride,
@@ -1031,11 +1177,11 @@ int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ld
       EVD_LAUNCHED(ctx);
       return 0;
     } else if (b <= 32) {
-      return launch_chase<32>(ctx, count, n, b, band, ldband, band_stride, mail, U, ldu, u_stride, com, ticket, D,
-                              d_stride, E, e_stride);
+      return launch_chase<32>(ctx, count, n, b, band, ldband, band_stride, mail, boxes(), U, ldu, u_stride, com, ticket,
+                              D, d_stride, E, e_stride);
     } else {
-      return launch_chase<64>(ctx, count, n, b, band, ldband, band_stride, mail, U, ldu, u_stride, com, ticket, D,
-                              d_stride, E, e_stride);
+      return launch_chase<64>(ctx, count, n, b, band, ldband, band_stride, mail, boxes(), U, ldu, u_stride, com, ticket,
+                              D, d_stride, E, e_stride);
     }
   }
   band_extract_batched_kernel<<<dim3((unsigned)std::min<long>((n + 255) / 256, 1024), (unsigned)count), 256, 0,
@@ -1047,6 +1193,16 @@ int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ld
 
 int sb2st(evd_ctx *ctx, long n, long b, double *band, long ldband, float *U, long ldu, double *D, double *E) {
   return sb2st_batched(ctx, 1, n, b, band, ldband, 0, U, ldu, 0, D, 0, E, 0, nullptr);
+}
+
+// arena of a chase called by itself: with the XCDs' boxes where it may grow to
+// that (no captured graph, lent arena or budget against it), else without
+static int chase_arena(evd_ctx *ctx, int count, long n, long b) {
+  const size_t need = sb2st_batched_workspace(count, n, b) + 4096, all = need + chase_boxes_bytes(count, n, b);
+  if (all > ctx->arena_bytes && ctx->graphs == 0 && !ctx->arena_external && !(ctx->budget && all > ctx->budget) &&
+      arena_ensure(ctx, all) == 0)
+    return 0;
+  return arena_ensure(ctx, need);
 }
 
 // ---- the chase without allocation: scratch in a file-scope device array.
@@ -1101,7 +1257,7 @@ extern "C" int evd_sb2st_f64(evd_ctx *ctx, long n, long b, double *band, long ld
   EVD_ARG(ctx, b >= 1 && b <= 64, 3);
   EVD_ARG(ctx, ldband >= 2 * b, 5);
   EVD_ARG(ctx, ldu >= n + b, 7);
-  if (ctx->arena_top == 0) EVD_TRY(arena_ensure(ctx, sb2st_batched_workspace(1, n, b) + 4096));
+  if (ctx->arena_top == 0) EVD_TRY(chase_arena(ctx, 1, n, b));
   EVD_TRY(sb2st(ctx, n, b, band, ldband, U, ldu, D, E));
   return check_device_error(ctx, "evd_sb2st_f64");
 }
@@ -1138,7 +1294,7 @@ extern "C" int evd_sb2st_batched_f64(evd_ctx *ctx, int count, long n, long b, do
   EVD_ARG(ctx, count <= 1 || d_stride >= n, 12);
   EVD_ARG(ctx, count <= 1 || e_stride >= std::max<long>(1, n - 1), 14);
   EVD_ARG(ctx, (long)count * std::max<long>(n, 1) < (1L << 30), 2);
-  if (ctx->arena_top == 0) EVD_TRY(arena_ensure(ctx, sb2st_batched_workspace(count, n, b) + 4096));
+  if (ctx->arena_top == 0) EVD_TRY(chase_arena(ctx, count, n, b));
   EVD_TRY(sb2st_batched(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, D, d_stride, E, e_stride,
                         nullptr));
   return check_device_error(ctx, "evd_sb2st_batched_f64");

@@ -6,7 +6,9 @@ the model grants is the kernel's: a step's sends are issued after the previous
 step's empties have completed.  Every interleaving must give the oracle's
 sequential result, no element may land in a slot that is not empty or be left
 behind in one that is loaded again, and without the start word or the ordering
-of empties before sends the model must fail."""
+of empties before sends the model must fail.  With units, the messages inside
+a run of sweeps go through the box of the run's XCD, those between runs through
+the common one.  A second model hands out the sweeps (next_sweep)."""
 import random
 
 import numpy as np
@@ -44,11 +46,16 @@ def _window(n, b, p):
     return w
 
 
-def chase(Bd, b, seed, start_word=True, ordered=True, window=7):
+def chase(Bd, b, seed, start_word=True, ordered=True, window=7, unit=None, members=1):
     n = Bd.shape[0]
     rng = random.Random(seed)
     nsw = n - 2
-    mem = {}  # (parity, slot | 'X', element) -> value; absent = EMPTY
+    mem = {}  # (box and parity, slot | 'X', element) -> value; absent = EMPTY
+
+    def half(s):
+        """Where sweep s sends: its parity, in the common box or that of its unit's XCD."""
+        return s % 2 if not unit or (s + 1) % unit == 0 else (s // unit % members, s % 2)
+
     for j in range(-(-n // b)):
         p = 1 + j * b
         if p < n:
@@ -81,7 +88,7 @@ def chase(Bd, b, seed, start_word=True, ordered=True, window=7):
     def program(s):
         """The sweep as a generator: yields None to be rescheduled."""
         x = st[s]
-        rd, wr = (s + 1) % 2, s % 2
+        rd, wr = half(s - 1), half(s)
         p = s + 1
         ln, ln2 = _lens(n, b, p)
         store = lambda kind, j, key, v=None: x["stores"].append((kind, j, key, v))
@@ -174,7 +181,7 @@ def chase(Bd, b, seed, start_word=True, ordered=True, window=7):
         idle += 1
         if idle > 2_000_000:
             raise Stale("no progress")
-    left = [k for k in mem if k[0] == nsw % 2]  # what sweep nsw - 2 sent: all of it was loaded
+    left = [k for k in mem if k[0] == half(nsw - 2)]  # what sweep nsw - 2 sent: all of it was loaded
     if left:
         raise Stale(f"{len(left)} elements left behind")
     return D, E, U
@@ -194,6 +201,15 @@ def test_messages_match_sequential_chase(n, b):
         assert max(np.abs(a - r).max() for a, r in zip(res, ref)) < 1e-11
 
 
+@pytest.mark.parametrize("unit,members", [(2, 1), (2, 3), (3, 2), (5, 2), (100, 1)])
+@pytest.mark.parametrize("n,b", [(9, 4), (24, 4), (26, 5), (17, 2)])
+def test_messages_through_unit_boxes(n, b, unit, members):
+    B = _band(n, b)
+    ref = O.sb2st(B, b)
+    res = chase(B, b, 7 * unit + members, unit=unit, members=members)
+    assert max(np.abs(a - r).max() for a, r in zip(res, ref)) < 1e-11
+
+
 @pytest.mark.parametrize("unsafe", [{"start_word": False}, {"ordered": False}])
 def test_model_catches_unsafe_protocols(unsafe):
     n, b = 25, 4
@@ -207,3 +223,77 @@ def test_model_catches_unsafe_protocols(unsafe):
         except Stale:
             bad += 1
     assert bad
+
+
+def hand_out(nsweeps, count, length, members, groups, seed):
+    """next_sweep for groups[x] workgroups on XCD x, every atomic access an
+    interleaving point, on a chain in which a sweep ends only after its
+    predecessor.  Returns {(problem, sweep): XCD}."""
+    rng = random.Random(seed)
+    total = -(-nsweeps // length) * count
+    DONE = 0x7FFFFFFF
+    word = {"unit": 0, "members": 0}
+    state = {x: (0, 0, 0) for x in range(len(groups))}  # member, unit + 1, handed out
+    owner, ended = {}, set()
+
+    def take(x):
+        while True:
+            m, unit, idx = state[x]
+            state[x] = (m, unit, idx + 1)
+            yield
+            if unit == DONE:
+                return None
+            if unit and idx < length:
+                s = (unit - 1) // count * length + idx
+                if s < nsweeps:
+                    return (unit - 1) % count, s
+                continue
+            if idx == (length if unit else 0):
+                if not unit:
+                    m, word["members"] = word["members"], word["members"] + 1
+                    yield
+                u = None
+                if m < members:
+                    t, word["unit"] = word["unit"], word["unit"] + 1
+                    yield
+                    u = t if t < total else None
+                state[x] = (m, DONE, 1) if u is None else (m, u + 1, 1)
+                yield
+                return None if u is None else (u % count, u // count * length)
+            while state[x][1] == unit:
+                yield
+
+    def workgroup(x):
+        while True:
+            job = yield from take(x)
+            if job is None:
+                return
+            assert job not in owner
+            owner[job] = x
+            q, s = job
+            while s > 0 and (q, s - 1) not in ended:
+                yield
+            ended.add(job)
+
+    live = [workgroup(x) for x in range(len(groups)) for _ in range(groups[x])]
+    for _ in range(2_000_000):
+        if not live:
+            return owner
+        g = rng.choice(live)
+        try:
+            next(g)
+        except StopIteration:
+            live.remove(g)
+    raise Stale("no progress")
+
+
+@pytest.mark.parametrize("nsweeps,count,length,members,groups", [
+    (1, 1, 2, 1, [1, 1]), (9, 1, 9, 1, [2, 3, 1]), (23, 1, 4, 3, [2, 1, 4, 1]), (10, 5, 3, 2, [3, 3, 3]),
+    (7, 3, 1, 1, [4]), (12, 2, 5, 2, [1, 0, 0]), (2, 6, 2, 8, [1] * 8)])
+def test_hand_out_reaches_every_sweep(nsweeps, count, length, members, groups):
+    for seed in range(5):
+        owner = hand_out(nsweeps, count, length, members, groups, seed)
+        assert set(owner) == {(q, s) for q in range(count) for s in range(nsweeps)}
+        assert len(set(owner.values())) <= members
+        for (q, s), x in owner.items():  # a unit stays on one XCD
+            assert s % length == 0 or owner[q, s - 1] == x
