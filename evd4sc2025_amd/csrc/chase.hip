@@ -146,10 +146,14 @@ __device__ __attribute__((always_inline)) inline double chase_reflector(double x
 // kernel is built for the latency of that chain: the steps of a sweep, and the
 // hand-off from a sweep to the next.
 //
-// Step.  u from LDS -> q = N u (FMAs, a DPP sum over the row's 8 lanes) ->
+// Step.  The window -> q = N u (FMAs, a DPP sum over the row's 8 lanes) ->
 // barrier -> the next column x = N[:, 0] - q u_0, its norm and the next u,
-// which every wave forms for itself.  Everything else (B1 <- H B1, the rank-2
-// update of S, the messages) fills the waits.  B1 is the previous N, passed
+// which every wave forms for itself.  Everything else fills the waits: B1 <-
+// H B1 and its part of a message need no window and come before it, the slot is
+// emptied in the shadow of the reflector, and the rest of the message goes out
+// with S(:, 0) and beta first, which complete what the next sweep waits for.
+// b = 32, n = 6000: 21.1 -> 16.3 ms, n = 1000: 3.33 -> 2.46 ms; b = 64, n = 8192:
+// 86.5 -> 67.7 ms.  B1 is the previous N, passed
 // through LDS transposed, so that its column sums u^T B1 are row sums of a
 // wave's own lanes as well.
 //
@@ -167,10 +171,11 @@ __device__ __attribute__((always_inline)) inline double chase_reflector(double x
 // to complete, then a flag, then a load (n = 16384, b = 32: store 0.33-0.48 us,
 // flag 0.5-0.66 us, loads behind it).  Having read a slot, the receiver empties it again.
 // Slots are doubled by the sweep's parity, and reuse is safe by the order of
-// the chain alone: a step's sends follow a barrier before which every wave has
-// waited for loads issued after the previous step's empties (memory
-// operations complete in order), so message j of sweep s, complete at step
-// (s, j + 1), proves that s has emptied slot j of the other parity.  Only a
+// the chain alone: a step's sends but those of B1 follow a barrier before which
+// every wave has waited for loads issued after the previous step's empties
+// (memory operations complete in order), so message j of sweep s, which S(:, 0)
+// and beta complete at step (s, j + 1), proves that s has emptied slot j of the
+// other parity; B1 goes to slot j - 1, which the step before proved empty.  Only a
 // sweep's first slots have no such message before them: the receiver waits for
 // the predecessor's start word, set once it holds its own first window.
 // What a sweep sends is exactly what the next one loads (both bounded by row
@@ -452,21 +457,60 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
     };
 
     // one step on the window in (S, N); the next one's is loaded into
-    // (Sn, Nn).  The sweep's first step has a copy of its own, so that the
-    // loop's steps all see the same number of memory operations behind a
-    // window's loads and wait for nothing newer.  0: go on, 1: last step,
-    // 2: aborted
+    // (Sn, Nn).  0: go on, 1: last step, 2: aborted
     auto step = [&](auto is_first, double(&S)[EPT], double(&N)[EPT], double(&Sn)[EPT], double(&Nn)[EPT])
                     __attribute__((always_inline)) -> int {
       constexpr bool first = decltype(is_first)::value;
       const bool last = (len2 == 0);
+      // ---- B1 <- H B1 (B1 transposed), for which u is all it takes: done and
+      // sent while the window is on its way
+      double uk[EPT];
+      const double ui = sU[wave][ri];
+#pragma unroll
+      for (int r = 0; r < EPT; r++) uk[r] = sU[wave][kc + 8 * r];
+      if constexpr (!first) {
+        double bt[EPT], t = 0.0;
+#pragma unroll
+        for (int r = 0; r < EPT; r++) bt[r] = sB[ri * LD + kc + 8 * r];
+#pragma unroll
+        for (int r = 0; r < EPT; r++) t += bt[r] * uk[r];
+        t = group_sum<8>(t);
+        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(wr - slot, 0, slot_bytes, kBufferWord3);
+#pragma unroll
+        for (int r = 0; r < EPT; r++) {
+          bt[r] -= uk[r] * t;
+          st_band_at<OUT>(rv, oB[r], bt[r]);
+        }
+        st_band_at<OUT>(rv, oM, bt[0]);
+      }
       if (!arrived(S, N)) {
         const unsigned long long t0 = clock100();
         do {
           load_window(rd, S, N);
         } while (!arrived(S, N) && !expired(t0));
       }
-      // empty the slot, then look for the next window
+      // ---- row sums q = N u, y = S u
+      double y = 0.0, qq = 0.0;
+#pragma unroll
+      for (int r = 0; r < EPT; r++) {
+        qq += N[r] * uk[r];
+        y += S[r] * uk[r];
+      }
+      qq = group_sum<8>(qq);
+      y = group_sum<8>(y);
+      if (kc == 0) {
+        sQ[ri] = qq;
+        sN0[ri] = N[0];
+        sY[ri] = y;
+      }
+      grp_barrier();
+      // ---- the next column and its reflector (every wave for itself), the
+      // slot emptied in its shadow
+      const double x = sN0[xi] - sQ[xi] * u0;
+      double yk[EPT];
+#pragma unroll
+      for (int r = 0; r < EPT; r++) yk[r] = sY[kc + 8 * r];
+      const int aborted = s_abort;
       {
         const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(rd, 0, slot_bytes, kBufferWord3);
 #pragma unroll
@@ -475,41 +519,6 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
           __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rs, oN[r], 0, IN);
         }
       }
-      rd += slot;
-      const int pn = p + len, len3 = max(0, min(b, n - pn - len2));
-      if (len3 != b) window_offsets(len2, len3);
-      load_window(rd, Sn, Nn);
-      // ---- row sums q = N u, y = S u, t = u^T B1 (B1 transposed)
-      double uk[EPT], bt[EPT];
-      const double ui = sU[wave][ri];
-      double t = 0.0, y = 0.0, qq = 0.0;
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        const int kk = kc + 8 * r;
-        uk[r] = sU[wave][kk];
-        bt[r] = first ? 0.0 : sB[ri * LD + kk];
-      }
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        qq += N[r] * uk[r];
-        y += S[r] * uk[r];
-        t += bt[r] * uk[r];
-      }
-      qq = group_sum<8>(qq);
-      y = group_sum<8>(y);
-      t = group_sum<8>(t);
-      if (kc == 0) {
-        sQ[ri] = qq;
-        sN0[ri] = N[0];
-        sY[ri] = y;
-      }
-      grp_barrier();
-      // ---- the next column and its reflector (every wave for itself)
-      const double x = sN0[xi] - sQ[xi] * u0;
-      double yk[EPT];
-#pragma unroll
-      for (int r = 0; r < EPT; r++) yk[r] = sY[kc + 8 * r];
-      const int aborted = s_abort;
       double un0 = 0.0, betan = 0.0, uu = 0.0;
       uu = chase_reflector<BW>(x, lane, un0, betan);
       if (len2 <= 1) {  // a single row is left as it is
@@ -517,29 +526,16 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
         betan = __shfl(x, 0, 64);
       }
       if (lane < BW) sU[wave][lane] = uu;
-      // ---- N <- N H, S <- H S H (rank-2 with w = y - (u^T y / 2) u)
+      // ---- S <- H S H (rank-2 with w = y - (u^T y / 2) u), N <- N H
       double psi = 0.0;
 #pragma unroll
       for (int r = 0; r < EPT; r++) psi += uk[r] * yk[r];
       psi = 0.5 * group_sum<8>(psi);
       const double wi = y - psi * ui;
-      const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(wr, 0, slot_bytes, kBufferWord3);
-      const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(first ? wr : wr - slot, 0, slot_bytes, kBufferWord3);
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        const int kk = kc + 8 * r;
-        N[r] -= qq * uk[r];
-        sB[kk * LD + ri] = N[r];
-        // ---- B1 <- H B1 (the first step has none and issues dropped stores)
-        bt[r] -= uk[r] * t;
-        st_band_at<OUT>(rv, first ? kOutOfRange : oB[r], bt[r]);
-      }
-      st_band_at<OUT>(rv, first ? kOutOfRange : oM, bt[0]);
 #pragma unroll
       for (int r = 0; r < EPT; r++) {
         const double wk = yk[r] - psi * uk[r];
         S[r] -= sym_pair(ui, wk, wi, uk[r]);
-        st_band_at<OUT>(rw, oA[r], S[r]);
       }
       // S(:, 0) and the next beta complete message j - 1 (X in the first step)
       {
@@ -550,6 +546,17 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
             kBufferWord3);
         st_band_at<OUT>(rc, oc, tid == 1 ? betan : S[0]);
       }
+#pragma unroll
+      for (int r = 0; r < EPT; r++) {
+        N[r] -= qq * uk[r];
+        sB[(kc + 8 * r) * LD + ri] = N[r];
+      }
+      {
+        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(wr, 0, slot_bytes, kBufferWord3);
+#pragma unroll
+        for (int r = 0; r < EPT; r++) st_band_at<OUT>(rw, oA[r], S[r]);
+      }
+      const int pn = p + len, len3 = max(0, min(b, n - pn - len2));
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)uu), ru,
                                             (wave == 0 && lane < len2) ? (unsigned)(pn + lane) * 4u : kOutOfRange, 0, 0);
       if constexpr (first) {
@@ -562,6 +569,11 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
           if (tid == 9) Dq[n - 1] = S[0];
         }
       }
+      // look for the next window (loads behind this step's empties: see above)
+      asm volatile("" ::: "memory");
+      rd += slot;
+      if (len3 != b) window_offsets(len2, len3);
+      load_window(rd, Sn, Nn);
       grp_barrier();
       if (aborted) return 2;
       if (last) return 1;

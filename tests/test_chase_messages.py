@@ -2,8 +2,8 @@
 sweeps run concurrently and hand each other the window of every step through
 slots that are doubled by the sweep's parity and hold EMPTY until a message
 element arrives.  Stores complete late and in random order; the only ordering
-the model grants is the kernel's: a step's sends are issued after the previous
-step's empties have completed.  Every interleaving must give the oracle's
+the model grants is the kernel's: a step's sends, but for those of B1, are issued
+after the previous step's empties have completed.  Every interleaving must give the oracle's
 sequential result, no element may land in a slot that is not empty or be left
 behind in one that is loaded again, and without the start word or the ordering
 of empties before sends the model must fail.  With units, the messages inside
@@ -108,6 +108,14 @@ def chase(Bd, b, seed, start_word=True, ordered=True, window=7, unit=None, membe
         E[s] = beta
         j, B1 = 0, None
         while True:
+            send = lambda key, v: store("send", j, key, v)
+            if j > 0:  # before the window, and before the empties are known to be complete
+                B1 = B1 - np.outer(u, u @ B1)
+                for k in range(1, b):
+                    send((wr, j - 1, "S", b - 1, k - 1), B1[0, k])
+                    send((wr, j - 1, "S", k - 1, b - 1), B1[0, k])
+                    for i in range(1, ln):
+                        send((wr, j - 1, "N", i - 1, k - 1), B1[i, k])
             keys = [(rd, j, *e) for e in _window(n, b, p)]
             got = {}
             while len(got) < len(keys):  # elements are seen one by one, in any order
@@ -126,7 +134,6 @@ def chase(Bd, b, seed, start_word=True, ordered=True, window=7, unit=None, membe
             w = y - 0.5 * (u @ y) * u
             S = S - np.outer(u, w) - np.outer(w, u)
             N = N - np.outer(N @ u, u)
-            send = lambda key, v: store("send", j, key, v)
             if j == 0:
                 started.add(s)
                 D[s + 1] = S[0, 0]
@@ -135,12 +142,6 @@ def chase(Bd, b, seed, start_word=True, ordered=True, window=7, unit=None, membe
                 if s == nsw - 1:
                     E[n - 2], D[n - 1] = S[1, 0], S[1, 1]
             else:
-                B1 = B1 - np.outer(u, u @ B1)
-                for k in range(1, b):
-                    send((wr, j - 1, "S", b - 1, k - 1), B1[0, k])
-                    send((wr, j - 1, "S", k - 1, b - 1), B1[0, k])
-                    for i in range(1, ln):
-                        send((wr, j - 1, "N", i - 1, k - 1), B1[i, k])
                 send((wr, j - 1, "S", b - 1, b - 1), S[0, 0])
                 for i in range(1, ln):
                     send((wr, j - 1, "N", i - 1, b - 1), S[i, 0])
