@@ -175,7 +175,9 @@ __device__ __attribute__((always_inline)) inline double chase_reflector(double x
 // every wave has waited for loads issued after the previous step's empties
 // (memory operations complete in order), so message j of sweep s, which S(:, 0)
 // and beta complete at step (s, j + 1), proves that s has emptied slot j of the
-// other parity; B1 goes to slot j - 1, which the step before proved empty.  Only a
+// other parity; B1 goes to slot j - 1, which the step before proved empty.  In
+// the last step, whose message nothing follows, a wave completes its empties
+// before it sends (every wave that empties elements there sends some).  Only a
 // sweep's first slots have no such message before them: the receiver waits for
 // the predecessor's start word, set once it holds its own first window.
 // What a sweep sends is exactly what the next one loads (both bounded by row
@@ -551,6 +553,8 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
         N[r] -= qq * uk[r];
         sB[(kc + 8 * r) * LD + ri] = N[r];
       }
+      // the last message has no step behind it to show that the slot is empty
+      if (last) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       {
         const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(wr, 0, slot_bytes, kBufferWord3);
 #pragma unroll
@@ -603,7 +607,15 @@ __global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
   while (true) {
     if (tid == 0) {
       int s, q, m;
-      s_sweep = next_sweep(ticket, xcd, units, count, nsweeps, err, s, q, m) ? s : -1;
+      if (LOCAL) {
+        s_sweep = next_sweep(ticket, xcd, units, count, nsweeps, err, s, q, m) ? s : -1;
+      } else {  // sweep by sweep over the problems
+        const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        s = (int)(t / count);
+        q = (int)(t % count);
+        m = 0;
+        s_sweep = s < nsweeps ? s : -1;
+      }
       s_problem = q;
       s_member = m;
       s_abort = 0;
@@ -1050,11 +1062,18 @@ static int launch_chase_group(evd_ctx *ctx, int count, long n, long b, double *b
 // Sweeps in flight of one problem (a sweep trails its predecessor by two to
 // three steps of b rows) and the XCDs that run the chase: 32 sweeps an XCD, one
 // per CU, keep a chain of up to 32 on one XCD; at b = 64, 16, whose slots (64
-// KiB, two steps apart, both parities) fit the 4 MiB of its L2.
+// KiB, two steps apart, both parities) fit the 4 MiB of its L2.  Where the eight
+// XCDs do not hold all that are in flight, the slots would not stay in the L2s: a
+// large batch runs as several launches, and single chases beyond that (n >
+// 20000 at b = 32) do without boxes.
 static long chase_inflight(long n, long b) { return (2 * n + 5 * b - 1) / (5 * b) + 4; }
 static int chase_members(int count, long n, long b) {
   const long per = b <= 32 ? 32 : 16;
-  return (int)std::min<long>(kXcds, (chase_inflight(n, b) * count + per - 1) / per);
+  return (int)((chase_inflight(n, b) * count + per - 1) / per);
+}
+// problems of a batch per launch: as many as the XCDs hold in flight
+static int chase_batch(int count, long n, long b) {
+  return (int)std::max<long>(1, std::min<long>(count, kXcds * (b <= 32 ? 32 : 16) / chase_inflight(n, b)));
 }
 
 template <int BW>
@@ -1062,21 +1081,20 @@ static int launch_chase(evd_ctx *ctx, int count, long n, long b, const double *b
                         double *mail, double *boxes, float *U, long ldu, long u_stride, int *com, unsigned *ticket,
                         double *D, long d_stride, double *E, long e_stride) {
   // workgroups: as many as sweeps are in flight (a workgroup takes its next
-  // sweep as soon as it finishes one), at most the resident count.  Those
-  // beyond that only poll and crowd out concurrent solves.  With boxes that many
-  // on each member XCD: workgroups are dealt to the XCDs in turn, so eight
-  // times as many are launched, of which those on other XCDs leave at once.
+  // sweep as soon as it finishes one), at most one per CU.  Those beyond that
+  // only poll and crowd out concurrent solves.  With boxes that many on each
+  // member XCD: workgroups are dealt to the XCDs in turn, so eight times as many
+  // are launched, of which those on other XCDs leave at once.
   int resident = 0;
   const void *kernel = boxes ? (const void *)chase_kernel<BW, true> : (const void *)chase_kernel<BW, false>;
   EVD_TRY(max_coresident_blocks(ctx, kernel, ChaseShape<BW>::NT, 0, &resident));
-  resident = std::max(ctx->num_cus, resident);
   const long nsweeps = n - 2, inflight = chase_inflight(n, b);
   const int members = boxes ? chase_members(count, n, b) : 1;
   // units: everything on one XCD where that holds a problem's sweeps in
   // flight; else as many sweeps as an XCD holds; batches mix the problems
-  long per = std::min<long>(inflight * count, resident), len = 1;
+  long per = std::min<long>(inflight * count, ctx->num_cus), len = 1;
   if (boxes) {
-    per = std::min<long>((per + members - 1) / members + 2, resident / kXcds);
+    per = std::min<long>((inflight * count + members - 1) / members + 2, resident / kXcds);
     len = count > 1 ? std::min(inflight, per) : members == 1 ? nsweeps : per;
     len = std::max<long>(2, std::min(len, nsweeps));
     per *= kXcds;
@@ -1143,6 +1161,7 @@ size_t sb2st_batched_workspace(int count, long n, long b) {
 // The XCDs' boxes are scratch on top of that, used where the arena has room
 // (a call never fails for want of them; the results are the same).
 static size_t chase_boxes_bytes(int count, long n, long b) {
+  count = chase_batch(count, n, b);
   return (size_t)chase_members(count, n, b) * count * 2 * mail_half(n, b) * sizeof(double);
 }
 
@@ -1172,6 +1191,7 @@ int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ld
     const int depth = std::min({ctx->tune.chase_depth > 0 ? ctx->tune.chase_depth : 1, group_depth_max(b), 3});
     if (b > 64) return set_error(ctx, EVD_E_UNSUPPORTED, "bandwidth %ld > 64", b);
     auto boxes = [&]() -> double * {
+      if (chase_members(chase_batch(count, n, b), n, b) > kXcds) return nullptr;
       const size_t bytes = chase_boxes_bytes(count, n, b);
       const size_t room = ctx->arena_bytes - std::min(ctx->arena_bytes, align256(ctx->arena_top));
       return ext_com || bytes > room ? nullptr : static_cast<double *>(arena_alloc(ctx, bytes));
@@ -1188,12 +1208,25 @@ int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ld
                            ctx->stream>>>((int)n, band, ldband, band_stride, U, ldu, u_stride, D, d_stride, E, e_stride);
       EVD_LAUNCHED(ctx);
       return 0;
-    } else if (b <= 32) {
-      return launch_chase<32>(ctx, count, n, b, band, ldband, band_stride, mail, boxes(), U, ldu, u_stride, com, ticket,
-                              D, d_stride, E, e_stride);
     } else {
-      return launch_chase<64>(ctx, count, n, b, band, ldband, band_stride, mail, boxes(), U, ldu, u_stride, com, ticket,
-                              D, d_stride, E, e_stride);
+      double *bx = boxes();
+      const int batch = bx ? chase_batch(count, n, b) : count;
+      for (int q0 = 0; q0 < count; q0 += batch) {
+        const int c = std::min(batch, count - q0);
+        if (q0 > 0) EVD_TRY(fill_u32(ctx, ticket, kTicketWords, 0u));
+        const double *bq = band + (long)q0 * band_stride;
+        double *mq = mail + (long)q0 * 2 * mail_half(n, b);
+        float *Uq = U + (long)q0 * u_stride;
+        int *cq = com + (long)q0 * com_stride;
+        double *Dq = D + (long)q0 * d_stride, *Eq = E + (long)q0 * e_stride;
+        if (b <= 32)
+          EVD_TRY(launch_chase<32>(ctx, c, n, b, bq, ldband, band_stride, mq, bx, Uq, ldu, u_stride, cq, ticket, Dq,
+                                   d_stride, Eq, e_stride));
+        else
+          EVD_TRY(launch_chase<64>(ctx, c, n, b, bq, ldband, band_stride, mq, bx, Uq, ldu, u_stride, cq, ticket, Dq,
+                                   d_stride, Eq, e_stride));
+      }
+      return 0;
     }
   }
   band_extract_batched_kernel<<<dim3((unsigned)std::min<long>((n + 255) / 256, 1024), (unsigned)count), 256, 0,
@@ -1211,7 +1244,7 @@ int sb2st(evd_ctx *ctx, long n, long b, double *band, long ldband, float *U, lon
 // that (no captured graph, lent arena or budget against it), else without
 static int chase_arena(evd_ctx *ctx, int count, long n, long b) {
   const size_t need = sb2st_batched_workspace(count, n, b) + 4096, all = need + chase_boxes_bytes(count, n, b);
-  if (all > ctx->arena_bytes && ctx->graphs == 0 && !ctx->arena_external && !(ctx->budget && all > ctx->budget) &&
+  if (chase_members(chase_batch(count, n, b), n, b) <= kXcds && all > ctx->arena_bytes && ctx->graphs == 0 && !ctx->arena_external && !(ctx->budget && all > ctx->budget) &&
       arena_ensure(ctx, all) == 0)
     return 0;
   return arena_ensure(ctx, need);
