@@ -574,10 +574,14 @@ static int sgemm_dispatch(evd_ctx *ctx, long m, long n, long k, float alpha, con
   if (m <= 32 && n > 64)
     return launch_sgemm<TA, TB, 32, 256, 1, 4>(ctx, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch,
                                                256, 2, kc);
-  long big_tiles = ((m + 127) / 128) * ((n + 127) / 128) * shape_batch(ctx, batch);
-  // the gemm_tile knob forces 128 x 128 (1) or 64 x 64 (2) output tiles
-  if (ctx->tune.gemm_tile == 1 ||
-      (ctx->tune.gemm_tile == 0 && (big_tiles >= target || (m > 64 && n > 64 && k < 1024))))
+  // 128 x 128 output tiles where they and a K split (chunks of 256) give every
+  // CU a workgroup; below that 64 x 64 tiles, whose workgroups do a quarter
+  // of the work one after the other (the merges and products of the back
+  // transformation at n = 1000: 40-55 us on 128 x 128 tiles for any k < 1024,
+  // 10-14 us on 64 x 64).  The gemm_tile knob forces 128 x 128 (1) or 64 x 64 (2).
+  const long big_tiles = ((m + 127) / 128) * ((n + 127) / 128) * shape_batch(ctx, batch);
+  const bool short_k = m > 64 && n > 64 && k < 1024 && big_tiles * std::max<long>(1, k / 256) >= ctx->num_cus;
+  if (ctx->tune.gemm_tile == 1 || (ctx->tune.gemm_tile == 0 && (big_tiles >= target || short_k)))
     return launch_sgemm<TA, TB, 128, 128, 2, 2>(ctx, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch,
                                                 256, 2, kc);
   return launch_sgemm<TA, TB, 64, 64, 2, 2>(ctx, m, n, k, alpha, A, lda, sA, B, ldb, sB, beta, C, ldc, sC, batch, 128,

@@ -259,9 +259,19 @@ long sbr_back_blk(long knob, long b, long wcols) {
   return bb;
 }
 
+// Columns of W and Y that hold panels (the rest of wcols is zero padding), and
+// the block width without the doublings that would only merge padding: at n =
+// 256 the merges and products of three 256 x 256 zero blocks, five launches of
+// 38 us, were a tenth of the whole solve.
+static long panel_cols(long n, long b) { return n - b > 1 ? (n - b - 2) / b * b + b : 0; }
+static long used_blk(long blk, long b, long used) {
+  while (blk % 2 == 0 && blk / 2 >= b && blk / 2 >= used) blk /= 2;
+  return blk;
+}
+
 int sbr_back(evd_ctx *ctx, long n, long b, long ncols, float *Z, long ldz, float *W, long ldw, const float *Y,
              long ldy, long wcols) {
-  const long blk = sbr_back_blk(ctx->tune.sbr_back_block, b, wcols);
+  const long blk = used_blk(sbr_back_blk(ctx->tune.sbr_back_block, b, wcols), b, panel_cols(n, b));
   // a block of b (no merge; b not dividing the padding, e.g. b = 24) is applied panel by panel
   if (blk != b && wcols % blk != 0)
     return set_error(ctx, EVD_E_UNSUPPORTED, "W/Y column padding %ld not a multiple of %ld", wcols, blk);
@@ -275,7 +285,7 @@ int sbr_back(evd_ctx *ctx, long n, long b, long ncols, float *Z, long ldz, float
 int sbr_back_batched(evd_ctx *ctx, int count, long n, long b, long ncols, float *Z, long ldz, long sZ, float *W,
                      long ldw, const float *Y, long ldy, long wcols) {
   if (count == 1) return sbr_back(ctx, n, b, ncols, Z, ldz, W, ldw, Y, ldy, wcols);
-  const long blk = sbr_back_blk(ctx->tune.sbr_back_block, b, wcols);
+  const long blk = used_blk(sbr_back_blk(ctx->tune.sbr_back_block, b, wcols), b, panel_cols(n, b));
   if (blk != b && wcols % blk != 0) return set_error(ctx, EVD_E_UNSUPPORTED, "W/Y column padding %ld not a multiple of %ld", wcols, blk);
   ArenaFrame frame(ctx);
   ShapeDiv shape(ctx, count);
