@@ -492,6 +492,12 @@ static int panel_halves(evd_ctx *ctx, long m, long nc, const float *A, long lda,
   return 0;
 }
 
+// Rows per workgroup of the column-exchange kernel: the panel_rows knob, 512 (two
+// per thread) by default, 256 where they are all the panel has (half the
+// additions of every step, the same sums; the seven panels of n = 256, one
+// of them factored here: 124 -> 116 us).
+static int panel_rows(const evd_ctx *ctx, long m) { return ctx->tune.panel_rows == 256 || m <= 256 ? 256 : 512; }
+
 // Panel factorisation used by the SBR drivers (FP32 and FP64 storage; the
 // arithmetic is FP64 in both) and by evd_panel_qr_f32 / _f64.
 template <typename T>
@@ -508,14 +514,12 @@ int panel_qr_t(evd_ctx *ctx, long m, long nc, const T *A, long lda, T *Y, long l
     int *bad = arena_alloc_n<int>(ctx, 1);
     if (!bad) return EVD_E_NOMEM;
     EVD_TRY(panel_cholqr<T>(ctx, 1, m, nc, A, lda, 0, Y, ldy, 0, W, ldw, 0, R, ldr, Aout, ldo, 0, tau_out, bad));
-    if (ctx->tune.panel_rows == 256)
+    if (panel_rows(ctx, m) == 256)
       return launch_panel<32, 1, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out, 1, 0, 0, 0, 0,
                                     bad);
     return launch_panel<32, 2, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out, 1, 0, 0, 0, 0, bad);
   }
-  // rows per workgroup (the panel_rows knob): 512 (two per thread) by
-  // default; 256 doubles the workgroups that share the column exchanges
-  if (nc <= 32 && ctx->tune.panel_rows == 256)
+  if (nc <= 32 && panel_rows(ctx, m) == 256)
     return launch_panel<32, 1, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out);
   if (nc <= 32) return launch_panel<32, 2, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out);
   if (nc <= 64) return launch_panel<64, 1, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out);
@@ -573,6 +577,9 @@ int panel_qr_batched(evd_ctx *ctx, int count, long m, long nc, float *A, long ld
     int maxres = 0;
     if (count > 1 && G > 1)
       EVD_TRY(max_coresident_blocks(ctx, (const void *)panel_qr_kernel<32, 2, float>, 256, 0, &maxres));
+    if (m <= 256)
+      return launch_panel<32, 1, float>(ctx, m, nc, A, lda, Y, ldy, W, ldw, nullptr, 0, A, lda, nullptr, count, sA,
+                                        sY, sW, sA, bad);
     if (count == 1 || G == 1 || (G * count <= maxres && G * count <= kTagWords))
       return launch_panel<32, 2, float>(ctx, m, nc, A, lda, Y, ldy, W, ldw, nullptr, 0, A, lda, nullptr, count, sA,
                                         sY, sW, sA, bad);
@@ -592,6 +599,9 @@ int panel_qr_batched(evd_ctx *ctx, int count, long m, long nc, float *A, long ld
     else
       EVD_TRY(max_coresident_blocks(ctx, (const void *)panel_qr_kernel<64, 1, float>, 256, 0, &maxres));
   }
+  if (count > 1 && nc <= 32 && m <= 256)
+    return launch_panel<32, 1, float>(ctx, m, nc, A, lda, Y, ldy, W, ldw, nullptr, 0, A, lda, nullptr, count, sA, sY,
+                                      sW, sA);
   if (count > 1 && nc <= 64 && (G == 1 || (G * count <= maxres && G * count <= kTagWords))) {
     if (nc <= 32)
       return launch_panel<32, 2, float>(ctx, m, nc, A, lda, Y, ldy, W, ldw, nullptr, 0, A, lda, nullptr, count, sA,
