@@ -1012,8 +1012,10 @@ __global__ __launch_bounds__((D + 1) * 64, 1) void chase_group_kernel(
   }
 }
 
-__global__ void band_pack_kernel(int n, int b, const float *__restrict__ A, long lda, double *__restrict__ band,
-                                 long ldb) {
+__global__ void band_pack_kernel(int n, int b, const float *__restrict__ A, long lda, long a_stride,
+                                 double *__restrict__ band, long ldb, long band_stride) {
+  A += blockIdx.z * a_stride;
+  band += blockIdx.z * band_stride;
   long c = blockIdx.y * (long)blockDim.y + threadIdx.y;
   for (; c < n; c += (long)gridDim.y * blockDim.y)
     for (int i = threadIdx.x; i < 2 * b; i += blockDim.x) {
@@ -1023,13 +1025,18 @@ __global__ void band_pack_kernel(int n, int b, const float *__restrict__ A, long
     }
 }
 
-int band_pack(evd_ctx *ctx, long n, long b, const float *A, long lda, double *band, long ldband) {
+int band_pack_batched(evd_ctx *ctx, int count, long n, long b, const float *A, long lda, long a_stride, double *band,
+                      long ldband, long band_stride) {
   if (n <= 0) return 0;
   dim3 blk(64, 4);
   unsigned gy = (unsigned)std::min<long>((n + 3) / 4, 65535);
-  band_pack_kernel<<<dim3(1, gy), blk, 0, ctx->stream>>>((int)n, (int)b, A, lda, band, ldband);
+  band_pack_kernel<<<dim3(1, gy, (unsigned)count), blk, 0, ctx->stream>>>((int)n, (int)b, A, lda, a_stride, band, ldband,
+                                                                          band_stride);
   EVD_LAUNCHED(ctx);
   return 0;
+}
+int band_pack(evd_ctx *ctx, long n, long b, const float *A, long lda, double *band, long ldband) {
+  return band_pack_batched(ctx, 1, n, b, A, lda, 0, band, ldband, 0);
 }
 
 // largest sweeps-per-group whose window fits kGW columns: (2D + 2) b - D + 1 <= kGW
@@ -1172,7 +1179,10 @@ static size_t chase_boxes_bytes(int count, long n, long b) {
 int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ldband, long band_stride, float *U,
                   long ldu, long u_stride, double *D, long d_stride, double *E, long e_stride, int *ext_com) {
   if (n <= 0 || count <= 0) return 0;
-  for (int q = 0; q < count; q++) EVD_TRY(fill_f32(ctx, U + (long)q * u_stride, ldu, n, ldu, 0.f));
+  if (u_stride == ldu * n)
+    EVD_TRY(fill_f32(ctx, U, ldu, n * count, ldu, 0.f));
+  else
+    for (int q = 0; q < count; q++) EVD_TRY(fill_f32(ctx, U + (long)q * u_stride, ldu, n, ldu, 0.f));
   if (n > 2) {
     ArenaFrame frame(ctx);
     // messages, then progress words com[q * n * kComStride + s * kComStride]

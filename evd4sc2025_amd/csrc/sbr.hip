@@ -146,8 +146,10 @@ int sy2sb_batched(evd_ctx *ctx, int count, long n, long b, long nb, float *A, lo
   if (n <= 0 || count <= 0) return 0;
   if (count == 1) return sy2sb(ctx, n, b, nb, A, lda, W, ldw, Y, ldy, wcols);
   for (int q = 0; q < count; q++) {
-    EVD_TRY(fill_f32(ctx, W + q * sW, n, wcols, ldw, 0.f));
-    EVD_TRY(fill_f32(ctx, Y + q * sY, n, wcols, ldy, 0.f));
+    const int c = sW == ldw * wcols && sY == ldy * wcols ? count : 1;  // contiguous: all at once
+    EVD_TRY(fill_f32(ctx, W + q * sW, n, wcols * c, ldw, 0.f));
+    EVD_TRY(fill_f32(ctx, Y + q * sY, n, wcols * c, ldy, 0.f));
+    if (c == count) break;
   }
   ArenaFrame frame(ctx);
   ShapeDiv shape(ctx, count);

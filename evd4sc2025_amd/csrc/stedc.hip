@@ -1248,7 +1248,10 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
     dc_tear_kernel<<<(unsigned)std::min<long>((nt + 255) / 256, 1024), 256, 0, ctx->stream>>>(nt, dsplit, E, D);
     EVD_LAUNCHED(ctx);
     // outside the leaves' diagonal blocks Z starts as zeros
-    for (int q = 0; vec && q < count; q++) EVD_TRY(fill_f64(ctx, Z + q * zs, n, n, ldz, 0.0));
+    if (vec && zs == n * ldz)
+      EVD_TRY(fill_f64(ctx, Z, n, n * count, ldz, 0.0));
+    else
+      for (int q = 0; vec && q < count; q++) EVD_TRY(fill_f64(ctx, Z + q * zs, n, n, ldz, 0.0));
   }
   dc_leaf_kernel<<<(unsigned)plan->nleaf, 64, 0, ctx->stream>>>(dleaf, E, D, Z, ldz, sc.zmul, rows, err);
   EVD_LAUNCHED(ctx);

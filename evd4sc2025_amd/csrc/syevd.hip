@@ -23,6 +23,8 @@ int sy2sb(evd_ctx *ctx, long n, long b, long nb, float *A, long lda, float *W, l
           long wcols);
 size_t sy2sb_workspace(long n, long b, long nb);
 int band_pack(evd_ctx *ctx, long n, long b, const float *A, long lda, double *band, long ldband);
+int band_pack_batched(evd_ctx *ctx, int count, long n, long b, const float *A, long lda, long a_stride, double *band,
+                      long ldband, long band_stride);
 int sb2st(evd_ctx *ctx, long n, long b, double *band, long ldband, float *U, long ldu, double *D, double *E);
 int stedc(evd_ctx *ctx, long n, double *D, double *E, double *Z, long ldz);
 size_t stedc_workspace(long n);
@@ -57,8 +59,11 @@ int sbr_back_batched(evd_ctx *ctx, int count, long n, long b, long ncols, float 
 static long wy_cols(long n) { return (n + 1023) / 1024 * 1024; }
 
 // ------------------------------------------------------------- helpers
+// problem blockIdx.z at the given strides
 __global__ void f64_to_f32_kernel(long rows, long cols, const double *__restrict__ s, long lds, float *__restrict__ d,
-                                  long ldd) {
+                                  long ldd, long s_stride = 0, long d_stride = 0) {
+  s += blockIdx.z * s_stride;
+  d += blockIdx.z * d_stride;
   for (long c = blockIdx.y; c < cols; c += gridDim.y)
     for (long r = blockIdx.x * (long)blockDim.x + threadIdx.x; r < rows; r += (long)gridDim.x * blockDim.x)
       d[r + c * ldd] = (float)s[r + c * lds];
@@ -73,33 +78,65 @@ static dim3 grid2d(long rows, long cols) {
   return dim3((unsigned)std::min<long>((rows + 255) / 256, 64), (unsigned)std::min<long>(cols, 8192));
 }
 
+// rows (and columns) that count toward max |a_ij|, per problem of one launch
+constexpr int kScreenBatch = 64;
+struct ScreenRows {
+  int n[kScreenBatch];
+};
+
 // Symmetric fill of the upper triangle from the lower one + non-finite
 // screen + max |a_ij| (as the bits of a non-negative float, which order like
-// unsigned integers) into *amax.  A non-finite entry raises EVD_E_NONFINITE
+// unsigned integers) into amax[q].  A non-finite entry raises EVD_E_NONFINITE
 // in the error word (read when the call ends) and is replaced by 0, so the
 // rest of the solve runs on finite data without a host round trip after the
 // screen.
-// Entries at rows (and columns) >= nmax do not count toward the maximum.
-__global__ void symmetrize_check_kernel(long n, float *__restrict__ A, long lda, unsigned *__restrict__ err,
-                                        unsigned *__restrict__ amax, long nmax) {
+// One workgroup per 64 x 64 tile of the lower triangle (grid x) and problem
+// (grid z); the mirrored tile goes through LDS, so both triangles are accessed
+// along columns (a thread per entry wrote the upper one at a stride of lda: n =
+// 1000: 58 us, now 9 us).
+__global__ __launch_bounds__(256) void symmetrize_check_kernel(int n, float *__restrict__ A, long lda, long a_stride,
+                                                               unsigned *__restrict__ err,
+                                                               unsigned *__restrict__ amax, ScreenRows rows) {
+  A += blockIdx.z * a_stride;
+  const int nmax = rows.n[blockIdx.z];
+  const int t = (int)blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int ti = (int)((sqrtf(8.f * (float)t + 1.f) - 1.f) * 0.5f);  // tile (ti, tj), tj <= ti
+  while ((ti + 1) * (ti + 2) / 2 <= t) ti++;
+  while (ti * (ti + 1) / 2 > t) ti--;
+  const int r0 = 64 * ti, c0 = 64 * (t - ti * (ti + 1) / 2);
+  __shared__ float tile[64][65];
   unsigned mx = 0;
-  for (long c = blockIdx.y; c < n; c += gridDim.y)
-    for (long r = c + blockIdx.x * (long)blockDim.x + threadIdx.x; r < n; r += (long)gridDim.x * blockDim.x) {
-      float v = A[r + c * lda];
-      if (!isfinite(v)) {
-        atomicOr(err, (unsigned)EVD_E_NONFINITE);
-        v = 0.f;
-        A[r + c * lda] = v;
-      }
-      A[c + r * lda] = v;
-      if (r < nmax) mx = max(mx, __float_as_uint(fabsf(v)));
+  const int r = r0 + lane;
+  float v[16];
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    const int c = c0 + w + 4 * k;
+    v[k] = (r < n && c <= r) ? A[r + c * lda] : 0.f;
+  }
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    const int c = c0 + w + 4 * k;
+    if (!isfinite(v[k])) {
+      atomicOr(err, (unsigned)EVD_E_NONFINITE);
+      v[k] = 0.f;
+      A[r + c * lda] = 0.f;
     }
+    if (r < nmax) mx = max(mx, __float_as_uint(fabsf(v[k])));
+    tile[w + 4 * k][lane] = v[k];
+  }
+  __syncthreads();
+  // lane runs along the columns of the tile, which are rows of the mirror
+#pragma unroll
+  for (int k = 0; k < 16; k++) {
+    const int c = c0 + lane, q = r0 + w + 4 * k;
+    if (q < n && c < q) A[c + q * lda] = tile[lane][w + 4 * k];
+  }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 64));
   // one atomic per wave at most, and only while it can still raise the
   // maximum (a stale read only lets an unneeded atomic through)
-  if ((threadIdx.x & 63) == 0 && mx > __hip_atomic_load(amax, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-    atomicMax(amax, mx);
+  unsigned *am = amax + blockIdx.z;
+  if (lane == 0 && mx > __hip_atomic_load(am, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(am, mx);
 }
 
 // Scaling into the safe range (the step of LAPACK ssyevd): with
@@ -156,10 +193,13 @@ __global__ void unscale_values_kernel(long n, double *__restrict__ w, long w_str
 static int prepare_inputs(evd_ctx *ctx, int count, long n, float *A, long lda, long a_stride, double *sigma,
                           unsigned *amax) {
   EVD_TRY(fill_u32(ctx, amax, (size_t)count, 0u));
-  for (int q = 0; q < count; q++) {
-    const long nmax = ctx->amax_rows ? std::min(n, ctx->amax_rows[q]) : n;
-    symmetrize_check_kernel<<<grid2d(n, n), 256, 0, ctx->stream>>>(n, A + q * a_stride, lda, ctx->ctrl + kCtrlError,
-                                                                     amax + q, nmax);
+  const long tiles = (n + 63) / 64;
+  for (int q0 = 0; q0 < count; q0 += kScreenBatch) {
+    const int c = std::min(kScreenBatch, count - q0);
+    ScreenRows rows;
+    for (int q = 0; q < c; q++) rows.n[q] = (int)(ctx->amax_rows ? std::min(n, ctx->amax_rows[q0 + q]) : n);
+    symmetrize_check_kernel<<<dim3((unsigned)(tiles * (tiles + 1) / 2), 1, (unsigned)c), 256, 0, ctx->stream>>>(
+        (int)n, A + q0 * a_stride, lda, a_stride, ctx->ctrl + kCtrlError, amax + q0, rows);
     EVD_LAUNCHED(ctx);
   }
   const dim3 g = grid2d(n, n);
@@ -176,7 +216,10 @@ static int unscale_values(evd_ctx *ctx, int count, long n, double *w, long w_str
   return 0;
 }
 
-__global__ void copy_f64_kernel(long n, const double *__restrict__ s, double *__restrict__ d) {
+__global__ void copy_f64_kernel(long n, const double *__restrict__ s, double *__restrict__ d, long s_stride = 0,
+                                long d_stride = 0) {
+  s += blockIdx.y * s_stride;
+  d += blockIdx.y * d_stride;
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) d[i] = s[i];
 }
 
@@ -323,22 +366,19 @@ int syevd_batched(evd_ctx *ctx, char jobz, int count, long n, long b, long nb, f
 
   stage_mark(ctx, 0);
   EVD_TRY(sy2sb_batched(ctx, count, n, b, nb, A, lda, a_stride, W, n, sWY, Y, n, sWY, wc));
-  for (int q = 0; q < count; q++) EVD_TRY(band_pack(ctx, n, b, A + q * a_stride, lda, band + q * band_stride, ldband));
+  EVD_TRY(band_pack_batched(ctx, count, n, b, A, lda, a_stride, band, ldband, band_stride));
   stage_mark(ctx, 1);
   EVD_TRY(sb2st_batched(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, D, n, E, e_stride, nullptr));
   stage_mark(ctx, 2);
   EVD_TRY(stedc_batched(ctx, count, n, D, E, Zt, n, n * n));
-  for (int q = 0; q < count; q++) {
-    copy_f64_kernel<<<(unsigned)std::min<long>((n + 255) / 256, 1024), 256, 0, ctx->stream>>>(n, D + q * n,
-                                                                                             w + q * w_stride);
-    EVD_LAUNCHED(ctx);
-  }
+  copy_f64_kernel<<<dim3((unsigned)std::min<long>((n + 255) / 256, 1024), (unsigned)count), 256, 0, ctx->stream>>>(
+      n, D, w, n, w_stride);
+  EVD_LAUNCHED(ctx);
   EVD_TRY(unscale_values(ctx, count, n, w, w_stride, sigma));
   if (vec) {
-    for (int q = 0; q < count; q++) {
-      f64_to_f32_kernel<<<grid2d(n, n), 256, 0, ctx->stream>>>(n, n, Zt + q * n * n, n, Z + q * z_stride, ldz);
-      EVD_LAUNCHED(ctx);
-    }
+    const dim3 gz = grid2d(n, n);
+    f64_to_f32_kernel<<<dim3(gz.x, gz.y, (unsigned)count), 256, 0, ctx->stream>>>(n, n, Zt, n, Z, ldz, n * n, z_stride);
+    EVD_LAUNCHED(ctx);
     stage_mark(ctx, 3);
     if (b != 32 && b != 64) {
       EVD_TRY(bc_back_small_batched(ctx, count, n, b, n, Z, ldz, z_stride, U, ldu, u_stride, true));
