@@ -310,31 +310,51 @@ __device__ __forceinline__ bool wave_cholesky(const double *G, double *R, int la
   return ok;
 }
 
-// X = U^-1 for an upper triangular 32 x 32 U on one wave: lane c forms column
-// c by right-looking back substitution (x_k is final once the rows below k
-// are applied, and the updates of the rows above it are independent, so the
-// dependent chain is one multiply-add per step; lane i divides for the
-// diagonal's reciprocal i).  UNIT_LT: U is the transpose of the unit lower
-// triangle stored in M (U[i][k] = M[k][i], unit diagonal); otherwise U is
+// v of lane ^ 32 (v_permlane32_swap exchanges one half of its destination with
+// the other half of its source; xor-ing out the own value leaves the partner's)
+__device__ __forceinline__ double other_half(double v) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  const auto rl = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto rh = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return __longlong_as_double((long long)(((unsigned long long)(rh[0] ^ rh[1] ^ hi) << 32) | (rl[0] ^ rl[1] ^ lo)));
+}
+
+// X = U^-1 for an upper triangular 32 x 32 U on one wave: lanes c and c + 32
+// form column c by right-looking back substitution, the even and the odd rows
+// (x_k is final once the rows below k are applied, and the updates of the
+// rows above it are independent, so the dependent chain is x_k to the other
+// half and one multiply-add per step; lane i divides for the diagonal's
+// reciprocal i).  The updates are what takes the time (all rows in one lane, the
+// upper half of the wave idle: 5.6 us; the pass with its two rounds of inverses
+// went from 39.4 to 35.3 us at m = 1000).  UNIT_LT: U is the transpose of the unit
+// lower triangle stored in M (U[i][k] = M[k][i], unit diagonal); otherwise U is
 // M's upper triangle.
 template <bool UNIT_LT>
 __device__ __forceinline__ void wave_upper_inverse(const double *M, double *X, int lane) {
-  const int c = lane & (kQ - 1);
+  const int c = lane & (kQ - 1), h = lane >> 5;
   const double rd = UNIT_LT ? 1.0 : 1.0 / M[c * kLD + c];
-  double s[kQ];
+  double s[kQ / 2];  // rows 2 m + h
 #pragma unroll
-  for (int i = 0; i < kQ; i++) s[i] = (i == c) ? 1.0 : 0.0;
+  for (int m = 0; m < kQ / 2; m++) s[m] = (2 * m + h == c) ? 1.0 : 0.0;
 #pragma unroll
   for (int k = kQ - 1; k >= 0; k--) {
-    const double xk = UNIT_LT ? s[k] : s[k] * lane_value(rd, k);
-    s[k] = xk;
+    const bool own = h == (k & 1);  // row k is in this half
+    const double x = UNIT_LT ? s[k / 2] : s[k / 2] * lane_value(rd, k);
+    const double y = other_half(x);
+    const double xk = own ? x : y;
+    if (k & 1) {  // row k - 1 shares the register
+      const double t = s[k / 2] - (UNIT_LT ? M[k * kLD + k - 1] : M[(k - 1) * kLD + k]) * xk;
+      s[k / 2] = own ? x : t;
+    } else {
+      s[k / 2] = own ? x : s[k / 2];
+    }
 #pragma unroll
-    for (int i = 0; i < k; i++) s[i] -= (UNIT_LT ? M[k * kLD + i] : M[i * kLD + k]) * xk;
+    for (int m = 0; m < k / 2; m++)
+      s[m] -= (UNIT_LT ? M[k * kLD + 2 * m + h] : M[(2 * m + h) * kLD + k]) * xk;
   }
-  if (lane < kQ) {
 #pragma unroll
-    for (int i = 0; i < kQ; i++) X[i * kLD + c] = s[i];
-  }
+  for (int m = 0; m < kQ / 2; m++) X[(2 * m + h) * kLD + c] = s[m];
 }
 
 // C = A B for 32 x 32 matrices in LDS (pitch kLD), by the whole workgroup:
