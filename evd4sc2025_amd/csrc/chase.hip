@@ -10,19 +10,24 @@
 //   N <- N H (block below S, which becomes the next B1 - the bulge).
 // u is stored in U[p .. p+len-1, s] ("noBandU" layout, FP32).
 //
-// MI355X design: sweeps are handed out by atomic tickets, runs of consecutive
-// ones to one XCD, in an order that leaves every sweep's predecessor finished
-// or owned by a running workgroup, so no co-residency (cooperative launch) is
-// needed.  A sweep does not update a band in memory: it receives the window of
-// each of its steps from its predecessor as a message and sends the next
-// sweep's windows on (chase_kernel below).  A message within an XCD goes
-// through its L2 (plain stores, loads that pass the CU's cache by); one that
-// crosses XCDs is device-coherent on both sides (sc1).
+// MI355X design: sweeps are handed out by an atomic ticket in increasing
+// order, so a sweep's predecessor is always owned by a running workgroup and
+// no co-residency (cooperative launch) is needed.  The band lives in HBM and
+// every access of the chase is device-coherent (sc1 loads and stores, which
+// bypass the non-coherent per-XCD caches; on this chip the L1-bypassing sc0
+// loads do not observe other CUs' stores, so an XCD-local exchange is not
+// available), and a vmcnt(0) wait orders a step's stores before its flag.
+// Per step the S and N windows are held in registers (a row per 256/BW
+// lanes), B1 and the next B1 in LDS; H B1 is applied by one wave while the
+// others wait for their window loads.  Step (s, p) needs step (s-1, p-1+2b)
+// only for one element, B1[0][0] of that step (row p+2b-1, column p+b-1),
+// which becomes beta; the owner publishes that beta at the end of its
+// previous step, so sweep s may start row p as soon as sweep s-1 has
+// published a next-row >= p + 2b - 1 (a lag of two steps, not three).
 // Every wait is bounded by a watchdog so the grid always drains.
 #include <climits>
 #include <map>
 #include <mutex>
-#include <type_traits>
 
 #include "common.hpp"
 
@@ -36,606 +41,197 @@ constexpr unsigned kBufferWord3 = 0x00020000u;  // raw buffer descriptor: 32-bit
 
 constexpr int kSc1 = 16;  // buffer-op cache policy: sc1, device-coherent
 
-// byte offset past every band (< 2 GiB): the buffer range check drops the
-// store or returns 0 for the load, so every lane issues every access
-constexpr unsigned kOutOfRange = 0x80000000u;
-
-__device__ __attribute__((always_inline)) inline double ld_band_at(__amdgpu_buffer_rsrc_t r, unsigned byte_off) {
-  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, byte_off, 0, kSc1));
+__device__ inline double ld_band(__amdgpu_buffer_rsrc_t r, unsigned off_elems) {
+  return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off_elems * 8u, 0, kSc1));
 }
-template <int POLICY>
-__device__ __attribute__((always_inline)) inline void st_band_at(__amdgpu_buffer_rsrc_t r, unsigned byte_off, double v) {
+__device__ inline void st_band(__amdgpu_buffer_rsrc_t r, unsigned off_elems, double v) {
   __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(__attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned, v),
-                                        r, byte_off, 0, POLICY);
+                                        r, off_elems * 8u, 0, kSc1);
 }
 
-__device__ __attribute__((always_inline)) inline void grp_barrier() {
-  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-}
-__device__ __attribute__((always_inline)) inline void wave_lds_order() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
-
-// s_waitcnt with only the vector-memory count: vmcnt(N), N <= 63
-template <int N>
-__device__ __attribute__((always_inline)) inline void wait_vm() {
-  static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-// 64-bit DPP move of v (rows outside RM read 0)
-template <int CTRL, int RM>
-__device__ __attribute__((always_inline)) inline double dpp_f64(double v) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)x, CTRL, RM, 0xf, false);
-  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), CTRL, RM, 0xf, false);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// v of lane ^ 32.  v_permlane32_swap exchanges one half of its destination
-// with the other half of its source; with both operands v, one result holds
-// this lane's own value and the other the partner's, so xor-ing out the own
-// value leaves the partner's whichever half was exchanged.
-__device__ __attribute__((always_inline)) inline double half_swap(double v) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)x, hi = (unsigned)(x >> 32);
-  const auto rl = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-  const auto rh = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-  const unsigned plo = rl[0] ^ rl[1] ^ lo, phi = rh[0] ^ rh[1] ^ hi;
-  return __builtin_bit_cast(double, ((unsigned long long)phi << 32) | plo);
-}
-// v of lane ^ 16 (v_permlane16_swap: the same, rows of 16 lanes)
-__device__ __attribute__((always_inline)) inline double row_swap(double v) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)x, hi = (unsigned)(x >> 32);
-  const auto rl = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-  const auto rh = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-  const unsigned plo = rl[0] ^ rl[1] ^ lo, phi = rh[0] ^ rh[1] ^ hi;
-  return __builtin_bit_cast(double, ((unsigned long long)phi << 32) | plo);
-}
-
-// sum over aligned groups of W lanes (8 .. 64), returned in every lane of the
-// group: each step adds the other half of a group whose halves already agree,
-// so mirrors serve as exchanges
-template <int W>
-__device__ __attribute__((always_inline)) inline double group_sum(double v) {
-  v += dpp_f64<0xb1, 0xf>(v);                  // quad_perm [1, 0, 3, 2]
-  v += dpp_f64<0x4e, 0xf>(v);                  // quad_perm [2, 3, 0, 1]
-  v += dpp_f64<0x141, 0xf>(v);                 // row_half_mirror
-  if (W >= 16) v += dpp_f64<0x140, 0xf>(v);    // row_mirror
-  if (W >= 32) v += row_swap(v);
-  if (W >= 64) v += half_swap(v);
-  return v;
-}
-
-// a b + c d with both products rounded, so that exchanging (a, d) and (b, c)
-// gives the same bits: the two halves of a symmetric block stay equal
-__device__ __attribute__((always_inline)) inline double sym_pair(double a, double b, double c, double d) {
-#pragma clang fp contract(off)
-  const double x = a * b, y = c * d;
-  return x + y;
-}
-
-// Reflector of the chase (reference sign convention) from the column whose
-// entry i is x in lane i (W entries, zeros past its length, repeated every W
-// lanes): u = (x/||x|| + sign(x0) e1) / sqrt(|x0/||x|| + sign(x0)|), so that
-// ||u||^2 = 2 and H x = beta e1.  Returns lane i's u_i; u0 = u_0.
-template <int W>
-__device__ __attribute__((always_inline)) inline double chase_reflector(double x, int lane, double &u0, double &beta) {
-  const double nn = group_sum<W>(x * x);
-  const unsigned long long xb = __builtin_bit_cast(unsigned long long, x);
-  const double x0 = __builtin_bit_cast(double, ((unsigned long long)(unsigned)__builtin_amdgcn_readlane(
-                                                    (int)(unsigned)(xb >> 32), 0)
-                                                << 32) |
-                                                   (unsigned)__builtin_amdgcn_readlane((int)(unsigned)xb, 0));
-  u0 = 0.0;
-  beta = x0;
-  if (!(nn > 0.0)) return 0.0;
-  double inv, nrm, scl, root;
-  rsqrt_sqrt(nn, inv, nrm);
-  const double a = x0 * inv + (x0 >= 0.0 ? 1.0 : -1.0);
-  rsqrt_sqrt(fabs(a), scl, root);
-  beta = x0 >= 0.0 ? -nrm : nrm;
-  u0 = a * scl;
-  return (lane & (W - 1)) == 0 ? u0 : x * inv * scl;
-}
-
-// ---------------------------------------------------------------------------
-// One workgroup per sweep in flight, 8 threads per row of a BW x BW block:
-// thread (ri, kc) holds row ri, columns kc + 8 r.
-//
-// The chase is a chain of dependent steps and nothing else bounds it, so the
-// kernel is built for the latency of that chain: the steps of a sweep, and the
-// hand-off from a sweep to the next.
-//
-// Step.  The window -> q = N u (FMAs, a DPP sum over the row's 8 lanes) ->
-// barrier -> the next column x = N[:, 0] - q u_0, its norm and the next u,
-// which every wave forms for itself.  Everything else fills the waits: B1 <-
-// H B1 and its part of a message need no window and come before it, the slot is
-// emptied in the shadow of the reflector, and the rest of the message goes out
-// with S(:, 0) and beta first, which complete what the next sweep waits for.
-// b = 32, n = 6000: 21.1 -> 16.3 ms, n = 1000: 3.33 -> 2.46 ms; b = 64, n = 8192:
-// 86.5 -> 67.7 ms.  B1 is the previous N, passed
-// through LDS transposed, so that its column sums u^T B1 are row sums of a
-// wave's own lanes as well.
-//
-// Hand-off.  Step (s + 1, j) works on the window of step (s, j) shifted by one
-// row and column: S'(i, k) = S(i+1, k+1) of step (s, j), its last row and
-// column from B1 and S(0, 0) of step (s, j+1); N'(i, k) = B1(i+1, k+1) of step
-// (s, j+1), its last column from S(:, 0) and the next beta of that step, its
-// last row zero otherwise.  Sweep s sends these elements as message j, in the
-// order in which the receiver's threads load them (plane r of a block is
-// element (i, 8 r + kc) at 8 i + kc), so every access of either side covers
-// whole runs of lines; X is the same for column s + 1 below the diagonal, from
-// which sweep s + 1 starts.  An empty slot holds kEmpty, a signalling NaN that
-// no arithmetic returns: the receiver loads its window until no element is
-// empty, so data and its arrival are one access and nobody waits for a store
-// to complete, then a flag, then a load (n = 16384, b = 32: store 0.33-0.48 us,
-// flag 0.5-0.66 us, loads behind it).  Having read a slot, the receiver empties it again.
-// Slots are doubled by the sweep's parity, and reuse is safe by the order of
-// the chain alone: a step's sends but those of B1 follow a barrier before which
-// every wave has waited for loads issued after the previous step's empties
-// (memory operations complete in order), so message j of sweep s, which S(:, 0)
-// and beta complete at step (s, j + 1), proves that s has emptied slot j of the
-// other parity; B1 goes to slot j - 1, which the step before proved empty.  In
-// the last step, whose message nothing follows, a wave completes its empties
-// before it sends (every wave that empties elements there sends some).  Only a
-// sweep's first slots have no such message before them: the receiver waits for
-// the predecessor's start word, set once it holds its own first window.
-// What a sweep sends is exactly what the next one loads (both bounded by row
-// < n), so no stale element stays behind.
-//
-// Measured against one workgroup per sweep on a band in HBM with progress
-// words (window loads, stores and a flag in every step's chain): b = 32,
-// n = 6000: 49.2 -> 25.6 ms, n = 16384: 137 -> 85 ms; b = 64, n = 8192:
-// 156 -> 92 ms (with every message between XCDs, see below).
-//
-// Where the messages go decides the hand-off: from one XCD to another a store
-// reaches a poll after 820 ns, through the XCD's own L2 after 340 ns (a message
-// of 64 doubles sent to and fro).  So consecutive sweeps run on one XCD, each
-// of which has a box of slots of its own: a slot of a box is only ever
-// accessed through one L2.  All messages between
-// XCDs -> this: b = 32: n = 1000 3.88 -> 3.33 ms, n = 6000 25.6 -> 21.1 ms,
-// n = 16384 85.7 -> 59.6 ms; b = 64, n = 8192: 93.5 -> 86.5 ms.
-//
-// A batch of `count` same-size problems shares one launch, its units mixed.
+// LAPACK-style reflector of the chase (reference sign convention): from the
+// column x = Bc[0..lenx) (LDS, stride LD), u = (x/||x|| + sign(x0) e1) /
+// sqrt(|x0/||x|| + sign(x0)|), ||u||^2 = 2, H x = beta e1.  Wave 0 only.
 template <int BW>
-struct ChaseShape {
-  static constexpr int EPT = BW / 8;    // window columns per thread
-  static constexpr int NT = BW * 8;     // threads
-  static constexpr int NW = NT / 64;    // waves
-  // stride of the transposed N in LDS: 8 mod 32 doubles, so that a wave's
-  // 8 x 8 elements fall on distinct banks in the write and in the read
-  static constexpr int LD = BW + 8;
-};
-
-constexpr unsigned kEmptyHi = 0x7FF7A5C3u;  // high word of an empty slot element
-constexpr int kXWords = 64;                 // doubles of an X slot
-
-// message slots of one problem: [parity][slot][S planes, N planes], each
-// parity followed by its X slot
-__host__ __device__ inline long mail_plane(long b) { return 8 * b; }
-__host__ __device__ inline long mail_slot(long b) { return 2 * ((b + 7) / 8) * mail_plane(b); }
-__host__ __device__ inline long mail_slots(long n, long b) { return (n + b - 1) / b; }
-__host__ __device__ inline long mail_half(long n, long b) { return mail_slots(n, b) * mail_slot(b) + kXWords; }
-
-// Messages of parity 1 for sweep 0, from the band, into the box between XCDs
-// (grid z = 0); everything else, the other boxes included, empty.
-__global__ __launch_bounds__(256) void mail_fill_kernel(int n, int b, const double *__restrict__ band_all, long ldb,
-                                                        long band_stride, double *__restrict__ mail_all,
-                                                        double *__restrict__ boxes, double *__restrict__ D_all,
-                                                        long d_stride) {
-  const long q = blockIdx.y;
-  const double *band = band_all + q * band_stride;
-  const long half = mail_half(n, b), slot = mail_slot(b), plane = mail_plane(b), nslots = mail_slots(n, b);
-  const double empty = __builtin_bit_cast(double, (unsigned long long)kEmptyHi << 32);
-  if (blockIdx.z > 0) {
-    double *box = boxes + ((blockIdx.z - 1L) * gridDim.y + q) * 2 * half;
-    for (long e = blockIdx.x * 256L + threadIdx.x; e < 2 * half; e += gridDim.x * 256L) box[e] = empty;
-    return;
+__device__ inline void chase_reflector(const double *Bc, int lenx, int lane, double *u, double *s_beta, float *U,
+                                       long urow, long ucol) {
+  constexpr int LD = BW + 1;
+  const double x = (lane < lenx) ? Bc[lane * LD] : 0.0;
+  const double nrm = sqrt(wave_sum(x * x));
+  const double x0 = Bc[0];
+  double uu = 0.0;
+  if (nrm > 0.0) {
+    const double inv = 1.0 / nrm;
+    const double u0 = x0 * inv + (x0 >= 0.0 ? 1.0 : -1.0);
+    const double scl = 1.0 / sqrt(fabs(u0));
+    uu = (lane == 0 ? u0 : x * inv) * scl;
   }
-  double *mail = mail_all + q * 2 * half;
-  if (blockIdx.x == 0 && threadIdx.x == 0) D_all[q * d_stride] = band[0];
-  for (long e = blockIdx.x * 256L + threadIdx.x; e < 2 * half; e += gridDim.x * 256L) {
-    double v = empty;
-    if (e >= half) {
-      const long f = e - half;
-      long row = -1, col = 0;  // element of the band, row < 0: none
-      if (f >= nslots * slot) {
-        const long i = f - nslots * slot;
-        if (i < b) row = 1 + i;
-      } else {
-        const long j = f / slot, w = f % slot;
-        const bool isn = w >= slot / 2;
-        const long v2 = isn ? w - slot / 2 : w;
-        const long i = (v2 % plane) / 8, k = (v2 / plane) * 8 + (v2 & 7);
-        const long p = 1 + j * b, len = min((long)b, n - p), len2 = max(0L, min((long)b, n - p - len));
-        if (k < len && i < (isn ? len2 : len) && !(isn && i == b - 1 && k < b - 1)) {
-          row = isn ? p + len + i : p + max(i, k);
-          col = isn ? p + k : p + min(i, k);
-        }
-      }
-      if (row >= 0 && row < n) {
-        v = band[(row - col) + col * ldb];
-        // a caller's NaN must not read as an empty slot
-        if (!(v == v)) v = __builtin_nan("");
-      }
-    }
-    mail[e] = v;
-  }
+  if (lane < BW) u[lane] = (lane < lenx) ? uu : 0.0;
+  if (lane < lenx) U[(urow + lane) + ucol] = (float)uu;
+  if (lane == 0) *s_beta = (nrm > 0.0) ? (x0 >= 0.0 ? -nrm : nrm) : x0;
 }
 
-// Handing out sweeps.  A unit is a run of `len` consecutive sweeps of one
-// problem; units are numbered run by run over the problems (run u / count of
-// problem u % count) and an XCD takes the next one when all sweeps of its last
-// are handed out.  So the first sweep that is not finished is running or next
-// in its XCD's unit, whose workgroups have only finished ones behind them:
-// the chain always moves.  Units go to the first `members` XCDs that ask; the
-// workgroups of the others leave.
-// Words at `ticket`: the next unit, the members so far, and at
-// kXcdWords (x + 1) the 64-bit state of XCD x: member number << 61 | unit + 1
-// << 30 | sweeps handed out (0: no unit yet).
-constexpr int kXcds = 8, kXcdWords = 32;
-constexpr long kTicketWords = (long)kXcdWords * (kXcds + 1);
-constexpr unsigned kNoUnit = 0x7fffffffu;
-
-struct ChaseUnits {
-  int len, total, members;
-};
-
-// sweep (s of problem q) for this workgroup, whose XCD is member m; false: no
-// more.  One thread calls.
-__device__ inline bool next_sweep(unsigned *ticket, int x, const ChaseUnits &units, int count, int nsweeps,
-                                  unsigned *err, int &s, int &q, int &m) {
-  unsigned long long *state = reinterpret_cast<unsigned long long *>(ticket + kXcdWords * (x + 1));
-  auto field = [](unsigned long long v) -> unsigned { return (unsigned)(v >> 30) & kNoUnit; };
-  while (true) {
-    const unsigned long long v = __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    const unsigned unit = field(v), idx = (unsigned)v & 0x3fffffffu;
-    m = (int)(v >> 61);
-    if (unit == kNoUnit) return false;
-    if (unit != 0 && idx < (unsigned)units.len) {
-      s = (int)((unit - 1) / count) * units.len + (int)idx;
-      q = (int)((unit - 1) % count);
-      if (s < nsweeps) return true;
-      continue;
-    }
-    if (idx == (unit == 0 ? 0u : (unsigned)units.len)) {  // fetch the XCD's next unit, and take its first sweep
-      if (unit == 0) m = (int)__hip_atomic_fetch_add(ticket + 1, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      unsigned u = kNoUnit - 1;
-      if (m < units.members) {
-        const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (t < (unsigned)units.total) u = t;
-      }
-      const bool none = u == kNoUnit - 1;
-      __hip_atomic_store(state, (none ? 0ull : (unsigned long long)m << 61) | (unsigned long long)(u + 1) << 30 | 1ull,
-                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (none) return false;
-      s = (int)(u / count) * units.len;
-      q = (int)(u % count);
-      return true;
-    }
-    // another workgroup fetches it
-    const unsigned long long t0 = clock100();
-    while (field(__hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) == unit) {
-      __builtin_amdgcn_s_sleep(2);
-      if (clock100() - t0 > kWatchdogTicks) {
-        atomicOr(err, (unsigned)EVD_E_TIMEOUT);
-        return false;
-      }
-    }
-  }
-}
-
-// LOCAL: messages between sweeps of one unit go through box m of the XCD's
-// member number (boxes; one per member and problem) and stay in its L2; the
-// first sweep of a unit receives, and the last one sends, through mail_all.
-// Otherwise every message goes through mail_all.
-template <int BW, bool LOCAL>
-__global__ __launch_bounds__(ChaseShape<BW>::NT) void chase_kernel(
-    int n, int b, double *__restrict__ mail_all, double *__restrict__ boxes, ChaseUnits units,
-    float *__restrict__ U_all, long ldu, long u_stride, int *__restrict__ com_all, unsigned *__restrict__ ticket,
-    unsigned *__restrict__ err, int count, double *__restrict__ D_all, long d_stride, double *__restrict__ E_all,
-    long e_stride) {
-  using Sh = ChaseShape<BW>;
-  constexpr int EPT = Sh::EPT, NT = Sh::NT, NW = Sh::NW, LD = Sh::LD;
-  __shared__ double sB[BW * LD];      // N^T of the last step: the next B1
-  __shared__ double sU[NW][BW];       // each wave's copy of u
-  __shared__ double sY[BW], sQ[BW], sN0[BW], sX[BW];
-  __shared__ int s_sweep, s_problem, s_member, s_abort;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int ri = tid >> 3, kc = tid & 7, xi = lane & (BW - 1);
+// A batch of `count` same-size problems shares one launch: ticket t is sweep
+// t / count of problem t % count, so each problem's sweeps are still handed
+// out in increasing order.  Problem q's band, reflectors and progress words
+// start at band + q * band_stride, U + q * u_stride, com + q * com_stride.
+template <int BW>
+__global__ __launch_bounds__(256, BW == 32 ? 4 : 1) void chase_kernel(int n, int b, double *__restrict__ band_all,
+                                                    long ldb, unsigned band_bytes, float *__restrict__ U_all,
+                                                    long ldu, int *__restrict__ com_all,
+                                                    unsigned *__restrict__ ticket, unsigned *__restrict__ err,
+                                                    int count, long band_stride, long u_stride, long com_stride) {
+  constexpr int LD = BW + 1;
+  constexpr int LPR = 256 / BW;  // lanes per window row
+  constexpr int EPT = BW / LPR;  // window columns per lane
+  constexpr int HALVES = 64 / BW;
+  __shared__ double sB[2][BW * LD];
+  __shared__ double u[BW], yv[BW], qv[BW];
+  __shared__ double s_beta;
+  __shared__ int s_ticket, s_ok;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int ri = tid / LPR, kc = tid % LPR;
   const int nsweeps = n - 2;
-  const long half = mail_half(n, b), slot = mail_slot(b);
-  const int slot_bytes = (int)(slot * 8);
-  const unsigned pb = (unsigned)(mail_plane(b) * 8), nb0 = (unsigned)slot_bytes / 2;  // bytes of a plane, start of N
-  typedef __attribute__((__vector_size__(2 * sizeof(unsigned)))) unsigned u2;
+  const unsigned ld = (unsigned)ldb;  // band offsets fit 32 bits (checked by the launcher)
 
-  // byte offset of S'(i, k) in a slot (N' at + nb0)
-  auto at = [&](int i, int k) -> unsigned { return (unsigned)(k >> 3) * pb + (unsigned)(i * 8 + (k & 7)) * 8u; };
-
-  const int xcd = LOCAL ? (int)__builtin_amdgcn_s_getreg((3 << 11) | 20) & (kXcds - 1) : 0;  // HW_REG_XCC_ID
-
-  // one sweep, messages in and out with these store policies (0: within the
-  // XCD, kSc1: device-coherent); true: aborted
-  auto sweep = [&](auto in_policy, auto out_policy, const int s, const int q, double *mail_in, double *mail_out)
-                   __attribute__((always_inline)) -> bool {
-    constexpr int IN = decltype(in_policy)::value, OUT = decltype(out_policy)::value;
-    // slot 0 of this sweep's messages in, out
-    double *rd = mail_in + ((s + 1) & 1) * half, *wr = mail_out + (s & 1) * half;
-    const __amdgpu_buffer_rsrc_t rxi =
-        __builtin_amdgcn_make_buffer_rsrc(rd + half - kXWords, 0, kXWords * 8, kBufferWord3);
-    const __amdgpu_buffer_rsrc_t ru = __builtin_amdgcn_make_buffer_rsrc(
-        U_all + (long)q * u_stride + (long)s * ldu, 0, (int)((n + b) * 4), kBufferWord3);
-    int *com = com_all + (long)q * n * kComStride;
-    double *Dq = D_all + q * d_stride, *Eq = E_all + q * e_stride;
-
-    int p = s + 1, len = min(b, n - p), len2 = max(0, min(b, n - p - len));
-
-    // watchdog of a wait; true = give up
-    auto expired = [&](unsigned long long t0) -> bool {
-      if (clock100() - t0 <= kWatchdogTicks) return false;
-      if (lane == 0) {
-        atomicOr(err, (unsigned)EVD_E_TIMEOUT);
-        s_abort = 1;
-      }
-      return true;
-    };
-    // offsets of a window's elements (kOutOfRange: not part of it)
-    unsigned oS[EPT], oN[EPT];
-    auto window_offsets = [&](int wlen, int wlen2) {
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        const int kk = kc + 8 * r;
-        oS[r] = (ri < wlen && kk < wlen) ? at(ri, kk) : kOutOfRange;
-        oN[r] = (ri < wlen2 && kk < wlen && !(ri == b - 1 && kk < b - 1)) ? nb0 + at(ri, kk) : kOutOfRange;
-      }
-    };
-    // offsets of a step's sends: S to slot j, B1 (thread = column ri, rows
-    // kk) to slot j - 1, row 0 of B1 mirrored, and thread kc = 0's S(ri, 0)
-    // (X in the first step)
-    unsigned oA[EPT], oB[EPT], oM, oC, oX;
-    auto send_offsets = [&](int wlen) {
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        const int kk = kc + 8 * r;
-        oA[r] = (ri >= 1 && kk >= 1 && ri < wlen && kk < wlen) ? at(ri - 1, kk - 1) : kOutOfRange;
-        oB[r] = (ri >= 1 && ri < b && kk < wlen) ? (kk == 0 ? at(b - 1, ri - 1) : nb0 + at(kk - 1, ri - 1)) : kOutOfRange;
-      }
-      oM = (kc == 0 && ri >= 1 && ri < b) ? at(ri - 1, b - 1) : kOutOfRange;
-      oC = (kc == 0 && ri < wlen) ? (ri == 0 ? at(b - 1, b - 1) : nb0 + at(ri - 1, b - 1)) : kOutOfRange;
-      oX = (kc == 0 && ri >= 1 && ri < wlen) ? (unsigned)(ri - 1) * 8u : kOutOfRange;
-    };
-    window_offsets(len, len2);
-    send_offsets(len);
-
-    // the predecessor's first slots are this sweep's to poll once it has started
-    if (s > 0) {
-      const unsigned long long t0 = clock100();
-      while (ld_dev(&com[(long)(s - 1) * kComStride]) == 0) {
-        if (expired(t0)) break;
-        __builtin_amdgcn_s_sleep(1);
-      }
-    }
-    // column s below the diagonal: wave 0 receives it for all
-    if (wave == 0) {
-      const unsigned ox = lane < min(b, n - p) ? (unsigned)lane * 8u : kOutOfRange;
-      const unsigned long long t0 = clock100();
-      double x;
-      while (true) {
-        x = ld_band_at(rxi, ox);
-        const bool ready = (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32) != kEmptyHi;
-        if (__all(ready) || expired(t0)) break;
-      }
-      __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rxi, ox, 0, IN);
-      if (lane < BW) sX[lane] = x;
-    }
-    grp_barrier();
-    double u0, beta;
-    {
-      const double uu = chase_reflector<BW>(sX[xi], lane, u0, beta);
-      if (lane < BW) sU[wave][lane] = uu;
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)uu), ru,
-                                            (wave == 0 && lane < len) ? (unsigned)(p + lane) * 4u : kOutOfRange, 0, 0);
-      if (tid == 0) Eq[s] = beta;
-    }
-
-    auto load_window = [&](const double *base, double(&S)[EPT], double(&N)[EPT]) {
-      const __amdgpu_buffer_rsrc_t rs =
-          __builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(base), 0, slot_bytes, kBufferWord3);
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        S[r] = ld_band_at(rs, oS[r]);
-        N[r] = ld_band_at(rs, oN[r]);
-      }
-    };
-    auto arrived = [&](const double(&S)[EPT], const double(&N)[EPT]) -> bool {
-      unsigned m = ~0u;
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        m = min(m, (unsigned)(__builtin_bit_cast(unsigned long long, S[r]) >> 32) ^ kEmptyHi);
-        m = min(m, (unsigned)(__builtin_bit_cast(unsigned long long, N[r]) >> 32) ^ kEmptyHi);
-      }
-      return __all(m != 0u);
-    };
-
-    // one step on the window in (S, N); the next one's is loaded into
-    // (Sn, Nn).  0: go on, 1: last step, 2: aborted
-    auto step = [&](auto is_first, double(&S)[EPT], double(&N)[EPT], double(&Sn)[EPT], double(&Nn)[EPT])
-                    __attribute__((always_inline)) -> int {
-      constexpr bool first = decltype(is_first)::value;
-      const bool last = (len2 == 0);
-      // ---- B1 <- H B1 (B1 transposed), for which u is all it takes: done and
-      // sent while the window is on its way
-      double uk[EPT];
-      const double ui = sU[wave][ri];
-#pragma unroll
-      for (int r = 0; r < EPT; r++) uk[r] = sU[wave][kc + 8 * r];
-      if constexpr (!first) {
-        double bt[EPT], t = 0.0;
-#pragma unroll
-        for (int r = 0; r < EPT; r++) bt[r] = sB[ri * LD + kc + 8 * r];
-#pragma unroll
-        for (int r = 0; r < EPT; r++) t += bt[r] * uk[r];
-        t = group_sum<8>(t);
-        const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(wr - slot, 0, slot_bytes, kBufferWord3);
-#pragma unroll
-        for (int r = 0; r < EPT; r++) {
-          bt[r] -= uk[r] * t;
-          st_band_at<OUT>(rv, oB[r], bt[r]);
-        }
-        st_band_at<OUT>(rv, oM, bt[0]);
-      }
-      if (!arrived(S, N)) {
+  // tid 0 polls the predecessor's progress word; false = watchdog expired
+  auto wait_prev = [&](const int *com, int s, int need) -> bool {
+    if (tid == 0) {
+      s_ok = 1;
+      if (s > 0) {
         const unsigned long long t0 = clock100();
-        do {
-          load_window(rd, S, N);
-        } while (!arrived(S, N) && !expired(t0));
-      }
-      // ---- row sums q = N u, y = S u
-      double y = 0.0, qq = 0.0;
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        qq += N[r] * uk[r];
-        y += S[r] * uk[r];
-      }
-      qq = group_sum<8>(qq);
-      y = group_sum<8>(y);
-      if (kc == 0) {
-        sQ[ri] = qq;
-        sN0[ri] = N[0];
-        sY[ri] = y;
-      }
-      grp_barrier();
-      // ---- the next column and its reflector (every wave for itself), the
-      // slot emptied in its shadow
-      const double x = sN0[xi] - sQ[xi] * u0;
-      double yk[EPT];
-#pragma unroll
-      for (int r = 0; r < EPT; r++) yk[r] = sY[kc + 8 * r];
-      const int aborted = s_abort;
-      {
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(rd, 0, slot_bytes, kBufferWord3);
-#pragma unroll
-        for (int r = 0; r < EPT; r++) {
-          __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rs, oS[r], 0, IN);
-          __builtin_amdgcn_raw_buffer_store_b64(u2{0u, kEmptyHi}, rs, oN[r], 0, IN);
+        while (ld_dev(&com[(long)(s - 1) * kComStride]) < need) {
+          __builtin_amdgcn_s_sleep(1);
+          if (clock100() - t0 > kWatchdogTicks) {
+            atomicOr(err, (unsigned)EVD_E_TIMEOUT);
+            s_ok = 0;
+            break;
+          }
         }
       }
-      double un0 = 0.0, betan = 0.0, uu = 0.0;
-      uu = chase_reflector<BW>(x, lane, un0, betan);
-      if (len2 <= 1) {  // a single row is left as it is
-        uu = un0 = 0.0;
-        betan = __shfl(x, 0, 64);
-      }
-      if (lane < BW) sU[wave][lane] = uu;
-      // ---- S <- H S H (rank-2 with w = y - (u^T y / 2) u), N <- N H
-      double psi = 0.0;
-#pragma unroll
-      for (int r = 0; r < EPT; r++) psi += uk[r] * yk[r];
-      psi = 0.5 * group_sum<8>(psi);
-      const double wi = y - psi * ui;
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        const double wk = yk[r] - psi * uk[r];
-        S[r] -= sym_pair(ui, wk, wi, uk[r]);
-      }
-      // S(:, 0) and the next beta complete message j - 1 (X in the first step)
-      {
-        const unsigned ob = first ? (unsigned)(b - 1) * 8u : nb0 + at(b - 1, b - 1);
-        const unsigned oc = tid == 1 ? (len2 > 0 ? ob : kOutOfRange) : (first ? oX : oC);
-        const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
-            first ? mail_out + (s & 1) * half + (half - kXWords) : wr - slot, 0, first ? kXWords * 8 : slot_bytes,
-            kBufferWord3);
-        st_band_at<OUT>(rc, oc, tid == 1 ? betan : S[0]);
-      }
-#pragma unroll
-      for (int r = 0; r < EPT; r++) {
-        N[r] -= qq * uk[r];
-        sB[(kc + 8 * r) * LD + ri] = N[r];
-      }
-      // the last message has no step behind it to show that the slot is empty
-      if (last) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      {
-        const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(wr, 0, slot_bytes, kBufferWord3);
-#pragma unroll
-        for (int r = 0; r < EPT; r++) st_band_at<OUT>(rw, oA[r], S[r]);
-      }
-      const int pn = p + len, len3 = max(0, min(b, n - pn - len2));
-      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, (float)uu), ru,
-                                            (wave == 0 && lane < len2) ? (unsigned)(pn + lane) * 4u : kOutOfRange, 0, 0);
-      if constexpr (first) {
-        if (tid == 0) {
-          Dq[s + 1] = S[0];
-          st_dev(&com[(long)s * kComStride], 1);
-        }
-        if (s == nsweeps - 1) {  // the last 2 x 2 block is final
-          if (tid == 8) Eq[n - 2] = S[0];
-          if (tid == 9) Dq[n - 1] = S[0];
-        }
-      }
-      // look for the next window (loads behind this step's empties: see above)
-      asm volatile("" ::: "memory");
-      rd += slot;
-      if (len3 != b) window_offsets(len2, len3);
-      load_window(rd, Sn, Nn);
-      grp_barrier();
-      if (aborted) return 2;
-      if (last) return 1;
-      wr += slot;
-      u0 = un0;
-      beta = betan;
-      p = pn;
-      len = len2;
-      len2 = len3;
-      if (len != b) send_offsets(len);
-      return 0;
-    };
-
-    double Sa[EPT], Na[EPT], Sb[EPT], Nb[EPT];
-    load_window(rd, Sa, Na);
-    int end = step(std::true_type{}, Sa, Na, Sb, Nb);
-    while (!end) {
-      end = step(std::false_type{}, Sb, Nb, Sa, Na);
-      if (end) break;
-      end = step(std::false_type{}, Sa, Na, Sb, Nb);
     }
-    return end == 2;
+    __syncthreads();
+    return s_ok != 0;
   };
 
-  const std::integral_constant<int, 0> local{};
-  const std::integral_constant<int, kSc1> coherent{};
   while (true) {
-    if (tid == 0) {
-      int s, q, m;
-      if (LOCAL) {
-        s_sweep = next_sweep(ticket, xcd, units, count, nsweeps, err, s, q, m) ? s : -1;
-      } else {  // sweep by sweep over the problems
-        const unsigned t = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        s = (int)(t / count);
-        q = (int)(t % count);
-        m = 0;
-        s_sweep = s < nsweeps ? s : -1;
-      }
-      s_problem = q;
-      s_member = m;
-      s_abort = 0;
+    if (tid == 0)
+      s_ticket = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int tk = s_ticket;
+    __syncthreads();
+    if (tk >= nsweeps * count) return;
+    const int q = tk % count, s = tk / count;
+    const __amdgpu_buffer_rsrc_t rb =
+        __builtin_amdgcn_make_buffer_rsrc(band_all + (long)q * band_stride, 0, (int)band_bytes, kBufferWord3);
+    float *U = U_all + (long)q * u_stride;
+    int *com = com_all + (long)q * com_stride;
+    int p = s + 1;
+    int len = min(b, n - p);
+    int colB1 = 1, cB1 = s;
+    bool first = true;
+    double *B1 = sB[0], *Bn = sB[1];
+    bool ok = wait_prev(com, s, p + 2 * b - 1);
+    if (ok) {
+      // column s below the diagonal is final: it becomes B1[:, 0]
+      for (int i = tid; i < BW; i += 256) B1[i * LD] = (i < len) ? ld_band(rb, (unsigned)(1 + i) + (unsigned)s * ld) : 0.0;
+      __syncthreads();
+      if (wave == 0) chase_reflector<BW>(B1, len, lane, u, &s_beta, U, p, (long)s * ldu);
+      __syncthreads();
     }
-    grp_barrier();
-    const int s = __builtin_amdgcn_readfirstlane(s_sweep), q = __builtin_amdgcn_readfirstlane(s_problem);
-    const int m = __builtin_amdgcn_readfirstlane(s_member);
-    grp_barrier();
-    if (s < 0) return;
-    double *mail = mail_all + (long)q * 2 * half, *box = boxes + ((long)m * count + q) * 2 * half;
-    bool aborted;
-    if (!LOCAL)
-      aborted = sweep(coherent, coherent, s, q, mail, mail);
-    else if (s % units.len == 0)
-      aborted = sweep(coherent, local, s, q, mail, box);
-    else if ((s + 1) % units.len == 0)
-      aborted = sweep(local, coherent, s, q, box, mail);
-    else
-      aborted = sweep(local, local, s, q, box, box);
-    if (aborted) return;
+    while (ok) {
+      const int len2 = max(0, min(b, n - p - len));
+      const bool last = (len2 <= 1);
+      // ---- S (symmetric, from the lower band) and N windows into registers
+      double Sr[EPT], Nr[EPT];
+#pragma unroll
+      for (int r = 0; r < EPT; r++) {
+        const int kk = kc + LPR * r;
+        const int lo = min(ri, kk), dd = ri > kk ? ri - kk : kk - ri;
+        Sr[r] = (ri < len && kk < len) ? ld_band(rb, (unsigned)dd + (unsigned)(p + lo) * ld) : 0.0;
+        Nr[r] = (ri < len2 && kk < len) ? ld_band(rb, (unsigned)(len + ri - kk) + (unsigned)(p + kk) * ld) : 0.0;
+      }
+      // ---- B1 <- H B1 and write-back (wave 3, while the loads are in flight):
+      // t_c = u^T B1[:, c] by lane c (rows split over HALVES lane sets), then
+      // the write-back with lanes along rows, so each store instruction
+      // covers whole runs of one or two band columns instead of one element
+      // of 32 or 64 columns
+      if (wave == 3) {
+        const int c = lane % BW, h = lane / BW;
+        double t = 0.0;
+#pragma unroll
+        for (int i = 0; i < BW; i += HALVES) t += u[i + h] * B1[(i + h) * LD + c];
+        if (HALVES == 2) t += __shfl_xor(t, 32, 64);
+        const double beta = s_beta;
+        const int ii = lane % BW;
+        const double uii = u[ii];
+#pragma unroll
+        for (int c0 = 0; c0 < BW; c0 += HALVES) {
+          const int cc = c0 + h;
+          const double tc = __shfl(t, cc, 64);
+          if (cc < colB1 && ii < len && !(cc == 0 && ii == 0 && !first)) {
+            const int col = cB1 + cc;
+            const double v = (cc == 0) ? (ii == 0 ? beta : 0.0) : B1[ii * LD + cc] - uii * tc;
+            st_band(rb, (unsigned)(p + ii - col) + (unsigned)col * ld, v);
+          }
+        }
+      }
+      // ---- y = S u and q = N u (row sums over the LPR lanes of a row)
+      double yp = 0.0, qp = 0.0;
+#pragma unroll
+      for (int r = 0; r < EPT; r++) {
+        const double uk = u[kc + LPR * r];
+        yp += Sr[r] * uk;
+        qp += Nr[r] * uk;
+      }
+#pragma unroll
+      for (int o = LPR / 2; o > 0; o >>= 1) {
+        yp += __shfl_xor(yp, o, 64);
+        qp += __shfl_xor(qp, o, 64);
+      }
+      if (kc == 0) {
+        yv[ri] = yp;
+        qv[ri] = qp;
+      }
+      __syncthreads();
+      // ---- S <- H S H (rank-2 with w = y - (u^T y / 2) u), N <- N H
+      const double psi = wave_sum((lane < BW) ? u[lane] * yv[lane] : 0.0);
+      const double ui = u[ri], wi = yv[ri] - 0.5 * psi * ui, qi = qv[ri];
+#pragma unroll
+      for (int r = 0; r < EPT; r++) {
+        const int kk = kc + LPR * r;
+        const double uk = u[kk], wk = yv[kk] - 0.5 * psi * uk;
+        Sr[r] -= ui * wk + wi * uk;
+        Nr[r] -= qi * uk;
+        if (ri >= kk && ri < len && kk < len) st_band(rb, (unsigned)(ri - kk) + (unsigned)(p + kk) * ld, Sr[r]);
+        Bn[ri * LD + kk] = Nr[r];
+        if (last && ri < len2 && kk < len) st_band(rb, (unsigned)(len + ri - kk) + (unsigned)(p + kk) * ld, Nr[r]);
+      }
+      __syncthreads();
+      // ---- next reflector from N[:, 0]; its beta (row p+len, column p) is
+      // published now, before the progress word, for the successor sweep
+      if (!last && wave == 0) {
+        chase_reflector<BW>(Bn, len2, lane, u, &s_beta, U, p + len, (long)s * ldu);
+        if (lane == 0) st_band(rb, (unsigned)len + (unsigned)p * ld, s_beta);
+      }
+      wait_mem();
+      __syncthreads();
+      if (tid == 0) st_dev(&com[(long)s * kComStride], last ? INT_MAX : p + len);
+      if (last) break;
+      double *t = B1;
+      B1 = Bn;
+      Bn = t;
+      colB1 = len;
+      cB1 = p;
+      p += len;
+      len = len2;
+      first = false;
+      ok = wait_prev(com, s, p + 2 * b - 1);
+    }
+    if (!ok) {
+      if (tid == 0) st_dev(&com[(long)s * kComStride], INT_MAX);
+      return;
+    }
   }
 }
 
@@ -680,6 +276,19 @@ constexpr int kGLD = 64;
 // most columns the front brings in at one step: b + 2 at b = 32 (the first
 // chunk s0 .. n of a sweep whose first step is also its last)
 constexpr int kGChunk = 34;
+constexpr unsigned kOutOfRange = 0x80000000u;  // byte offset past every band (< 2 GiB)
+
+__device__ __attribute__((always_inline)) inline void grp_barrier() {
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+__device__ __attribute__((always_inline)) inline void wave_lds_order() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
+// s_waitcnt with only the vector-memory count: vmcnt(N), N <= 63
+template <int N>
+__device__ __attribute__((always_inline)) inline void wait_vm() {
+  static_assert(N >= 0 && N <= 63, "vmcnt is 6 bits");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
 
 __device__ inline int sweep_nsteps(int n, int b, int s) {
   int p = s + 1, len = min(b, n - p), k = 1;
@@ -690,6 +299,15 @@ __device__ inline int sweep_nsteps(int n, int b, int s) {
     len = len2;
     k++;
   }
+}
+
+// 64-bit DPP move of v (rows outside RM read 0)
+template <int CTRL, int RM>
+__device__ __attribute__((always_inline)) inline double dpp_f64(double v) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)x, CTRL, RM, 0xf, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), CTRL, RM, 0xf, false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
 // sum over the 64 lanes, returned in every lane: quad, half-row and row
@@ -706,6 +324,19 @@ __device__ __attribute__((always_inline)) inline double wave_total(double v) {
   const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, 63);
   const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), 63);
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// v of lane ^ 32.  v_permlane32_swap exchanges one half of its destination
+// with the other half of its source; with both operands v, one result holds
+// this lane's own value and the other the partner's, so xor-ing out the own
+// value leaves the partner's whichever half was exchanged.
+__device__ __attribute__((always_inline)) inline double half_swap(double v) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)x, hi = (unsigned)(x >> 32);
+  const auto rl = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto rh = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  const unsigned plo = rl[0] ^ rl[1] ^ lo, phi = rh[0] ^ rh[1] ^ hi;
+  return __builtin_bit_cast(double, ((unsigned long long)phi << 32) | plo);
 }
 
 // reflector of the chase's convention from x (lane < lenx, zero elsewhere),
@@ -1066,62 +697,31 @@ static int launch_chase_group(evd_ctx *ctx, int count, long n, long b, double *b
   return 0;
 }
 
-// Sweeps in flight of one problem (a sweep trails its predecessor by two to
-// three steps of b rows) and the XCDs that run the chase: 32 sweeps an XCD, one
-// per CU, keep a chain of up to 32 on one XCD; at b = 64, 16, whose slots (64
-// KiB, two steps apart, both parities) fit the 4 MiB of its L2.  Where the eight
-// XCDs do not hold all that are in flight, the slots would not stay in the L2s: a
-// large batch runs as several launches, and single chases beyond that (n >
-// 20000 at b = 32) do without boxes.
-static long chase_inflight(long n, long b) { return (2 * n + 5 * b - 1) / (5 * b) + 4; }
-static int chase_members(int count, long n, long b) {
-  const long per = b <= 32 ? 32 : 16;
-  return (int)((chase_inflight(n, b) * count + per - 1) / per);
-}
-// problems of a batch per launch: as many as the XCDs hold in flight
-static int chase_batch(int count, long n, long b) {
-  return (int)std::max<long>(1, std::min<long>(count, kXcds * (b <= 32 ? 32 : 16) / chase_inflight(n, b)));
-}
-
 template <int BW>
-static int launch_chase(evd_ctx *ctx, int count, long n, long b, const double *band, long ldb, long band_stride,
-                        double *mail, double *boxes, float *U, long ldu, long u_stride, int *com, unsigned *ticket,
-                        double *D, long d_stride, double *E, long e_stride) {
-  // workgroups: as many as sweeps are in flight (a workgroup takes its next
-  // sweep as soon as it finishes one), at most one per CU.  Those beyond that
-  // only poll and crowd out concurrent solves.  With boxes that many on each
-  // member XCD: workgroups are dealt to the XCDs in turn, so eight times as many
-  // are launched, of which those on other XCDs leave at once.
+static int launch_chase(evd_ctx *ctx, int count, long n, long b, double *band, long ldb, long band_stride, float *U,
+                        long ldu, long u_stride, int *com, long com_stride, unsigned *ticket) {
+  const long bytes = ldb * n * (long)sizeof(double);
+  if (bytes >= (1L << 31))
+    return set_error(ctx, EVD_E_UNSUPPORTED, "band of %ld bytes exceeds the 2 GiB buffer range of the chase", bytes);
+  // workgroups: sweep s+1 trails sweep s by two b-row steps, so at most
+  // about n / (2b) sweeps of a problem are in flight; by default that many
+  // plus a few per problem (a workgroup takes its next sweep by ticket as
+  // soon as it finishes one), at most the resident count.  Workgroups beyond
+  // that only spin on progress words, slow the chase through the polling
+  // traffic (n = 16384: 148 ms with 260 workgroups, 163 ms with 1.25x,
+  // 191 ms with all resident ones) and crowd out concurrent solves.
   int resident = 0;
-  const void *kernel = boxes ? (const void *)chase_kernel<BW, true> : (const void *)chase_kernel<BW, false>;
-  EVD_TRY(max_coresident_blocks(ctx, kernel, ChaseShape<BW>::NT, 0, &resident));
-  const long nsweeps = n - 2, inflight = chase_inflight(n, b);
-  const int members = boxes ? chase_members(count, n, b) : 1;
-  // units: everything on one XCD where that holds a problem's sweeps in
-  // flight; else as many sweeps as an XCD holds; batches mix the problems
-  long per = std::min<long>(inflight * count, ctx->num_cus), len = 1;
-  if (boxes) {
-    per = std::min<long>((inflight * count + members - 1) / members + 2, resident / kXcds);
-    len = count > 1 ? std::min(inflight, per) : members == 1 ? nsweeps : per;
-    len = std::max<long>(2, std::min(len, nsweeps));
-    per *= kXcds;
-  }
-  long G = ctx->tune.chase_groups > 0 ? ctx->tune.chase_groups : per;
-  G = std::min<long>(G, std::max<long>(1, nsweeps * count * (boxes ? kXcds : 1)));
-  const ChaseUnits units{(int)len, (int)(((nsweeps + len - 1) / len) * count), members};
+  EVD_TRY(max_coresident_blocks(ctx, (const void *)chase_kernel<BW>, 256, 0, &resident));
+  const long inflight = ((n + 2 * b - 1) / (2 * b) + 4) * count;
+  long G = ctx->tune.chase_groups > 0 ? ctx->tune.chase_groups
+                                      : std::min<long>(inflight, (long)std::max(ctx->num_cus, resident));
+  G = std::min<long>(G, std::max<long>(1, (n - 2) * count));
+  int ni = (int)n, bi = (int)b;
+  unsigned nbytes = (unsigned)bytes;
   unsigned *err = ctx->ctrl + kCtrlError;
-  const long words = 2 * mail_half(n, b);
-  mail_fill_kernel<<<dim3((unsigned)std::min<long>((words + 255) / 256, 4096), (unsigned)count,
-                          boxes ? members + 1u : 1u),
-                     256, 0, ctx->stream>>>((int)n, (int)b, band, ldb, band_stride, mail, boxes, D, d_stride);
-  EVD_LAUNCHED(ctx);
   if (ctx->timing && !ctx->capturing) hipEventRecord(ctx->cev[0], ctx->stream);
-  if (boxes)
-    chase_kernel<BW, true><<<(unsigned)G, ChaseShape<BW>::NT, 0, ctx->stream>>>(
-        (int)n, (int)b, mail, boxes, units, U, ldu, u_stride, com, ticket, err, count, D, d_stride, E, e_stride);
-  else
-    chase_kernel<BW, false><<<(unsigned)G, ChaseShape<BW>::NT, 0, ctx->stream>>>(
-        (int)n, (int)b, mail, boxes, units, U, ldu, u_stride, com, ticket, err, count, D, d_stride, E, e_stride);
+  chase_kernel<BW><<<(unsigned)G, 256, 0, ctx->stream>>>(ni, bi, band, ldb, nbytes, U, ldu, com, ticket, err, count,
+                                                          band_stride, u_stride, com_stride);
   EVD_LAUNCHED(ctx);
   if (ctx->timing && !ctx->capturing) hipEventRecord(ctx->cev[1], ctx->stream);
   return 0;
@@ -1140,42 +740,10 @@ __global__ void band_extract_batched_kernel(int n, const double *__restrict__ ba
   }
 }
 
-// A band of width 1 is tridiagonal already; the sweeps' reflectors have length
-// 1 and flip signs (H = -1 where the entry below the diagonal is not zero).
-__global__ void chase_signs_kernel(int n, const double *__restrict__ band, long ldb, long band_stride,
-                                   float *__restrict__ U, long ldu, long u_stride, double *__restrict__ D,
-                                   long d_stride, double *__restrict__ E, long e_stride) {
-  const long q = blockIdx.y;
-  band += q * band_stride;
-  for (long s = blockIdx.x * (long)blockDim.x + threadIdx.x; s < n; s += (long)gridDim.x * blockDim.x) {
-    D[q * d_stride + s] = band[s * ldb];
-    if (s >= n - 1) continue;
-    double x = band[1 + s * ldb];
-    if (s > 0 && band[1 + (s - 1) * ldb] != 0.0) x = -x;
-    if (s < n - 2 && x != 0.0) {
-      U[q * u_stride + s + 1 + s * ldu] = (float)(x >= 0.0 ? 1.41421356237309504880 : -1.41421356237309504880);
-      x = -x;
-    }
-    E[q * e_stride + s] = x;
-  }
-}
-
-size_t sb2st_batched_workspace(int count, long n, long b) {
-  return align256((size_t)count * 2 * mail_half(n, b) * sizeof(double) +
-                  ((size_t)count * n * kComStride + kTicketWords) * sizeof(int));
-}
-
-// The XCDs' boxes are scratch on top of that, used where the arena has room
-// (a call never fails for want of them; the results are the same).
-static size_t chase_boxes_bytes(int count, long n, long b) {
-  count = chase_batch(count, n, b);
-  return (size_t)chase_members(count, n, b) * count * 2 * mail_half(n, b) * sizeof(double);
-}
-
 // Bulge chasing of `count` same-size bands in one persistent launch (problem q
 // at band + q band_stride, U + q u_stride, D + q d_stride, E + q e_stride).
 // The progress words and the ticket come from the arena, or from ext_com
-// (at least sb2st_batched_workspace(count, n, b) bytes) when it is given.
+// (at least sb2st_batched_workspace(count, n) bytes) when it is given.
 int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ldband, long band_stride, float *U,
                   long ldu, long u_stride, double *D, long d_stride, double *E, long e_stride, int *ext_com) {
   if (n <= 0 || count <= 0) return 0;
@@ -1185,59 +753,29 @@ int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ld
     for (int q = 0; q < count; q++) EVD_TRY(fill_f32(ctx, U + (long)q * u_stride, ldu, n, ldu, 0.f));
   if (n > 2) {
     ArenaFrame frame(ctx);
-    // messages, then progress words com[q * n * kComStride + s * kComStride]
-    // and the ticket
+    // progress words com[q * n * kComStride + s * kComStride], then the ticket
     const long com_stride = n * kComStride;
-    const size_t words = (size_t)count * com_stride + kTicketWords;
-    double *mail = ext_com ? reinterpret_cast<double *>(ext_com)
-                           : arena_alloc_n<double>(ctx, sb2st_batched_workspace(count, n, b) / sizeof(double));
-    if (!mail) return EVD_E_NOMEM;
-    int *com = reinterpret_cast<int *>(mail + 2 * mail_half(n, b) * count);
+    const size_t words = (size_t)count * com_stride + 1;
+    int *com = ext_com ? ext_com : arena_alloc_n<int>(ctx, words);
+    if (!com) return EVD_E_NOMEM;
     unsigned *ticket = reinterpret_cast<unsigned *>(com + (size_t)count * com_stride);
     EVD_TRY(fill_u32(ctx, reinterpret_cast<unsigned *>(com), words, 0u));
     // sweeps per workgroup: the knob (0 = 1, one sweep per workgroup), at most
     // what the LDS window holds and at most 3 (with more than four waves a
     // workgroup's waves share SIMDs and the grouped kernel's registers spill)
     const int depth = std::min({ctx->tune.chase_depth > 0 ? ctx->tune.chase_depth : 1, group_depth_max(b), 3});
-    if (b > 64) return set_error(ctx, EVD_E_UNSUPPORTED, "bandwidth %ld > 64", b);
-    auto boxes = [&]() -> double * {
-      if (chase_members(chase_batch(count, n, b), n, b) > kXcds) return nullptr;
-      const size_t bytes = chase_boxes_bytes(count, n, b);
-      const size_t room = ctx->arena_bytes - std::min(ctx->arena_bytes, align256(ctx->arena_top));
-      return ext_com || bytes > room ? nullptr : static_cast<double *>(arena_alloc(ctx, bytes));
-    };
-    if (b <= 32 && depth > 1) {
-      if (depth == 3)
-        EVD_TRY(launch_chase_group<3>(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, com, com_stride,
-                                      ticket));
-      else
-        EVD_TRY(launch_chase_group<2>(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, com, com_stride,
-                                      ticket));
-    } else if (b == 1) {
-      chase_signs_kernel<<<dim3((unsigned)std::min<long>((n + 255) / 256, 1024), (unsigned)count), 256, 0,
-                           ctx->stream>>>((int)n, band, ldband, band_stride, U, ldu, u_stride, D, d_stride, E, e_stride);
-      EVD_LAUNCHED(ctx);
-      return 0;
-    } else {
-      double *bx = boxes();
-      const int batch = bx ? chase_batch(count, n, b) : count;
-      for (int q0 = 0; q0 < count; q0 += batch) {
-        const int c = std::min(batch, count - q0);
-        if (q0 > 0) EVD_TRY(fill_u32(ctx, ticket, kTicketWords, 0u));
-        const double *bq = band + (long)q0 * band_stride;
-        double *mq = mail + (long)q0 * 2 * mail_half(n, b);
-        float *Uq = U + (long)q0 * u_stride;
-        int *cq = com + (long)q0 * com_stride;
-        double *Dq = D + (long)q0 * d_stride, *Eq = E + (long)q0 * e_stride;
-        if (b <= 32)
-          EVD_TRY(launch_chase<32>(ctx, c, n, b, bq, ldband, band_stride, mq, bx, Uq, ldu, u_stride, cq, ticket, Dq,
-                                   d_stride, Eq, e_stride));
-        else
-          EVD_TRY(launch_chase<64>(ctx, c, n, b, bq, ldband, band_stride, mq, bx, Uq, ldu, u_stride, cq, ticket, Dq,
-                                   d_stride, Eq, e_stride));
-      }
-      return 0;
-    }
+    if (b <= 32 && depth == 3)
+      EVD_TRY(launch_chase_group<3>(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, com, com_stride,
+                                    ticket));
+    else if (b <= 32 && depth == 2)
+      EVD_TRY(launch_chase_group<2>(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, com, com_stride,
+                                    ticket));
+    else if (b <= 32)
+      EVD_TRY(launch_chase<32>(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, com, com_stride, ticket));
+    else if (b <= 64)
+      EVD_TRY(launch_chase<64>(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, com, com_stride, ticket));
+    else
+      return set_error(ctx, EVD_E_UNSUPPORTED, "bandwidth %ld > 64", b);
   }
   band_extract_batched_kernel<<<dim3((unsigned)std::min<long>((n + 255) / 256, 1024), (unsigned)count), 256, 0,
                                 ctx->stream>>>((int)n, band, ldband, band_stride, D, d_stride, E, e_stride);
@@ -1245,29 +783,20 @@ int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ld
   return 0;
 }
 
+size_t sb2st_batched_workspace(int count, long n) { return align256(((size_t)count * n * kComStride + 1) * sizeof(int)); }
 
 int sb2st(evd_ctx *ctx, long n, long b, double *band, long ldband, float *U, long ldu, double *D, double *E) {
   return sb2st_batched(ctx, 1, n, b, band, ldband, 0, U, ldu, 0, D, 0, E, 0, nullptr);
 }
 
-// arena of a chase called by itself: with the XCDs' boxes where it may grow to
-// that (no captured graph, lent arena or budget against it), else without
-static int chase_arena(evd_ctx *ctx, int count, long n, long b) {
-  const size_t need = sb2st_batched_workspace(count, n, b) + 4096, all = need + chase_boxes_bytes(count, n, b);
-  if (chase_members(chase_batch(count, n, b), n, b) <= kXcds && all > ctx->arena_bytes && ctx->graphs == 0 && !ctx->arena_external && !(ctx->budget && all > ctx->budget) &&
-      arena_ensure(ctx, all) == 0)
-    return 0;
-  return arena_ensure(ctx, need);
-}
-
 // ---- the chase without allocation: scratch in a file-scope device array.
-// Messages, progress words (one per sweep, kComStride apart) and the sweep
-// ticket of one problem of order <= kNoAllocMaxN: 69 MiB per device, held
-// until the process ends.  Host code never passes the array's name to a kernel (it is a
+// Progress words (one per sweep, kComStride apart) and the sweep ticket of
+// one problem of order <= kNoAllocMaxN: 4 MiB per device, held until the
+// process ends.  Host code never passes the array's name to a kernel (it is a
 // host-side stand-in); it uses the device address that hipGetSymbolAddress
 // returns, looked up once per device with that device current.
 constexpr long kNoAllocMaxN = 32768;
-constexpr size_t kNoAllocWords = (size_t)kNoAllocMaxN * (kComStride + 4 * 2 * 64) + 131072;
+constexpr size_t kNoAllocWords = (size_t)kNoAllocMaxN * kComStride + 64;
 static __device__ __align__(256) int scratch[kNoAllocWords];
 
 static int noalloc_scratch(evd_ctx *ctx, int **out) {
@@ -1312,7 +841,7 @@ extern "C" int evd_sb2st_f64(evd_ctx *ctx, long n, long b, double *band, long ld
   EVD_ARG(ctx, b >= 1 && b <= 64, 3);
   EVD_ARG(ctx, ldband >= 2 * b, 5);
   EVD_ARG(ctx, ldu >= n + b, 7);
-  if (ctx->arena_top == 0) EVD_TRY(chase_arena(ctx, 1, n, b));
+  if (ctx->arena_top == 0) EVD_TRY(arena_ensure(ctx, sb2st_batched_workspace(1, n) + 4096));
   EVD_TRY(sb2st(ctx, n, b, band, ldband, U, ldu, D, E));
   return check_device_error(ctx, "evd_sb2st_f64");
 }
@@ -1327,8 +856,8 @@ extern "C" int evd_sb2st_f64_noalloc(evd_ctx *ctx, long n, long b, double *band,
   if (n > kNoAllocMaxN)
     return set_error(ctx, EVD_E_UNSUPPORTED, "evd_sb2st_f64_noalloc: n = %ld exceeds the scratch limit n <= %ld", n,
                      kNoAllocMaxN);
-  if (sb2st_batched_workspace(1, n, b) > kNoAllocWords * sizeof(int))
-    return set_error(ctx, EVD_E_UNSUPPORTED, "evd_sb2st_f64_noalloc: n = %ld, b = %ld exceed the scratch", n, b);
+  static_assert(kNoAllocWords * sizeof(int) >= ((size_t)kNoAllocMaxN * kComStride + 1) * sizeof(int),
+                "scratch holds the progress words and the ticket of the largest order");
   int *com = nullptr;
   EVD_TRY(noalloc_scratch(ctx, &com));
   EVD_TRY(sb2st_batched(ctx, 1, n, b, band, ldband, 0, U, ldu, 0, D, 0, E, 0, com));
@@ -1349,7 +878,7 @@ extern "C" int evd_sb2st_batched_f64(evd_ctx *ctx, int count, long n, long b, do
   EVD_ARG(ctx, count <= 1 || d_stride >= n, 12);
   EVD_ARG(ctx, count <= 1 || e_stride >= std::max<long>(1, n - 1), 14);
   EVD_ARG(ctx, (long)count * std::max<long>(n, 1) < (1L << 30), 2);
-  if (ctx->arena_top == 0) EVD_TRY(chase_arena(ctx, count, n, b));
+  if (ctx->arena_top == 0) EVD_TRY(arena_ensure(ctx, sb2st_batched_workspace(count, n) + 4096));
   EVD_TRY(sb2st_batched(ctx, count, n, b, band, ldband, band_stride, U, ldu, u_stride, D, d_stride, E, e_stride,
                         nullptr));
   return check_device_error(ctx, "evd_sb2st_batched_f64");

@@ -37,7 +37,7 @@ long sbr_back_blk(long knob, long b, long wcols);
 bool tune_lookup(long n, long b, int precision, int *nb, Tuning *t);
 int sb2st_batched(evd_ctx *ctx, int count, long n, long b, double *band, long ldband, long band_stride, float *U,
                   long ldu, long u_stride, double *D, long d_stride, double *E, long e_stride, int *ext_com);
-size_t sb2st_batched_workspace(int count, long n, long b);
+size_t sb2st_batched_workspace(int count, long n);
 bool bc_back_wy_fits(long n, long ldq);
 int bc_back_wy_batched(evd_ctx *ctx, int count, long n, long ncols, float *Q, long ldq, long q_stride, const float *U,
                        long ldu, long u_stride, bool split16);
@@ -231,7 +231,7 @@ size_t syevd_workspace(long n, long b, long nb, char jobz, int precision, long s
   s += align256((size_t)2 * b * n * sizeof(double));          // band
   s += align256((size_t)(n + b) * n * sizeof(float));         // U
   s += align256((size_t)n * sizeof(double)) * 2;              // D, E
-  size_t later = std::max(sy2sb_workspace(n, b, nb), sb2st_batched_workspace(1, n, b));
+  size_t later = std::max(sy2sb_workspace(n, b, nb), sb2st_batched_workspace(1, n));
   later = std::max(later, stedc_values_workspace(1, n));
   if (jobz == 'V' || jobz == 'v') {
     s += align256((size_t)n * n * sizeof(double));  // Z_T
@@ -323,7 +323,7 @@ size_t syevd_batched_workspace(int count, long n, long b, long nb, char jobz, in
   size_t per = align256((size_t)n * wc * sizeof(float)) * 2 + align256((size_t)2 * b * n * sizeof(double)) +
                align256((size_t)(n + b) * n * sizeof(float)) + align256((size_t)n * sizeof(double)) * 2;
   size_t s = per * count + 4 * 256;
-  size_t later = std::max(sy2sb_batched_workspace(count, n, b, nb), sb2st_batched_workspace(count, n, b) + ((size_t)1 << 20));
+  size_t later = std::max(sy2sb_batched_workspace(count, n, b, nb), sb2st_batched_workspace(count, n) + ((size_t)1 << 20));
   later = std::max(later, stedc_values_workspace(count, n) + ((size_t)1 << 20));
   if (vec) {
     s += align256((size_t)n * n * count * sizeof(double));  // tridiagonal eigenvectors
