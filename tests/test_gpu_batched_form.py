@@ -19,8 +19,6 @@ def _sizes(count=512, seed=1):
     return [int(x) for x in np.exp(rng.uniform(np.log(64), np.log(2048), size=count)).round()]
 
 
-@pytest.mark.skip(reason="did not end within 120 s while a large batch's chase was one launch of up to three workgroups "
-                  "per CU; that launch form is gone (chase_batch in chase.hip), but its failure is not explained")
 def test_batched_form_512_matrices(ctx):
     import torch
     from threadpoolctl import threadpool_limits
