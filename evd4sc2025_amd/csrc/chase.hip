@@ -49,21 +49,62 @@ __device__ inline void st_band(__amdgpu_buffer_rsrc_t r, unsigned off_elems, dou
                                         r, off_elems * 8u, 0, kSc1);
 }
 
+// 64-bit DPP move of v (rows outside RM read 0)
+template <int CTRL, int RM>
+__device__ __attribute__((always_inline)) inline double dpp_f64(double v) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)x, CTRL, RM, 0xf, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), CTRL, RM, 0xf, false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// sum over the 64 lanes, returned in every lane: quad, half-row and row
+// reductions by DPP, then row 15 -> rows 1 and 3 and lane 31 -> rows 2 and 3
+// broadcasts; lane 63 holds the total
+__device__ __attribute__((always_inline)) inline double wave_total(double v) {
+  v += dpp_f64<0xb1, 0xf>(v);   // quad_perm [1, 0, 3, 2]
+  v += dpp_f64<0x4e, 0xf>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_f64<0x141, 0xf>(v);  // row_half_mirror
+  v += dpp_f64<0x140, 0xf>(v);  // row_mirror
+  v += dpp_f64<0x142, 0xa>(v);  // row_bcast:15
+  v += dpp_f64<0x143, 0xc>(v);  // row_bcast:31
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, 63);
+  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), 63);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// sum over aligned groups of W lanes (4 or 8), returned in every lane of the
+// group: each step adds the other half of a group whose halves already agree,
+// so the mirror serves as an exchange
+template <int W>
+__device__ __attribute__((always_inline)) inline double group_sum(double v) {
+  static_assert(W == 4 || W == 8, "lanes of a window row");
+  v += dpp_f64<0xb1, 0xf>(v);                // quad_perm [1, 0, 3, 2]
+  v += dpp_f64<0x4e, 0xf>(v);                // quad_perm [2, 3, 0, 1]
+  if (W == 8) v += dpp_f64<0x141, 0xf>(v);   // row_half_mirror
+  return v;
+}
+
 // LAPACK-style reflector of the chase (reference sign convention): from the
 // column x = Bc[0..lenx) (LDS, stride LD), u = (x/||x|| + sign(x0) e1) /
-// sqrt(|x0/||x|| + sign(x0)|), ||u||^2 = 2, H x = beta e1.  Wave 0 only.
+// sqrt(|x0/||x|| + sign(x0)|), ||u||^2 = 2, H x = beta e1.  Wave 0 only.  It
+// sits in the chain of the steps: sums by DPP instead of shuffles through LDS
+// and refined reciprocal roots instead of two roots and two divisions (with the
+// same sums in the step, n = 6000, b = 32: 49.3 -> 44.0 ms).
 template <int BW>
 __device__ inline void chase_reflector(const double *Bc, int lenx, int lane, double *u, double *s_beta, float *U,
                                        long urow, long ucol) {
   constexpr int LD = BW + 1;
   const double x = (lane < lenx) ? Bc[lane * LD] : 0.0;
-  const double nrm = sqrt(wave_sum(x * x));
+  const double nn = wave_total(x * x);
   const double x0 = Bc[0];
-  double uu = 0.0;
-  if (nrm > 0.0) {
-    const double inv = 1.0 / nrm;
+  double uu = 0.0, nrm = 0.0;
+  if (nn > 0.0) {
+    double inv, scl, root;
+    rsqrt_sqrt(nn, inv, nrm);
     const double u0 = x0 * inv + (x0 >= 0.0 ? 1.0 : -1.0);
-    const double scl = 1.0 / sqrt(fabs(u0));
+    rsqrt_sqrt(fabs(u0), scl, root);
     uu = (lane == 0 ? u0 : x * inv) * scl;
   }
   if (lane < BW) u[lane] = (lane < lenx) ? uu : 0.0;
@@ -184,18 +225,15 @@ __global__ __launch_bounds__(256, BW == 32 ? 4 : 1) void chase_kernel(int n, int
         yp += Sr[r] * uk;
         qp += Nr[r] * uk;
       }
-#pragma unroll
-      for (int o = LPR / 2; o > 0; o >>= 1) {
-        yp += __shfl_xor(yp, o, 64);
-        qp += __shfl_xor(qp, o, 64);
-      }
+      yp = group_sum<LPR>(yp);
+      qp = group_sum<LPR>(qp);
       if (kc == 0) {
         yv[ri] = yp;
         qv[ri] = qp;
       }
       __syncthreads();
       // ---- S <- H S H (rank-2 with w = y - (u^T y / 2) u), N <- N H
-      const double psi = wave_sum((lane < BW) ? u[lane] * yv[lane] : 0.0);
+      const double psi = wave_total((lane < BW) ? u[lane] * yv[lane] : 0.0);
       const double ui = u[ri], wi = yv[ri] - 0.5 * psi * ui, qi = qv[ri];
 #pragma unroll
       for (int r = 0; r < EPT; r++) {
@@ -299,31 +337,6 @@ __device__ inline int sweep_nsteps(int n, int b, int s) {
     len = len2;
     k++;
   }
-}
-
-// 64-bit DPP move of v (rows outside RM read 0)
-template <int CTRL, int RM>
-__device__ __attribute__((always_inline)) inline double dpp_f64(double v) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)x, CTRL, RM, 0xf, false);
-  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), CTRL, RM, 0xf, false);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
-// sum over the 64 lanes, returned in every lane: quad, half-row and row
-// reductions by DPP, then row 15 -> rows 1 and 3 and lane 31 -> rows 2 and 3
-// broadcasts; lane 63 holds the total
-__device__ __attribute__((always_inline)) inline double wave_total(double v) {
-  v += dpp_f64<0xb1, 0xf>(v);   // quad_perm [1, 0, 3, 2]
-  v += dpp_f64<0x4e, 0xf>(v);   // quad_perm [2, 3, 0, 1]
-  v += dpp_f64<0x141, 0xf>(v);  // row_half_mirror
-  v += dpp_f64<0x140, 0xf>(v);  // row_mirror
-  v += dpp_f64<0x142, 0xa>(v);  // row_bcast:15
-  v += dpp_f64<0x143, 0xc>(v);  // row_bcast:31
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)x, 63);
-  const unsigned hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(x >> 32), 63);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
 // v of lane ^ 32.  v_permlane32_swap exchanges one half of its destination
