@@ -49,15 +49,6 @@ __device__ inline void st_band(__amdgpu_buffer_rsrc_t r, unsigned off_elems, dou
                                         r, off_elems * 8u, 0, kSc1);
 }
 
-// 64-bit DPP move of v (rows outside RM read 0)
-template <int CTRL, int RM>
-__device__ __attribute__((always_inline)) inline double dpp_f64(double v) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)x, CTRL, RM, 0xf, false);
-  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), CTRL, RM, 0xf, false);
-  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
-}
-
 // sum over the 64 lanes, returned in every lane: quad, half-row and row
 // reductions by DPP, then row 15 -> rows 1 and 3 and lane 31 -> rows 2 and 3
 // broadcasts; lane 63 holds the total

@@ -264,6 +264,33 @@ __device__ inline double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
+// 64-bit DPP move of v (rows outside RM read 0)
+template <int CTRL, int RM>
+__device__ __attribute__((always_inline)) inline double dpp_f64(double v) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)x, CTRL, RM, 0xf, false);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(unsigned)(x >> 32), CTRL, RM, 0xf, false);
+  return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+}
+
+// butterfly over a row of 16 lanes, the result in every lane, with the bits of
+// one by xor of the lane index 8, 4, 2, 1 (after the first step lanes 8 apart
+// agree, so a rotation by 4 serves as xor 4)
+__device__ __attribute__((always_inline)) inline double row_sum16(double v) {
+  v += dpp_f64<0x128, 0xf>(v);  // row_ror:8
+  v += dpp_f64<0x124, 0xf>(v);  // row_ror:4
+  v += dpp_f64<0x4e, 0xf>(v);   // quad_perm [2, 3, 0, 1]
+  v += dpp_f64<0xb1, 0xf>(v);   // quad_perm [1, 0, 3, 2]
+  return v;
+}
+__device__ __attribute__((always_inline)) inline double row_max16(double v) {
+  v = fmax(v, dpp_f64<0x128, 0xf>(v));
+  v = fmax(v, dpp_f64<0x124, 0xf>(v));
+  v = fmax(v, dpp_f64<0x4e, 0xf>(v));
+  v = fmax(v, dpp_f64<0xb1, 0xf>(v));
+  return v;
+}
+
 // 1 / sqrt(x) and sqrt(x) for x > 0: the hardware estimate refined by two
 // coupled Newton steps (Goldschmidt's iteration), the root corrected once more
 // by its residual.  One short chain instead of a square root and a division.

@@ -15,8 +15,9 @@
 //  * Q_new = Q' [U 0; 0 I] by grouped FP64 MFMA GEMMs over the top and bottom
 //    row blocks (column types 1/2/3 as in dlaed2/dlaed3).
 //
-// GPU layout: the binary split tree is built on the host down to leaves of at
-// most kDcLeaf rows, which one wave each solves by the QR algorithm; all merges of one
+// GPU layout: the binary split tree goes down to single rows.  The merges of the
+// subtrees of at most kDcLeaf rows (the leaves of the host's tree) run in one launch, a
+// workgroup per leaf; above them all merges of one
 // tree height run in the same launches (grid.y = merge), every merge working
 // in the index range [start, start+N) of n-long scratch arrays and in the
 // diagonal block of the n x n Q / scratch matrices.  The deflation scan is
@@ -31,6 +32,13 @@
 
 namespace evd {
 
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// order of a wave's LDS accesses
+static __device__ __attribute__((always_inline)) inline void lds_order() {
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+}
+
 struct MergeDesc {
   int start, n1, n2, pad;
   double rho;  // |e| at the split
@@ -40,12 +48,10 @@ struct MergeDesc {
 struct LeafDesc {
   int start, size, problem;
 };
-// Rows of a leaf.  A small merge level costs 35 to 60 us of dependent launches
-// whatever its size; the QR algorithm's rotations form one chain of about
-// 0.85 m^2 for a leaf of m rows, 0.1 us each, so leaves of 16 rows replace four
-// levels by one launch of 25 us, and leaves of 32 would spend 80 us to save one
-// level more.  With the parallel scans, products and copies below, whole solves of
-// T: n = 256 0.61 -> 0.25 ms, n = 2500 2.6 -> 1.3 ms.
+// Rows of a leaf: a row of 16 lanes holds the poles of its largest merge.  A small
+// merge level costs 35 to 60 us of dependent launches whatever its size; one
+// launch does the four below 16 rows in 40 us (n = 256 and 2500; 50 us for 32
+// problems of order 256).
 constexpr int kDcLeaf = 16;
 struct MergeOut {
   int K, K1, K2, K3, ndefl, nrot;
@@ -84,15 +90,15 @@ struct DCRows {
   double *first = nullptr, *last = nullptr, *rot_first = nullptr, *rot_last = nullptr;
 };
 
-// Tearing of every split at once, one thread per diagonal entry (an entry
-// between two splits is adjusted by both): split[k] != 0 marks a split between
-// rows k-1 and k.
-__global__ void dc_tear_kernel(long n, const int *__restrict__ split, const double *__restrict__ E,
-                               double *__restrict__ D) {
-  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+// Tearing of every split at once, one thread per diagonal entry: the tree's
+// splits are all the boundaries between rows of a problem, and an entry between two of
+// them is adjusted by both.
+__global__ void dc_tear_kernel(long n, long total, const double *__restrict__ E, double *__restrict__ D) {
+  for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < total; i += (long)gridDim.x * blockDim.x) {
     double d = D[i];
-    if (i > 0 && split[i]) d -= fabs(E[i - 1]);
-    if (i + 1 < n && split[i + 1]) d -= fabs(E[i]);
+    const long r = i % n;
+    if (r > 0) d -= fabs(E[i - 1]);
+    if (r + 1 < n) d -= fabs(E[i]);
     D[i] = d;
   }
 }
@@ -134,94 +140,6 @@ __global__ void dc_denormalize_kernel(long n, double *__restrict__ D, const doub
   if (s == 0.0 || s == 1.0) return;
   for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x)
     D[q * n + i] *= s;
-}
-
-// Eigen-decomposition of one leaf (a symmetric tridiagonal of at most kDcLeaf
-// rows) by the implicit symmetric QR algorithm with Wilkinson's shift (Golub &
-// Van Loan, Matrix Computations, section 8.3): one wave, every lane runs the same
-// scalar recurrence and lane r applies its rotations to row r of the
-// vectors.  D and the vectors leave sorted.  Bound by the chain of rotations
-// (a reciprocal root each); the column a rotation finishes leaves for LDS while
-// the other one stays in a register as the next rotation's first.
-__global__ __launch_bounds__(64) void dc_leaf_kernel(const LeafDesc *__restrict__ lf, const double *__restrict__ E,
-                                                     double *__restrict__ D, double *__restrict__ Z, long ldz,
-                                                     long zmul, DCRows rows, unsigned *__restrict__ err) {
-  __shared__ double d[kDcLeaf], e[kDcLeaf + 1], q[kDcLeaf][kDcLeaf + 1];
-  __shared__ int rank[kDcLeaf];
-  const LeafDesc l = lf[blockIdx.x];
-  const int m = l.size, st = l.start, lane = threadIdx.x;
-  const double eps = DBL_EPSILON * 0.5;
-  // entries whose square could underflow are zero beside the problem's norm, 1
-  const double tiny = 1e-140;
-  if (lane < m) {
-    d[lane] = D[st + lane];
-    e[lane] = lane < m - 1 ? E[st + lane] : 0.0;
-    for (int c = 0; c < m; c++) q[c][lane] = (c == lane) ? 1.0 : 0.0;
-  }
-  __syncthreads();
-  int hi = m - 1, it = 0;
-  while (hi > 0) {
-    const bool small = lane < hi && fabs(e[lane]) <= eps * (fabs(d[lane]) + fabs(d[lane + 1])) + tiny;
-    const unsigned long long cut = __ballot(small);
-    if ((cut >> (hi - 1)) & 1) {
-      hi--;
-      continue;
-    }
-    if (++it > 40 * kDcLeaf) {
-      if (lane == 0) atomicOr(err, (unsigned)EVD_E_NOCONVERGE);
-      break;
-    }
-    // the unreduced block lo .. hi
-    const int lo = cut ? 64 - __clzll((long long)cut) : 0;
-    const double eh = e[hi - 1], dh = d[hi], del = 0.5 * (d[hi - 1] - dh);
-    const double mu = dh - eh * (eh / (del + copysign(sqrt(del * del + eh * eh), del)));
-    double dk = d[lo], ek = e[lo], x = dk - mu, z = ek;
-    double qk = lane < m ? q[lo][lane] : 0.0;
-    for (int k = lo; k < hi; k++) {
-      const double dn = d[k + 1], en = e[k + 1], qn = lane < m ? q[k + 1][lane] : 0.0;
-      double c = 1.0, s = 0.0, r = 0.0;
-      const double rr = x * x + z * z;
-      if (rr > 0.0) {
-        double inv;
-        rsqrt_sqrt(rr, inv, r);
-        c = x * inv;
-        s = -z * inv;
-      }
-      if (k > lo) e[k - 1] = r;
-      const double cs = c * s, t = 2.0 * cs * ek, cc = c * c, ss = s * s;
-      d[k] = cc * dk - t + ss * dn;
-      x = cs * (dk - dn) + (cc - ss) * ek;
-      dk = ss * dk + t + cc * dn;
-      if (lane < m) q[k][lane] = c * qk - s * qn;
-      qk = s * qk + c * qn;
-      z = -s * en;
-      ek = c * en;
-    }
-    e[hi - 1] = x;
-    d[hi] = dk;
-    if (lane < m) q[hi][lane] = qk;
-    __syncthreads();
-  }
-  if (lane < m) {
-    int pos = 0;
-    const double v = d[lane];
-    for (int i = 0; i < m; i++) pos += (d[i] < v || (d[i] == v && i < lane)) ? 1 : 0;
-    rank[lane] = pos;
-    D[st + pos] = v;
-  }
-  __syncthreads();
-  if (rows.first) {
-    if (lane < m) {
-      rows.first[st + rank[lane]] = q[lane][0];
-      rows.last[st + rank[lane]] = q[lane][m - 1];
-    }
-    return;
-  }
-  double *Zb = Z + ((long)l.problem * zmul + st + (long)st * ldz);
-  for (int i = lane; i < m * m; i += 64) {
-    const int row = i % m, c = i / m;
-    Zb[row + (long)rank[c] * ldz] = q[c][row];
-  }
 }
 
 // |e| and sign(e) at every split, read on the device so no host round trip
@@ -319,7 +237,7 @@ __device__ inline unsigned long long block_scan256(unsigned long long v, unsigne
 __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__restrict__ md, MergeOut *__restrict__ mo,
                                                          const double *__restrict__ D, const double *__restrict__ Z,
                                                          long ldz, int sort, DCScratch sc, DCRows rows) {
-  __shared__ double red[4];
+  __shared__ double red[4], zpart[256];
   __shared__ unsigned long long sh[4];
   __shared__ int s_nc, s_K, s_nrot;
   const MergeDesc m = md[blockIdx.x];
@@ -513,13 +431,15 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
     const int ty = types[nd_col[kk]];
     qpos[kk] = (ty == 1) ? e1++ : (ty == 2) ? K1 + e2++ : K1 + K2 + e3++;
   }
-  // z sum in a fixed order (deterministic): per-thread chunks, waves, workgroup
-  zs2 = wave_sum(zs2);
+  // z sum in a fixed order (deterministic): per-thread chunks, then thread order
   __syncthreads();
-  if (lane == 0) red[wave] = zs2;
+  zpart[tid] = zs2;
   __syncthreads();
   if (tid == 0) {
-    const double zsum = ((red[0] + red[1]) + red[2]) + red[3];
+    const int np = kp > 0 ? (K + kp - 1) / kp : 0;  // threads that had a chunk
+    double zsum = 0.0;
+#pragma unroll 8
+    for (int t = 0; t < np; t++) zsum += zpart[t];
     MergeOut o;
     o.K = K;
     o.K1 = K1;
@@ -582,16 +502,18 @@ __global__ __launch_bounds__(256) void dc_gather_kernel(const MergeDesc *__restr
 }
 
 // f(tau) pieces relative to pole `org`: psi over poles <= lower, phi over the rest.
-// The secular function and its split derivatives at d[org] + tau, summed by
-// one wave: lane l takes poles l, l+64, ...; a butterfly allreduce leaves the
-// same sums in every lane, so the root iteration stays wave-uniform.
+// The secular function and its split derivatives at d[org] + tau, summed by W
+// lanes: lane l takes poles l, l + W, ...; a butterfly allreduce leaves the same
+// sums in every lane, so the root iteration stays uniform.  For K <= 16 both forms
+// give the same bits: the butterfly's steps over lanes without a pole add zeros.
+template <int W>
 __device__ inline void secular_eval(const double *__restrict__ d, const double *__restrict__ z, int K, int org,
                                     int lower, double tau, double rho, double &f, double &psi, double &dpsi,
-                                    double &phi, double &dphi) {
+                                    double &phi, double &dphi, int lane) {
+  static_assert(W == 64 || W == 16, "a wave or a row of lanes");
   const double dorg = d[org];
   psi = dpsi = phi = dphi = 0.0;
-  const int lane = threadIdx.x & 63;
-  for (int k = lane; k < K; k += 64) {
+  for (int k = lane; k < K; k += W) {
     const double del = (d[k] - dorg) - tau;
     const double zk = z[k];
     const double t = zk / del;
@@ -605,15 +527,112 @@ __device__ inline void secular_eval(const double *__restrict__ d, const double *
       dphi += dterm;
     }
   }
-  psi = wave_sum(psi);
-  dpsi = wave_sum(dpsi);
-  phi = wave_sum(phi);
-  dphi = wave_sum(dphi);
+  psi = W == 64 ? wave_sum(psi) : row_sum16(psi);
+  dpsi = W == 64 ? wave_sum(dpsi) : row_sum16(dpsi);
+  phi = W == 64 ? wave_sum(phi) : row_sum16(phi);
+  dphi = W == 64 ? wave_sum(dphi) : row_sum16(dphi);
   psi *= rho;
   dpsi *= rho;
   phi *= rho;
   dphi *= rho;
   f = 1.0 + psi + phi;
+}
+
+// Root i of the secular equation by W lanes: lambda = d[org] + tau.  Returns
+// whether the iteration converged.
+template <int W>
+__device__ inline bool secular_root(const double *__restrict__ d, const double *__restrict__ z, int K, int i,
+                                    double rho, double zsum, int lane, int &org, double &tau) {
+  const double eps = DBL_EPSILON * 0.5;
+  double lo, hi;
+  if (i < K - 1) {
+    const double gap = d[i + 1] - d[i];
+    const double mid = 0.5 * gap;
+    double f, psi, dpsi, phi, dphi;
+    secular_eval<W>(d, z, K, i, i, mid, rho, f, psi, dpsi, phi, dphi, lane);
+    if (f >= 0.0) {
+      org = i;
+      lo = 0.0;
+      hi = mid;
+    } else {
+      org = i + 1;
+      lo = mid - gap;  // relative to d[i+1]
+      hi = 0.0;
+    }
+  } else {
+    org = K - 1;
+    lo = 0.0;
+    hi = rho * zsum;
+    if (hi <= 0.0) hi = rho;
+  }
+  const int lower = i;  // poles d[0..i] lie below the root
+  tau = 0.5 * (lo + hi);
+  bool conv = false;
+  for (int it = 0; it < 200; it++) {
+    double f, psi, dpsi, phi, dphi;
+    secular_eval<W>(d, z, K, org, lower, tau, rho, f, psi, dpsi, phi, dphi, lane);
+    if (f < 0.0)
+      lo = tau;
+    else
+      hi = tau;
+    const double erretm = 10.0 * (fabs(psi) + fabs(phi)) + 4.0;
+    if (fabs(f) <= eps * erretm || (hi - lo) <= 4.0 * eps * fmax(fabs(lo), fabs(hi))) {
+      conv = true;
+      break;
+    }
+    // two-pole rational model around the current point
+    const double dl = (d[i] - d[org]) - tau;  // < 0
+    double tn;
+    bool ok = false;
+    if (i < K - 1) {
+      const double du = (d[i + 1] - d[org]) - tau;  // > 0
+      const double q = dl * dl * dpsi, s = du * du * dphi;
+      const double C = f - dl * dpsi - du * dphi;
+      const double a2 = C, a1 = -(C * (dl + du) + q + s), a0 = C * dl * du + q * du + s * dl;
+      double eta = 0.0;
+      if (fabs(a2) < 1e-300) {
+        if (a1 != 0.0) {
+          eta = -a0 / a1;
+          ok = true;
+        }
+      } else {
+        const double disc = a1 * a1 - 4.0 * a2 * a0;
+        if (disc >= 0.0) {
+          const double sq = sqrt(disc);
+          const double qq = -0.5 * (a1 + (a1 >= 0.0 ? sq : -sq));
+          const double r1 = qq / a2;
+          const double r2 = (qq != 0.0) ? a0 / qq : r1;
+          const bool in1 = (r1 > dl && r1 < du), in2 = (r2 > dl && r2 < du);
+          if (in1 && (!in2 || fabs(r1) <= fabs(r2))) {
+            eta = r1;
+            ok = true;
+          } else if (in2) {
+            eta = r2;
+            ok = true;
+          }
+        }
+      }
+      tn = tau + eta;
+    } else {
+      // single pole below: C + q/(dl - eta) = 0
+      const double q = dl * dl * dpsi;
+      const double C = f - dl * dpsi;
+      if (C > 0.0) {
+        tn = tau + dl + q / C;
+        ok = true;
+      } else {
+        tn = tau;
+      }
+    }
+    if (!ok || !(tn > lo && tn < hi)) tn = 0.5 * (lo + hi);
+    if (tn == tau || tn <= lo || tn >= hi) {
+      // the bracket cannot be split further in FP64: tau is as good as it gets
+      conv = true;
+      break;
+    }
+    tau = tn;
+  }
+  return conv;
 }
 
 __global__ void dc_secular_kernel(const MergeDesc *__restrict__ md, const MergeOut *__restrict__ mo, DCScratch sc,
@@ -622,100 +641,12 @@ __global__ void dc_secular_kernel(const MergeDesc *__restrict__ md, const MergeO
   const MergeOut o = mo[blockIdx.y];
   const int st = m.start, K = o.K;
   const double *d = sc.nd_d + st, *z = sc.nd_z + st;
-  const double rho = o.rho2;
-  const double eps = DBL_EPSILON * 0.5;
   // one wave per root
   const int waves = blockDim.x >> 6, lane = threadIdx.x & 63;
   for (int i = blockIdx.x * waves + (threadIdx.x >> 6); i < K; i += gridDim.x * waves) {
     int org;
-    double lo, hi;
-    if (i < K - 1) {
-      const double gap = d[i + 1] - d[i];
-      const double mid = 0.5 * gap;
-      double f, psi, dpsi, phi, dphi;
-      secular_eval(d, z, K, i, i, mid, rho, f, psi, dpsi, phi, dphi);
-      if (f >= 0.0) {
-        org = i;
-        lo = 0.0;
-        hi = mid;
-      } else {
-        org = i + 1;
-        lo = mid - gap;  // relative to d[i+1]
-        hi = 0.0;
-      }
-    } else {
-      org = K - 1;
-      lo = 0.0;
-      hi = rho * o.zsum;
-      if (hi <= 0.0) hi = rho;
-    }
-    const int lower = i;  // poles d[0..i] lie below the root
-    double tau = 0.5 * (lo + hi);
-    bool conv = false;
-    for (int it = 0; it < 200; it++) {
-      double f, psi, dpsi, phi, dphi;
-      secular_eval(d, z, K, org, lower, tau, rho, f, psi, dpsi, phi, dphi);
-      if (f < 0.0)
-        lo = tau;
-      else
-        hi = tau;
-      const double erretm = 10.0 * (fabs(psi) + fabs(phi)) + 4.0;
-      if (fabs(f) <= eps * erretm || (hi - lo) <= 4.0 * eps * fmax(fabs(lo), fabs(hi))) {
-        conv = true;
-        break;
-      }
-      // two-pole rational model around the current point
-      const double dl = (d[i] - d[org]) - tau;  // < 0
-      double tn;
-      bool ok = false;
-      if (i < K - 1) {
-        const double du = (d[i + 1] - d[org]) - tau;  // > 0
-        const double q = dl * dl * dpsi, s = du * du * dphi;
-        const double C = f - dl * dpsi - du * dphi;
-        const double a2 = C, a1 = -(C * (dl + du) + q + s), a0 = C * dl * du + q * du + s * dl;
-        double eta = 0.0;
-        if (fabs(a2) < 1e-300) {
-          if (a1 != 0.0) {
-            eta = -a0 / a1;
-            ok = true;
-          }
-        } else {
-          const double disc = a1 * a1 - 4.0 * a2 * a0;
-          if (disc >= 0.0) {
-            const double sq = sqrt(disc);
-            const double qq = -0.5 * (a1 + (a1 >= 0.0 ? sq : -sq));
-            const double r1 = qq / a2;
-            const double r2 = (qq != 0.0) ? a0 / qq : r1;
-            const bool in1 = (r1 > dl && r1 < du), in2 = (r2 > dl && r2 < du);
-            if (in1 && (!in2 || fabs(r1) <= fabs(r2))) {
-              eta = r1;
-              ok = true;
-            } else if (in2) {
-              eta = r2;
-              ok = true;
-            }
-          }
-        }
-        tn = tau + eta;
-      } else {
-        // single pole below: C + q/(dl - eta) = 0
-        const double q = dl * dl * dpsi;
-        const double C = f - dl * dpsi;
-        if (C > 0.0) {
-          tn = tau + dl + q / C;
-          ok = true;
-        } else {
-          tn = tau;
-        }
-      }
-      if (!ok || !(tn > lo && tn < hi)) tn = 0.5 * (lo + hi);
-      if (tn == tau || tn <= lo || tn >= hi) {
-        // the bracket cannot be split further in FP64: tau is as good as it gets
-        conv = true;
-        break;
-      }
-      tau = tn;
-    }
+    double tau;
+    const bool conv = secular_root<64>(d, z, K, i, o.rho2, o.zsum, lane, org, tau);
     if (lane == 0) {
       if (!conv) atomicOr(err, (unsigned)EVD_E_NOCONVERGE);
       sc.orig[st + i] = org;
@@ -725,30 +656,43 @@ __global__ void dc_secular_kernel(const MergeDesc *__restrict__ md, const MergeO
   }
 }
 
-// zhat_j^2 = prod_i (lambda_i - d_j) / (rho prod_{k != j} (d_k - d_j)): one wave
-// per j, lane l takes the ratios k = l, l + 64, ... (each within the spread of
-// the poles, as is any product of them) and the lanes' products are multiplied in
-// a fixed order.  One thread per j had taken 73 us at n = 2500, a serial chain of
-// K divisions on K / 256 workgroups.
+// zhat_j^2 = prod_i (lambda_i - d_j) / (rho prod_{k != j} (d_k - d_j)), the factor
+// of j first, then those of k = 0, 1, ... in order: one wave per four j.  Lane l
+// divides for k = k0 + l, then the wave multiplies the 64 quotients of each j in
+// order (j by lane & 3).  The divisions are what takes the time, the products
+// only K dependent multiplications; the order of the products decides the last
+// bits of zhat, and with them what the next merge deflates.  n = 2500: 124 us over
+// eight levels (a thread per j, which also divided: 73 us at the top one alone;
+// products of every 64th quotient, in another order: 74 us over all).
+constexpr int kLoewnerJ = 4;
 __global__ __launch_bounds__(256) void dc_loewner_kernel(const MergeDesc *__restrict__ md,
                                                          const MergeOut *__restrict__ mo, DCScratch sc) {
   const MergeDesc m = md[blockIdx.y];
   const MergeOut o = mo[blockIdx.y];
-  const int st = m.start, K = o.K, lane = threadIdx.x & 63;
+  const int st = m.start, K = o.K, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const double *d = sc.nd_d + st, *z = sc.nd_z + st;
   const int *orig = sc.orig + st;
   const double *tau = sc.tau + st;
-  for (int j = blockIdx.x * 4 + (threadIdx.x >> 6); j < K; j += gridDim.x * 4) {
-    const double dj = d[j];
-    double prod = 1.0;
-    for (int k = lane; k < K; k += 64) {
-      const double lk = (d[orig[k]] - dj) + tau[k];  // lambda_k - d_j
-      prod *= (k == j) ? lk / o.rho2 : lk / (d[k] - dj);
-    }
+  __shared__ double quot[4][kLoewnerJ][65];
+  for (int j0 = (blockIdx.x * 4 + wave) * kLoewnerJ; j0 < K; j0 += gridDim.x * 4 * kLoewnerJ) {
+    const int jl = min(j0 + (lane & (kLoewnerJ - 1)), K - 1);
+    double prod = ((d[orig[jl]] - d[jl]) + tau[jl]) / o.rho2;  // (lambda_j - d_j) / rho
+    for (int k0 = 0; k0 < K; k0 += 64) {
+      const int k = min(k0 + lane, K - 1);
+      const double dk = d[k], ok = d[orig[k]], tk = tau[k];
 #pragma unroll
-    for (int s = 32; s > 0; s >>= 1) prod *= __shfl_xor(prod, s, 64);
+      for (int u = 0; u < kLoewnerJ; u++) {
+        const int j = min(j0 + u, K - 1);
+        const double dj = d[j];
+        quot[wave][u][lane] = (k == j || k0 + lane >= K) ? 1.0 : ((ok - dj) + tk) / (dk - dj);
+      }
+      lds_order();
+#pragma unroll 16
+      for (int t = 0; t < 64; t++) prod *= quot[wave][lane & (kLoewnerJ - 1)][t];
+      lds_order();
+    }
     const double zh = sqrt(fabs(prod));
-    if (lane == 0) sc.zhat[st + j] = (z[j] >= 0.0) ? zh : -zh;
+    if (lane < kLoewnerJ && j0 + lane < K) sc.zhat[st + jl] = (z[jl] >= 0.0) ? zh : -zh;
   }
 }
 
@@ -983,6 +927,320 @@ __global__ void dc_copy_deflated_kernel(const MergeDesc *__restrict__ md, const 
   }
 }
 
+// One merge of a leaf's subtree.
+struct LeafMerge {
+  int off, n1, n2;  // rows off .. off + n1 - 1 and the n2 after them
+  int K, K1, K2, ndefl;
+  double rho2, zsum;
+};
+
+// The subtrees of the leaves: one workgroup per leaf of m <= kDcLeaf rows, the
+// four tree levels below it one after the other in LDS, each step of a merge as the
+// kernels of the levels above do it, operation for operation.  With it the tree ends
+// at single rows, and the sign of every vector follows from the merges alone: a
+// non-deflated one has v^T x < 0, a deflated one its child's sign, a single row is 1.
+// (Leaves by the QR algorithm gave other signs to the vectors that deflate all
+// the way up, and other last bits to the rest, which decide whether an entry at
+// the edge of the deflation tolerance is deflated: 8 of 4.1 million vectors of order
+// 256 changed sign.)
+// A row of 16 lanes serves one merge in the sort and the deflation, and one
+// root, one column and one position of the leaf in the other steps (16 rows of lanes,
+// 16 positions): no step loops over more than the 16 poles of a merge.  As one
+// launch instead of 4 x 8, which are bound by their launch gaps at these sizes.
+// Bound by the chain of the roots' iterations.
+__global__ __launch_bounds__(256) void dc_leaf_kernel(const LeafDesc *__restrict__ lf, const double *__restrict__ E,
+                                                      double *__restrict__ D, double *__restrict__ Z, long ldz,
+                                                      long zmul, DCRows rows, unsigned *__restrict__ err) {
+  constexpr int L = kDcLeaf;
+  __shared__ double e[L], d[L], ds[L], zs[L], sq[L], nd_d[L], nd_z[L], df_d[L], tmp_d[L], tau[L], lam[L], zhat[L];
+  __shared__ double rot_c[L], rot_s[L], quot[L][L + 1];
+  __shared__ double V[L][L + 1], Q[L][L + 1], U[L][L + 1];  // by column
+  __shared__ int cs[L], types[L], nd_col[L], qpos[L], df_col[L], tmp_c[L], cand[L], rot_p[L], rot_n[L], org[L], pos[L];
+  __shared__ LeafMerge mg[L / 2];
+  const LeafDesc leaf = lf[blockIdx.x];
+  const int m = leaf.size, st = leaf.start, tid = threadIdx.x, g = tid >> 4, l = tid & 15;
+  const int lane = tid & 63, wave = tid >> 6;
+  // the votes of this row of lanes
+  auto votes = [&](bool p) { return (unsigned)(__ballot(p) >> (16 * (g & 3))) & 0xffffu; };
+  const unsigned below = (1u << l) - 1u;
+  if (tid < m) {
+    d[tid] = D[st + tid];
+    e[tid] = tid < m - 1 ? E[st + tid] : 0.0;
+  }
+  if (g < m) V[g][l] = (g == l) ? 1.0 : 0.0;
+  __syncthreads();
+  for (int depth = 3; depth >= 0; depth--) {
+    if ((m + (1 << depth) - 1) >> depth < 2) continue;  // no node of this depth has two rows
+    // ---- node g of this depth: sort and deflation
+    if (g < (1 << depth)) {
+      int off = 0, N = m;
+      for (int b = depth - 1; b >= 0; b--) {
+        const int n1 = N / 2;
+        if ((g >> b) & 1) {
+          off += n1;
+          N -= n1;
+        } else {
+          N = n1;
+        }
+      }
+      LeafMerge o;
+      o.off = off;
+      o.n1 = N / 2;
+      o.n2 = N - o.n1;
+      o.K = o.K1 = o.K2 = o.ndefl = 0;
+      o.rho2 = o.zsum = 0.0;
+      if (N >= 2) {
+        const double es = e[off + o.n1 - 1];
+        const double rho = 2.0 * fabs(es);
+        o.rho2 = rho;
+        if (l < N) {
+          // every place holds a column also where a NaN leaves one out below
+          ds[off + l] = d[off + l];
+          zs[off + l] = 0.0;
+          cs[off + l] = l;
+          lds_order();
+          const double dv = d[off + l];
+          double z;
+          int at = 0;
+          if (l < o.n1) {
+            z = V[off + l][off + o.n1 - 1];
+            for (int i = 0; i < o.n2; i++) at += d[off + o.n1 + i] < dv ? 1 : 0;
+            at += l;
+          } else {
+            z = ((es >= 0.0) ? 1.0 : -1.0) * V[off + l][off + o.n1];
+            for (int i = 0; i < o.n1; i++) at += d[off + i] <= dv ? 1 : 0;
+            at += l - o.n1;
+          }
+          ds[off + at] = dv;
+          zs[off + at] = z * 0.70710678118654752440;
+          cs[off + at] = l;
+          types[off + l] = (l < o.n1) ? 1 : 3;
+        }
+        lds_order();
+        const double dl = l < N ? ds[off + l] : 0.0, zl = l < N ? zs[off + l] : 0.0;
+        const double dmax = row_max16(fabs(dl)), zmax = row_max16(fabs(zl));
+        const double eps = DBL_EPSILON * 0.5;
+        const double tol = 8.0 * eps * fmax(dmax, zmax);
+        const bool zd = l < N && (rho * zmax <= tol || rho * fabs(zl) <= tol), cd = l < N && !zd;
+        const unsigned mz = votes(zd), mc = votes(cd);
+        const int nzd = __popc(mz), nc = __popc(mc);
+        if (zd) {
+          df_d[off + __popc(mz & below)] = dl;
+          df_col[off + __popc(mz & below)] = cs[off + l];
+        }
+        if (cd) cand[off + __popc(mc & below)] = l;
+        lds_order();
+        // pairs of neighbours in order: all before the first rotation, the
+        // rotation, the rest after it
+        int K = 0, nrot = 0, pj = nc > 0 ? cand[off] : -1, k = 1;
+        while (k < nc) {
+          const int nvalid = nc - k;
+          const bool valid = l < nvalid;
+          const int j = valid ? cand[off + k + l] : 0;
+          const int prv = (l == 0) ? pj : (valid ? cand[off + k + l - 1] : 0);
+          bool rot = false;
+          double c = 0.0, sn = 0.0, ta = 0.0;
+          if (valid) {
+            sn = zs[off + prv];
+            c = zs[off + j];
+            ta = hypot(c, sn);
+            const double t = ds[off + j] - ds[off + prv];
+            c /= ta;
+            sn = -sn / ta;
+            rot = fabs(t * c * sn) <= tol;
+          }
+          const unsigned mask = votes(rot);
+          const int first = mask ? __ffs((int)mask) - 1 : nvalid;
+          if (l < first) {
+            nd_d[off + K + l] = ds[off + prv];
+            nd_z[off + K + l] = zs[off + prv];
+            nd_col[off + K + l] = cs[off + prv];
+          }
+          K += first;
+          if (first < nvalid) {
+            if (l == first) {
+              zs[off + j] = ta;
+              zs[off + prv] = 0.0;
+              const int cp = cs[off + prv], cn = cs[off + j];
+              if (types[off + cp] != types[off + cn]) types[off + cn] = 2;
+              types[off + cp] = 4;
+              rot_p[off + nrot] = cp;
+              rot_n[off + nrot] = cn;
+              rot_c[off + nrot] = c;
+              rot_s[off + nrot] = sn;
+              const double tt = ds[off + prv] * c * c + ds[off + j] * sn * sn;
+              ds[off + j] = ds[off + prv] * sn * sn + ds[off + j] * c * c;
+              ds[off + prv] = tt;
+              df_d[off + nzd + nrot] = tt;
+              df_col[off + nzd + nrot] = cp;
+            }
+            nrot++;
+            pj = __shfl(j, first, 16);
+            k += first + 1;
+            lds_order();
+          } else {
+            pj = __shfl(j, nvalid - 1, 16);
+            k = nc;
+          }
+        }
+        if (pj >= 0) {
+          if (l == 0) {
+            nd_d[off + K] = ds[off + pj];
+            nd_z[off + K] = zs[off + pj];
+            nd_col[off + K] = cs[off + pj];
+          }
+          K++;
+        }
+        lds_order();
+        const int nd = nzd + nrot;
+        if (nrot > 0) {
+          // the rotations on the vectors' columns, one row per lane
+          if (l < N)
+            for (int t = 0; t < nrot; t++) {
+              const double x = V[off + rot_p[off + t]][off + l], y = V[off + rot_n[off + t]][off + l];
+              const double c = rot_c[off + t], s = rot_s[off + t];
+              V[off + rot_p[off + t]][off + l] = c * x + s * y;
+              V[off + rot_n[off + t]][off + l] = c * y - s * x;
+            }
+          // deflated list ascending: the rotated entries among themselves, then
+          // merged with the z-deflated run (ties keep the run first)
+          if (l < nd) {
+            const double v = df_d[off + l];
+            int at = 0;
+            tmp_d[off + l] = v;
+            tmp_c[off + l] = df_col[off + l];
+            lds_order();
+            if (l < nzd) {
+              at = l;
+              for (int i = nzd; i < nd; i++) at += df_d[off + i] < v ? 1 : 0;
+            } else {
+              for (int i = 0; i < nzd; i++) at += df_d[off + i] <= v ? 1 : 0;
+              for (int i = nzd; i < nd; i++)
+                at += (df_d[off + i] < v || (df_d[off + i] == v && i < l)) ? 1 : 0;
+            }
+            tmp_d[off + at] = v;
+            tmp_c[off + at] = df_col[off + l];
+          }
+          lds_order();
+          if (l < nd) {
+            df_d[off + l] = tmp_d[off + l];
+            df_col[off + l] = tmp_c[off + l];
+          }
+        }
+        // types, positions by type, sum of the squares in order
+        const int ty = l < K ? types[off + nd_col[off + l]] : 0;
+        const unsigned m1 = votes(ty == 1), m2 = votes(ty == 2), m3 = votes(ty == 3);
+        o.K = K;
+        o.K1 = __popc(m1);
+        o.K2 = __popc(m2);
+        o.ndefl = nd;
+        if (l < K) {
+          qpos[off + l] = (ty == 1)   ? __popc(m1 & below)
+                          : (ty == 2) ? o.K1 + __popc(m2 & below)
+                                      : o.K1 + o.K2 + __popc(m3 & below);
+          sq[off + l] = nd_z[off + l] * nd_z[off + l];
+        }
+        lds_order();
+        for (int i = 0; i < K; i++) o.zsum += sq[off + i];
+      }
+      if (l == 0) mg[g] = o;
+    }
+    __syncthreads();
+    // ---- position g: its node, its column, its root
+    int node = 0, off = 0, N = m;
+    for (int b = 0; b < depth; b++) {
+      const int n1 = N / 2, right = g - off >= n1 ? 1 : 0;
+      node = 2 * node + right;
+      off += right ? n1 : 0;
+      N = right ? N - n1 : n1;
+    }
+    const bool on = g < m && N >= 2;
+    const LeafMerge o = mg[node];
+    const int i = g - off, K = o.K;
+    if (on) {
+      const int src = i < K ? nd_col[off + i] : df_col[off + i - K], dst = i < K ? qpos[off + i] : i;
+      if (l < N) Q[off + dst][off + l] = V[off + src][off + l];
+      if (i < K) {
+        int og;
+        double t;
+        const bool conv = secular_root<16>(nd_d + off, nd_z + off, K, i, o.rho2, o.zsum, l, og, t);
+        if (l == 0) {
+          if (!conv) atomicOr(err, (unsigned)EVD_E_NOCONVERGE);
+          org[g] = og;
+          tau[g] = t;
+          lam[g] = nd_d[off + og] + t;
+        }
+      }
+    }
+    __syncthreads();
+    if (on && i < K) {
+      const double dj = nd_d[off + i];
+      if (l < K) {
+        const double lk = (nd_d[off + org[off + l]] - dj) + tau[off + l];
+        quot[g][l] = lk / (l == i ? o.rho2 : nd_d[off + l] - dj);
+      }
+      lds_order();
+      double prod = quot[g][i];
+      for (int k = 0; k < K; k++)
+        if (k != i) prod *= quot[g][k];
+      const double zh = sqrt(fabs(prod));
+      if (l == 0) zhat[g] = (nd_z[g] >= 0.0) ? zh : -zh;
+    }
+    __syncthreads();
+    if (on) {
+      int at = i < K ? i : i - K;
+      if (i < K) {
+        const double dorg = nd_d[off + org[g]], ti = tau[g];
+        const double v = l < K ? zhat[off + l] / ((nd_d[off + l] - dorg) - ti) : 0.0;
+        // the square rounded by itself, as where it is added to a sum of zero
+        const double inv = 1.0 / sqrt(row_sum16(__builtin_fma(v, v, 0.0)));
+        if (l < K) U[g][qpos[off + l]] = v * inv;
+        for (int u = 0; u < o.ndefl; u++) at += df_d[off + u] < lam[g] ? 1 : 0;
+      } else {
+        for (int u = 0; u < K; u++) at += lam[off + u] <= df_d[g - K] ? 1 : 0;
+      }
+      if (l == 0) {
+        pos[g] = off + at;
+        d[off + at] = i < K ? lam[g] : df_d[g - K];
+      }
+    }
+    __syncthreads();
+    // ---- vectors: columns that deflated keep theirs, the others are products
+    // with the rows of each child
+    if (on && i >= K && l < N) V[pos[g]][off + l] = Q[g][off + l];
+    for (int t = wave; t < (2 << depth); t += 4) {
+      const LeafMerge p = mg[t >> 1];
+      if (p.K == 0) continue;
+      const int r0 = p.off + ((t & 1) ? p.n1 : 0), nr = (t & 1) ? p.n2 : p.n1;
+      const int k0 = (t & 1) ? p.K1 : 0, nk = (t & 1) ? p.K - p.K1 : p.K1 + p.K2;
+      const int r = lane & 15;
+      f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+      for (int ks = 0; ks < nk; ks += 4) {
+        const int k = ks + (lane >> 4);
+        const double a = (k < nk && r < nr) ? Q[p.off + k0 + k][r0 + r] : 0.0;
+        const double b = (k < nk && r < p.K) ? U[p.off + r][k0 + k] : 0.0;
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(b, a, acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int c = 0; c < 4; c++) {
+        const int col = (lane >> 4) + 4 * c;
+        if (r < nr && col < p.K) V[pos[p.off + col]][r0 + r] = acc[c];
+      }
+    }
+    __syncthreads();
+  }
+  if (tid < m) D[st + tid] = d[tid];
+  if (rows.first) {
+    if (tid < m) {
+      rows.first[st + tid] = V[tid][0];
+      rows.last[st + tid] = V[tid][m - 1];
+    }
+    return;
+  }
+  double *Zb = Z + ((long)leaf.problem * zmul + st + (long)st * ldz);
+  if (g < m && l < m) Zb[l + (long)g * ldz] = V[g][l];
+}
+
 struct TreeNode {
   int start, size, left, right, height;
 };
@@ -1030,7 +1288,7 @@ size_t stedc_values_workspace(int count, long n) {
 size_t stedc_workspace(long n) { return dc_per_problem(n) + align256(dc_lib_temp_words(n) * sizeof(double)) + (1 << 16); }
 
 // Merge plan of order n, built once per context: the tree (halving splits
-// down to leaves), merges grouped by height, the split flags and the
+// down to leaves), merges grouped by height, the leaves and the
 // per-level tile offsets of the grouped GEMMs, copied to device memory that
 // lives as long as the context.  Only the split values (rho, sign) change per
 // solve; dc_rho_kernel writes them into the device descriptors.
@@ -1087,17 +1345,12 @@ int dc_plan(evd_ctx *ctx, long n, int count, const DcPlan **out) {
   }
   plan.level_off[H + 1] = (int)all.size();
   plan.nmerge = (int)all.size();
-  const long nt = n * count;
-  std::vector<int> split(nt, 0);
-  for (const MergeDesc &m : all) split[m.start + m.n1] = 1;
-  const size_t b_md = align256(sizeof(MergeDesc) * all.size()), b_split = align256(sizeof(int) * nt),
-               b_tiles = align256(sizeof(int) * tiles.size());
+  const size_t b_md = align256(sizeof(MergeDesc) * all.size()), b_tiles = align256(sizeof(int) * tiles.size());
   std::vector<char> &host = plan.host;
-  host.assign(b_md + b_split + b_tiles + sizeof(LeafDesc) * leaves.size(), 0);
+  host.assign(b_md + b_tiles + sizeof(LeafDesc) * leaves.size(), 0);
   if (!all.empty()) memcpy(host.data(), all.data(), sizeof(MergeDesc) * all.size());
-  memcpy(host.data() + b_md, split.data(), sizeof(int) * nt);
-  if (!tiles.empty()) memcpy(host.data() + b_md + b_split, tiles.data(), sizeof(int) * tiles.size());
-  memcpy(host.data() + b_md + b_split + b_tiles, leaves.data(), sizeof(LeafDesc) * leaves.size());
+  if (!tiles.empty()) memcpy(host.data() + b_md, tiles.data(), sizeof(int) * tiles.size());
+  memcpy(host.data() + b_md + b_tiles, leaves.data(), sizeof(LeafDesc) * leaves.size());
   // device copy: carved from the context's plan pool (one allocation for all
   // plans), else an allocation of its own; the upload is stream-ordered and
   // its source stays alive with the plan
@@ -1222,9 +1475,7 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
   const int nmerge = plan->nmerge, H = plan->H;
   char *pdev = static_cast<char *>(plan->dev);
   MergeDesc *dmd = reinterpret_cast<MergeDesc *>(pdev);
-  const int *dsplit = reinterpret_cast<const int *>(pdev + align256(sizeof(MergeDesc) * nmerge));
-  const int *dtiles = reinterpret_cast<const int *>(pdev + align256(sizeof(MergeDesc) * nmerge) +
-                                                    align256(sizeof(int) * nt));
+  const int *dtiles = reinterpret_cast<const int *>(pdev + align256(sizeof(MergeDesc) * nmerge));
   const LeafDesc *dleaf = reinterpret_cast<const LeafDesc *>(reinterpret_cast<const char *>(dtiles) +
                                                              align256(sizeof(int) * 2 * nmerge));
   MergeOut *dmo = static_cast<MergeOut *>(arena_alloc(ctx, sizeof(MergeOut) * std::max(1, nmerge)));
@@ -1242,10 +1493,10 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
   // split values and signs, tearing of every split, then the leaves
   dc_normalize_kernel<<<(unsigned)count, 256, 0, ctx->stream>>>(n, D, E, nrm);
   EVD_LAUNCHED(ctx);
+  dc_tear_kernel<<<(unsigned)std::min<long>((nt + 255) / 256, 1024), 256, 0, ctx->stream>>>(n, nt, E, D);
+  EVD_LAUNCHED(ctx);
   if (nmerge > 0) {
     dc_rho_kernel<<<(unsigned)std::min((nmerge + 255) / 256, 1024), 256, 0, ctx->stream>>>(nmerge, dmd, E);
-    EVD_LAUNCHED(ctx);
-    dc_tear_kernel<<<(unsigned)std::min<long>((nt + 255) / 256, 1024), 256, 0, ctx->stream>>>(nt, dsplit, E, D);
     EVD_LAUNCHED(ctx);
     // outside the leaves' diagonal blocks Z starts as zeros
     if (vec && zs == n * ldz)
@@ -1253,7 +1504,7 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
     else
       for (int q = 0; vec && q < count; q++) EVD_TRY(fill_f64(ctx, Z + q * zs, n, n, ldz, 0.0));
   }
-  dc_leaf_kernel<<<(unsigned)plan->nleaf, 64, 0, ctx->stream>>>(dleaf, E, D, Z, ldz, sc.zmul, rows, err);
+  dc_leaf_kernel<<<(unsigned)plan->nleaf, 256, 0, ctx->stream>>>(dleaf, E, D, Z, ldz, sc.zmul, rows, err);
   EVD_LAUNCHED(ctx);
 
   // Merges level by level (by height).  Launch shapes come from the largest
@@ -1287,7 +1538,8 @@ int stedc_batched(evd_ctx *ctx, int count, long n, double *D, double *E, double 
     dc_secular_kernel<<<dim3(gw, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc, err);
     EVD_LAUNCHED(ctx);
     if (vec || h < H) {  // the last merge's vectors are not needed for the values
-      dc_loewner_kernel<<<dim3(gw, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc);
+      const unsigned gl = (unsigned)std::min(16384, (maxN + 4 * kLoewnerJ - 1) / (4 * kLoewnerJ));
+      dc_loewner_kernel<<<dim3(gl, nm), 256, 0, ctx->stream>>>(lmd, lmo, sc);
       EVD_LAUNCHED(ctx);
     }
     if (!vec) {
