@@ -65,37 +65,71 @@ __device__ __attribute__((always_inline)) inline double wave_total(double v) {
   return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
 }
 
+// v of lane ^ 32.  v_permlane32_swap exchanges one half of its destination
+// with the other half of its source; with both operands v, one result holds
+// this lane's own value and the other the partner's, so xor-ing out the own
+// value leaves the partner's whichever half was exchanged.
+__device__ __attribute__((always_inline)) inline double half_swap(double v) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)x, hi = (unsigned)(x >> 32);
+  const auto rl = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto rh = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  const unsigned plo = rl[0] ^ rl[1] ^ lo, phi = rh[0] ^ rh[1] ^ hi;
+  return __builtin_bit_cast(double, ((unsigned long long)phi << 32) | plo);
+}
+
+// v of lane ^ 16 (v_permlane16_swap exchanges odd rows of its destination with
+// even rows of its source)
+__device__ __attribute__((always_inline)) inline double row_swap(double v) {
+  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+  const unsigned lo = (unsigned)x, hi = (unsigned)(x >> 32);
+  const auto rl = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto rh = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  const unsigned plo = rl[0] ^ rl[1] ^ lo, phi = rh[0] ^ rh[1] ^ hi;
+  return __builtin_bit_cast(double, ((unsigned long long)phi << 32) | plo);
+}
+
+// wave_sum's butterfly (lane ^ 32, 16, 8, 4, 2, 1), bit for bit, by swaps of
+// half waves and rows and by DPP
+__device__ __attribute__((always_inline)) inline double wave_butterfly(double v) {
+  v += half_swap(v);
+  v += row_swap(v);
+  return row_sum16(v);
+}
+
 // sum over aligned groups of W lanes (4 or 8), returned in every lane of the
-// group: each step adds the other half of a group whose halves already agree,
-// so the mirror serves as an exchange
+// group, by lane ^ 4, 2, 1 in this order (a mirrored half row of reversed quads
+// is lane ^ 4)
 template <int W>
 __device__ __attribute__((always_inline)) inline double group_sum(double v) {
   static_assert(W == 4 || W == 8, "lanes of a window row");
-  v += dpp_f64<0xb1, 0xf>(v);                // quad_perm [1, 0, 3, 2]
-  v += dpp_f64<0x4e, 0xf>(v);                // quad_perm [2, 3, 0, 1]
-  if (W == 8) v += dpp_f64<0x141, 0xf>(v);   // row_half_mirror
+  if (W == 8) v += dpp_f64<0x141, 0xf>(dpp_f64<0x1b, 0xf>(v));
+  v += dpp_f64<0x4e, 0xf>(v);  // quad_perm [2, 3, 0, 1]
+  v += dpp_f64<0xb1, 0xf>(v);  // quad_perm [1, 0, 3, 2]
   return v;
 }
 
 // LAPACK-style reflector of the chase (reference sign convention): from the
 // column x = Bc[0..lenx) (LDS, stride LD), u = (x/||x|| + sign(x0) e1) /
 // sqrt(|x0/||x|| + sign(x0)|), ||u||^2 = 2, H x = beta e1.  Wave 0 only.  It
-// sits in the chain of the steps: sums by DPP instead of shuffles through LDS
-// and refined reciprocal roots instead of two roots and two divisions (with the
-// same sums in the step, n = 6000, b = 32: 49.3 -> 44.0 ms).
+// sits in the chain of the steps: sums by swaps and DPP instead of shuffles
+// through LDS, and short chains for two roots and two reciprocals (with the same
+// sums in the step, n = 6000, b = 32: 49.3 -> 45.8 ms).  All have the bits of the
+// plain forms: a last bit of T decides which entries the tridiagonal solver
+// deflates, and so now and then the sign of a vector.
 template <int BW>
 __device__ inline void chase_reflector(const double *Bc, int lenx, int lane, double *u, double *s_beta, float *U,
                                        long urow, long ucol) {
   constexpr int LD = BW + 1;
   const double x = (lane < lenx) ? Bc[lane * LD] : 0.0;
-  const double nn = wave_total(x * x);
+  const double nn = wave_butterfly(x * x);
   const double x0 = Bc[0];
   double uu = 0.0, nrm = 0.0;
   if (nn > 0.0) {
     double inv, scl, root;
-    rsqrt_sqrt(nn, inv, nrm);
+    sqrt_and_recip(nn, nrm, inv);
     const double u0 = x0 * inv + (x0 >= 0.0 ? 1.0 : -1.0);
-    rsqrt_sqrt(fabs(u0), scl, root);
+    sqrt_and_recip(fabs(u0), root, scl);
     uu = (lane == 0 ? u0 : x * inv) * scl;
   }
   if (lane < BW) u[lane] = (lane < lenx) ? uu : 0.0;
@@ -224,7 +258,7 @@ __global__ __launch_bounds__(256, BW == 32 ? 4 : 1) void chase_kernel(int n, int
       }
       __syncthreads();
       // ---- S <- H S H (rank-2 with w = y - (u^T y / 2) u), N <- N H
-      const double psi = wave_total((lane < BW) ? u[lane] * yv[lane] : 0.0);
+      const double psi = wave_butterfly((lane < BW) ? u[lane] * yv[lane] : 0.0);
       const double ui = u[ri], wi = yv[ri] - 0.5 * psi * ui, qi = qv[ri];
 #pragma unroll
       for (int r = 0; r < EPT; r++) {
@@ -328,19 +362,6 @@ __device__ inline int sweep_nsteps(int n, int b, int s) {
     len = len2;
     k++;
   }
-}
-
-// v of lane ^ 32.  v_permlane32_swap exchanges one half of its destination
-// with the other half of its source; with both operands v, one result holds
-// this lane's own value and the other the partner's, so xor-ing out the own
-// value leaves the partner's whichever half was exchanged.
-__device__ __attribute__((always_inline)) inline double half_swap(double v) {
-  const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)x, hi = (unsigned)(x >> 32);
-  const auto rl = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
-  const auto rh = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
-  const unsigned plo = rl[0] ^ rl[1] ^ lo, phi = rh[0] ^ rh[1] ^ hi;
-  return __builtin_bit_cast(double, ((unsigned long long)phi << 32) | plo);
 }
 
 // reflector of the chase's convention from x (lane < lenx, zero elsewhere),

@@ -291,20 +291,30 @@ __device__ __attribute__((always_inline)) inline double row_max16(double v) {
   return v;
 }
 
-// 1 / sqrt(x) and sqrt(x) for x > 0: the hardware estimate refined by two
-// coupled Newton steps (Goldschmidt's iteration), the root corrected once more
-// by its residual.  One short chain instead of a square root and a division.
-__device__ __attribute__((always_inline)) inline void rsqrt_sqrt(double x, double &inv, double &root) {
+// root = sqrt(x) and inv = 1 / root for x > 0, both as the IEEE operations round
+// them: where no step can leave the normal range, Goldschmidt's iteration from the
+// hardware estimate, two corrections of the root by its residual, and two of
+// the reciprocal (Markstein 1990: a correction by fma of a value within an ulp is
+// the rounded reciprocal, but for a significand of all ones).  One short chain
+// instead of a square root and a division.
+__device__ __attribute__((always_inline)) inline void sqrt_and_recip(double x, double &root, double &inv) {
+  if (x < 0x1p-700 || x > 0x1p700) {
+    root = sqrt(x);
+    inv = 1.0 / root;
+    return;
+  }
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
-  double r = __builtin_fma(-g, h, 0.5);
+  const double r = __builtin_fma(-h, g, 0.5);
   g = __builtin_fma(g, r, g);
   h = __builtin_fma(h, r, h);
-  r = __builtin_fma(-g, h, 0.5);
-  g = __builtin_fma(g, r, g);
-  h = __builtin_fma(h, r, h);
-  root = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-  inv = 2.0 * h;
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  double v = 2.0 * h;
+  v = __builtin_fma(__builtin_fma(-g, v, 1.0), v, v);
+  v = __builtin_fma(__builtin_fma(-g, v, 1.0), v, v);
+  root = g;
+  inv = v;
 }
 
 __device__ inline float wave_sum(float v) {
