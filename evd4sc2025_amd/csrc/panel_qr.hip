@@ -2,7 +2,7 @@
 // my_hou_kernel in the reference: api/panelQR.cu:20-246,
 // api/inc/TallShinnyQR.h:9-134, util/inc/kernelQR.h:215-414).
 //
-// Design (MI355X): one cooperative launch of G workgroups; workgroup g keeps
+// Design (MI355X): one launch of G workgroups (cooperative for G > 1); workgroup g keeps
 // rows [g*256*RPT, (g+1)*256*RPT) of the m x nb panel in registers as FP64 for
 // the whole factorisation (the panel is read once and written once).  Column
 // j needs sigma = ||x||^2 and p_c = x^T a_c for the trailing columns, x = the
@@ -392,9 +392,6 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
   }
 }
 
-// launches of the column-exchange kernel that may run on one card at once
-constexpr int kPanelLaunches = 16;
-
 template <int NB, int RPT, typename T>
 static int launch_panel(evd_ctx *ctx, long m, long nc, const T *A, long lda, T *Y, long ldy, T *W, long ldw, T *R,
                         long ldr, T *Aout, long ldo, double *tau_out, int count = 1, long s_in = 0, long s_y = 0,
@@ -419,16 +416,14 @@ static int launch_panel(evd_ctx *ctx, long m, long nc, const T *A, long lda, T *
   void *args[] = {&mi, &ni, (void *)&A, &lda, &Y, &ldy, &W, &ldw, &R, &ldr, &Aout, &ldo, &part, &tau_out,
                   &tags, &epoch_word, &err, &s_in, &s_y, &s_w, &s_out, (void *)&only_bad};
   // The groups of a launch wait for each other, so all of them have to become
-  // resident.  A cooperative launch sees to that, but goes through a queue of
-  // its own: 11 us before and 11 us after a kernel that, as the fallback of
-  // the Cholesky QR path, mostly has nothing to do.  A regular launch is as
-  // safe while all launches that can run at once fit together: every other
-  // kernel here ends by itself (the chase waits on running workgroups only), so
-  // groups that have to wait for room get it as long as these launches
-  // alone never fill the card.  HIP runs at most four kernels of a process at
-  // once (its hardware queues); 1/16 of the card leaves room for four
-  // processes that do: 32 groups, m <= 16384.  Larger panels stay cooperative.
-  if (G == 1 || (long)G * count <= maxres / kPanelLaunches)
+  // resident.  A cooperative launch sees to that: those of one process go through a
+  // queue of their own, one after another, and every other kernel ends by itself (the
+  // chase waits on running workgroups only), so the groups always get their room.
+  // A regular launch of waiting groups beside a cooperative one does not: each can
+  // hold a part of the card that the other waits for.  One workgroup waits for
+  // nobody: a regular launch, which may overlap with the work of other streams and
+  // saves the way through the other queue (11 us before and 11 us after it).
+  if (G == 1)
     EVD_HIP(ctx, hipLaunchKernel((const void *)panel_qr_kernel<NB, RPT, T>, dim3(G, count), dim3(256), args, 0,
                                  ctx->stream));
   else
