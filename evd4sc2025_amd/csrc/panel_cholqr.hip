@@ -622,8 +622,9 @@ __global__ __launch_bounds__(256) void cq_out_kernel(int m, int nc, const T *__r
 #pragma unroll
   for (int k = 0; k < 8; k++) {
     const int c = 8 * w + k;
-    if (top) xs[lane * kLD + c] = v1[k];
-    const double v = top ? v1[k] : xs[lane * kLD + c];
+    // (values, not a choice of addresses, which would keep v1 in private memory)
+    const double own = xs[lane * kLD + c], first = v1[k], v = top ? first : own;
+    if (top) xs[lane * kLD + c] = first;
     if (rin && c < nc && Y) Y[r + (long)c * ldy] = (T)v;
   }
   __syncthreads();
