@@ -33,6 +33,7 @@ struct Tuning {
   int gemm_tile = 0;       // output tile of the large FP32 products (0 = auto, 1 = 128 x 128, 2 = 64 x 64)
   int own_gemm = 0;        // 1: large plain FP32 products on this library's MFMA kernels, not rocBLAS
   int panel_exchange = 0;  // 1: panels on the column-exchange kernel only (no Cholesky QR path)
+  int panel_alone = 0;     // 1: flagged panels by one workgroup, as if the others had found no room
 };
 
 // Merge plan of the tridiagonal divide and conquer for one order n (host

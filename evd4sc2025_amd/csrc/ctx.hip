@@ -350,7 +350,7 @@ int evd_ctx_set_knob(evd_ctx *ctx, const char *name, int value) {
                {"bc_valu", &ctx->tune.bc_valu, 0, 1},           {"skinny_split", &ctx->tune.skinny_split, 0, 4},
                {"chase_depth", &ctx->tune.chase_depth, 0, 6},   {"panel_rows", &ctx->tune.panel_rows, 0, 512},
                {"gemm_tile", &ctx->tune.gemm_tile, 0, 2},       {"own_gemm", &ctx->tune.own_gemm, 0, 1},
-               {"panel_exchange", &ctx->tune.panel_exchange, 0, 1}};
+               {"panel_exchange", &ctx->tune.panel_exchange, 0, 1}, {"panel_alone", &ctx->tune.panel_alone, 0, 1}};
   for (auto &kb : knobs)
     if (!strcmp(kb.name, name)) {
       if (value < kb.lo || value > kb.hi) return -3;

@@ -536,8 +536,9 @@ template <int MODE, typename T>
 __global__ __launch_bounds__(256) void cq_pass_kernel(int m, int nc, const T *__restrict__ A, long lda, long s_in,
                                                       double *__restrict__ fac, double *__restrict__ part,
                                                       long s_part, unsigned *__restrict__ cnt,
-                                                      int *__restrict__ state, double one_pass_max) {
+                                                      int *__restrict__ state, long gate, double one_pass_max) {
   const int g = blockIdx.x, q = blockIdx.y, ng = gridDim.x, tid = threadIdx.x;
+  if (MODE == 0 && g == 0 && tid == 0) state[gate + q] = 0;  // the fallback's gate opens
   const int ngroups = (ng + kGroup - 1) / kGroup;
   if (MODE == 1 && state[q] != kNeedPass2) return;
   A += q * s_in;
@@ -650,7 +651,7 @@ __global__ __launch_bounds__(256) void cq_out_kernel(int m, int nc, const T *__r
 // Panels of `count` problems (A of problem q at q s_in, ...; R and tau only
 // for count = 1).  Returns 0 after enqueueing; the state words `bad` (count
 // ints, device) end as 1 for the problems the caller's fallback must factor
-// (and 2 for the others).
+// (and 2 for the others), the count ints after them, the fallback's gates, as 0.
 template <typename T>
 int panel_cholqr(evd_ctx *ctx, int count, long m, long nc, const T *A, long lda, long s_in, T *Y, long ldy, long s_y,
                  T *W, long ldw, long s_w, T *R, long ldr, T *Aout, long ldo, long s_out, double *tau_out,
@@ -676,10 +677,10 @@ int panel_cholqr(evd_ctx *ctx, int count, long m, long nc, const T *A, long lda,
     T *Yq = Y + q0 * s_y, *Wq = W + q0 * s_w, *Oq = Aout ? Aout + q0 * s_out : nullptr;
     int *st = bad + q0;
     const dim3 rows_grid((unsigned)ng, (unsigned)cq), out_grid((unsigned)((m + kOut - 1) / kOut), (unsigned)cq);
-    cq_pass_kernel<0, T><<<rows_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, part, s_part, cnt, st,
+    cq_pass_kernel<0, T><<<rows_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, part, s_part, cnt, st, count,
                                                              one_pass_max);
     EVD_LAUNCHED(ctx);
-    cq_pass_kernel<1, T><<<rows_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, part, s_part, cnt, st,
+    cq_pass_kernel<1, T><<<rows_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, part, s_part, cnt, st, count,
                                                              one_pass_max);
     EVD_LAUNCHED(ctx);
     cq_out_kernel<T><<<out_grid, 256, 0, ctx->stream>>>(mi, ni, Aq, lda, s_in, fac, Yq, ldy, s_y, Wq, ldw, s_w, Oq,

@@ -2,7 +2,7 @@
 // my_hou_kernel in the reference: api/panelQR.cu:20-246,
 // api/inc/TallShinnyQR.h:9-134, util/inc/kernelQR.h:215-414).
 //
-// Design (MI355X): one launch of G workgroups (cooperative for G > 1); workgroup g keeps
+// Design (MI355X): one launch of G workgroups (see launch_panel for its kind); workgroup g keeps
 // rows [g*256*RPT, (g+1)*256*RPT) of the m x nb panel in registers as FP64 for
 // the whole factorisation (the panel is read once and written once).  Column
 // j needs sigma = ||x||^2 and p_c = x^T a_c for the trailing columns, x = the
@@ -54,6 +54,108 @@ constexpr unsigned long long panel_sentinel(unsigned epoch, int step) {
          (unsigned long long)((unsigned)step & 0xFFFFFFu);
 }
 
+// LAPACK dlarfg from the pivot alpha and sigma = ||x below it||^2
+__device__ inline void panel_reflector(double alpha, double sigma, double &beta, double &tau, double &scale) {
+  if (sigma == 0.0) {
+    beta = alpha;
+    tau = 0.0;
+    scale = 0.0;
+  } else {
+    const double nrm = sqrt(alpha * alpha + sigma);
+    beta = alpha >= 0.0 ? -nrm : nrm;
+    tau = (beta - alpha) / beta;
+    scale = 1.0 / (alpha - beta);
+  }
+}
+
+// T by the dlarft forward/columnwise recurrence, one row per thread:
+// T[i][j] = -tau_j sum_{l=i}^{j-1} T[i][l] (v_l^T v_j)
+template <int NB>
+__device__ inline void panel_t_factor(int k, int tid, const double *taus, const double (*gram)[NB + 1],
+                                      double (*Tt)[NB + 1]) {
+  if (tid < k) {
+    const int i = tid;
+    Tt[i][i] = taus[i];
+    for (int jj = i + 1; jj < k; jj++) {
+      double s = 0.0;
+      for (int l = i; l < jj; l++) s += Tt[l][i] * gram[l][jj];
+      Tt[jj][i] = -taus[jj] * s;
+    }
+  }
+}
+
+// Outputs of a thread's rows (columns in natural order): R / [R; 0], then a[]
+// becomes V in place, Y = V, W = V T
+template <int NB, int RPT, typename T>
+__device__ inline void panel_outputs(int m, int nc, int k, const long (&rowv)[RPT], double (&a)[RPT][NB],
+                                     const double (*Tt)[NB + 1], T *__restrict__ R, long ldr, T *__restrict__ Aout,
+                                     long ldo, T *__restrict__ Y, long ldy, T *__restrict__ W, long ldw) {
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const long r = rowv[q];
+    if (r < m) {
+#pragma unroll
+      for (int c = 0; c < NB; c++) {
+        if (c >= nc) continue;
+        const double rv = (r <= c) ? a[q][c] : 0.0;
+        if (R && r < nc) R[r + (long)c * ldr] = (T)rv;
+        if (Aout) Aout[r + (long)c * ldo] = (T)rv;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < NB; c++) a[q][c] = (c < k) ? ((r > c) ? a[q][c] : (r == c ? 1.0 : 0.0)) : 0.0;
+    if (r < m && Y) {
+#pragma unroll
+      for (int c = 0; c < NB; c++)
+        if (c < nc) Y[r + (long)c * ldy] = (T)a[q][c];
+    }
+  }
+  if (W) {
+    for (int c = 0; c < nc; c++) {
+#pragma unroll
+      for (int q = 0; q < RPT; q++) {
+        const long r = rowv[q];
+        double w = 0.0;
+#pragma unroll
+        for (int l = 0; l < NB; l++) w += a[q][l] * Tt[c][l];
+        if (r < m) W[r + (long)c * ldw] = (T)w;
+      }
+    }
+  }
+}
+
+// How the groups of a regular launch come together.  They may wait for each other
+// only once all of them run: each counts itself into the problem's gate word and
+// polls it; when not all have come within kGatherTicks a group, one of them closes the gate
+// (the count cannot be complete then), every other one leaves, also those that come
+// later, and that one factors the panel alone.  So no group waits for one that
+// has no room, whatever else is on the card, and all of these waits are bounded.
+enum : int { kLeave, kTogether, kAlone };
+constexpr unsigned kGateClosed = 0x80000000u;
+// of the 100 MHz clock: half a millisecond, what a group of 512 rows adds to the work
+// of one alone (m = 1024: 1.2 ms, 16384: 15.9 ms; together 0.2 ms), so waiting
+// at most doubles it
+constexpr unsigned long long kGatherTicks = 50000;
+
+__device__ inline int gather_groups(unsigned *gate, unsigned G, bool alone) {
+  const unsigned before = __hip_atomic_fetch_add(gate, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (alone) return before == 0 ? kAlone : kLeave;
+  if (before & kGateClosed) return kLeave;
+  const unsigned long long t0 = clock100();
+  while (true) {
+    unsigned w = ld_dev(gate);
+    if (w & kGateClosed) return kLeave;
+    if (w == G) return kTogether;
+    if (clock100() - t0 > kGatherTicks * G) {
+      if (__hip_atomic_compare_exchange_strong(gate, &w, w | kGateClosed, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT))
+        return kAlone;
+      continue;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
 // Register layout: every thread holds RPT rows of the panel, a[q][s], s a
 // rotating slot index.  At the start of step j, column j + s sits in slot s
 // for s < NB - j (the active columns; slot 0 is the pivot column) and
@@ -71,7 +173,8 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
                                                        double *__restrict__ tau_out, unsigned *__restrict__ tags,
                                                        unsigned *__restrict__ epoch_word, unsigned *__restrict__ err,
                                                        long s_in, long s_y, long s_w, long s_out,
-                                                       const int *__restrict__ only_bad) {
+                                                       const int *__restrict__ only_bad,
+                                                       unsigned *__restrict__ gate, int alone) {
   constexpr int CH = NB < 32 ? NB : 32;  // slots per in-wave reduction
   constexpr int PASSG = 32;              // group records gathered per pass
   static_assert(NB <= 256, "the pivot rows must live in group 0");
@@ -103,15 +206,6 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
   // (factored there) load nothing and leave after counting into the launch
   // epoch below
   const bool skip = only_bad && only_bad[blockIdx.y] != 1;
-  double a[RPT][NB];
-  long rowv[RPT];
-#pragma unroll
-  for (int q = 0; q < RPT; q++) {
-    const long r = (long)g * 256 * RPT + q * 256 + tid;
-    rowv[q] = r;
-#pragma unroll
-    for (int c = 0; c < NB; c++) a[q][c] = (!skip && r < m && c < nc) ? (double)Ain[r + (long)c * lda] : 0.0;
-  }
   for (int i = tid; i < NB * (NB + 1); i += 256) {
     (&gram[0][0])[i] = 0.0;
     (&Tt[0][0])[i] = 0.0;
@@ -140,6 +234,136 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
   const unsigned epoch = s_epoch;
   // (every group has counted itself into the epoch above, so the word advances)
   if (skip) return;
+  if (G > 1 && gate) {
+    if (tid == 0) s_ok = gather_groups(gate + blockIdx.y, (unsigned)G, alone != 0);
+    __syncthreads();
+    const int role = __builtin_amdgcn_readfirstlane(s_ok);
+    __syncthreads();
+    if (role == kLeave) return;
+    if (NB == 32 && role == kAlone) {
+      // ---- This group factors all rows: each thread takes its rows of group
+      // 0, 1, ... in turn, with the sums of the exchange in their order, so the
+      // bits are those of the groups together.  A step is one pass over the
+      // rows (the last reflector on them, then the sums); in between they are kept,
+      // as FP64, in the places of Y (and, for FP32 storage, of W for the low words).
+      auto keep = [&](long r, int c, double v) {
+        if constexpr (sizeof(T) == 8) {
+          Y[r + (long)c * ldy] = (T)v;
+        } else {
+          const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
+          Y[r + (long)c * ldy] = __builtin_bit_cast(float, (unsigned)(x >> 32));
+          W[r + (long)c * ldw] = __builtin_bit_cast(float, (unsigned)x);
+        }
+      };
+      auto kept = [&](long r, int c) -> double {
+        if constexpr (sizeof(T) == 8) {
+          return (double)Y[r + (long)c * ldy];
+        } else {
+          const unsigned hi = __builtin_bit_cast(unsigned, (float)Y[r + (long)c * ldy]);
+          const unsigned lo = __builtin_bit_cast(unsigned, (float)W[r + (long)c * ldw]);
+          return __builtin_bit_cast(double, ((unsigned long long)hi << 32) | lo);
+        }
+      };
+      // column c of row r before H_{j-1}
+      auto column = [&](long r, int j, int c) -> double {
+        return (r < m && c < nc) ? (j == 0 ? (double)Ain[r + (long)c * lda] : kept(r, c)) : 0.0;
+      };
+      // H_{j-1} at row r with its column j - 1 at x: the factor of the others and
+      // what becomes of that column
+      auto reflect = [&](long r, int j, double x, double &vv, double &fin) {
+        const double beta = sc[0], scale = sc[1];
+        vv = (r > j - 1) ? x * scale : (r == j - 1 ? 1.0 : 0.0);
+        fin = (r > j - 1) ? vv : (r == j - 1 ? beta : x);
+      };
+      constexpr int H = 16;  // columns at a time
+      for (int j = 0; j < k; j++) {
+        double tacc = 0.0;
+        for (int v = 0; v < G; v++) {
+          double vv[RPT], fin[RPT], xq[RPT];
+#pragma unroll
+          for (int q = 0; q < RPT; q++) {
+            const long r = (long)v * 256 * RPT + q * 256 + tid;
+            vv[q] = fin[q] = 0.0;
+            double x = column(r, j, j);
+            if (j > 0) {
+              reflect(r, j, column(r, j, j - 1), vv[q], fin[q]);
+              x = x - vv[q] * wv[j];
+            }
+            xq[q] = (r < m && r > j) ? x : 0.0;
+          }
+#pragma unroll 1
+          for (int h = 0; h < NB; h += H) {
+            double e[H];
+#pragma unroll
+            for (int c = 0; c < H; c++) e[c] = 0.0;
+#pragma unroll
+            for (int q = 0; q < RPT; q++) {
+              const long r = (long)v * 256 * RPT + q * 256 + tid;
+#pragma unroll
+              for (int cc = 0; cc < H; cc++) {
+                const int c = h + cc;
+                double x = column(r, j, c);
+                if (j > 0) x = (c == j - 1) ? fin[q] : x - vv[q] * wv[c];
+                if (r < m && c < nc) keep(r, c, x);
+                if (r == j) piv[c] = x;
+                e[cc] += xq[q] * x;
+              }
+            }
+            const double mine = wave_reduce_scatter<H>(e, lane);
+            if ((lane & (64 / H - 1)) == 0) red[wave][h + lane / (64 / H)] = mine;
+          }
+          __syncthreads();
+          if (tid < NB) {
+            // record v of a pass: partial sum v % 8, the eight in order at its end
+            constexpr int P = 256 / NB;
+            const int gg = v % PASSG;
+            const double rec1 = red[0][tid] + red[1][tid] + red[2][tid] + red[3][tid];
+            gsum[(gg % P) * NB + tid] = (gg < P ? 0.0 : gsum[(gg % P) * NB + tid]) + rec1;
+            if (gg == PASSG - 1 || v == G - 1)
+              for (int p = 0; p < min(P, gg + 1); p++) tacc += gsum[p * NB + tid];
+          }
+          __syncthreads();
+        }
+        if (tid < NB) tot[tid] = tacc;
+        __syncthreads();
+        if (tid < NB) {
+          const double alpha = piv[j], sigma = tot[j], ts = tot[tid];
+          double beta, tau, scale;
+          panel_reflector(alpha, sigma, beta, tau, scale);
+          wv[tid] = (tid > j) ? tau * (piv[tid] + scale * ts) : 0.0;
+          if (tid < j) gram[tid][j] = piv[tid] + scale * ts;
+          if (tid == j) {
+            sc[0] = beta;
+            sc[1] = scale;
+            taus[j] = tau;
+          }
+        }
+        __syncthreads();
+      }
+      panel_t_factor<NB>(k, tid, taus, gram, Tt);
+      if (tid < k && tau_out) tau_out[tid] = taus[tid];
+      __syncthreads();
+#pragma unroll 1
+      for (int v = 0; v < G * RPT; v++) {
+        const long r[1] = {(long)v * 256 + tid};
+        double x[1][NB], vv, fin;
+        reflect(r[0], k, column(r[0], k, k - 1), vv, fin);
+#pragma unroll
+        for (int c = 0; c < NB; c++) x[0][c] = (c == k - 1) ? fin : column(r[0], k, c) - vv * wv[c];
+        panel_outputs<NB, 1>(m, nc, k, r, x, Tt, R, ldr, Aout, ldo, Y, ldy, W, ldw);
+      }
+      return;
+    }
+  }
+  double a[RPT][NB];
+  long rowv[RPT];
+#pragma unroll
+  for (int q = 0; q < RPT; q++) {
+    const long r = (long)g * 256 * RPT + q * 256 + tid;
+    rowv[q] = r;
+#pragma unroll
+    for (int c = 0; c < NB; c++) a[q][c] = (r < m && c < nc) ? (double)Ain[r + (long)c * lda] : 0.0;
+  }
   if (G > 1) {
     // sentinels of steps 0 and 1 in this group's records, then a one-time
     // start barrier so nobody polls a slot before its owner marked it
@@ -299,16 +523,7 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
       }
       const double alpha = piv[0], sigma = t0;
       double beta, tau, scale;
-      if (sigma == 0.0) {
-        beta = alpha;
-        tau = 0.0;
-        scale = 0.0;
-      } else {
-        const double nrm = sqrt(alpha * alpha + sigma);
-        beta = alpha >= 0.0 ? -nrm : nrm;
-        tau = (beta - alpha) / beta;
-        scale = 1.0 / (alpha - beta);
-      }
+      panel_reflector(alpha, sigma, beta, tau, scale);
       wv[s] = (s >= 1 && s < nact) ? tau * (piv[s] + scale * ts) : 0.0;
       if (s >= nact) gram[s - nact][j] = piv[s] + scale * ts;
       if (s == 0) {
@@ -343,59 +558,17 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
   }
   __syncthreads();
 
-  // ---- T by the dlarft forward/columnwise recurrence, one row per thread:
-  // T[i][j] = -tau_j sum_{l=i}^{j-1} T[i][l] (v_l^T v_j)
-  if (tid < k) {
-    const int i = tid;
-    Tt[i][i] = taus[i];
-    for (int jj = i + 1; jj < k; jj++) {
-      double s = 0.0;
-      for (int l = i; l < jj; l++) s += Tt[l][i] * gram[l][jj];
-      Tt[jj][i] = -taus[jj] * s;
-    }
-    if (g == 0 && tau_out) tau_out[i] = taus[i];
-  }
+  panel_t_factor<NB>(k, tid, taus, gram, Tt);
+  if (tid < k && g == 0 && tau_out) tau_out[tid] = taus[tid];
   __syncthreads();
 
-  // ---- outputs: R / [R;0], then a[] becomes V in place, Y = V, W = V T
-#pragma unroll
-  for (int q = 0; q < RPT; q++) {
-    const long r = rowv[q];
-    if (r < m) {
-#pragma unroll
-      for (int c = 0; c < NB; c++) {
-        if (c >= nc) continue;
-        const double rv = (r <= c) ? a[q][c] : 0.0;
-        if (R && r < nc) R[r + (long)c * ldr] = (T)rv;
-        if (Aout) Aout[r + (long)c * ldo] = (T)rv;
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < NB; c++) a[q][c] = (c < k) ? ((r > c) ? a[q][c] : (r == c ? 1.0 : 0.0)) : 0.0;
-    if (r < m && Y) {
-#pragma unroll
-      for (int c = 0; c < NB; c++)
-        if (c < nc) Y[r + (long)c * ldy] = (T)a[q][c];
-    }
-  }
-  if (W) {
-    for (int c = 0; c < nc; c++) {
-#pragma unroll
-      for (int q = 0; q < RPT; q++) {
-        const long r = rowv[q];
-        double w = 0.0;
-#pragma unroll
-        for (int l = 0; l < NB; l++) w += a[q][l] * Tt[c][l];
-        if (r < m) W[r + (long)c * ldw] = (T)w;
-      }
-    }
-  }
+  panel_outputs<NB, RPT>(m, nc, k, rowv, a, Tt, R, ldr, Aout, ldo, Y, ldy, W, ldw);
 }
 
 template <int NB, int RPT, typename T>
 static int launch_panel(evd_ctx *ctx, long m, long nc, const T *A, long lda, T *Y, long ldy, T *W, long ldw, T *R,
                         long ldr, T *Aout, long ldo, double *tau_out, int count = 1, long s_in = 0, long s_y = 0,
-                        long s_w = 0, long s_out = 0, const int *only_bad = nullptr) {
+                        long s_w = 0, long s_out = 0, const int *only_bad = nullptr, unsigned *gate = nullptr) {
   const long rows_per = 256L * RPT;
   int G = (int)((m + rows_per - 1) / rows_per);
   if (count > 1 && (R || tau_out)) return set_error(ctx, EVD_E_UNSUPPORTED, "batched panels write no R / tau output");
@@ -412,18 +585,21 @@ static int launch_panel(evd_ctx *ctx, long m, long nc, const T *A, long lda, T *
   unsigned *tags = ctx->tags;
   unsigned *epoch_word = ctx->ctrl + kCtrlEpoch;
   unsigned *err = ctx->ctrl + kCtrlError;
-  int mi = (int)m, ni = (int)nc;
+  int mi = (int)m, ni = (int)nc, alone = ctx->tune.panel_alone;
+  if (!Y || !W) gate = nullptr;  // one group alone keeps its rows there
   void *args[] = {&mi, &ni, (void *)&A, &lda, &Y, &ldy, &W, &ldw, &R, &ldr, &Aout, &ldo, &part, &tau_out,
-                  &tags, &epoch_word, &err, &s_in, &s_y, &s_w, &s_out, (void *)&only_bad};
+                  &tags, &epoch_word, &err, &s_in, &s_y, &s_w, &s_out, (void *)&only_bad, &gate, &alone};
   // The groups of a launch wait for each other, so all of them have to become
   // resident.  A cooperative launch sees to that: those of one process go through a
   // queue of their own, one after another, and every other kernel ends by itself (the
   // chase waits on running workgroups only), so the groups always get their room.
   // A regular launch of waiting groups beside a cooperative one does not: each can
-  // hold a part of the card that the other waits for.  One workgroup waits for
-  // nobody: a regular launch, which may overlap with the work of other streams and
-  // saves the way through the other queue (11 us before and 11 us after it).
-  if (G == 1)
+  // hold a part of the card that the other waits for.  Regular are therefore one
+  // workgroup, which waits for nobody, and groups that come together at a gate, which
+  // wait for running ones only.  The gate is for the fallback of the Cholesky QR
+  // path, which mostly has nothing to do: the other queue costs 11 us before and 11
+  // us after it (values of n = 3001: 38.4 -> 35.8 ms, FP64 band of n = 1500: 6.9 -> 5.8).
+  if (G == 1 || gate)
     EVD_HIP(ctx, hipLaunchKernel((const void *)panel_qr_kernel<NB, RPT, T>, dim3(G, count), dim3(256), args, 0,
                                  ctx->stream));
   else
@@ -506,13 +682,15 @@ int panel_qr_t(evd_ctx *ctx, long m, long nc, const T *A, long lda, T *Y, long l
     // Cholesky QR + reconstruction; the column-exchange kernel runs after it
     // and factors the panel only if it was flagged
     ArenaFrame frame(ctx);
-    int *bad = arena_alloc_n<int>(ctx, 1);
+    int *bad = arena_alloc_n<int>(ctx, 2);  // state, gate
     if (!bad) return EVD_E_NOMEM;
+    unsigned *gate = reinterpret_cast<unsigned *>(bad + 1);
     EVD_TRY(panel_cholqr<T>(ctx, 1, m, nc, A, lda, 0, Y, ldy, 0, W, ldw, 0, R, ldr, Aout, ldo, 0, tau_out, bad));
     if (panel_rows(ctx, m) == 256)
       return launch_panel<32, 1, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out, 1, 0, 0, 0, 0,
-                                    bad);
-    return launch_panel<32, 2, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out, 1, 0, 0, 0, 0, bad);
+                                    bad, gate);
+    return launch_panel<32, 2, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out, 1, 0, 0, 0, 0, bad,
+                                  gate);
   }
   if (nc <= 32 && panel_rows(ctx, m) == 256)
     return launch_panel<32, 1, T>(ctx, m, nc, A, lda, Y, ldy, W, ldw, R, ldr, Aout, ldo, tau_out);
@@ -564,8 +742,9 @@ int panel_qr_batched(evd_ctx *ctx, int count, long m, long nc, float *A, long ld
     // then the fallback for the flagged ones (one launch when the groups of
     // all problems can be co-resident, else per problem)
     ArenaFrame frame(ctx);
-    int *bad = arena_alloc_n<int>(ctx, (size_t)count);
+    int *bad = arena_alloc_n<int>(ctx, (size_t)2 * count);  // states, gates
     if (!bad) return EVD_E_NOMEM;
+    unsigned *gate = reinterpret_cast<unsigned *>(bad + count);
     EVD_TRY(panel_cholqr<float>(ctx, count, m, nc, A, lda, sA, Y, ldy, sY, W, ldw, sW, nullptr, 0, A, lda, sA,
                                 nullptr, bad));
     const long G = (m + 511) / 512;
@@ -574,13 +753,14 @@ int panel_qr_batched(evd_ctx *ctx, int count, long m, long nc, float *A, long ld
       EVD_TRY(max_coresident_blocks(ctx, (const void *)panel_qr_kernel<32, 2, float>, 256, 0, &maxres));
     if (m <= 256)
       return launch_panel<32, 1, float>(ctx, m, nc, A, lda, Y, ldy, W, ldw, nullptr, 0, A, lda, nullptr, count, sA,
-                                        sY, sW, sA, bad);
+                                        sY, sW, sA, bad, gate);
     if (count == 1 || G == 1 || (G * count <= maxres && G * count <= kTagWords))
       return launch_panel<32, 2, float>(ctx, m, nc, A, lda, Y, ldy, W, ldw, nullptr, 0, A, lda, nullptr, count, sA,
-                                        sY, sW, sA, bad);
+                                        sY, sW, sA, bad, gate);
     for (int q = 0; q < count; q++) {
       const int st = launch_panel<32, 2, float>(ctx, m, nc, A + q * sA, lda, Y + q * sY, ldy, W + q * sW, ldw,
-                                                nullptr, 0, A + q * sA, lda, nullptr, 1, 0, 0, 0, 0, bad + q);
+                                                nullptr, 0, A + q * sA, lda, nullptr, 1, 0, 0, 0, 0, bad + q,
+                                                gate + q);
       if (st) return st;
     }
     return 0;
