@@ -698,17 +698,21 @@ class Server:
         self._keep[rid.value] = (A, w, Z)
         return rid.value, w, Z
 
+    def _error(self, rc: int) -> str:
+        # a positive status is a request's, a negative one the call's own argument
+        return self._lib.evd_server_last_error(self._h).decode() if rc > 0 else ""
+
     def wait(self, rid: int) -> int:
         rc = self._lib.evd_server_wait(self._h, rid)
         if rc:
-            raise EvdError("evd_server_wait", rc, "")
+            raise EvdError("evd_server_wait", rc, self._error(rc))
         self._keep.pop(rid, None)
         return rc
 
     def wait_all(self):
         rc = self._lib.evd_server_wait_all(self._h)
         if rc:
-            raise EvdError("evd_server_wait_all", rc, "")
+            raise EvdError("evd_server_wait_all", rc, self._error(rc))
         self._keep.clear()
 
     def latency_ms(self, rid: int) -> float:

@@ -90,6 +90,7 @@ SIGNATURES = {
     "evd_server_submit": (_i, [_vp, _l, _l, _l, _vp, _l, _vp, _vp, _l, C.POINTER(_l)]),
     "evd_server_wait": (_i, [_vp, _l]),
     "evd_server_wait_all": (_i, [_vp]),
+    "evd_server_last_error": (C.c_char_p, [_vp]),
     "evd_server_request_ms": (_i, [_vp, _l, C.POINTER(C.c_double)]),
     "evd_server_stats": (_i, [_vp, C.POINTER(_l), C.POINTER(C.c_double), C.POINTER(C.c_double),
                               C.POINTER(C.c_double), C.POINTER(C.c_size_t)]),

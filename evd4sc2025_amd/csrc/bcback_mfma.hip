@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void bcw_prep_kernel(int n, const float *__res
     out[(2 * f) * kFrag + lane] = hi;
     out[(2 * f + 1) * kFrag + lane] = lo;
   }
-  if (bad) atomicOr(err, (unsigned)EVD_E_RANGE);
+  if (bad) atomicOr(err, kErrRange);
 }
 
 // ------------------------------------------------------------------ main

@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256, BW == 32 ? 4 : 1) void chase_kernel(int n, int
         while (ld_dev(&com[(long)(s - 1) * kComStride]) < need) {
           __builtin_amdgcn_s_sleep(1);
           if (clock100() - t0 > kWatchdogTicks) {
-            atomicOr(err, (unsigned)EVD_E_TIMEOUT);
+            atomicOr(err, kErrTimeout);
             s_ok = 0;
             break;
           }
@@ -628,7 +628,7 @@ __global__ __launch_bounds__((D + 1) * 64, 1) void chase_group_kernel(
             if (known >= need) break;
             if (clock100() - t0 > kWatchdogTicks) {
               if (lane == 0) {
-                atomicOr(err, (unsigned)EVD_E_TIMEOUT);
+                atomicOr(err, kErrTimeout);
                 s_abort = 1;
               }
               break;

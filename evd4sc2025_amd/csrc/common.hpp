@@ -14,6 +14,7 @@
 #include <vector>
 
 #include "../../include/evd4sc.h"
+#include "errors.hpp"
 
 typedef struct _rocblas_handle *rocblas_handle;
 
@@ -106,7 +107,7 @@ namespace evd {
 
 // control block layout (words)
 enum : int {
-  kCtrlError = 0,      // device-side error word (EVD_E_*), sticky until read
+  kCtrlError = 0,      // device-side error word (kErr* bits), sticky until read
   kCtrlEpoch = 8,      // launch epoch of the panel factorisation's exchange
   kCtrlBarrier = 16,   // grid barrier: [count, generation] pairs, 64 slots
   kCtrlWordsTotal = 16 + 2 * 64,
@@ -377,7 +378,7 @@ __device__ inline bool grid_barrier(unsigned *words, unsigned nblocks, unsigned 
       while (ld_dev(&words[1]) == gen) {
         __builtin_amdgcn_s_sleep(1);
         if (clock100() - t0 > kWatchdogTicks) {
-          atomicOr(err, (unsigned)EVD_E_TIMEOUT);
+          atomicOr(err, kErrTimeout);
           s_ok = 0;
           break;
         }

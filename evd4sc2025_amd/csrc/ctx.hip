@@ -177,8 +177,7 @@ int check_device_error(evd_ctx *ctx, const char *where) {
     unsigned z = 0;
     EVD_HIP(ctx, hipMemcpyAsync(ctx->ctrl + kCtrlError, &z, sizeof(unsigned), hipMemcpyHostToDevice, ctx->stream));
     EVD_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    int code = (h & EVD_E_TIMEOUT) ? EVD_E_TIMEOUT : (h & EVD_E_NONFINITE) ? EVD_E_NONFINITE : (int)h;
-    return set_error(ctx, code, "device reported error word 0x%x in %s", h, where);
+    return set_error(ctx, device_error_code(h), "%s (device error word 0x%x) in %s", device_error_text(h), h, where);
   }
   return 0;
 }

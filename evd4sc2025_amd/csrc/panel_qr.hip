@@ -383,7 +383,7 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
       while (ld_dev(&tags[gg]) != epoch) {
         __builtin_amdgcn_s_sleep(1);
         if (clock100() - t0 > kWatchdogTicks) {
-          atomicOr(err, (unsigned)EVD_E_TIMEOUT);
+          atomicOr(err, kErrTimeout);
           s_ok = 0;
           break;
         }
@@ -475,7 +475,7 @@ __global__ __launch_bounds__(256) void panel_qr_kernel(int m, int nc, const T *_
                 __builtin_amdgcn_s_sleep(1);
                 v[u] = ld_dev(src);
                 if (clock100() - t0 > kWatchdogTicks) {
-                  atomicOr(err, (unsigned)EVD_E_TIMEOUT);
+                  atomicOr(err, kErrTimeout);
                   s_ok = 0;
                   break;
                 }

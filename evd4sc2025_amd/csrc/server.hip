@@ -37,6 +37,7 @@
 #include <deque>
 #include <map>
 #include <mutex>
+#include <string>
 #include <thread>
 #include <unordered_map>
 #include <vector>
@@ -61,6 +62,7 @@ struct Request {
 
 struct Done {
   int status;
+  std::string error;  // what the slot's context reported (status != 0)
   double latency_ms;
   clk::time_point t_done;
 };
@@ -128,6 +130,7 @@ struct evd_server {
   bool stop = false;
   bool have_first = false;
   clk::time_point t_first, t_last;
+  std::string last_error;  // of the failed request that a wait reported last
   std::vector<double> lat;
 };
 
@@ -139,13 +142,17 @@ static bool same_class(const Request &a, const Request &b) {
   return a.n == b.n && a.b == b.b && a.nb == b.nb && (a.Z != nullptr) == (b.Z != nullptr);
 }
 
-static void finish(evd_server *s, const std::vector<Request> &batch, int st) {
+static void finish(evd_server *s, const std::vector<Request> &batch, int st, const char *error) {
   const clk::time_point t1 = clk::now();
+  std::string text;
+  if (st)
+    text = "order " + std::to_string(batch[0].n) + (batch[0].Z ? ", jobz V" : ", jobz N") + ", batch of " +
+           std::to_string(batch.size()) + ": " + error;
   {
     std::lock_guard<std::mutex> lk(s->mu);
     for (const Request &r : batch) {
       const double ms = std::chrono::duration<double, std::milli>(t1 - r.t_submit).count();
-      s->done[r.id] = Done{st, ms, t1};
+      s->done[r.id] = Done{st, text, ms, t1};
       s->lat.push_back(ms);
     }
     s->t_last = t1;
@@ -178,6 +185,12 @@ static int run_batch(evd_server *s, int slot, const std::vector<Request> &batch)
     if (vec) EVD_TRY(evd::copy_f32(ctx, Z + (long)q * n * n, n, batch[q].Z, batch[q].ldz, n, n));
   }
   return evd_ctx_synchronize(ctx);
+}
+
+// status of a finished request; a failed one's text becomes the server's
+static int report(evd_server *s, long id, const Done &d) {
+  if (d.status) s->last_error = "request " + std::to_string(id) + " (" + d.error + ")";
+  return d.status;
 }
 
 // queue positions in admission order
@@ -228,6 +241,7 @@ static void worker_main(evd_server *s, int slot) {
         s->cv_work.wait(lk);
       }
     }
+    evd::set_error(ctx, 0, "%s", "");  // of this batch only
     int st = s->pool ? evd::ctx_lend_arena(ctx, s->pool + off, need) : evd_ctx_reserve(ctx, need);
     if (st == 0) {
       if (batch.size() == 1) {
@@ -243,7 +257,7 @@ static void worker_main(evd_server *s, int slot) {
       std::lock_guard<std::mutex> lk(s->mu);
       s->free.release(off, need);
     }
-    finish(s, batch, st);
+    finish(s, batch, st, evd_ctx_last_error(ctx));
   }
 }
 
@@ -365,7 +379,7 @@ int evd_server_wait(evd_server *s, long id) {
   std::unique_lock<std::mutex> lk(s->mu);
   if (id < 0 || id >= s->next_id) return -2;
   s->cv_done.wait(lk, [&] { return s->done.count(id) > 0; });
-  return s->done[id].status;
+  return report(s, id, s->done[id]);
 }
 
 int evd_server_wait_all(evd_server *s) {
@@ -373,8 +387,17 @@ int evd_server_wait_all(evd_server *s) {
   std::unique_lock<std::mutex> lk(s->mu);
   s->cv_done.wait(lk, [&] { return s->queue.empty() && s->running == 0; });
   for (auto &kv : s->done)
-    if (kv.second.status) return kv.second.status;
+    if (kv.second.status) return report(s, kv.first, kv.second);
   return 0;
+}
+
+const char *evd_server_last_error(evd_server *s) {
+  if (!s) return "null server";
+  std::lock_guard<std::mutex> lk(s->mu);
+  // a copy per calling thread: a later wait of another thread replaces the text
+  static thread_local std::string text;
+  text = s->last_error;
+  return text.c_str();
 }
 
 int evd_server_request_ms(evd_server *s, long id, double *latency_ms) {

@@ -648,7 +648,7 @@ __global__ void dc_secular_kernel(const MergeDesc *__restrict__ md, const MergeO
     double tau;
     const bool conv = secular_root<64>(d, z, K, i, o.rho2, o.zsum, lane, org, tau);
     if (lane == 0) {
-      if (!conv) atomicOr(err, (unsigned)EVD_E_NOCONVERGE);
+      if (!conv) atomicOr(err, kErrNoconverge);
       sc.orig[st + i] = org;
       sc.tau[st + i] = tau;
       sc.lam[st + i] = d[org] + tau;
@@ -1165,7 +1165,7 @@ __global__ __launch_bounds__(256) void dc_leaf_kernel(const LeafDesc *__restrict
         double t;
         const bool conv = secular_root<16>(nd_d + off, nd_z + off, K, i, o.rho2, o.zsum, l, og, t);
         if (l == 0) {
-          if (!conv) atomicOr(err, (unsigned)EVD_E_NOCONVERGE);
+          if (!conv) atomicOr(err, kErrNoconverge);
           org[g] = og;
           tau[g] = t;
           lam[g] = nd_d[off + og] + t;

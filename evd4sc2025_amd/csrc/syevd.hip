@@ -86,7 +86,7 @@ struct ScreenRows {
 
 // Symmetric fill of the upper triangle from the lower one + non-finite
 // screen + max |a_ij| (as the bits of a non-negative float, which order like
-// unsigned integers) into amax[q].  A non-finite entry raises EVD_E_NONFINITE
+// unsigned integers) into amax[q].  A non-finite entry raises kErrNonfinite
 // in the error word (read when the call ends) and is replaced by 0, so the
 // rest of the solve runs on finite data without a host round trip after the
 // screen.
@@ -117,7 +117,7 @@ __global__ __launch_bounds__(256) void symmetrize_check_kernel(int n, float *__r
   for (int k = 0; k < 16; k++) {
     const int c = c0 + w + 4 * k;
     if (!isfinite(v[k])) {
-      atomicOr(err, (unsigned)EVD_E_NONFINITE);
+      atomicOr(err, kErrNonfinite);
       v[k] = 0.f;
       A[r + c * lda] = 0.f;
     }

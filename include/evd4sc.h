@@ -393,6 +393,10 @@ int evd_server_submit(evd_server *srv, long n, long b, long nb, float *A, long l
                       long *id);
 int evd_server_wait(evd_server *srv, long id); /* status of the request */
 int evd_server_wait_all(evd_server *srv);      /* first nonzero status, else 0 */
+/* What the failed request that a wait reported last ran into: its id, order and
+ * batch, and the message of its slot's context.  Valid until this thread's next
+ * call. */
+const char *evd_server_last_error(evd_server *srv);
 int evd_server_request_ms(evd_server *srv, long id, double *latency_ms);
 /* completed requests, solves/s from first submission to last completion,
  * p50 / p99 latency (submission to completion), bytes held by slot arenas */
