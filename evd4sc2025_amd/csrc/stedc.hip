@@ -248,7 +248,10 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
     __syncthreads();
   }
   double *ds = sc.ds + st, *zs = sc.zs + st;
-  const int *cs = sc.cs + st;
+  // sorted -> local column; a NaN among d leaves places of the order unwritten, so
+  // what is read there is kept within the merge
+  const int *order = sc.cs + st;
+  auto cs = [&](int i) { return (int)min((unsigned)order[i], (unsigned)(N - 1)); };
   int *types = sc.types + st;
   double *nd_d = sc.nd_d + st, *nd_z = sc.nd_z + st;
   int *nd_col = sc.nd_col + st, *qpos = sc.qpos + st;
@@ -283,7 +286,7 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
   for (int i = i0; i < i1; i++) {
     if (all_defl || rho * fabs(zs[i]) <= tol) {
       df_d[zoff] = ds[i];
-      df_col[zoff] = cs[i];
+      df_col[zoff] = cs(i);
       zoff++;
     } else {
       cand[coff++] = i;
@@ -319,14 +322,14 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
       if (lane < first) {
         nd_d[K + lane] = ds[prv];
         nd_z[K + lane] = zs[prv];
-        nd_col[K + lane] = cs[prv];
+        nd_col[K + lane] = cs(prv);
       }
       K += first;
       if (first < nvalid) {
         if (lane == first) {
           zs[j] = tau;
           zs[prv] = 0.0;
-          const int cp = cs[prv], cn = cs[j];
+          const int cp = cs(prv), cn = cs(j);
           if (types[cp] != types[cn]) types[cn] = 2;
           types[cp] = 4;
           rot_p[nrot] = cp;
@@ -353,7 +356,7 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
       if (lane == 0) {
         nd_d[K] = ds[pj];
         nd_z[K] = zs[pj];
-        nd_col[K] = cs[pj];
+        nd_col[K] = cs(pj);
       }
       K++;
     }
@@ -407,7 +410,7 @@ __global__ __launch_bounds__(256) void dc_deflate_kernel(const MergeDesc *__rest
     __syncthreads();
     for (int e = tid; e < nd; e += 256) {
       df_d[e] = tmp_d[e];
-      df_col[e] = tmp_c[e];
+      df_col[e] = (int)min((unsigned)tmp_c[e], (unsigned)(N - 1));
     }
   }
 
