@@ -78,23 +78,31 @@ __device__ __attribute__((always_inline)) inline double half_swap(double v) {
   return __builtin_bit_cast(double, ((unsigned long long)phi << 32) | plo);
 }
 
-// v of lane ^ 16 (v_permlane16_swap exchanges odd rows of its destination with
-// even rows of its source)
-__device__ __attribute__((always_inline)) inline double row_swap(double v) {
+// v + v of lane ^ 16 (v_permlane16_swap exchanges odd rows of its destination with
+// even rows of its source: with both v, one result holds the even row of each pair
+// in both of its rows and the other the odd row)
+__device__ __attribute__((always_inline)) inline double row_pair_sum(double v) {
   const unsigned long long x = __builtin_bit_cast(unsigned long long, v);
-  const unsigned lo = (unsigned)x, hi = (unsigned)(x >> 32);
-  const auto rl = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
-  const auto rh = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
-  const unsigned plo = rl[0] ^ rl[1] ^ lo, phi = rh[0] ^ rh[1] ^ hi;
-  return __builtin_bit_cast(double, ((unsigned long long)phi << 32) | plo);
+  const auto rl = __builtin_amdgcn_permlane16_swap((unsigned)x, (unsigned)x, false, false);
+  const auto rh = __builtin_amdgcn_permlane16_swap((unsigned)(x >> 32), (unsigned)(x >> 32), false, false);
+  return __builtin_bit_cast(double, ((unsigned long long)rh[0] << 32) | rl[0]) +
+         __builtin_bit_cast(double, ((unsigned long long)rh[1] << 32) | rl[1]);
 }
 
-// wave_sum's butterfly (lane ^ 32, 16, 8, 4, 2, 1), bit for bit, by swaps of
-// half waves and rows and by DPP
-__device__ __attribute__((always_inline)) inline double wave_butterfly(double v) {
-  v += half_swap(v);
-  v += row_swap(v);
-  return row_sum16(v);
+// sum of the products a b over BW lanes, in every lane, with the bits of wave_sum
+// over the wave (lane ^ 32, 16, 8, 4, 2, 1) where lanes from BW on add zeros.  BW =
+// 32: both halves of the wave hold the same a and b, so the step over lane ^ 32,
+// which adds a zero, is left out.
+template <int BW>
+__device__ __attribute__((always_inline)) inline double wave_dot(double a, double b) {
+  double v;
+  if (BW == 32) {
+    v = __builtin_fma(a, b, 0.0);  // rounded by itself
+  } else {
+    v = a * b;
+    v += half_swap(v);
+  }
+  return row_sum16(row_pair_sum(v));
 }
 
 // sum over aligned groups of W lanes (4 or 8), returned in every lane of the
@@ -114,23 +122,31 @@ __device__ __attribute__((always_inline)) inline double group_sum(double v) {
 // sqrt(|x0/||x|| + sign(x0)|), ||u||^2 = 2, H x = beta e1.  Wave 0 only.  It
 // sits in the chain of the steps: sums by swaps and DPP instead of shuffles
 // through LDS, and short chains for two roots and two reciprocals (with the same
-// sums in the step, n = 6000, b = 32: 49.3 -> 45.8 ms).  All have the bits of the
+// sums in the step, n = 6000, b = 32: 49.3 -> 44.8 ms).  All have the bits of the
 // plain forms: a last bit of T decides which entries the tridiagonal solver
 // deflates, and so now and then the sign of a vector.
 template <int BW>
 __device__ inline void chase_reflector(const double *Bc, int lenx, int lane, double *u, double *s_beta, float *U,
                                        long urow, long ucol) {
   constexpr int LD = BW + 1;
-  const double x = (lane < lenx) ? Bc[lane * LD] : 0.0;
-  const double nn = wave_butterfly(x * x);
+  const int row = lane % BW;
+  const double x = (row < lenx) ? Bc[row * LD] : 0.0;
+  const double nn = wave_dot<BW>(x, x);
   const double x0 = Bc[0];
-  double uu = 0.0, nrm = 0.0;
-  if (nn > 0.0) {
-    double inv, scl, root;
-    sqrt_and_recip(nn, nrm, inv);
-    const double u0 = x0 * inv + (x0 >= 0.0 ? 1.0 : -1.0);
-    sqrt_and_recip(fabs(u0), root, scl);
-    uu = (lane == 0 ? u0 : x * inv) * scl;
+  double nrm, inv, root, scl;
+  sqrt_and_recip(nn, nrm, inv);
+  double u0 = x0 * inv + (x0 >= 0.0 ? 1.0 : -1.0);
+  sqrt_and_recip(fabs(u0), root, scl);  // 1 <= |u0| <= 2
+  double uu = (row == 0 ? u0 : x * inv) * scl;
+  if (!(nn >= 0x1p-700 && nn <= 0x1p700)) {  // a zero column, or norms out of the short chain's range
+    uu = nrm = 0.0;
+    if (nn > 0.0) {
+      nrm = sqrt(nn);
+      inv = 1.0 / nrm;
+      u0 = x0 * inv + (x0 >= 0.0 ? 1.0 : -1.0);
+      scl = 1.0 / sqrt(fabs(u0));
+      uu = (row == 0 ? u0 : x * inv) * scl;
+    }
   }
   if (lane < BW) u[lane] = (lane < lenx) ? uu : 0.0;
   if (lane < lenx) U[(urow + lane) + ucol] = (float)uu;
@@ -258,7 +274,7 @@ __global__ __launch_bounds__(256, BW == 32 ? 4 : 1) void chase_kernel(int n, int
       }
       __syncthreads();
       // ---- S <- H S H (rank-2 with w = y - (u^T y / 2) u), N <- N H
-      const double psi = wave_butterfly((lane < BW) ? u[lane] * yv[lane] : 0.0);
+      const double psi = wave_dot<BW>(u[lane % BW], yv[lane % BW]);
       const double ui = u[ri], wi = yv[ri] - 0.5 * psi * ui, qi = qv[ri];
 #pragma unroll
       for (int r = 0; r < EPT; r++) {

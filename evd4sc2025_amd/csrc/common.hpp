@@ -293,18 +293,13 @@ __device__ __attribute__((always_inline)) inline double row_max16(double v) {
   return v;
 }
 
-// root = sqrt(x) and inv = 1 / root for x > 0, both as the IEEE operations round
-// them: where no step can leave the normal range, Goldschmidt's iteration from the
-// hardware estimate, two corrections of the root by its residual, and two of
-// the reciprocal (Markstein 1990: a correction by fma of a value within an ulp is
-// the rounded reciprocal, but for a significand of all ones).  One short chain
+// root = sqrt(x) and inv = 1 / root as the IEEE operations round them, for x where
+// no step leaves the normal range (2^-700 <= x <= 2^700): Goldschmidt's iteration
+// from the hardware estimate, two corrections of the root by its residual, and two
+// of the reciprocal (Markstein 1990: a correction by fma of a value within an ulp
+// is the rounded reciprocal, but for a significand of all ones).  One short chain
 // instead of a square root and a division.
 __device__ __attribute__((always_inline)) inline void sqrt_and_recip(double x, double &root, double &inv) {
-  if (x < 0x1p-700 || x > 0x1p700) {
-    root = sqrt(x);
-    inv = 1.0 / root;
-    return;
-  }
   const double y = __builtin_amdgcn_rsq(x);
   double g = x * y, h = 0.5 * y;
   const double r = __builtin_fma(-h, g, 0.5);
