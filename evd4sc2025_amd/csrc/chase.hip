@@ -14,9 +14,10 @@
 // order, so a sweep's predecessor is always owned by a running workgroup and
 // no co-residency (cooperative launch) is needed.  The band lives in HBM and
 // every access of the chase is device-coherent (sc1 loads and stores, which
-// bypass the non-coherent per-XCD caches; on this chip the L1-bypassing sc0
-// loads do not observe other CUs' stores, so an XCD-local exchange is not
-// available), and a vmcnt(0) wait orders a step's stores before its flag.
+// do not depend on which XCD a workgroup runs on; sc0 loads, which reach other
+// CUs' stores on some chips, do not observe them here, and plain stores with sc1
+// loads only within an XCD), and a vmcnt(0) wait orders a step's stores before
+// its flag.
 // Per step the S and N windows are held in registers (a row per 256/BW
 // lanes), B1 and the next B1 in LDS; H B1 is applied by one wave while the
 // others wait for their window loads.  Step (s, p) needs step (s-1, p-1+2b)

@@ -38,8 +38,8 @@ struct Tuning {
 };
 
 // Merge plan of the tridiagonal divide and conquer for one order n (host
-// level table + device copy of the merge descriptors, split flags and tile
-// offsets), kept per context.
+// level table + device copy of the merge descriptors, tile offsets and
+// leaves), kept per context.
 struct DcPlan {
   int nmerge = 0, H = 0, nleaf = 0;
   std::vector<int> level_off;    // merges of height h: [level_off[h], level_off[h + 1])

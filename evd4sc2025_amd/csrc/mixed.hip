@@ -33,8 +33,8 @@ long bucket_order(long n) {
 // norm[q] = max(norm[q], ||A_q||_inf) of the symmetric matrices held in the
 // lower triangles: row i sums |A[i, 0:i]| + |A[i:n, i]|.  A workgroup takes 64
 // rows of one problem (grid (ceil(N / 64), count)): lanes along the rows left of
-// the diagonal block, a wave per column below.  The matrix is read once, at
-// unit stride in both parts; one workgroup a matrix with a thread per row
+// the diagonal block, a wave per column below.  The lower triangle is read
+// twice, at unit stride both times; one workgroup a matrix with a thread per row
 // (strided in the second part) took 909 us a group over the 17 groups of 40
 // matrices of order 64 to 2048, this 76 us.
 __global__ __launch_bounds__(256) void inf_norm_kernel(const long *__restrict__ n_of, float *const *__restrict__ A_of,

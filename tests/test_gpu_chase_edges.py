@@ -1,5 +1,5 @@
-"""The bulge chase at the edges of its message layout: bandwidths that do not
-fill a block or a plane of 8 columns, orders around multiples of the bandwidth
+"""The bulge chase at the edges of its windows: bandwidths that do not fill a
+block or a lane group of 8, orders around multiples of the bandwidth
 (a last block of one row, of none, sweeps of a single step), bands of width 1,
 leading dimensions above 2 b, rows past the matrix that hold anything."""
 import numpy as np
@@ -45,8 +45,7 @@ def test_chase_edges_match_oracle(ctx, b):
 
 
 def test_band_that_holds_the_empty_pattern_does_not_stall(ctx):
-    """A signalling NaN with the bits of an empty message element is an
-    ordinary NaN to the chase."""
+    """A NaN of any bits in the band goes through the chase, which ends."""
     import evd4sc2025_amd as E
 
     n, b = 100, 32

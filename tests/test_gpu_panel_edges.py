@@ -1,8 +1,7 @@
 """Cholesky QR panels at the edges of their tiles: rows around the 64 of an
 output workgroup, the 256 of a Gram workgroup and the 2048 of a reduction
 group, fewer columns than the 32 of a tile, and rank-deficient panels whose
-fallback runs in one workgroup, in several on a regular launch, and above the
-limit of regular launches."""
+fallback runs in one workgroup and in up to 34 that come together."""
 import numpy as np
 import pytest
 
