@@ -117,6 +117,9 @@ struct evd_server {
   char *pool = nullptr;
   FreeList free;
   std::vector<evd_ctx *> ctx;
+  // answers size queries of submit: the slots' contexts change their knobs during a
+  // call, from the tuning cache's entry of its class
+  evd_ctx sizes;
   bool batching = true;
   int precision = EVD_PREC_FP32;  // GEMM precision of every slot (evd_ctx_set_precision)
   int policy = 0;                 // 0: largest order first, 1: FIFO
@@ -314,7 +317,7 @@ int evd_server_set_precision(evd_server *s, int precision) {
   std::lock_guard<std::mutex> lk(s->mu);
   if (s->running != 0 || !s->queue.empty()) return EVD_E_UNSUPPORTED;  // only between workloads
   for (evd_ctx *c : s->ctx) EVD_TRY(evd_ctx_set_precision(c, precision));
-  s->precision = precision;
+  s->precision = s->sizes.precision = precision;
   return 0;
 }
 
@@ -357,7 +360,7 @@ int evd_server_submit(evd_server *s, long n, long b, long nb, float *A, long lda
   size_t ws;
   {
     std::lock_guard<std::mutex> lk(s->mu);
-    ws = evd::syevd_call_workspace(s->ctx[0], n, b, nb, Z ? 'V' : 'N') + ((size_t)1 << 20);
+    ws = evd::syevd_call_workspace(&s->sizes, n, b, nb, Z ? 'V' : 'N') + ((size_t)1 << 20);
   }
   if (s->pool && ws > s->budget) return EVD_E_NOMEM;
   {

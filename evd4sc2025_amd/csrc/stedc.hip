@@ -72,7 +72,7 @@ struct DCScratch {
   int *orig;
   double *tau, *lam, *zhat;
   int *colmap, *dmap;
-  double *Qc, *Uc;  // n x n, ld n
+  double *Qc = nullptr, *Uc = nullptr;  // n x n, ld n (with vectors)
   // Same-size batches run as one concatenated index space: merge starts (and
   // every vector above) are global, problem q = MergeDesc::pad owns indices
   // [q n, q n + n).  Its matrices sit at their own offsets; adding
